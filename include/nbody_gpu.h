@@ -73,7 +73,9 @@ typedef struct nb_params {
   int32_t jsplit;         /* FP32 force kernel: source-range slices; 0 = tuned */
   int32_t block;          /* FP32 force kernel: threads per workgroup (64..256); 0 = tuned */
   int32_t variant;        /* FP32 force kernel: 0 = tuned, 1 = scalar-cache j stream,
-                             2 = LDS-staged j tiles */
+                             2 = LDS-staged j tiles, 3 = each unordered pair once (eps > 0, no
+                             overlap cutoff; tile_j 64, block 256).  With none of the five fields
+                             pinned, 3 where it applies */
   int32_t events;         /* 1 = the reference's subsume and fragmentation events on the device
                              (Compute's dispatch, body.go:172-183; ResolveSubsume :228-244;
                              doFragment / fragment, fragcalc.go:54-117); 0 = elastic collisions

@@ -69,7 +69,7 @@ static void free_all(Ctx *c) {
   void *ptrs[] = {c->x,    c->y,      c->z,     c->vx,   c->vy,        c->vz,   c->m,
                   c->r,    c->rest,   c->frag,  c->beh,  c->flags,     c->collided,
                   c->js,   c->rmax_tile, c->acc, c->fcnt, c->flist, c->recs, c->pairs, c->ctr,
-                  c->diag, c->pairs_tmp, c->pairs_sw, c->res_words};
+                  c->diag, c->pairs_tmp, c->pairs_sw, c->res_words, c->layer};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   c->x = c->y = c->z = c->vx = c->vy = c->vz = c->m = c->r = c->rest = c->frag = nullptr;
@@ -84,6 +84,9 @@ static void free_all(Ctx *c) {
   c->res_words = nullptr;
   c->ctr = nullptr;
   c->diag = nullptr;
+  c->layer = nullptr;
+  c->acc_split = c->rec_split = 0;
+  c->layer_words = 0;
 }
 
 static bool detect_needed(const Ctx *c) {
@@ -93,10 +96,11 @@ static bool drop_needed(const Ctx *c) { return c->p.overlap_cutoff || c->p.eps =
 
 static int tiles_of(const Ctx *c) { return (int)(c->npad / c->shape.tile_j); }
 
-// Default launch shape: the one nb_autotune picks at 65,536 and 262,144 bodies (LDS-staged
-// sources, one target per lane, 512-source tiles), with enough source slices for about 16
-// workgroups per CU on 256 CUs.  npad is a multiple of 1024, so every field divides it.
-static ForceShape default_shape(int64_t npad) {
+// Launch shape with one evaluation per ordered pair: the one nb_autotune picks among those at
+// 65,536 and 262,144 bodies (LDS-staged sources, one target per lane, 512-source tiles), with
+// enough source slices for about 16 workgroups per CU on 256 CUs.  npad is a multiple of 1024, so
+// every field divides it.
+ForceShape default_shape(int64_t npad) {
   ForceShape s;
   s.ipl = 1;
   s.block = 256;
@@ -109,28 +113,75 @@ static ForceShape default_shape(int64_t npad) {
   return s;
 }
 
+// Each pair once (variant 3).
+static bool sym_possible(const Ctx *c) {
+  return c->p.precision == NB_PREC_FP32 && c->p.eps > 0.0 && !c->p.overlap_cutoff;
+}
+static int64_t sym_blocks(const ForceShape &s, int64_t n) {
+  const int64_t T = s.ipl * s.block / 64;
+  return ((n + 63) / 64 + T - 1) / T;
+}
+// Targets per lane: four keep the most arithmetic per LDS read and per moved sum, but a block is
+// then 1,024 bodies, too coarse for small n.  Measured best of 1 / 2 / 4 (ms): 0.046 / 0.049 /
+// 0.054 at n = 10,000, 0.084 / 0.083 / 0.082 at 16,384, 0.175 / 0.167 / 0.172 at 25,000,
+// 0.254 / 0.244 / 0.239 at 32,768, 0.934 / 0.863 / 0.826 at 65,536.
+// Slices: about 8,192 workgroups, at least 12 and at most 48 slices a row (small n: 16, where each
+// more costs a longer fold): with 12 / 24 / 48 slices at 262,144 12.6 / 12.25 / 12.2 ms.
+static ForceShape sym_shape(int64_t n) {
+  ForceShape s;
+  s.variant = 3;
+  s.tile_j = 64;
+  s.block = 256;
+  s.ipl = n < 12288 ? 1 : n < 28672 ? 2 : 4;
+  const int64_t nb = std::max<int64_t>(sym_blocks(s, n), 1);
+  s.jsplit = s.ipl == 1 ? 16 : s.ipl == 2 ? 24
+                             : (int)std::min<int64_t>(48, std::max<int64_t>(12, 8192 / nb));
+  return s;
+}
+
 static bool shape_valid(const ForceShape &s, int64_t npad) {
   if (s.ipl != 1 && s.ipl != 2 && s.ipl != 4) return false;
+  if (s.jsplit < 1 || s.jsplit > kMaxSplit) return false;
+  if (s.variant == 3)
+    return s.tile_j == 64 && s.block == 256;
   if (s.block < 64 || s.block > 256 || (s.block & 63)) return false;
   if (s.tile_j < 64 || s.tile_j > 1024 || (s.tile_j & 63) || npad % s.tile_j) return false;
   if (npad % (s.block * s.ipl)) return false;
-  if (s.jsplit < 1 || s.jsplit > kMaxSplit || s.jsplit > npad / s.tile_j) return false;
+  if (s.jsplit > npad / s.tile_j) return false;
   if (s.variant != 1 && s.variant != 2) return false;
   return true;
 }
 
+int ensure_acc(Ctx *c, int split) {
+  if (split <= c->acc_split && c->acc) return NB_OK;
+  NB_HIP(c, dalloc(&c->acc, (size_t)split * 3 * c->cap));
+  c->acc_split = split;
+  return NB_OK;
+}
+
 // (Re)size the per-slice and per-tile buffers for the current shape.
 static int prepare_shape(Ctx *c) {
-  if (!shape_valid(c->shape, c->npad))
+  if (!shape_valid(c->shape, c->npad) || (c->shape.variant == 3 && !sym_possible(c)))
     return fail(c, NB_E_INVALID, "invalid FP32 force kernel shape for this body count");
-  const int split = c->p.precision == NB_PREC_FP64 ? 1 : c->shape.jsplit;
-  if (split > c->acc_split || !c->acc) {
-    const int alloc_split = std::max(split, 1);
-    NB_HIP(c, dalloc(&c->acc, (size_t)alloc_split * 3 * c->cap));
-    NB_HIP(c, dalloc(&c->fcnt, (size_t)alloc_split * c->cap));
-    NB_HIP(c, dalloc(&c->flist, (size_t)alloc_split * c->cap * kFlagSlots));
-    NB_HIP(c, dalloc(&c->recs, (size_t)alloc_split * c->cap));
-    c->acc_split = alloc_split;
+  const int split = c->p.precision == NB_PREC_FP64 ? 1
+                    : c->shape.variant == 3        ? c->shape.jsplit + 1
+                                                   : c->shape.jsplit;
+  int rc = ensure_acc(c, split);
+  if (rc) return rc;
+  if (c->shape.variant == 3) {
+    const int64_t want = std::min<int64_t>(sym_blocks(c->shape, c->n) / 2 * 3 * c->npad,
+                                           std::max<int64_t>(kLayerWords, 3 * c->npad));
+    if (want > c->layer_words) {
+      c->layer_words = 0;
+      NB_HIP(c, dalloc(&c->layer, (size_t)want));
+      c->layer_words = want;
+    }
+  } else if (split > c->rec_split) {
+    c->rec_split = 0;
+    NB_HIP(c, dalloc(&c->fcnt, (size_t)split * c->cap));
+    NB_HIP(c, dalloc(&c->flist, (size_t)split * c->cap * kFlagSlots));
+    NB_HIP(c, dalloc(&c->recs, (size_t)split * c->cap));
+    c->rec_split = split;
   }
   const int tiles = tiles_of(c);
   if (c->rmax_tile_j != c->shape.tile_j) {
@@ -146,9 +197,11 @@ static int prepare_shape(Ctx *c) {
 // pinned fields.
 static void choose_shape(Ctx *c) {
   if (c->shape_tuned && shape_valid(c->shape, c->npad)) return;
-  c->shape = default_shape(c->npad);
-  c->shape_tuned = false;
   const nb_params &p = c->p;
+  const bool pinned = p.ipl || p.tile_j || p.jsplit || p.block || p.variant;
+  c->shape = (!pinned && sym_possible(c)) || p.variant == 3 ? sym_shape(c->n)
+                                                           : default_shape(c->npad);
+  c->shape_tuned = false;
   if (p.ipl) c->shape.ipl = p.ipl;
   if (p.tile_j) c->shape.tile_j = p.tile_j;
   if (p.jsplit) c->shape.jsplit = p.jsplit;
@@ -173,7 +226,7 @@ static int size_pairs(Ctx *c, int64_t n) {
   return NB_OK;
 }
 
-ForceArgs make_force_args(Ctx *c) {
+ForceArgs make_force_args(Ctx *c, const ForceShape &s) {
   ForceArgs a;
   a.js = c->js;
   a.rmax_tile = c->rmax_tile;
@@ -183,18 +236,44 @@ ForceArgs make_force_args(Ctx *c) {
   a.flist = c->flist;
   a.npad = (int)c->npad;
   a.n = (int)c->n;
-  a.tile_j = c->shape.tile_j;
-  a.tiles = tiles_of(c);
-  a.tiles_per_slice = (a.tiles + c->shape.jsplit - 1) / c->shape.jsplit;
+  a.tile_j = s.tile_j;
+  a.tiles = (int)(c->npad / s.tile_j);
+  a.tiles_per_slice = (a.tiles + s.jsplit - 1) / s.jsplit;
   const double e2 = c->p.eps * c->p.eps;
   a.eps2 = (float)e2;
   a.detect = detect_needed(c) ? 1 : 0;
   a.drop_flagged = drop_needed(c) ? 1 : 0;
   a.recs = c->recs;
-  a.rec_cap = (int64_t)c->acc_split * c->cap;
+  a.rec_cap = (int64_t)c->rec_split * c->cap;
   a.ctr = c->ctr;
   a.run_flag = nullptr;
   return a;
+}
+
+hipError_t launch_plain(Ctx *c, bool detect, const uint32_t *run_flag) {
+  if (c->shape.variant == 3) {
+    SymArgs a{};
+    a.js = c->js;
+    a.rmax_tile = c->rmax_tile;
+    a.x = c->x; a.y = c->y; a.z = c->z; a.r = c->r;
+    a.beh = c->beh;
+    a.flags = c->flags;
+    a.acc = c->acc + 3 * c->npad;  // slice 0 receives the result
+    a.layer = c->layer;
+    a.pairs = c->pairs;
+    a.ctr = c->ctr;
+    a.run_flag = run_flag;
+    a.pair_cap = c->pair_cap;
+    a.npad = (int)c->npad;
+    a.n = (int)c->n;
+    a.eps2 = (float)(c->p.eps * c->p.eps);
+    a.events = c->p.events;
+    return launch_force_sym(c->shape, a, c->acc, c->layer_words, detect, c->stream);
+  }
+  ForceArgs a = make_force_args(c, c->shape);
+  a.run_flag = run_flag;
+  if (!detect) a.detect = a.drop_flagged = 0;
+  return launch_force_f32(c->shape, a, c->stream);
 }
 
 // Force phase of one cycle (force + detection + sorted pair list).
@@ -222,11 +301,11 @@ static int force_phase(Ctx *c, bool timed, int ev_slot) {
     NB_HIP(c, launch_force_f64(a, c->stream));
     if (timed) NB_HIP(c, hipEventRecord(c->ev[2 * ev_slot + 1], c->stream));
   } else {
-    ForceArgs a = make_force_args(c);
     if (timed) NB_HIP(c, hipEventRecord(c->ev[2 * ev_slot], c->stream));
-    NB_HIP(c, launch_force_f32(c->shape, a, c->stream));
+    NB_HIP(c, launch_plain(c, detect_needed(c), nullptr));
     if (timed) NB_HIP(c, hipEventRecord(c->ev[2 * ev_slot + 1], c->stream));
-    if (a.detect) {
+    if (detect_needed(c) && c->shape.variant != 3) {
+      const ForceArgs a = make_force_args(c, c->shape);
       FixupArgs f;
       f.x = c->x; f.y = c->y; f.z = c->z; f.m = c->m; f.r = c->r;
       f.beh = c->beh;
@@ -263,7 +342,7 @@ int sort_pairs(Ctx *c) {
 }
 
 static int split_now(const Ctx *c) {
-  return (c->p.precision == NB_PREC_FP64 || c->sur_on) ? 1 : c->shape.jsplit;
+  return (c->p.precision == NB_PREC_FP64 || c->sur_on) ? 1 : plain_split(c);
 }
 
 static int64_t count_active(int64_t n, const uint8_t *flags) {
@@ -385,7 +464,6 @@ int nb_load(nb_ctx *c, int64_t n, const double *x, const double *y, const double
   if (npad > c->cap) {
     free_all(c);
     c->cap = npad;
-    c->acc_split = 0;
     c->rmax_tile_j = 0;
     c->pair_cap_pow2 = 0;
     NB_HIP(c, dalloc(&c->x, c->cap));
@@ -793,6 +871,18 @@ int nb_autotune(nb_ctx *c, int32_t reps, int32_t *cfg) {
             if (shape_valid(s, npad)) cand.push_back(s);
           }
         }
+  if (sym_possible(c))
+    for (int ipl : {1, 2, 4})
+      for (int split : {12, 16, 24, 32, 48}) {
+        ForceShape s = sym_shape(c->n);
+        s.ipl = ipl;
+        s.jsplit = split;
+        cand.push_back(s);
+      }
+  // the timed launches may list pairs: the context's counters are put back afterwards
+  DevCounters saved;
+  NB_HIP(c, hipMemcpyAsync(&saved, c->ctr, sizeof saved, hipMemcpyDeviceToHost, c->stream));
+  NB_HIP(c, hipStreamSynchronize(c->stream));
   hipEvent_t e0, e1;
   NB_HIP(c, hipEventCreate(&e0));
   NB_HIP(c, hipEventCreate(&e1));
@@ -809,10 +899,9 @@ int nb_autotune(nb_ctx *c, int32_t reps, int32_t *cfg) {
     if (dup) continue;
     c->shape = s;
     if (prepare_shape(c)) continue;
-    ForceArgs a = make_force_args(c);
-    if (launch_force_f32(s, a, c->stream) != hipSuccess) continue;  // warm-up
+    if (launch_plain(c, detect_needed(c), nullptr) != hipSuccess) continue;  // warm-up
     NB_HIP(c, hipEventRecord(e0, c->stream));
-    for (int k = 0; k < reps; k++) (void)launch_force_f32(s, a, c->stream);
+    for (int k = 0; k < reps; k++) (void)launch_plain(c, detect_needed(c), nullptr);
     NB_HIP(c, hipEventRecord(e1, c->stream));
     NB_HIP(c, hipEventSynchronize(e1));
     float ms = 0;
@@ -824,6 +913,8 @@ int nb_autotune(nb_ctx *c, int32_t reps, int32_t *cfg) {
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
+  NB_HIP(c, hipMemcpyAsync(c->ctr, &saved, sizeof saved, hipMemcpyHostToDevice, c->stream));
+  NB_HIP(c, hipStreamSynchronize(c->stream));
   c->shape = best_s;
   c->shape_tuned = true;
   int rc = prepare_shape(c);
@@ -1018,7 +1109,7 @@ int nb_cycle(nb_ctx *c, double R, int64_t *n_out) {
     NB_HIP(c, dalloc(&c->js, c->cap));
     c->diag_len = c->cap * 8 + 64;
     NB_HIP(c, dalloc(&c->diag, c->diag_len));
-    c->acc_split = 0;   // per-slice buffers are re-sized by prepare_shape
+    c->acc_split = c->rec_split = 0;   // per-slice buffers are re-sized by prepare_shape
     c->rmax_tile_j = 0;
   }
   {

@@ -16,6 +16,7 @@ constexpr int kPad = 1024;           // body arrays are padded to a multiple of 
 constexpr int kFlagSlots = 4;        // flagged tiles remembered per (slice, target)
 constexpr int kMaxSplit = 64;        // max source-range slices
 constexpr int kSortLdsKeys = 8192;   // pair keys sorted in LDS by one workgroup
+constexpr int64_t kLayerWords = (int64_t)1 << 28;  // floats of variant 3's workspace (1 GiB)
 constexpr float kSentinel = 1.0e18f; // position of padding / inactive sources in the FP32 stream
 
 // Device counters, one struct per context (zeroed by a fill kernel, never by hipMemset, so the
@@ -83,7 +84,7 @@ struct ForceShape {
   int tile_j = 256; // sources per Kahan tile
   int jsplit = 1;   // source-range slices (grid.y)
   int block = 256;  // threads per workgroup
-  int variant = 1;  // 1 = scalar-cache j stream, 2 = LDS-staged tiles
+  int variant = 1;  // 1 = scalar-cache j stream, 2 = LDS-staged tiles, 3 = each pair once
 };
 
 struct Ctx {
@@ -113,6 +114,10 @@ struct Ctx {
   // per-slice accelerations (FP32 path) or force (FP64 path): [split][3][npad] doubles
   double *acc = nullptr;
   int acc_split = 0;
+  int rec_split = 0;  // slices the flagged-tile arrays hold
+  // variant 3: the tiles' sums per block distance
+  float *layer = nullptr;
+  int64_t layer_words = 0;
   // flagged tiles: counts [split][npad], lists [split][npad][kFlagSlots], records [split*npad]
   int32_t *fcnt = nullptr, *flist = nullptr;
   int2 *recs = nullptr;
@@ -222,13 +227,43 @@ struct ForceArgs {
   const uint32_t *run_flag;  // if set, the launch does nothing unless *run_flag != 0
 };
 hipError_t launch_force_f32(const ForceShape &s, const ForceArgs &a, hipStream_t st);
-ForceArgs make_force_args(Ctx *c);
+ForceArgs make_force_args(Ctx *c, const ForceShape &s);
+// The FP32 direct sum in the context's shape into acc; run_flag: nothing unless it is nonzero.
+// detect: flag candidates (variants 1 and 2) or list the pairs (variant 3).
+hipError_t launch_plain(Ctx *c, bool detect, const uint32_t *run_flag);
+// Slices of acc the direct sum leaves (variant 3 folds its own).
+inline int plain_split(const Ctx *c) { return c->shape.variant == 3 ? 1 : c->shape.jsplit; }
+ForceShape default_shape(int64_t npad);  // one evaluation per ordered pair
+int ensure_acc(Ctx *c, int split);       // acc with room for split slices
 int fail_msg(Ctx *c, int code, const char *msg);
 void set_global_error(const char *msg);  // the message nb_last_error(NULL) returns
 void sur_free(Sur *s);
 int sur_force_phase(Ctx *c, bool timed, int ev_slot);
 void bh_free(Bh *b);
 int bh_force_phase(Ctx *c, bool timed, int ev_slot);
+
+// Each unordered pair once (nb_sym.hip): eps > 0, no overlap gate.
+struct SymArgs {
+  const float4 *js;
+  const float *rmax_tile;  // per 64-body tile (detection)
+  const double *x, *y, *z, *r;
+  const int32_t *beh;
+  const uint8_t *flags;
+  double *acc;   // [slices][3][npad]: the targets' sums
+  float *layer;  // [distance][3][npad]: the tiles' sums
+  uint64_t *pairs;
+  DevCounters *ctr;
+  const uint32_t *run_flag;
+  int64_t pair_cap;
+  int npad, n;
+  float eps2;
+  int events;
+  // set by launch_force_sym
+  int ntiles, nb, slices, d0, d1;
+};
+// out: [3][npad] accelerations / G, apart from a.acc.  layer_words: floats in a.layer.
+hipError_t launch_force_sym(const ForceShape &s, SymArgs a, double *out, int64_t layer_words,
+                            bool detect, hipStream_t st);
 
 struct FixupArgs {
   const double *x, *y, *z, *m, *r;

@@ -1529,12 +1529,9 @@ int sur_force_phase(Ctx *c, bool timed, int ev_slot) {
     rc = sur_check_launch(c, s->p.check_samples, s->p.tol, s->p.tol_body, true);
     if (rc) return rc;
     // direct-sum redo of this cycle's force when the flag is up (the kernel exits otherwise)
-    ForceArgs fa = make_force_args(c);
-    fa.run_flag = s->flag;
-    fa.detect = 0;  // the near field already listed every colliding pair
-    fa.drop_flagged = 0;
-    NB_HIP(c, launch_force_f32(c->shape, fa, st));
-    hipLaunchKernelGGL(k_sur_fold, dim3(nb256(c->n)), dim3(256), 0, st, c->acc, c->shape.jsplit,
+    // (no detection: the near field already listed every colliding pair)
+    NB_HIP(c, launch_plain(c, false, s->flag));
+    hipLaunchKernelGGL(k_sur_fold, dim3(nb256(c->n)), dim3(256), 0, st, c->acc, plain_split(c),
                        (int)c->npad, (int)c->n, s->flag, c->ctr);
     NB_HIP(c, hipGetLastError());
     s->checks++;
@@ -1699,11 +1696,16 @@ int nb_sur_collect(nb_ctx *c, int64_t samples, uint64_t seed) {
   NB_HIP(c, hipSetDevice(c->device));
   int rc = sur_pipeline(c, true, false, false, false);
   if (rc) return rc;
-  ForceArgs fa = make_force_args(c);
+  // labels come from the kernel with one evaluation per ordered pair: a network trained from the
+  // same seeds keeps its bits whichever kernel the steps run
+  const ForceShape ls = c->shape.variant == 3 ? default_shape(c->npad) : c->shape;
+  rc = ensure_acc(c, ls.jsplit);
+  if (rc) return rc;
+  ForceArgs fa = make_force_args(c, ls);
   fa.run_flag = nullptr;
   fa.detect = 0;
   fa.drop_flagged = 0;
-  NB_HIP(c, launch_force_f32(c->shape, fa, c->stream));
+  NB_HIP(c, launch_force_f32(ls, fa, c->stream));
   int32_t nact = 0;
   NB_HIP(c, hipMemcpyAsync(&nact, s->cstart + s->ncell, 4, hipMemcpyDeviceToHost, c->stream));
   NB_HIP(c, hipStreamSynchronize(c->stream));
@@ -1739,7 +1741,7 @@ int nb_sur_collect(nb_ctx *c, int64_t samples, uint64_t seed) {
                                 c->stream);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_sur_label, dim3(nb256(S)), dim3(256), 0, c->stream, dpick, (int)S,
-                       s->perm, s->keys2, s->ncell, s->base, s->feat, c->acc, c->shape.jsplit,
+                       s->perm, s->keys2, s->ncell, s->base, s->feat, c->acc, ls.jsplit,
                        (int)c->npad, s->tx + (size_t)s->trows * kFeat, s->ty + (size_t)s->trows * 3);
     e = hipGetLastError();
   }
