@@ -32,7 +32,7 @@ __device__ static void emit(uint64_t *pairs, DevCounters *ctr, int64_t cap, int 
 }
 
 // ---------------------------------------------------------------------------------------------
-// FP64 force in the reference's operation order, one thread per target, sources in index order.
+// FP64 force in the reference's operation order, sources added in index order.
 //   eps == 0 && cutoff: calcForceFrom (body.go:214-225)
 //       dist = sqrt(dx*dx+dy*dy+dz*dz); if dist > Ri+Rj: force = G*mi*mj/(dist*dist);
 //       fx += force*dx/dist
@@ -40,80 +40,146 @@ __device__ static void emit(uint64_t *pairs, DevCounters *ctr, int64_t cap, int 
 //       distSq = d2 + eps*eps; dist = sqrt(distSq); force = G*mi*mj/distSq; fx += force*dx/dist
 // Pairs are emitted from the lower index (Collided, body.go:192-208).
 // ---------------------------------------------------------------------------------------------
-// Sources are staged in LDS 256 at a time by the workgroup and read back as broadcasts; each
-// lane still sums its sources in array order, op for op as calcForceFrom.
-__global__ __launch_bounds__(256) void k_force_f64(Force64Args a) {
-  __shared__ double sx[256], sy[256], sz[256], sm[256], sr[256];
-  __shared__ int32_t sb[256];
-  __shared__ uint8_t sf[256];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;  // npad is a multiple of 256
-  double fx = 0, fy = 0, fz = 0;
+// Three quotients by one divisor, bit-identical to three divisions.  A correctly rounded FP64
+// division n / d is v_div_scale of both operands, v_rcp, two Newton steps, the quotient, its
+// residual, v_div_fmas and v_div_fixup; with d in [2^-400, 2^400] and |n| in [2^-400, 2^300] the
+// scalings and the fix-up are identities, so the steps that depend on d alone are done once.  Zero
+// numerators (a body on a coordinate plane of the other) take the division, like everything else
+// outside that range.
+// need: lanes whose quotients are used (the others may hold anything).
+__device__ __forceinline__ void three_quotients(const double n[3], double d, bool need,
+                                                double q[3]) {
+  double y = __builtin_amdgcn_rcp(d);
+  y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+  y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+  int ok = (int)(d >= 0x1p-400) & (int)(d <= 0x1p400);
+#pragma unroll
+  for (int c = 0; c < 3; c++) ok &= (int)(fabs(n[c]) >= 0x1p-400) & (int)(fabs(n[c]) <= 0x1p300);
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    const double v = n[c] * y;
+    q[c] = __builtin_fma(__builtin_fma(-d, v, n[c]), y, v);
+  }
+  if (__builtin_amdgcn_ballot_w64(need && !ok)) {
+    __asm__ volatile("");  // a real branch: these divisions are rare
+    if (!ok) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) q[c] = n[c] / d;
+    }
+  }
+}
+
+// A target's terms are computed by many lanes and added by one, in index order.
+// A workgroup owns TL targets.  Its 13 term waves take the next 13 * 64 / TL sources of a round
+// (lane = target + TL * source; UN passes per round), and write the three components of each term
+// to LDS; a skipped pair (self, inactive, behind the gate) writes +0.0, which leaves the sum's
+// bits alone: a sum that starts at +0.0 is never -0.0.  Meanwhile its 3 sum waves, one per
+// component, add the previous round's terms in index order.  The buffers alternate, so there is
+// one barrier per round.
+// One lane per target (sources staged in LDS) left most of the chip idle below 65,536 bodies, each
+// lane in a serial chain of square roots and divisions: 0.413 ms at n = 1,000, 6.69 at 16,384,
+// 26.6 at 65,536, 283 at 262,144.  This form, same bits: 0.018, 1.22, 16.7 and 256 ms.  What bounds
+// it now is FP64 issue (about 110 VALU instructions a pair), and for small n the serial additions.
+constexpr int kF64Term = 13, kF64Sum = 3;
+template <int TL, int UN>
+__global__ __launch_bounds__(64 * (kF64Term + kF64Sum)) void k_force_f64(Force64Args a) {
+  constexpr int SL = 64 / TL;            // sources per wave
+  constexpr int C = kF64Term * SL;       // sources per pass of the term waves
+  __shared__ double terms[2][3][C * UN][TL];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = blockIdx.x * TL + (lane & (TL - 1));
+  const int rounds = (a.n + C * UN - 1) / (C * UN);
+  if (wave >= kF64Term) {  // a component's sums
+    const int c = wave - kF64Term;
+    double f = 0;
+    for (int r = 0; r <= rounds; r++) {
+      if (r > 0 && lane < TL) {
+        const double *t = &terms[(r - 1) & 1][c][0][lane];
+#pragma unroll 13
+        for (int e = 0; e < C * UN; e++) f += t[e * TL];
+      }
+      __syncthreads();
+    }
+    if (lane < TL && i < a.npad) a.acc[(size_t)c * a.npad + i] = f;
+    return;
+  }
   const bool ai = i < a.n && active_f(a.flags[i]);
-  const bool wave_on = __builtin_amdgcn_ballot_w64(ai) != 0;
   const double xi = ai ? a.x[i] : 0, yi = ai ? a.y[i] : 0, zi = ai ? a.z[i] : 0;
   const double mi = ai ? a.m[i] : 0, ri = ai ? a.r[i] : 0;
   const int32_t bi = ai ? a.beh[i] : NB_CB_NONE;
-  const bool ci = ai && nb_may_pair(bi, a.events);
-  const double G = a.G, eps2 = a.eps * a.eps;
+  const bool ci = ai && a.collisions && nb_may_pair(bi, a.events);
+  const double Gm = a.G * mi, eps2 = a.eps * a.eps;
   const bool ref = a.eps == 0.0 && a.cutoff;
-  // the unsoftened distance is only needed for the overlap gate and for detection
   const bool need_d0 = ref || a.cutoff || a.collisions;
-  for (int t0 = 0; t0 < a.n; t0 += 256) {
-    __syncthreads();
-    const int js = t0 + threadIdx.x;
-    if (js < a.n) {
-      sx[threadIdx.x] = a.x[js];
-      sy[threadIdx.x] = a.y[js];
-      sz[threadIdx.x] = a.z[js];
-      sm[threadIdx.x] = a.m[js];
-      sr[threadIdx.x] = a.r[js];
-      sb[threadIdx.x] = a.beh[js];
-      sf[threadIdx.x] = a.flags[js];
-    }
-    __syncthreads();
-    if (!wave_on) continue;
-    const int cnt = min(256, a.n - t0);
-    for (int jj = 0; jj < cnt; jj++) {
-      if (!active_f(sf[jj])) continue;
-      const int j = t0 + jj;
-      const double dx = sx[jj] - xi;
-      const double dy = sy[jj] - yi;
-      const double dz = sz[jj] - zi;
-      const double d2 = dx * dx + dy * dy + dz * dz;
-      const double rs = ri + sr[jj];
-      if (j != i && ai) {
+  // a source's words are requested one pass ahead, so no term waits for memory
+  double sx, sy, sz, sm, sr;
+  int sf;
+  const int j0 = wave * SL + lane / TL;
+  auto fetch = [&](int j) {
+    const int q = min(j, a.n - 1);
+    sx = a.x[q];
+    sy = a.y[q];
+    sz = a.z[q];
+    sm = a.m[q];
+    sr = a.r[q];
+    sf = a.flags[q];
+  };
+  fetch(j0);
+  for (int r = 0; r <= rounds; r++) {
+    if (r < rounds) {
+#pragma unroll
+      for (int u = 0; u < UN; u++) {
+        const int j = (r * UN + u) * C + j0;
+        const double dx = sx - xi, dy = sy - yi, dz = sz - zi, mj = sm, rj = sr;
+        const bool valid = j < a.n && j != i && ai && active_f((uint8_t)sf);
+        fetch(j + C);
+        const double d2 = dx * dx + dy * dy + dz * dz;
+        const double rs = ri + rj;
         const double dist0 = need_d0 ? __builtin_sqrt(d2) : 0.0;
         const bool overlap = need_d0 && !(dist0 > rs);
-        if (ref) {
-          if (!overlap) {
-            const double force = G * mi * sm[jj] / (dist0 * dist0);
-            fx += force * dx / dist0;
-            fy += force * dy / dist0;
-            fz += force * dz / dist0;
-          }
-        } else {
-          if (!(a.cutoff && overlap)) {
-            const double distSq = d2 + eps2;
-            const double dist = __builtin_sqrt(distSq);
-            const double force = G * mi * sm[jj] / distSq;
-            fx += force * dx / dist;
-            fy += force * dy / dist;
-            fz += force * dz / dist;
-          }
-        }
-        if (a.collisions && overlap && i < j && ci &&
-            nb_pair_event(bi, sb[jj], ri, sr[jj], dist0, a.events))
+        // eps == 0 with the gate divides by the rounded distance's square (body.go:221),
+        // otherwise by the squared distance itself (octree.go:317-319)
+        const double distSq = ref ? dist0 * dist0 : d2 + eps2;
+        const double dist = ref ? dist0 : __builtin_sqrt(distSq);
+        const double force = Gm * mj / distSq;
+        const double n[3] = {force * dx, force * dy, force * dz};
+        double q[3];
+        three_quotients(n, dist, valid, q);
+        const bool adds = valid && !(a.cutoff && overlap);
+        const int e = u * C + j0;
+#pragma unroll
+        for (int c = 0; c < 3; c++) terms[r & 1][c][e][lane & (TL - 1)] = adds ? q[c] : 0.0;
+        if (valid && overlap && i < j && ci &&
+            nb_pair_event(bi, a.beh[j], ri, rj, dist0, a.events))
           emit(a.pairs, a.ctr, a.pair_cap, i, j);
       }
     }
+    __syncthreads();
   }
-  a.acc[i] = fx;
-  a.acc[a.npad + i] = fy;
-  a.acc[2 * a.npad + i] = fz;
 }
 
 hipError_t launch_force_f64(const Force64Args &a, hipStream_t st) {
-  hipLaunchKernelGGL(k_force_f64, dim3((unsigned)(a.npad / 256)), dim3(256), 0, st, a);
+  // Targets per workgroup: the busiest of the 256 CUs takes k = ceil(n / (256 TL)) workgroups, and
+  // the time measured from n = 200 to 40,000 is n (a + b k): a one round's latency, b the work of
+  // TL targets, in units of 0.1 us per 1,000 sources.  Small TL spreads few targets over the chip,
+  // large TL reads each source for more of them.
+  const struct { int tl, a, b; } cost[] = {{64, 207, 559}, {32, 110, 336}, {16, 65, 169},
+                                           {8, 43, 103}, {4, 75, 69}};
+  int tl = 64;
+  int64_t best = INT64_MAX;
+  for (const auto &q : cost) {
+    const int64_t k = ((int64_t)a.n + 256 * q.tl - 1) / (256 * q.tl), v = q.a + q.b * k;
+    if (v < best) best = v, tl = q.tl;
+  }
+  const dim3 grid((unsigned)(a.npad / tl)), block(64 * (kF64Term + kF64Sum));
+  switch (tl) {
+    case 64: hipLaunchKernelGGL((k_force_f64<64, 2>), grid, block, 0, st, a); break;
+    case 32: hipLaunchKernelGGL((k_force_f64<32, 1>), grid, block, 0, st, a); break;
+    case 16: hipLaunchKernelGGL((k_force_f64<16, 1>), grid, block, 0, st, a); break;
+    case 8: hipLaunchKernelGGL((k_force_f64<8, 1>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((k_force_f64<4, 1>), grid, block, 0, st, a); break;
+  }
   return hipGetLastError();
 }
 
