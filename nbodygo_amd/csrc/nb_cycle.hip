@@ -23,14 +23,6 @@ __device__ __forceinline__ bool collide_b(int32_t b) {
   return b == NB_CB_ELASTIC || b == NB_CB_FRAGMENT;
 }
 
-__device__ static void emit(uint64_t *pairs, DevCounters *ctr, int64_t cap, int i, int j) {
-  uint32_t q = atomicAdd(&ctr->pair_count, 1u);
-  if ((int64_t)q < cap)
-    pairs[q] = ((uint64_t)(uint32_t)i << 32) | (uint32_t)j;
-  else
-    atomicOr(&ctr->pair_overflow, 1u);
-}
-
 // ---------------------------------------------------------------------------------------------
 // FP64 force in the reference's operation order, sources added in index order.
 //   eps == 0 && cutoff: calcForceFrom (body.go:214-225)
@@ -82,14 +74,18 @@ __device__ __forceinline__ void three_quotients(const double n[3], double d, boo
 // it now is FP64 issue (about 110 VALU instructions a pair), and for small n the serial additions.
 constexpr int kF64Term = 13, kF64Sum = 3;
 template <int TL, int UN>
-__global__ __launch_bounds__(64 * (kF64Term + kF64Sum)) void k_force_f64(Force64Args a) {
+__global__ __launch_bounds__(64 * (kF64Term + kF64Sum)) __attribute__((amdgpu_waves_per_eu(8)))
+void k_force_f64(Force64Args a) {
   constexpr int SL = 64 / TL;            // sources per wave
   constexpr int C = kF64Term * SL;       // sources per pass of the term waves
   __shared__ double terms[2][3][C * UN][TL];
+  __shared__ PairBuf<192> found;  // (two workgroups' LDS just fits a CU with TL = 64)
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = blockIdx.x * TL + (lane & (TL - 1));
   const int rounds = (a.n + C * UN - 1) / (C * UN);
+  if (threadIdx.x == 0) found.clear();
+  __syncthreads();
   if (wave >= kF64Term) {  // a component's sums
     const int c = wave - kF64Term;
     double f = 0;
@@ -102,61 +98,62 @@ __global__ __launch_bounds__(64 * (kF64Term + kF64Sum)) void k_force_f64(Force64
       __syncthreads();
     }
     if (lane < TL && i < a.npad) a.acc[(size_t)c * a.npad + i] = f;
-    return;
-  }
-  const bool ai = i < a.n && active_f(a.flags[i]);
-  const double xi = ai ? a.x[i] : 0, yi = ai ? a.y[i] : 0, zi = ai ? a.z[i] : 0;
-  const double mi = ai ? a.m[i] : 0, ri = ai ? a.r[i] : 0;
-  const int32_t bi = ai ? a.beh[i] : NB_CB_NONE;
-  const bool ci = ai && a.collisions && nb_may_pair(bi, a.events);
-  const double Gm = a.G * mi, eps2 = a.eps * a.eps;
-  const bool ref = a.eps == 0.0 && a.cutoff;
-  const bool need_d0 = ref || a.cutoff || a.collisions;
-  // a source's words are requested one pass ahead, so no term waits for memory
-  double sx, sy, sz, sm, sr;
-  int sf;
-  const int j0 = wave * SL + lane / TL;
-  auto fetch = [&](int j) {
-    const int q = min(j, a.n - 1);
-    sx = a.x[q];
-    sy = a.y[q];
-    sz = a.z[q];
-    sm = a.m[q];
-    sr = a.r[q];
-    sf = a.flags[q];
-  };
-  fetch(j0);
-  for (int r = 0; r <= rounds; r++) {
-    if (r < rounds) {
+  } else {
+    const bool ai = i < a.n && active_f(a.flags[i]);
+    const double xi = ai ? a.x[i] : 0, yi = ai ? a.y[i] : 0, zi = ai ? a.z[i] : 0;
+    const double mi = ai ? a.m[i] : 0, ri = ai ? a.r[i] : 0;
+    const int32_t bi = ai ? a.beh[i] : NB_CB_NONE;
+    const bool ci = ai && a.collisions && nb_may_pair(bi, a.events);
+    const double Gm = a.G * mi, eps2 = a.eps * a.eps;
+    const bool ref = a.eps == 0.0 && a.cutoff;
+    const bool need_d0 = ref || a.cutoff || a.collisions;
+    // a source's words are requested one pass ahead, so no term waits for memory
+    double sx, sy, sz, sm, sr;
+    int sf;
+    const int j0 = wave * SL + lane / TL;
+    auto fetch = [&](int j) {
+      const int q = min(j, a.n - 1);
+      sx = a.x[q];
+      sy = a.y[q];
+      sz = a.z[q];
+      sm = a.m[q];
+      sr = a.r[q];
+      sf = a.flags[q];
+    };
+    fetch(j0);
+    for (int r = 0; r <= rounds; r++) {
+      if (r < rounds) {
 #pragma unroll
-      for (int u = 0; u < UN; u++) {
-        const int j = (r * UN + u) * C + j0;
-        const double dx = sx - xi, dy = sy - yi, dz = sz - zi, mj = sm, rj = sr;
-        const bool valid = j < a.n && j != i && ai && active_f((uint8_t)sf);
-        fetch(j + C);
-        const double d2 = dx * dx + dy * dy + dz * dz;
-        const double rs = ri + rj;
-        const double dist0 = need_d0 ? __builtin_sqrt(d2) : 0.0;
-        const bool overlap = need_d0 && !(dist0 > rs);
-        // eps == 0 with the gate divides by the rounded distance's square (body.go:221),
-        // otherwise by the squared distance itself (octree.go:317-319)
-        const double distSq = ref ? dist0 * dist0 : d2 + eps2;
-        const double dist = ref ? dist0 : __builtin_sqrt(distSq);
-        const double force = Gm * mj / distSq;
-        const double n[3] = {force * dx, force * dy, force * dz};
-        double q[3];
-        three_quotients(n, dist, valid, q);
-        const bool adds = valid && !(a.cutoff && overlap);
-        const int e = u * C + j0;
+        for (int u = 0; u < UN; u++) {
+          const int j = (r * UN + u) * C + j0;
+          const double dx = sx - xi, dy = sy - yi, dz = sz - zi, mj = sm, rj = sr;
+          const bool valid = j < a.n && j != i && ai && active_f((uint8_t)sf);
+          fetch(j + C);
+          const double d2 = dx * dx + dy * dy + dz * dz;
+          const double rs = ri + rj;
+          const double dist0 = need_d0 ? __builtin_sqrt(d2) : 0.0;
+          const bool overlap = need_d0 && !(dist0 > rs);
+          // eps == 0 with the gate divides by the rounded distance's square (body.go:221),
+          // otherwise by the squared distance itself (octree.go:317-319)
+          const double distSq = ref ? dist0 * dist0 : d2 + eps2;
+          const double dist = ref ? dist0 : __builtin_sqrt(distSq);
+          const double force = Gm * mj / distSq;
+          const double n[3] = {force * dx, force * dy, force * dz};
+          double q[3];
+          three_quotients(n, dist, valid, q);
+          const bool adds = valid && !(a.cutoff && overlap);
+          const int e = u * C + j0;
 #pragma unroll
-        for (int c = 0; c < 3; c++) terms[r & 1][c][e][lane & (TL - 1)] = adds ? q[c] : 0.0;
-        if (valid && overlap && i < j && ci &&
-            nb_pair_event(bi, a.beh[j], ri, rj, dist0, a.events))
-          emit(a.pairs, a.ctr, a.pair_cap, i, j);
+          for (int c = 0; c < 3; c++) terms[r & 1][c][e][lane & (TL - 1)] = adds ? q[c] : 0.0;
+          if (valid && overlap && i < j && ci &&
+              nb_pair_event(bi, a.beh[j], ri, rj, dist0, a.events))
+            found.add(a.pairs, a.ctr, a.pair_cap, i, j);
+        }
       }
+      __syncthreads();
     }
-    __syncthreads();
   }
+  found.flush(a.pairs, a.ctr, a.pair_cap);
 }
 
 hipError_t launch_force_f64(const Force64Args &a, hipStream_t st) {

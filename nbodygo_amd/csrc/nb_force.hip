@@ -217,6 +217,7 @@ __global__ __launch_bounds__(256) void k_force_scalar(ForceArgs a) {
 // Variant 2: source tiles are staged in LDS by the workgroup (one coalesced 16-byte load per
 // lane per row), then read back as wave-uniform broadcasts (ds_read_b128, no bank conflicts).
 constexpr int kLdsTileMax = 1024;
+constexpr int kLdsStage = 512;
 template <int IPL, bool DETECT>
 __global__ __launch_bounds__(256) void k_force_lds(ForceArgs a) {
   __shared__ float4 sh[kLdsTileMax];
@@ -229,28 +230,34 @@ __global__ __launch_bounds__(256) void k_force_lds(ForceArgs a) {
   const int t0 = blockIdx.y * a.tiles_per_slice;
   const int t1 = min(t0 + a.tiles_per_slice, a.tiles);
   cfp rmt = (cfp)a.rmax_tile;
-  for (int t = t0; t < t1; t++) {
+  // short tiles are staged several at a time: two barriers per 512 sources
+  const int per = a.tile_j < kLdsStage ? kLdsStage / a.tile_j : 1;
+  for (int ts = t0; ts < t1; ts += per) {
+    const int te = min(ts + per, t1), staged = (te - ts) * a.tile_j;
     __syncthreads();
-    const float4 *src = a.js + (size_t)t * a.tile_j;
-    for (int q = threadIdx.x; q < a.tile_j; q += blockDim.x) sh[q] = src[q];
+    const float4 *src = a.js + (size_t)ts * a.tile_j;
+    for (int q = threadIdx.x; q < staged; q += blockDim.x) sh[q] = src[q];
     __syncthreads();
-    float px[IPL], py[IPL], pz[IPL], rmin[IPL];
+    for (int t = ts; t < te; t++) {
+      const float4 *tl = sh + (t - ts) * a.tile_j;
+      float px[IPL], py[IPL], pz[IPL], rmin[IPL];
 #pragma unroll
-    for (int k = 0; k < IPL; k++) px[k] = py[k] = pz[k] = 0.f, rmin[k] = FLT_MAX;
-    // tile_j is a multiple of 64.  Eight sources per step are read first (eight ds_read_b128 in
-    // flight, one LDS base address with immediate offsets), then used in order.
-    for (int jj = 0; jj < a.tile_j; jj += 8) {
-      float4 b8[8];
+      for (int k = 0; k < IPL; k++) px[k] = py[k] = pz[k] = 0.f, rmin[k] = FLT_MAX;
+      // tile_j is a multiple of 64.  Eight sources per step are read first (eight ds_read_b128 in
+      // flight, one LDS base address with immediate offsets), then used in order.
+      for (int jj = 0; jj < a.tile_j; jj += 8) {
+        float4 b8[8];
 #pragma unroll
-      for (int u = 0; u < 8; u++) b8[u] = sh[jj + u];
+        for (int u = 0; u < 8; u++) b8[u] = tl[jj + u];
 #pragma unroll
-      for (int u = 0; u < 8; u++) NB_INTERACT(b8[u].x, b8[u].y, b8[u].z, b8[u].w)
+        for (int u = 0; u < 8; u++) NB_INTERACT(b8[u].x, b8[u].y, b8[u].z, b8[u].w)
+      }
+      self_tile_rmin<IPL, DETECT>(T, rmin, base, stride, t, a.tile_j, eps2, [&](int jj) -> f4v {
+        const float4 b = tl[jj];
+        return f4v{b.x, b.y, b.z, b.w};
+      });
+      tile_end<IPL, DETECT>(T, px, py, pz, rmin, DETECT ? rmt[t] : 0.f, eps2, a.drop_flagged, t);
     }
-    self_tile_rmin<IPL, DETECT>(T, rmin, base, stride, t, a.tile_j, eps2, [&](int jj) -> f4v {
-      const float4 b = sh[jj];
-      return f4v{b.x, b.y, b.z, b.w};
-    });
-    tile_end<IPL, DETECT>(T, px, py, pz, rmin, DETECT ? rmt[t] : 0.f, eps2, a.drop_flagged, t);
   }
   store_targets<IPL, DETECT>(T, a, base, stride);
 }
@@ -291,14 +298,6 @@ __device__ __forceinline__ bool can_collide(int32_t b) {
   return b == NB_CB_ELASTIC || b == NB_CB_FRAGMENT;
 }
 
-__device__ void emit_pair(uint64_t *pairs, DevCounters *ctr, int64_t cap, int i, int j) {
-  uint32_t q = atomicAdd(&ctr->pair_count, 1u);
-  if ((int64_t)q < cap)
-    pairs[q] = ((uint64_t)(uint32_t)i << 32) | (uint32_t)j;
-  else
-    atomicOr(&ctr->pair_overflow, 1u);
-}
-
 // One wavefront per record: the 64 lanes split each flagged tile's sources, and the FP64 partial
 // sums are combined with a fixed butterfly, so the result does not depend on scheduling.  The
 // grid is fixed; waves stride over the record count the force kernel left in device memory.
@@ -308,7 +307,13 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// Pairs and the tile count go through LDS: an atomic per record took most of the kernel's 0.88 ms
+// at n = 10,007 in the reference scene (55,000 records).  Without them, and with a source's words
+// requested together, 0.15 ms: 220 G pair tests/s, FP64 issue.
 __global__ __launch_bounds__(256) void k_fixup(FixupArgs a) {
+  __shared__ PairBuf<512> found;
+  if (threadIdx.x == 0) found.clear();
+  __syncthreads();
   const int lane = threadIdx.x & 63;
   const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   const int nwaves = (int)((gridDim.x * blockDim.x) >> 6);
@@ -334,24 +339,28 @@ __global__ __launch_bounds__(256) void k_fixup(FixupArgs a) {
       else t = u == 0 ? lst.x : u == 1 ? lst.y : u == 2 ? lst.z : lst.w;
       const int j0 = t * a.tile_j;
       const int j1 = min(j0 + a.tile_j, a.n);
-      for (int j = j0 + lane; j < j1; j += 64) {
-        if (j == i || !active_body(a.flags[j])) continue;
-        const double dx = a.x[j] - xi;
-        const double dy = a.y[j] - yi;
-        const double dz = a.z[j] - zi;
+      for (int jb = j0; jb < j1; jb += 64) {
+        // every word of the source is requested at once; lanes past the end read the last one
+        const int j = jb + lane, q = min(j, j1 - 1);
+        const double xj = a.x[q], yj = a.y[q], zj = a.z[q], rj = a.r[q], mj = a.m[q];
+        const uint8_t fj = a.flags[q];
+        const bool valid = j < j1 && j != i && active_body(fj);
+        const double dx = xj - xi;
+        const double dy = yj - yi;
+        const double dz = zj - zi;
         const double d2 = dx * dx + dy * dy + dz * dz;
         const double dist = __builtin_sqrt(d2);
-        const double rj = a.r[j];
         const bool overlap = !(dist > ri + rj);
-        if (overlap && a.collisions && i < j && ci &&
+        if (valid && overlap && a.collisions && i < j && ci &&
             nb_pair_event(bi, a.beh[j], ri, rj, dist, a.events))
-          emit_pair(a.pairs, a.ctr, a.pair_cap, i, j);
-        if (a.recompute && !(overlap && a.cutoff)) {
+          found.add(a.pairs, a.ctr, a.pair_cap, i, j);
+        if (a.recompute) {
           const double ds = d2 + a.eps2;
-          const double w = a.m[j] / (ds * __builtin_sqrt(ds));
-          ax += w * dx;
-          ay += w * dy;
-          az += w * dz;
+          const double w = mj / (ds * __builtin_sqrt(ds));
+          const bool add = valid && !(overlap && a.cutoff);
+          ax += add ? w * dx : 0.0;
+          ay += add ? w * dy : 0.0;
+          az += add ? w * dz : 0.0;
         }
       }
     }
@@ -361,7 +370,7 @@ __global__ __launch_bounds__(256) void k_fixup(FixupArgs a) {
       az = wave_sum(az);
     }
     if (lane == 0) {
-      atomicAdd((unsigned long long *)&a.ctr->fixup_tiles, (unsigned long long)ntile);
+      atomicAdd(&found.tiles, (uint32_t)ntile);
       if (a.recompute) {
         double *o = a.acc + (size_t)slice * 3 * a.npad;
         if (all) {
@@ -376,11 +385,13 @@ __global__ __launch_bounds__(256) void k_fixup(FixupArgs a) {
       }
     }
   }
+  found.flush(a.pairs, a.ctr, a.pair_cap);
 }
 
 hipError_t launch_fixup(const FixupArgs &a, hipStream_t st) {
-  // 8 waves per CU on 256 CUs; the kernel strides over however many records there are.
-  hipLaunchKernelGGL(k_fixup, dim3(512), dim3(256), 0, st, a);
+  // 32 waves per CU on 256 CUs, enough to cover a record's chain of loads; the kernel strides over
+  // however many records there are.
+  hipLaunchKernelGGL(k_fixup, dim3(2048), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 

@@ -55,7 +55,8 @@ __device__ __forceinline__ float from_next_lane(float v) {
 
 // The reference's overlap test of target i against the 64 bodies of tile t, one per lane; `own`:
 // the tile lies in the target's own block, where each pair is met from both sides.
-__device__ __forceinline__ void exact_tile(const SymArgs &a, int i, int t, bool own) {
+template <class Buf>
+__device__ __forceinline__ void exact_tile(const SymArgs &a, Buf &found, int i, int t, bool own) {
   const int j = t * 64 + (int)(threadIdx.x & 63);
   if (j >= a.n || j == i || (own && j < i)) return;
   const uint8_t fj = a.flags[j];
@@ -66,11 +67,7 @@ __device__ __forceinline__ void exact_tile(const SymArgs &a, int i, int t, bool 
   const double d = __builtin_sqrt(dx * dx + dy * dy + dz * dz);
   const double ri = a.r[i], rj = a.r[j];
   if (d > ri + rj || !nb_pair_event(bi, a.beh[j], ri, rj, d, a.events)) return;
-  const uint32_t q = atomicAdd(&a.ctr->pair_count, 1u);
-  if ((int64_t)q < a.pair_cap)
-    a.pairs[q] = ((uint64_t)(uint32_t)min(i, j) << 32) | (uint32_t)max(i, j);
-  else
-    atomicOr(&a.ctr->pair_overflow, 1u);
+  found.add(a.pairs, a.ctr, a.pair_cap, min(i, j), max(i, j));
 }
 
 // One row of independent instructions ends here: the scheduler keeps rows apart.
@@ -84,6 +81,7 @@ void k_force_sym(SymArgs a) {
   __shared__ float4 sh[2][128];
   __shared__ float red[2][W][3][64];
   __shared__ double sums[W][IPL][3][64];  // the targets' sums over the tiles so far
+  __shared__ PairBuf<DETECT ? 256 : 1> found;
   if (a.run_flag && *a.run_flag == 0u) return;  // conditional launch (surrogate fallback)
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -141,6 +139,7 @@ void k_force_sym(SymArgs a) {
 
   int t = first + u0;
   if (t >= ntiles) t -= ntiles;
+  if (DETECT && threadIdx.x == 0) found.clear();
   if (u0 < u1 && wave == 0) {
     const float4 b = a.js[(size_t)t * 64 + lane];
     sh[0][lane] = b;
@@ -288,12 +287,11 @@ void k_force_sym(SymArgs a) {
         const float thr = __builtin_fmaf(w, w, eps2) * 1.0000039f;
         uint64_t hit = __ballot(rmin[k] <= thr && (live >> k & 1));
         if (hit && lane == 0)
-          atomicAdd((unsigned long long *)&a.ctr->fixup_tiles,
-                    (unsigned long long)__builtin_popcountll(hit));
+          atomicAdd(&found.tiles, (uint32_t)__builtin_popcountll(hit));
         while (hit) {
           const int l = __builtin_ctzll(hit);
           hit &= hit - 1;
-          exact_tile(a, (row * T + wave * IPL + k) * 64 + l, t, d == 0);
+          exact_tile(a, found, (row * T + wave * IPL + k) * 64 + l, t, d == 0);
         }
       }
     }
@@ -320,6 +318,7 @@ void k_force_sym(SymArgs a) {
     o[a.npad + i] = sums[wave][k][1][lane];
     o[2 * (size_t)a.npad + i] = sums[wave][k][2][lane];
   }
+  if (DETECT) found.flush(a.pairs, a.ctr, a.pair_cap);
 }
 
 // out = (first panel: 0, later: out) + the target slices + the distances that reached the body's
