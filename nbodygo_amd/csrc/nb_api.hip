@@ -69,7 +69,7 @@ static void free_all(Ctx *c) {
   void *ptrs[] = {c->x,    c->y,      c->z,     c->vx,   c->vy,        c->vz,   c->m,
                   c->r,    c->rest,   c->frag,  c->beh,  c->flags,     c->collided,
                   c->js,   c->rmax_tile, c->acc, c->fcnt, c->flist, c->recs, c->pairs, c->ctr,
-                  c->diag, c->pairs_tmp, c->pairs_sw, c->res_words, c->layer};
+                  c->diag, c->pairs_sorted, c->pair_words, c->pair_body, c->pair_geom, c->layer};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   c->x = c->y = c->z = c->vx = c->vy = c->vz = c->m = c->r = c->rest = c->frag = nullptr;
@@ -80,8 +80,10 @@ static void free_all(Ctx *c) {
   c->acc = nullptr;
   c->fcnt = c->flist = nullptr;
   c->recs = nullptr;
-  c->pairs = c->pairs_tmp = c->pairs_sw = nullptr;
-  c->res_words = nullptr;
+  c->pairs = c->pairs_sorted = nullptr;
+  c->pair_words = c->pair_body = nullptr;
+  c->pair_geom = nullptr;
+  c->pair_cap_pow2 = c->pair_body_cap = 0;
   c->ctr = nullptr;
   c->diag = nullptr;
   c->layer = nullptr;
@@ -209,21 +211,60 @@ static void choose_shape(Ctx *c) {
   if (p.variant) c->shape.variant = p.variant;
 }
 
-// Pair buffer for n bodies: a power of two so the global bitonic network can pad in place.
+// Pair buffers for n bodies (collisions on), grown in powers of two.
+constexpr int kPairWords = 11;  // int32 words per pair of PairArgs' per-pair arrays
 static int size_pairs(Ctx *c, int64_t n) {
   const int64_t pcap =
       c->p.pair_capacity > 0 ? c->p.pair_capacity : std::max<int64_t>(4 * n, 65536);
+  c->pair_cap = pcap;
+  if (!c->p.collisions) return NB_OK;
   int64_t pow2 = 1;
   while (pow2 < pcap) pow2 <<= 1;
   if (pow2 > c->pair_cap_pow2) {
+    c->pair_cap_pow2 = 0;
     NB_HIP(c, dalloc(&c->pairs, (size_t)pow2));
-    NB_HIP(c, dalloc(&c->pairs_tmp, (size_t)pow2));
-    NB_HIP(c, dalloc(&c->pairs_sw, (size_t)pow2));
-    NB_HIP(c, dalloc(&c->res_words, (size_t)pow2 * 5));
+    NB_HIP(c, dalloc(&c->pairs_sorted, (size_t)pow2));
+    NB_HIP(c, dalloc(&c->pair_words, (size_t)pow2 * kPairWords));
+    NB_HIP(c, dalloc(&c->pair_geom, (size_t)std::min(pow2, kPairGeom) * 6));
     c->pair_cap_pow2 = pow2;
   }
-  c->pair_cap = pcap;
+  if (c->cap > c->pair_body_cap) {
+    c->pair_body_cap = 0;
+    const size_t words = (size_t)4 * (c->cap + 2) + 2 * (c->cap / 1024 + 2);
+    NB_HIP(c, dalloc(&c->pair_body, words));
+    NB_HIP(c, hipMemsetAsync(c->pair_body, 0, words * sizeof(int32_t), c->stream));
+    c->pair_body_cap = c->cap;
+  }
   return NB_OK;
+}
+
+static PairArgs make_pair_args(Ctx *c) {
+  PairArgs a;
+  a.raw = c->pairs;
+  a.keys = c->pairs_sorted;
+  a.cap = c->pair_cap;
+  a.n = (int)c->n;
+  a.ctr = c->ctr;
+  const int64_t body = c->pair_body_cap + 2, pair = c->pair_cap_pow2;  // both even: int2 alignment
+  a.own = c->pair_body;
+  a.reach = a.own + body;
+  a.own_off = a.reach + body;
+  a.reach_off = a.own_off + body;
+  a.bsum = reinterpret_cast<int2 *>(a.reach_off + body);
+  int32_t *w = c->pair_words;
+  a.succ = reinterpret_cast<int2 *>(w);
+  a.role = reinterpret_cast<int2 *>(w + 2 * pair);
+  w += 4 * pair;
+  a.slot_own = w;
+  a.slot_reach = w + pair;
+  a.list_own = w + 2 * pair;
+  a.list_reach = w + 3 * pair;
+  a.by_hi = w + 4 * pair;
+  a.place = w + 5 * pair;
+  a.pend = w + 6 * pair;
+  a.geom = c->pair_geom;
+  a.geom_cap = std::min(pair, kPairGeom);
+  return a;
 }
 
 ForceArgs make_force_args(Ctx *c, const ForceShape &s) {
@@ -276,7 +317,7 @@ hipError_t launch_plain(Ctx *c, bool detect, const uint32_t *run_flag) {
   return launch_force_f32(c->shape, a, c->stream);
 }
 
-// Force phase of one cycle (force + detection + sorted pair list).
+// Force phase of one cycle (force + detection; the pairs in any order).
 static int force_phase(Ctx *c, bool timed, int ev_slot) {
   if (c->sur_on) return sur_force_phase(c, timed, ev_slot);
   if (c->bh_on) return bh_force_phase(c, timed, ev_slot);
@@ -332,12 +373,6 @@ static int force_phase(Ctx *c, bool timed, int ev_slot) {
       NB_HIP(c, launch_fixup(f, c->stream));
     }
   }
-  if (c->p.collisions) return sort_pairs(c);
-  return NB_OK;
-}
-
-int sort_pairs(Ctx *c) {
-  NB_HIP(c, launch_sort_pairs(c->pairs, c->pairs_tmp, c->pair_cap, c->ctr, c->stream));
   return NB_OK;
 }
 
@@ -465,7 +500,6 @@ int nb_load(nb_ctx *c, int64_t n, const double *x, const double *y, const double
     free_all(c);
     c->cap = npad;
     c->rmax_tile_j = 0;
-    c->pair_cap_pow2 = 0;
     NB_HIP(c, dalloc(&c->x, c->cap));
     NB_HIP(c, dalloc(&c->y, c->cap));
     NB_HIP(c, dalloc(&c->z, c->cap));
@@ -579,7 +613,7 @@ int nb_step(nb_ctx *c, double dt, double R, int32_t nsteps, nb_stats *out) {
       ra.beh = c->beh;
       ra.flags = c->flags;
       ra.collided = c->collided;
-      ra.pairs = c->pairs;
+      ra.pairs = c->pairs_sorted;
       ra.ctr = c->ctr;
       ra.pair_cap = c->pair_cap;
       ra.events = c->p.events;
@@ -588,15 +622,9 @@ int nb_step(nb_ctx *c, double dt, double R, int32_t nsteps, nb_stats *out) {
       ra.acc = c->acc;
       ra.split = split_now(c);
       ra.npad = (int)c->npad;
-      ra.pairs_sw = c->pairs_sw;
-      ra.sort_tmp = c->pairs_tmp;
-      ra.succ = c->res_words;
-      ra.pending = c->res_words + 2 * c->pair_cap_pow2;
-      ra.list_a = c->res_words + 3 * c->pair_cap_pow2;
-      ra.list_b = c->res_words + 4 * c->pair_cap_pow2;
       ra.serial = c->p.resolve == 1 ? 1 : 0;
       if (timed) NB_HIP(c, hipEventRecord(c->ev_res[2 * s], c->stream));
-      NB_HIP(c, launch_resolve(ra, c->stream));
+      NB_HIP(c, launch_pairs(make_pair_args(c), &ra, c->pairs_seen, c->stream));
       if (timed) NB_HIP(c, hipEventRecord(c->ev_res[2 * s + 1], c->stream));
     }
     UpdateArgs u;
@@ -637,6 +665,7 @@ int nb_step(nb_ctx *c, double dt, double R, int32_t nsteps, nb_stats *out) {
   const int64_t removed = (int64_t)(after.removed_total - before.removed_total) +
                           (int64_t)(after.inactive_events - before.inactive_events);
   c->n_active = std::max<int64_t>(0, c->n_active - removed);
+  c->pairs_seen = after.pair_count;
   if (c->p.events) events_refresh_host(c, after);
   if (out) {
     memset(out, 0, sizeof *out);
@@ -670,6 +699,8 @@ int nb_compute_forces(nb_ctx *c, double *fx, double *fy, double *fz) {
   NB_HIP(c, hipSetDevice(c->device));
   int rc = force_phase(c, false, 0);
   if (rc) return rc;
+  if (c->p.collisions)
+    NB_HIP(c, launch_pairs(make_pair_args(c), nullptr, c->pairs_seen, c->stream));
   double *tmp = c->diag;  // 3 n doubles of the context's scratch
   NB_HIP(c, launch_combine_force(c->acc, split_now(c), (int)c->npad, (int)c->n, c->m, c->p.G,
                                  c->p.precision == NB_PREC_FP64 ? 1 : 0, tmp, c->stream));
@@ -680,6 +711,7 @@ int nb_compute_forces(nb_ctx *c, double *fx, double *fy, double *fz) {
   NB_HIP(c, hipStreamSynchronize(c->stream));
   DevCounters ctr;
   NB_HIP(c, hipMemcpy(&ctr, c->ctr, sizeof ctr, hipMemcpyDeviceToHost));
+  c->pairs_seen = ctr.pair_count;
   if (ctr.pair_overflow)
     return fail(c, NB_E_PAIR_OVERFLOW, "collision pairs exceeded pair_capacity");
   return NB_OK;
@@ -736,7 +768,7 @@ int nb_get_pairs(nb_ctx *c, int32_t *ij, int64_t cap, int64_t *n) {
   const int64_t k = c->p.collisions ? std::min(stored, cap) : 0;
   if (k > 0) {
     std::vector<uint64_t> keys((size_t)k);
-    NB_HIP(c, hipMemcpy(keys.data(), c->pairs, (size_t)k * sizeof(uint64_t), hipMemcpyDeviceToHost));
+    NB_HIP(c, hipMemcpy(keys.data(), c->pairs_sorted, (size_t)k * sizeof(uint64_t), hipMemcpyDeviceToHost));
     for (int64_t q = 0; q < k; q++) {
       ij[2 * q] = (int32_t)(keys[q] >> 32);
       ij[2 * q + 1] = (int32_t)(keys[q] & 0xffffffffu);

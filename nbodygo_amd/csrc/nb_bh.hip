@@ -1309,10 +1309,6 @@ int bh_force_phase(Ctx *c, bool timed, int ev_slot) {
     da.events = c->p.events;
     hipLaunchKernelGGL(k_bh_detect, dim3(nb256(n)), dim3(256), 0, st, da);
     NB_HIP(c, hipGetLastError());
-    {
-      const int rcs = sort_pairs(c);
-      if (rcs) return rcs;
-    }
   }
   b->builds++;
   return NB_OK;

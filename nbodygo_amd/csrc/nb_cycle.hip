@@ -213,108 +213,6 @@ hipError_t launch_accel_f64(const Accel64Args &a, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Pair sort: keys (i << 32 | j) ascending = canonical order.  The count is known on the device
-// only, so the host launches a fixed sequence sized by the capacity and each kernel reads the
-// count: kSortLdsKeys-key chunks are sorted in LDS by one workgroup each (one workgroup sorts the
-// whole list when it fits), then runs of doubling length are merged (each key finds its place by
-// a binary search in the other run), one launch per run length up to the capacity.  A pass whose
-// runs already span the list copies it, so the buffers alternate in a fixed order and the result
-// always ends in the key buffer.
-// ---------------------------------------------------------------------------------------------
-// Sorts sh[0, P) ascending (P a power of two) with the block's threads.
-__device__ static void bitonic_lds(uint64_t *sh, int64_t P) {
-  const int tid = threadIdx.x, nt = blockDim.x;
-  for (int64_t k = 2; k <= P; k <<= 1) {
-    for (int64_t j = k >> 1; j > 0; j >>= 1) {
-      for (int64_t q = tid; q < P; q += nt) {
-        const int64_t o = q ^ j;
-        if (o > q) {
-          const uint64_t u = sh[q], v = sh[o];
-          const bool up = (q & k) == 0;
-          if ((u > v) == up) {
-            sh[q] = v;
-            sh[o] = u;
-          }
-        }
-      }
-      __syncthreads();
-    }
-  }
-}
-
-// src[base, base + cnt) (cnt <= kSortLdsKeys) sorted through LDS into dst[base, base + cnt).
-__device__ static void sort_chunk_lds(uint64_t *sh, const uint64_t *src, uint64_t *dst,
-                                      int64_t base, int64_t cnt) {
-  const int tid = threadIdx.x, nt = blockDim.x;
-  int64_t P = 1;
-  while (P < cnt) P <<= 1;
-  for (int64_t q = tid; q < P; q += nt) sh[q] = q < cnt ? src[base + q] : ~0ull;
-  __syncthreads();
-  bitonic_lds(sh, P);
-  for (int64_t q = tid; q < cnt; q += nt) dst[base + q] = sh[q];
-}
-
-__global__ __launch_bounds__(1024) void k_sort_chunks(const uint64_t *keys, uint64_t *dst,
-                                                      int64_t cap, const DevCounters *ctr) {
-  __shared__ uint64_t sh[kSortLdsKeys];
-  const int64_t cnt = min((int64_t)ctr->pair_count, cap);
-  const int64_t base = (int64_t)blockIdx.x * kSortLdsKeys;
-  if (base >= cnt) return;
-  sort_chunk_lds(sh, keys, dst, base, min((int64_t)kSortLdsKeys, cnt - base));
-}
-
-// Number of entries of the sorted run r[0, n) below key (strict) or, with upper, not above it.
-__device__ __forceinline__ int64_t run_rank(const uint64_t *r, int64_t n, uint64_t key,
-                                            bool upper) {
-  int64_t lo = 0, hi = n;
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) >> 1;
-    const uint64_t v = r[mid];
-    if (v < key || (upper && v == key)) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
-}
-
-// Runs of length L in src merged pairwise into dst (copied when one run spans the list).
-__global__ __launch_bounds__(256) void k_merge_pass(const uint64_t *src, uint64_t *dst,
-                                                    int64_t L, int64_t cap,
-                                                    const DevCounters *ctr) {
-  const int64_t cnt = min((int64_t)ctr->pair_count, cap);
-  const int64_t gs = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < cnt; q += gs) {
-    const uint64_t key = src[q];
-    if (cnt <= L) {
-      dst[q] = key;
-      continue;
-    }
-    const int64_t r = q / L, m0 = (r & ~(int64_t)1) * L;
-    if (!(r & 1)) {  // left run: place after the right run's smaller keys
-      const int64_t rb = m0 + L;
-      dst[rb < cnt ? q + run_rank(src + rb, min(L, cnt - rb), key, false) : q] = key;
-    } else {  // right run: after the left run's keys not above it (stable)
-      dst[q - L + run_rank(src + m0, L, key, true)] = key;
-    }
-  }
-}
-
-hipError_t launch_sort_pairs(uint64_t *keys, uint64_t *tmp, int64_t cap, const DevCounters *ctr,
-                             hipStream_t st) {
-  int passes = 0;
-  for (int64_t L = kSortLdsKeys; L < cap; L <<= 1) passes++;
-  // the chunks go to whichever buffer makes the last pass land in keys
-  uint64_t *buf[2] = {(passes & 1) ? tmp : keys, (passes & 1) ? keys : tmp};
-  const unsigned chunks = (unsigned)((cap + kSortLdsKeys - 1) / kSortLdsKeys);
-  hipLaunchKernelGGL(k_sort_chunks, dim3(chunks), dim3(1024), 0, st, keys, buf[0], cap, ctr);
-  const unsigned g = (unsigned)std::min<int64_t>(2048, (cap + 255) / 256);
-  int64_t L = kSortLdsKeys;
-  for (int p = 0; p < passes; p++, L <<= 1)
-    hipLaunchKernelGGL(k_merge_pass, dim3(g), dim3(256), 0, st, buf[p & 1], buf[(p + 1) & 1], L,
-                       cap, ctr);
-  return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------------------------
 // Elastic collision resolution (ProcessMods, body_collection.go:212-233), one thread walking the
 // sorted pair list: each unordered pair is resolved once, as lo.ResolveCollision(hi) when lo is
 // Elastic, else hi.ResolveCollision(lo) (only an Elastic first body resolves, body.go:252-253).
@@ -323,23 +221,42 @@ struct Elastic {
   double v1[3], v2[3], cm[3];
 };
 
-// calcElasticCollision, cmd/body/collisioncalc.go:42-186 (coll3d).
-__device__ static bool elastic(const ResolveArgs &a, int b, int o, Elastic &res) {
-  double r12, m21, d, v, theta2, phi2, st, ct, sp, cp, vx1r, vy1r, vz1r, fvz1r, thetav, phiv, dr,
-      alpha, beta, sbeta, cbeta, aa, dvz2, vx2r, vy2r, vz2r, x21, y21, z21, vx21, vy21, vz21,
-      vx_cm, vy_cm, vz_cm;
-  const double m1 = a.m[b], m2 = a.m[o];
+// calcElasticCollision, cmd/body/collisioncalc.go:42-186 (coll3d), in two parts: what depends on
+// the two positions and radii alone, which a pass evaluates for all its pairs at once, and the
+// rest.  The operations and their order are the reference's.
+struct ElasticGeom {
+  double d, r12, st, ct, sp, cp;
+};
+
+__device__ static ElasticGeom elastic_geom(const ResolveArgs &a, int b, int o) {
   const double r1 = a.r[b], r2 = a.r[o];
   const double x1 = a.x[b], y1 = a.y[b], z1 = a.z[b];
-  double x2 = a.x[o], y2 = a.y[o], z2 = a.z[o];
+  const double x21 = a.x[o] - x1, y21 = a.y[o] - y1, z21 = a.z[o] - z1;
+  ElasticGeom g;
+  g.r12 = r1 + r2;
+  g.d = sqrt(x21 * x21 + y21 * y21 + z21 * z21);
+  const double theta2 = acos(z21 / g.d);
+  double phi2;
+  if (x21 == 0 && y21 == 0)
+    phi2 = 0;
+  else
+    phi2 = atan2(y21, x21);
+  g.st = sin(theta2);
+  g.ct = cos(theta2);
+  g.sp = sin(phi2);
+  g.cp = cos(phi2);
+  return g;
+}
+
+__device__ static bool elastic(const ResolveArgs &a, int b, int o, const ElasticGeom &g,
+                               Elastic &res) {
+  double m21, v, st, ct, sp, cp, vx1r, vy1r, vz1r, fvz1r, thetav, phiv, dr, alpha, beta, sbeta,
+      cbeta, aa, dvz2, vx2r, vy2r, vz2r, vx21, vy21, vz21, vx_cm, vy_cm, vz_cm;
+  const double m1 = a.m[b], m2 = a.m[o];
   double vx1 = a.vx[b], vy1 = a.vy[b], vz1 = a.vz[b];
   const double vx2 = a.vx[o], vy2 = a.vy[o], vz2 = a.vz[o];
 
-  r12 = r1 + r2;
   m21 = m2 / m1;
-  x21 = x2 - x1;
-  y21 = y2 - y1;
-  z21 = z2 - z1;
   vx21 = vx2 - vx1;
   vy21 = vy2 - vy1;
   vz21 = vz2 - vz1;
@@ -348,26 +265,17 @@ __device__ static bool elastic(const ResolveArgs &a, int b, int o, Elastic &res)
   vy_cm = (m1 * vy1 + m2 * vy2) / (m1 + m2);
   vz_cm = (m1 * vz1 + m2 * vz2) / (m1 + m2);
 
-  d = sqrt(x21 * x21 + y21 * y21 + z21 * z21);
   v = sqrt(vx21 * vx21 + vy21 * vy21 + vz21 * vz21);
   if (v == 0) return false;
 
-  x2 = x21;
-  y2 = y21;
-  z2 = z21;
   vx1 = -vx21;
   vy1 = -vy21;
   vz1 = -vz21;
 
-  theta2 = acos(z2 / d);
-  if (x2 == 0 && y2 == 0)
-    phi2 = 0;
-  else
-    phi2 = atan2(y2, x2);
-  st = sin(theta2);
-  ct = cos(theta2);
-  sp = sin(phi2);
-  cp = cos(phi2);
+  st = g.st;
+  ct = g.ct;
+  sp = g.sp;
+  cp = g.cp;
 
   vx1r = ct * cp * vx1 + ct * sp * vy1 - st * vz1;
   vy1r = cp * vy1 - sp * vx1;
@@ -377,13 +285,16 @@ __device__ static bool elastic(const ResolveArgs &a, int b, int o, Elastic &res)
     fvz1r = 1;
   else if (fvz1r < -1)
     fvz1r = -1;
+  // separating (thetav > pi / 2 below) is settled before any angle: acos(x) is pi / 2 - x near 0,
+  // so at -1e-14 it exceeds M_PI / 2 by 45 of its ulps
+  if (fvz1r < -1e-14) return false;
   thetav = acos(fvz1r);
   if (vx1r == 0 && vy1r == 0)
     phiv = 0;
   else
     phiv = atan2(vy1r, vx1r);
 
-  dr = d * sin(thetav) / r12;
+  dr = g.d * sin(thetav) / g.r12;
   if (thetav > M_PI / 2 || fabs(dr) > 1) return false;
 
   alpha = asin(-dr);
@@ -496,23 +407,11 @@ __device__ static bool elastic_pair(const ResolveArgs &a, int lo, int hi, int *b
   return (a.flags[*b] & NB_F_EXISTS) && (a.flags[*o] & NB_F_EXISTS);
 }
 
-// One canonical pair, as ProcessMods handles its event (body_collection.go:212-233).
-__device__ static void resolve_pair(const ResolveArgs &a, int lo, int hi, ResolveTally &t) {
-  if (a.events && !(collide_b(a.beh[lo]) && collide_b(a.beh[hi]))) {
-    // a subsume pair: ResolveSubsume (body.go:228-244) by the larger body, no existence check
-    const int b = a.r[lo] > a.r[hi] ? lo : hi, o = b == lo ? hi : lo;
-    a.m[b] = a.m[b] + a.m[o];
-    const uint8_t fo = a.flags[o];
-    if ((fo & NB_F_EXISTS) && !(fo & NB_F_FRAGMENTING)) t.inactive++;
-    a.flags[o] = (uint8_t)(fo & ~NB_F_EXISTS);  // SetNotExists (body.go:93-96)
-    a.m[o] = 0.0;
-    t.subsumed++;
-    return;
-  }
-  int b, o;
-  if (!elastic_pair(a, lo, hi, &b, &o)) return;
+// A pair that can act, b resolving (ResolveCollision, body.go:248-264).
+__device__ static void resolve_elastic(const ResolveArgs &a, int b, int o, const ElasticGeom &g,
+                                       ResolveTally &t) {
   Elastic e;
-  if (!elastic(a, b, o, e)) return;
+  if (!elastic(a, b, o, g, e)) return;
   t.resolved++;
   double tf = 0, of = 0;
   if (should_fragment(a, b, o, e, &tf, &of)) {
@@ -535,6 +434,24 @@ __device__ static void resolve_pair(const ResolveArgs &a, int lo, int hi, Resolv
   a.vz[o] = (e.v2[2] - e.cm[2]) * rr + e.cm[2];
   a.collided[b] = 1;
   a.collided[o] = 1;
+}
+
+// One canonical pair, as ProcessMods handles its event (body_collection.go:212-233).
+__device__ static void resolve_pair(const ResolveArgs &a, int lo, int hi, ResolveTally &t) {
+  if (a.events && !(collide_b(a.beh[lo]) && collide_b(a.beh[hi]))) {
+    // a subsume pair: ResolveSubsume (body.go:228-244) by the larger body, no existence check
+    const int b = a.r[lo] > a.r[hi] ? lo : hi, o = b == lo ? hi : lo;
+    a.m[b] = a.m[b] + a.m[o];
+    const uint8_t fo = a.flags[o];
+    if ((fo & NB_F_EXISTS) && !(fo & NB_F_FRAGMENTING)) t.inactive++;
+    a.flags[o] = (uint8_t)(fo & ~NB_F_EXISTS);  // SetNotExists (body.go:93-96)
+    a.m[o] = 0.0;
+    t.subsumed++;
+    return;
+  }
+  int b, o;
+  if (!elastic_pair(a, lo, hi, &b, &o)) return;
+  resolve_elastic(a, b, o, elastic_geom(a, b, o), t);
 }
 
 __device__ static void add_tally(DevCounters *ctr, uint32_t found, const ResolveTally &t) {
@@ -561,137 +478,346 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
   add_tally(a.ctr, found, t);
 }
 
-// The same pass with pairs that share no body resolved together (events off).  A pair reads and
-// writes only its two bodies, and nothing in the pass changes which pairs act, so the state is
-// bit-identical to the one-by-one pass as long as every pair sees both its bodies exactly as the
-// pairs before it in canonical order left them.  The pairs touching one body b form a chain in
-// canonical order: the pairs (x, b), x ascending, then b's own pairs (b, y), y ascending.  A pair
-// therefore waits for at most two predecessors (the previous pair on each of its bodies) and
-// releases at most two successors.  The chains come from two sorted lists: the pair keys
-// (lo << 32 | hi) and the same keys swapped (hi << 32 | lo), where b's pairs (x, b) are one run.
-// Then one workgroup resolves the ready pairs round by round: pairs of one round share no body.
-__device__ __forceinline__ int64_t key_lower_bound(const uint64_t *k, int64_t n, uint64_t key) {
-  int64_t lo = 0, hi = n;
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) >> 1;
-    if (k[mid] < key) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
+// ---------------------------------------------------------------------------------------------
+// The pair list in canonical order, and the pairs' chains.
+//
+// The force phase leaves the pairs (lo << 32 | hi) in any order.  They are counted per body, twice:
+// as lo's (a body's own pairs) and as hi's (the pairs that reach it); prefix sums of the two counts
+// place each pair in its body's two lists, and its rank among the list's partners gives its place
+// in order.  Own lists one after another, partners ascending, are the canonical order.  A list is
+// as long as its body's pairs, so ranking costs a few reads per pair; nothing depends on the list's
+// capacity, only on the bodies and the pairs there are.
+//
+// With events off, pairs that share no body resolve together.  A pair reads and writes only its two
+// bodies, and nothing in the pass changes which pairs act, so the state is bit-identical to the
+// one-by-one pass as long as every pair sees both its bodies exactly as the pairs before it in
+// canonical order left them.  The pairs touching one body form a chain in canonical order: the
+// pairs (x, b) that reach it, x ascending, then its own pairs (b, y), y ascending.  A pair waits for
+// at most two predecessors (the previous pair on each of its bodies) and releases at most two
+// successors.  One workgroup resolves the ready pairs round by round.
+//
+// Up to kPairSmallN bodies one workgroup does all of it in one launch, the counts in LDS; above, or
+// when the last cycle had more than kPairSmallPairs pairs, the list takes five launches, the chains
+// and the rounds one each (one workgroup / seven launches, reference scene: 0.020 / 0.033 ms with 63
+// pairs, 0.045 / 0.057 with 1,074, 0.072 / 0.074 with 2,439, 0.184 / 0.114 with 6,998).
+// A sort of the keys, one of the swapped keys and binary searches took 11 to 23 launches.
+//
+// A round costs one coll3d of latency (FP64 transcendentals): the half of it that depends on
+// positions alone is evaluated beforehand for all pairs, and 512 threads leave it the registers it
+// needs.  List and rounds together, before and now: 0.103 -> 0.019 ms at n = 1,000 (63 pairs, 3
+// rounds), 0.63 -> 0.11 at 10,007 (6,998 pairs, 16 rounds), 1.30 -> 0.24 at 16,384 (18,696 pairs,
+// 40 rounds).
+// ---------------------------------------------------------------------------------------------
+constexpr int kPairSmallN = 16384;        // bodies whose two count arrays fit one workgroup's LDS
+constexpr int kPairThreads = 512;         // coll3d keeps its 140 VGPRs (1,024 threads would spill)
+constexpr int kPairLdsPend = 128 * 1024;  // pairs whose predecessor counts fit in LDS, one byte each
+
+__device__ __forceinline__ int64_t pair_total(const PairArgs &a) {
+  return min((int64_t)a.ctr->pair_count, a.cap);
 }
 
-// keys_sw[k] = the k-th pair key with its halves swapped (sorted afterwards).
-__global__ void k_pairs_swap(const uint64_t *keys, uint64_t *keys_sw, int64_t cap,
-                             const DevCounters *ctr) {
-  const int64_t cnt = min((int64_t)ctr->pair_count, cap);
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < cnt;
-       k += (int64_t)gridDim.x * blockDim.x) {
-    const uint64_t v = keys[k];
-    keys_sw[k] = (v << 32) | (v >> 32);
+// A pair's place in its two bodies' lists, in arrival order.
+template <class P>
+__device__ __forceinline__ void pair_count(const PairArgs &a, int64_t cnt, P own, P reach,
+                                           int64_t k0, int64_t step) {
+  for (int64_t k = k0; k < cnt; k += step) {
+    const uint64_t key = a.raw[k];
+    a.slot_own[k] = atomicAdd(&own[(int)(key >> 32)], 1);
+    a.slot_reach[k] = atomicAdd(&reach[(int)(key & 0xffffffffu)], 1);
   }
 }
 
-// For each pair: its successor on each of its two bodies (-1: none) and how many predecessors it
-// waits for.  keys: sorted pair keys; sw: sorted swapped keys.
-__global__ void k_pair_dag(const uint64_t *keys, const uint64_t *sw, int64_t cap,
-                           const DevCounters *ctr, int32_t *succ, int32_t *pending) {
-  const int64_t cnt = min((int64_t)ctr->pair_count, cap);
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < cnt;
-       k += (int64_t)gridDim.x * blockDim.x) {
-    const uint64_t key = keys[k];
-    const uint32_t lo = (uint32_t)(key >> 32), hi = (uint32_t)key;
-    int npred = 0;
-    // chain of lo: k lies in lo's own run (lo, y)
-    int32_t s_lo = -1;
-    if (k + 1 < cnt && (uint32_t)(keys[k + 1] >> 32) == lo) s_lo = (int32_t)(k + 1);
-    if (k > 0 && (uint32_t)(keys[k - 1] >> 32) == lo) {
-      npred++;
-    } else {  // the first of lo's own run: after the last pair (x, lo), if there is one
-      const int64_t e = key_lower_bound(sw, cnt, ((uint64_t)lo + 1) << 32) - 1;
-      if (e >= 0 && (uint32_t)(sw[e] >> 32) == lo) npred++;
+template <class P>
+__device__ __forceinline__ void pair_fill(const PairArgs &a, int64_t cnt, P own, P reach,
+                                          int64_t k0, int64_t step) {
+  for (int64_t k = k0; k < cnt; k += step) {
+    const uint64_t key = a.raw[k];
+    const int lo = (int)(key >> 32), hi = (int)(key & 0xffffffffu);
+    a.list_own[own[lo] + a.slot_own[k]] = hi;
+    a.list_reach[reach[hi] + a.slot_reach[k]] = lo;
+  }
+}
+
+// Ranks: the pair's canonical index, and the index by place in hi's list.
+template <class P>
+__device__ __forceinline__ void pair_rank(const PairArgs &a, int64_t cnt, P own, P reach,
+                                          int64_t k0, int64_t step) {
+  for (int64_t k = k0; k < cnt; k += step) {
+    const uint64_t key = a.raw[k];
+    const int lo = (int)(key >> 32), hi = (int)(key & 0xffffffffu);
+    const int u0 = own[lo], u1 = own[lo + 1], l0 = reach[hi], l1 = reach[hi + 1];
+    int p = u0, q = l0;
+    for (int e = u0; e < u1; e++) p += a.list_own[e] < hi ? 1 : 0;
+    for (int e = l0; e < l1; e++) q += a.list_reach[e] < lo ? 1 : 0;
+    a.keys[p] = key;
+    a.by_hi[q] = p;
+    a.place[p] = q;
+  }
+}
+
+// Chains, roles and positions' half of coll3d of the sorted pairs.
+template <class P>
+__device__ __forceinline__ void pair_link(const PairArgs &a, const ResolveArgs &r, int64_t cnt,
+                                          P own, P reach, int64_t k0, int64_t step) {
+  for (int64_t k = k0; k < cnt; k += step) {
+    const uint64_t key = a.keys[k];
+    const int lo = (int)(key >> 32), hi = (int)(key & 0xffffffffu);
+    const int q = a.place[k];
+    // lo's chain: its own pairs in order, after the pairs that reach it
+    int pend = (int)k > own[lo] || reach[lo + 1] > reach[lo] ? 1 : 0;
+    int2 succ;
+    succ.x = (int)k + 1 < own[lo + 1] ? (int)k + 1 : -1;
+    // hi's chain: the pairs that reach it in order, then its own
+    pend += q > reach[hi] ? 1 : 0;
+    succ.y = q + 1 < reach[hi + 1] ? a.by_hi[q + 1] : own[hi] < own[hi + 1] ? own[hi] : -1;
+    a.succ[k] = succ;
+    a.pend[k] = pend;
+    int b, o;
+    const bool acts = elastic_pair(r, lo, hi, &b, &o);
+    a.role[k] = acts ? make_int2(b, o) : make_int2(-1, -1);
+    if (acts && k < a.geom_cap) {
+      const ElasticGeom g = elastic_geom(r, b, o);
+      double *w = a.geom + k * 6;
+      w[0] = g.d;
+      w[1] = g.r12;
+      w[2] = g.st;
+      w[3] = g.ct;
+      w[4] = g.sp;
+      w[5] = g.cp;
     }
-    // chain of hi: k is the pair (lo, hi) among hi's pairs (x, hi), at position p of sw
-    const int64_t p = key_lower_bound(sw, cnt, ((uint64_t)hi << 32) | lo);
-    int32_t s_hi = -1;
-    if (p > 0 && (uint32_t)(sw[p - 1] >> 32) == hi) npred++;
-    if (p + 1 < cnt && (uint32_t)(sw[p + 1] >> 32) == hi) {
-      const uint64_t nk = ((uint64_t)(uint32_t)sw[p + 1] << 32) | hi;  // the pair (x', hi)
-      s_hi = (int32_t)key_lower_bound(keys, cnt, nk);
-    } else {  // the last pair (x, hi): next comes hi's own run (hi, y), if there is one
-      const int64_t f = key_lower_bound(keys, cnt, (uint64_t)hi << 32);
-      if (f < cnt && (uint32_t)(keys[f] >> 32) == hi) s_hi = (int32_t)f;
-    }
-    succ[2 * k] = s_lo;
-    succ[2 * k + 1] = s_hi;
-    pending[k] = npred;
   }
 }
 
-__device__ __forceinline__ void sync_all() {
-  __threadfence();
-  __syncthreads();
-}
-
-__global__ __launch_bounds__(1024) void k_resolve_dag(ResolveArgs a) {
-  __shared__ int s_len;
-  __shared__ unsigned long long s_res, s_frag;
+// The rounds, by one workgroup.  pend8: kPairLdsPend bytes of LDS (predecessor counts).
+__device__ static void pair_rounds(const PairArgs &a, const ResolveArgs &r, int cnt,
+                                   uint32_t *pend8, int *s_len, unsigned long long *s_tally) {
   const int tid = threadIdx.x, nt = blockDim.x;
-  const uint32_t found = a.ctr->pair_count;
-  const int cnt = (int)min((int64_t)found, a.pair_cap);
-  if (tid == 0) s_len = 0, s_res = 0, s_frag = 0;
+  const bool lds = cnt <= kPairLdsPend;
+  if (tid == 0) *s_len = 0, s_tally[0] = s_tally[1] = 0;
   __syncthreads();
-  int32_t *cur = a.list_a, *nxt = a.list_b;
-  for (int k = tid; k < cnt; k += nt)
-    if (a.pending[k] == 0) cur[atomicAdd(&s_len, 1)] = k;
-  sync_all();
-  int m = s_len;
+  int32_t *cur = a.list_own, *nxt = a.list_reach;  // (the lists have done their work)
+  for (int w = tid; w * 4 < cnt; w += nt) {
+    uint32_t v = 0;
+    for (int e = 0; e < 4 && w * 4 + e < cnt; e++) {
+      const int p = a.pend[w * 4 + e];
+      v |= (uint32_t)p << (8 * e);
+      if (p == 0) cur[atomicAdd(s_len, 1)] = w * 4 + e;
+    }
+    if (lds) pend8[w] = v;
+  }
+  __syncthreads();
+  int m = *s_len;
   ResolveTally t;
   while (m > 0) {
     __syncthreads();  // every thread has read s_len
-    if (tid == 0) s_len = 0;
+    if (tid == 0) *s_len = 0;
     __syncthreads();
     for (int q = tid; q < m; q += nt) {
       const int k = cur[q];
-      const uint64_t key = a.pairs[k];
-      resolve_pair(a, (int)(key >> 32), (int)(key & 0xffffffffu), t);
+      const int2 role = a.role[k], succ = a.succ[k];
+      if (role.x >= 0) {
+        ElasticGeom g;
+        if (k < a.geom_cap) {
+          const double *w = a.geom + (int64_t)k * 6;
+          g.d = w[0];
+          g.r12 = w[1];
+          g.st = w[2];
+          g.ct = w[3];
+          g.sp = w[4];
+          g.cp = w[5];
+        } else {
+          g = elastic_geom(r, role.x, role.y);
+        }
+        resolve_elastic(r, role.x, role.y, g, t);
+      }
+#pragma unroll
       for (int e = 0; e < 2; e++) {
-        const int sk = a.succ[2 * k + e];
-        if (sk >= 0 && atomicSub(&a.pending[sk], 1) == 1) nxt[atomicAdd(&s_len, 1)] = sk;
+        const int sk = e ? succ.y : succ.x;
+        if (sk < 0) continue;
+        bool ready;
+        if (lds) {
+          const int sh = 8 * (sk & 3);
+          ready = (atomicSub(&pend8[sk >> 2], 1u << sh) >> sh & 255u) == 1u;
+        } else {
+          ready = atomicSub(&a.pend[sk], 1) == 1;
+        }
+        if (ready) nxt[atomicAdd(s_len, 1)] = sk;
       }
     }
-    sync_all();
-    m = s_len;
+    __syncthreads();  // the workgroup's writes are seen by its next reads
+    m = *s_len;
     int32_t *sw = cur;
     cur = nxt;
     nxt = sw;
   }
-  atomicAdd(&s_res, (unsigned long long)t.resolved);
-  atomicAdd(&s_frag, (unsigned long long)t.fragreq);
+  atomicAdd(&s_tally[0], (unsigned long long)t.resolved);
+  atomicAdd(&s_tally[1], (unsigned long long)t.fragreq);
   __syncthreads();
   if (tid == 0) {
     ResolveTally all;
-    all.resolved = s_res;
-    all.fragreq = s_frag;
-    add_tally(a.ctr, found, all);
+    all.resolved = s_tally[0];
+    all.fragreq = s_tally[1];
+    add_tally(a.ctr, a.ctr->pair_count, all);
   }
 }
 
-hipError_t launch_resolve(const ResolveArgs &a, hipStream_t st) {
-  if (a.events || a.serial || !a.succ) {
-    hipLaunchKernelGGL(k_resolve, dim3(1), dim3(64), 0, st, a);
-    return hipGetLastError();
+// Exclusive prefix sums of each thread's pair of values over the workgroup; total gets the sums.
+__device__ static int2 block_scan2(int2 v, int2 *waves, int2 *total) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  int2 s = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int x = __shfl_up(s.x, d, 64), y = __shfl_up(s.y, d, 64);
+    if (lane >= d) s.x += x, s.y += y;
   }
-  // the chains: swapped keys, sorted; successors and predecessor counts; then the rounds
-  const unsigned g = (unsigned)std::min<int64_t>(4096, (a.pair_cap + 255) / 256);
-  hipLaunchKernelGGL(k_pairs_swap, dim3(g), dim3(256), 0, st, a.pairs, a.pairs_sw, a.pair_cap,
-                     a.ctr);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  e = launch_sort_pairs(a.pairs_sw, a.sort_tmp, a.pair_cap, a.ctr, st);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_pair_dag, dim3(g), dim3(256), 0, st, a.pairs, a.pairs_sw, a.pair_cap,
-                     a.ctr, a.succ, a.pending);
-  hipLaunchKernelGGL(k_resolve_dag, dim3(1), dim3(1024), 0, st, a);
+  if (lane == 63) waves[w] = s;
+  __syncthreads();
+  int2 base = make_int2(0, 0), all = make_int2(0, 0);
+  for (int q = 0; q < nw; q++) {
+    const int2 u = waves[q];
+    if (q < w) base.x += u.x, base.y += u.y;
+    all.x += u.x;
+    all.y += u.y;
+  }
+  __syncthreads();
+  *total = all;
+  return make_int2(base.x + s.x - v.x, base.y + s.y - v.y);
+}
+
+// One workgroup, one launch: list (mode 0), or list and rounds (mode 1).
+__global__ __launch_bounds__(kPairThreads) void k_pairs_small(PairArgs a, ResolveArgs r, int mode) {
+  __shared__ int counts[2 * (kPairSmallN + 1)];
+  __shared__ int2 waves[16];
+  __shared__ int s_len;
+  __shared__ unsigned long long s_tally[2];
+  static_assert(kPairLdsPend <= sizeof(counts), "the predecessor counts reuse the count arrays");
+  int *own = counts, *reach = counts + kPairSmallN + 1;
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const int cnt = (int)pair_total(a);
+  if (cnt == 0) {
+    if (mode == 1 && tid == 0) add_tally(a.ctr, 0, ResolveTally{});
+    return;
+  }
+  for (int i = tid; i <= a.n; i += nt) own[i] = reach[i] = 0;
+  __syncthreads();
+  pair_count(a, cnt, own, reach, tid, nt);
+  __syncthreads();
+  const int per = (a.n + nt - 1) / nt, i0 = min(tid * per, a.n), i1 = min(i0 + per, a.n);
+  int2 v = make_int2(0, 0), total;
+  for (int i = i0; i < i1; i++) v.x += own[i], v.y += reach[i];
+  int2 at = block_scan2(v, waves, &total);
+  for (int i = i0; i < i1; i++) {
+    const int x = own[i], y = reach[i];
+    own[i] = at.x;
+    reach[i] = at.y;
+    at.x += x;
+    at.y += y;
+  }
+  if (tid == 0) own[a.n] = total.x, reach[a.n] = total.y;
+  __syncthreads();
+  pair_fill(a, cnt, own, reach, tid, nt);
+  __syncthreads();
+  pair_rank(a, cnt, own, reach, tid, nt);
+  if (mode == 0) return;
+  __syncthreads();
+  pair_link(a, r, cnt, own, reach, tid, nt);
+  __syncthreads();
+  pair_rounds(a, r, cnt, reinterpret_cast<uint32_t *>(counts), &s_len, s_tally);
+}
+
+// The same over the whole chip.  The counts are zero between uses.
+__global__ __launch_bounds__(256) void k_pair_count(PairArgs a) {
+  pair_count(a, pair_total(a), a.own, a.reach, (int64_t)blockIdx.x * 256 + threadIdx.x,
+             (int64_t)gridDim.x * 256);
+}
+
+constexpr int kPairScan = 4096;  // bodies per workgroup of the prefix sums, four per thread
+__global__ __launch_bounds__(1024) void k_pair_sums(PairArgs a) {
+  __shared__ int2 waves[16];
+  if (pair_total(a) == 0) return;
+  const int i0 = blockIdx.x * kPairScan + (int)threadIdx.x * 4;
+  int2 v = make_int2(0, 0), total;
+  for (int e = 0; e < 4; e++)
+    if (i0 + e < a.n) v.x += a.own[i0 + e], v.y += a.reach[i0 + e];
+  block_scan2(v, waves, &total);
+  if (threadIdx.x == 0) a.bsum[blockIdx.x] = total;
+}
+
+__global__ __launch_bounds__(1024) void k_pair_offsets(PairArgs a) {
+  __shared__ int2 waves[16];
+  if (pair_total(a) == 0) return;
+  int2 before = make_int2(0, 0), base, total;
+  for (int q = threadIdx.x; q < (int)blockIdx.x; q += 1024)
+    before.x += a.bsum[q].x, before.y += a.bsum[q].y;
+  block_scan2(before, waves, &base);  // the sums of the workgroups before this one
+  const int i0 = blockIdx.x * kPairScan + (int)threadIdx.x * 4;
+  int2 c[4], v = make_int2(0, 0);
+  for (int e = 0; e < 4; e++) {
+    c[e] = i0 + e < a.n ? make_int2(a.own[i0 + e], a.reach[i0 + e]) : make_int2(0, 0);
+    v.x += c[e].x;
+    v.y += c[e].y;
+  }
+  int2 at = block_scan2(v, waves, &total);
+  at.x += base.x;
+  at.y += base.y;
+  for (int e = 0; e < 4; e++) {
+    if (i0 + e < a.n) {
+      a.own[i0 + e] = a.reach[i0 + e] = 0;  // as the next use expects them
+      a.own_off[i0 + e] = at.x;
+      a.reach_off[i0 + e] = at.y;
+    }
+    at.x += c[e].x;
+    at.y += c[e].y;
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+    a.own_off[a.n] = base.x + total.x;
+    a.reach_off[a.n] = base.y + total.y;
+  }
+}
+
+__global__ __launch_bounds__(256) void k_pair_fill(PairArgs a) {
+  pair_fill(a, pair_total(a), a.own_off, a.reach_off, (int64_t)blockIdx.x * 256 + threadIdx.x,
+            (int64_t)gridDim.x * 256);
+}
+__global__ __launch_bounds__(256) void k_pair_rank(PairArgs a) {
+  pair_rank(a, pair_total(a), a.own_off, a.reach_off, (int64_t)blockIdx.x * 256 + threadIdx.x,
+            (int64_t)gridDim.x * 256);
+}
+__global__ __launch_bounds__(256) void k_pair_link(PairArgs a, ResolveArgs r) {
+  pair_link(a, r, pair_total(a), a.own_off, a.reach_off,
+            (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256);
+}
+__global__ __launch_bounds__(kPairThreads) void k_pair_rounds(PairArgs a, ResolveArgs r) {
+  __shared__ uint32_t pend8[kPairLdsPend / 4];
+  __shared__ int s_len;
+  __shared__ unsigned long long s_tally[2];
+  const int cnt = (int)pair_total(a);
+  if (cnt == 0) {
+    if (threadIdx.x == 0) add_tally(a.ctr, 0, ResolveTally{});
+    return;
+  }
+  pair_rounds(a, r, cnt, pend8, &s_len, s_tally);
+}
+
+hipError_t launch_pairs(const PairArgs &a, const ResolveArgs *r, int64_t expect, hipStream_t st) {
+  const bool together = r && !r->events && !r->serial;
+  if (a.n <= kPairSmallN && expect <= kPairSmallPairs) {
+    hipLaunchKernelGGL(k_pairs_small, dim3(1), dim3(kPairThreads), 0, st, a, r ? *r : ResolveArgs{},
+                       together ? 1 : 0);
+  } else {
+    const unsigned g = (unsigned)std::min<int64_t>(1024, (a.cap + 255) / 256);
+    const unsigned gs = (unsigned)((a.n + kPairScan - 1) / kPairScan);
+    hipLaunchKernelGGL(k_pair_count, dim3(g), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_pair_sums, dim3(gs), dim3(1024), 0, st, a);
+    hipLaunchKernelGGL(k_pair_offsets, dim3(gs), dim3(1024), 0, st, a);
+    hipLaunchKernelGGL(k_pair_fill, dim3(g), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_pair_rank, dim3(g), dim3(256), 0, st, a);
+    if (together) {
+      hipLaunchKernelGGL(k_pair_link, dim3(g), dim3(256), 0, st, a, *r);
+      hipLaunchKernelGGL(k_pair_rounds, dim3(1), dim3(kPairThreads), 0, st, a, *r);
+    }
+  }
+  if (r && !together) hipLaunchKernelGGL(k_resolve, dim3(1), dim3(64), 0, st, *r);
   return hipGetLastError();
 }
 

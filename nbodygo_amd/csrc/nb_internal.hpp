@@ -15,7 +15,6 @@ namespace nb {
 constexpr int kPad = 1024;           // body arrays are padded to a multiple of this
 constexpr int kFlagSlots = 4;        // flagged tiles remembered per (slice, target)
 constexpr int kMaxSplit = 64;        // max source-range slices
-constexpr int kSortLdsKeys = 8192;   // pair keys sorted in LDS by one workgroup
 constexpr int64_t kLayerWords = (int64_t)1 << 28;  // floats of variant 3's workspace (1 GiB)
 constexpr float kSentinel = 1.0e18f; // position of padding / inactive sources in the FP32 stream
 
@@ -165,11 +164,13 @@ struct Ctx {
   int32_t *fcnt = nullptr, *flist = nullptr;
   int2 *recs = nullptr;
 
-  // collision pairs as 64-bit keys (i << 32 | j); the sort's merge buffer and the resolution's
-  // swapped keys (same size); the resolution's per-pair words: 5 int32 per pair (two successors,
-  // a predecessor count, two frontier lists)
-  uint64_t *pairs = nullptr, *pairs_tmp = nullptr, *pairs_sw = nullptr;
-  int32_t *res_words = nullptr;
+  // collision pairs as 64-bit keys (i << 32 | j), as found and in canonical order; the words of
+  // the pair list's chains per pair and per body
+  uint64_t *pairs = nullptr, *pairs_sorted = nullptr;
+  int32_t *pair_words = nullptr, *pair_body = nullptr;
+  double *pair_geom = nullptr;
+  int64_t pair_body_cap = 0;
+  int64_t pairs_seen = 0;  // pairs of the last cycle read back (chooses the list's launches)
   int64_t pair_cap = 0;
   int64_t pair_cap_pow2 = 0;
 
@@ -355,10 +356,6 @@ struct Accel64Args {
 };
 hipError_t launch_accel_f64(const Accel64Args &a, hipStream_t st);
 
-hipError_t launch_sort_pairs(uint64_t *keys, uint64_t *tmp, int64_t cap, const DevCounters *ctr,
-                             hipStream_t st);
-int sort_pairs(Ctx *c);  // the context's pair list into canonical order
-
 struct ResolveArgs {
   double *x, *y, *z, *vx, *vy, *vz, *m, *r, *rest, *frag;
   int32_t *beh;
@@ -372,14 +369,29 @@ struct ResolveArgs {
   FragState *fst;
   const double *acc;  // this cycle's force slices, kept by a body that starts fragmenting
   int split, npad;
-  // events off: pairs that share no body resolve together.  pairs_sw / sort_tmp: pair_cap keys
-  // each (the swapped keys and the sort's merge buffer); succ: 2 per pair; pending, list_a,
-  // list_b: 1 per pair.  serial = one lane in canonical order.
-  uint64_t *pairs_sw, *sort_tmp;
-  int32_t *succ, *pending, *list_a, *list_b;
-  int serial;
+  int serial;  // one pair at a time on one lane
 };
-hipError_t launch_resolve(const ResolveArgs &a, hipStream_t st);
+
+// The pair list in canonical order and the pairs' chains (nb_cycle.hip).
+struct PairArgs {
+  const uint64_t *raw;  // pairs as the force phase found them
+  uint64_t *keys;       // the same in canonical order
+  int64_t cap;
+  int n;
+  DevCounters *ctr;
+  int32_t *own, *reach;          // per body: pairs as the lower, as the higher index (zero at rest)
+  int32_t *own_off, *reach_off;  // their prefix sums, n + 1 each
+  int2 *bsum;
+  // per pair
+  int32_t *slot_own, *slot_reach, *list_own, *list_reach, *by_hi, *place, *pend;
+  int2 *succ, *role;
+  double *geom;  // 6 words for the first geom_cap pairs
+  int64_t geom_cap;
+};
+constexpr int64_t kPairSmallPairs = 2500;  // pairs up to which one workgroup does the whole pass
+constexpr int64_t kPairGeom = 1 << 18;     // pairs whose positions' half of coll3d is kept
+// r: resolve too.  expect: about how many pairs there are (chooses the launches, not the result).
+hipError_t launch_pairs(const PairArgs &a, const ResolveArgs *r, int64_t expect, hipStream_t st);
 
 struct UpdateArgs {
   double *x, *y, *z, *vx, *vy, *vz;

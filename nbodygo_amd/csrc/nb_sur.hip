@@ -1536,10 +1536,6 @@ int sur_force_phase(Ctx *c, bool timed, int ev_slot) {
     NB_HIP(c, hipGetLastError());
     s->checks++;
   }
-  if (detect) {
-    const int rcs = sort_pairs(c);
-    if (rcs) return rcs;
-  }
   s->steps++;
   return NB_OK;
 }
