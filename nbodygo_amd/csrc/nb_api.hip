@@ -462,6 +462,7 @@ int nb_create(const nb_params *p, nb_ctx **out) {
     delete c;
     return NB_E_HIP;
   }
+  stage_user(1);
   *out = c;
   return NB_OK;
 }
@@ -483,6 +484,7 @@ void nb_destroy(nb_ctx *c) {
   for (hipEvent_t e : c->ev_res) (void)hipEventDestroy(e);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
+  stage_user(-1);
 }
 
 int nb_load(nb_ctx *c, int64_t n, const double *x, const double *y, const double *z,
@@ -495,6 +497,7 @@ int nb_load(nb_ctx *c, int64_t n, const double *x, const double *y, const double
   if (n > 0 && (!x || !y || !z || !vx || !vy || !vz || !m || !r || !beh || !flags))
     return fail(c, NB_E_INVALID, "nb_load: NULL array");
   NB_HIP(c, hipSetDevice(c->device));
+  c->ctr_last_ok = false;
   const int64_t npad = std::max<int64_t>(round_up(n, kPad), kPad);
   if (npad > c->cap) {
     free_all(c);
@@ -578,9 +581,9 @@ int nb_step(nb_ctx *c, double dt, double R, int32_t nsteps, nb_stats *out) {
     return fail(c, NB_E_INVALID, "nb_step: dt and R must be finite");
   NB_HIP(c, hipSetDevice(c->device));
   auto t0 = std::chrono::steady_clock::now();
-  DevCounters before;
-  NB_HIP(c, hipMemcpyAsync(&before, c->ctr, sizeof before, hipMemcpyDeviceToHost, c->stream));
-  NB_HIP(c, hipStreamSynchronize(c->stream));
+  DevCounters before = c->ctr_last;
+  if (!c->ctr_last_ok) NB_HIP(c, stage_counters(c->ctr, c->stream, &before));
+  c->ctr_last_ok = false;
   const bool timed = c->timing && nsteps > 0 && c->n > 0;
   if (timed) {
     while ((int)c->ev.size() < 2 * nsteps) {
@@ -647,8 +650,9 @@ int nb_step(nb_ctx *c, double dt, double R, int32_t nsteps, nb_stats *out) {
     NB_HIP(c, launch_update(u, c->stream));
   }
   DevCounters after;
-  NB_HIP(c, hipMemcpyAsync(&after, c->ctr, sizeof after, hipMemcpyDeviceToHost, c->stream));
-  NB_HIP(c, hipStreamSynchronize(c->stream));
+  NB_HIP(c, stage_counters(c->ctr, c->stream, &after));
+  c->ctr_last = after;
+  c->ctr_last_ok = true;
   auto t1 = std::chrono::steady_clock::now();
   double force_ms = 0, resolve_ms = 0;
   if (timed) {
@@ -697,6 +701,7 @@ int nb_compute_forces(nb_ctx *c, double *fx, double *fy, double *fz) {
   if (c->n && (!fx || !fy || !fz)) return fail(c, NB_E_INVALID, "nb_compute_forces: NULL output");
   if (c->n == 0) return NB_OK;
   NB_HIP(c, hipSetDevice(c->device));
+  c->ctr_last_ok = false;
   int rc = force_phase(c, false, 0);
   if (rc) return rc;
   if (c->p.collisions)
@@ -705,12 +710,10 @@ int nb_compute_forces(nb_ctx *c, double *fx, double *fy, double *fz) {
   NB_HIP(c, launch_combine_force(c->acc, split_now(c), (int)c->npad, (int)c->n, c->m, c->p.G,
                                  c->p.precision == NB_PREC_FP64 ? 1 : 0, tmp, c->stream));
   const size_t db = (size_t)c->n * sizeof(double);
-  NB_HIP(c, hipMemcpyAsync(fx, tmp, db, hipMemcpyDeviceToHost, c->stream));
-  NB_HIP(c, hipMemcpyAsync(fy, tmp + c->n, db, hipMemcpyDeviceToHost, c->stream));
-  NB_HIP(c, hipMemcpyAsync(fz, tmp + 2 * c->n, db, hipMemcpyDeviceToHost, c->stream));
-  NB_HIP(c, hipStreamSynchronize(c->stream));
+  const Fetch seg[3] = {{fx, tmp, db}, {fy, tmp + c->n, db}, {fz, tmp + 2 * c->n, db}};
+  NB_HIP(c, stage_fetch(seg, 3, c->stream));
   DevCounters ctr;
-  NB_HIP(c, hipMemcpy(&ctr, c->ctr, sizeof ctr, hipMemcpyDeviceToHost));
+  NB_HIP(c, stage_counters(c->ctr, c->stream, &ctr));
   c->pairs_seen = ctr.pair_count;
   if (ctr.pair_overflow)
     return fail(c, NB_E_PAIR_OVERFLOW, "collision pairs exceeded pair_capacity");
@@ -786,10 +789,12 @@ int nb_store(nb_ctx *c, double *x, double *y, double *z, double *vx, double *vy,
   const size_t db = (size_t)c->n * sizeof(double);
   double *dst[7] = {x, y, z, vx, vy, vz, rest};
   const double *src[7] = {c->x, c->y, c->z, c->vx, c->vy, c->vz, c->rest};
+  Fetch seg[8];
+  int n = 0;
   for (int k = 0; k < 7; k++)
-    if (dst[k]) NB_HIP(c, hipMemcpyAsync(dst[k], src[k], db, hipMemcpyDeviceToHost, c->stream));
-  if (flags) NB_HIP(c, hipMemcpyAsync(flags, c->flags, (size_t)c->n, hipMemcpyDeviceToHost, c->stream));
-  NB_HIP(c, hipStreamSynchronize(c->stream));
+    if (dst[k]) seg[n++] = {dst[k], src[k], db};
+  if (flags) seg[n++] = {flags, c->flags, (size_t)c->n};
+  NB_HIP(c, stage_fetch(seg, n, c->stream));
   return NB_OK;
 }
 
@@ -803,19 +808,19 @@ int nb_store_bodies(nb_ctx *c, double *x, double *y, double *z, double *vx, doub
   const size_t db = (size_t)c->n * sizeof(double);
   double *dst[10] = {x, y, z, vx, vy, vz, m, r, rest, frag};
   const double *src[10] = {c->x, c->y, c->z, c->vx, c->vy, c->vz, c->m, c->r, c->rest, c->frag};
+  Fetch seg[13];
+  int n = 0;
   for (int k = 0; k < 10; k++)
-    if (dst[k]) NB_HIP(c, hipMemcpyAsync(dst[k], src[k], db, hipMemcpyDeviceToHost, c->stream));
-  if (beh)
-    NB_HIP(c, hipMemcpyAsync(beh, c->beh, (size_t)c->n * sizeof(int32_t), hipMemcpyDeviceToHost,
-                             c->stream));
-  if (flags) NB_HIP(c, hipMemcpyAsync(flags, c->flags, (size_t)c->n, hipMemcpyDeviceToHost, c->stream));
+    if (dst[k]) seg[n++] = {dst[k], src[k], db};
+  if (beh) seg[n++] = {beh, c->beh, (size_t)c->n * sizeof(int32_t)};
+  if (flags) seg[n++] = {flags, c->flags, (size_t)c->n};
   if (frag_step) {
     if (c->fstep)
-      NB_HIP(c, hipMemcpyAsync(frag_step, c->fstep, db, hipMemcpyDeviceToHost, c->stream));
+      seg[n++] = {frag_step, c->fstep, db};
     else
       memset(frag_step, 0, db);
   }
-  NB_HIP(c, hipStreamSynchronize(c->stream));
+  NB_HIP(c, stage_fetch(seg, n, c->stream));
   return NB_OK;
 }
 
@@ -825,16 +830,11 @@ int nb_store_render(nb_ctx *c, float *xyz, uint8_t *exists) {
   if (c->n == 0) return NB_OK;
   if (!xyz) return fail(c, NB_E_INVALID, "nb_store_render: NULL xyz");
   NB_HIP(c, hipSetDevice(c->device));
-  float *tmp = reinterpret_cast<float *>(c->diag);  // 3 n floats of the context's scratch
-  NB_HIP(c, launch_render(c->x, c->y, c->z, c->flags, (int)c->n, tmp, c->stream));
-  NB_HIP(c, hipMemcpyAsync(xyz, tmp, (size_t)3 * c->n * sizeof(float), hipMemcpyDeviceToHost,
-                           c->stream));
-  NB_HIP(c, hipStreamSynchronize(c->stream));
-  if (exists) {
-    std::vector<uint8_t> f((size_t)c->n);
-    NB_HIP(c, hipMemcpy(f.data(), c->flags, (size_t)c->n, hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < c->n; i++) exists[i] = (f[(size_t)i] & NB_F_EXISTS) ? 1 : 0;
-  }
+  float *tmp = reinterpret_cast<float *>(c->diag);  // 3 n floats and n bytes of the scratch
+  uint8_t *ex = reinterpret_cast<uint8_t *>(tmp + 3 * c->cap);
+  NB_HIP(c, launch_render(c->x, c->y, c->z, c->flags, (int)c->n, tmp, ex, c->stream));
+  const Fetch seg[2] = {{xyz, tmp, (size_t)3 * c->n * sizeof(float)}, {exists, ex, (size_t)c->n}};
+  NB_HIP(c, stage_fetch(seg, exists ? 2 : 1, c->stream));
   return NB_OK;
 }
 
@@ -882,6 +882,7 @@ int nb_autotune(nb_ctx *c, int32_t reps, int32_t *cfg) {
   }
   if (reps < 1) reps = 1;
   NB_HIP(c, hipSetDevice(c->device));
+  c->ctr_last_ok = false;
   const ForceShape keep = c->shape;
   const int64_t npad = c->npad;
   std::vector<ForceShape> cand;
@@ -1000,6 +1001,7 @@ int nb_cycle(nb_ctx *c, double R, int64_t *n_out) {
   if (!c->loaded) return fail(c, NB_E_STATE, "nb_cycle: no bodies loaded");
   if (!std::isfinite(R)) return fail(c, NB_E_INVALID, "nb_cycle: R must be finite");
   NB_HIP(c, hipSetDevice(c->device));
+  c->ctr_last_ok = false;
   hipStream_t st = c->stream;
   const int64_t n = c->n, nadd = c->adds.count();
   int64_t nk = 0;

@@ -242,6 +242,34 @@ __global__ void k_batch_reset(BatchQueue *q) {
   if (threadIdx.x == 0) q->next = 0;
 }
 
+// The caller's body order (simulations back to back) from the padded one: each output word's
+// simulation by binary search in its offset, one array per grid.y.
+struct BatchUnpadArgs {
+  const double *src[6];
+  const uint8_t *flags;
+  double *out;       // [6][n]
+  uint8_t *out_flags;
+  const int64_t *off, *poff;  // nsims + 1 each
+  int nsims;
+  int64_t n;
+};
+__global__ __launch_bounds__(256) void k_batch_unpad(BatchUnpadArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= a.n) return;
+  int lo = 0, hi = a.nsims;  // off[lo] <= i < off[hi]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (a.off[mid] <= i) lo = mid;
+    else hi = mid;
+  }
+  const int64_t p = a.poff[lo] + (i - a.off[lo]);
+  const int c = blockIdx.y;
+  if (c < 6)
+    a.out[(int64_t)c * a.n + i] = a.src[c][p];
+  else
+    a.out_flags[i] = a.flags[p];
+}
+
 }  // namespace nb
 
 // ---------------------------------------------------------------------------------------------
@@ -263,6 +291,9 @@ struct nb_batch {
   uint8_t *flags = nullptr, *collided = nullptr;
   float4 *js = nullptr;
   DevCounters *ctr = nullptr;
+  int64_t *sim_off = nullptr;  // off and poff on the device
+  double *unpad = nullptr;     // [6][bodies] and the flags in the caller's order
+  DevCounters ctr_last{};      // as the last step (or the load) left them
   BatchItem *items = nullptr;
   BatchQueue *queue = nullptr;
   int nitems = 0;
@@ -312,7 +343,8 @@ void drop_graph(nb_batch *b) {
 void free_batch(nb_batch *b) {
   drop_graph(b);
   void *ptrs[] = {b->x, b->y, b->z, b->vx, b->vy, b->vz, b->m, b->rest, b->acc,
-                  b->flags, b->collided, b->js, b->ctr, b->items, b->queue};
+                  b->flags, b->collided, b->js, b->ctr, b->items, b->queue,
+                  b->sim_off, b->unpad};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   b->x = b->y = b->z = b->vx = b->vy = b->vz = b->m = b->rest = b->acc = nullptr;
@@ -321,6 +353,8 @@ void free_batch(nb_batch *b) {
   b->ctr = nullptr;
   b->items = nullptr;
   b->queue = nullptr;
+  b->sim_off = nullptr;
+  b->unpad = nullptr;
 }
 
 // Build the item list (longest first) with the per-bucket IPL and tile.
@@ -453,6 +487,7 @@ int nb_batch_create(const nb_params *p, nb_batch **out) {
     return NB_E_HIP;
   }
   b->cus = prop.multiProcessorCount;
+  stage_user(1);
   *out = b;
   return NB_OK;
 }
@@ -464,6 +499,7 @@ void nb_batch_destroy(nb_batch *b) {
   free_batch(b);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
+  stage_user(-1);
 }
 
 const char *nb_batch_last_error(const nb_batch *b) { return b ? b->err.c_str() : "NULL batch"; }
@@ -525,7 +561,14 @@ int nb_batch_load(nb_batch *b, int32_t nsims, const int64_t *offsets, const doub
   NB_BHIP(b, hipMemsetAsync(b->acc, 0, (size_t)3 * n * sizeof(double), b->stream));
   // worst case item count: one item per 64 targets
   NB_BHIP(b, hipMalloc((void **)&b->items, (size_t)(n / 64 + nsims + 1) * sizeof(BatchItem)));
+  NB_BHIP(b, hipMalloc((void **)&b->sim_off, (size_t)2 * (nsims + 1) * sizeof(int64_t)));
+  NB_BHIP(b, hipMemcpyAsync(b->sim_off, b->off.data(), (size_t)(nsims + 1) * sizeof(int64_t),
+                            hipMemcpyHostToDevice, b->stream));
+  NB_BHIP(b, hipMemcpyAsync(b->sim_off + nsims + 1, b->poff.data(),
+                            (size_t)(nsims + 1) * sizeof(int64_t), hipMemcpyHostToDevice,
+                            b->stream));
   NB_BHIP(b, launch_zero_counters(b->ctr, 1, b->stream));
+  b->ctr_last = DevCounters{};
   NB_BHIP(b, launch_write_stream(b->x, b->y, b->z, b->m, b->flags, b->js, (int)n, (int)n,
                                  b->stream));
   return build_items(b, -1, 0);
@@ -545,8 +588,8 @@ int nb_batch_step(nb_batch *b, double dt, double R, int32_t nsteps, nb_stats *ou
     return bfail(b, NB_E_INVALID, "nb_batch_step: bad arguments");
   NB_BHIP(b, hipSetDevice(b->device));
   auto t0 = std::chrono::steady_clock::now();
-  DevCounters before, after;
-  NB_BHIP(b, hipMemcpyAsync(&before, b->ctr, sizeof before, hipMemcpyDeviceToHost, b->stream));
+  const DevCounters before = b->ctr_last;
+  DevCounters after;
   if (nsteps > 0) {
     if (b->use_graph) {
       if (!b->exec || b->graph_steps != nsteps || b->graph_dt != dt || b->graph_R != R) {
@@ -569,8 +612,8 @@ int nb_batch_step(nb_batch *b, double dt, double R, int32_t nsteps, nb_stats *ou
       for (int s = 0; s < nsteps; s++) NB_BHIP(b, enqueue_cycle(b, dt, R));
     }
   }
-  NB_BHIP(b, hipMemcpyAsync(&after, b->ctr, sizeof after, hipMemcpyDeviceToHost, b->stream));
-  NB_BHIP(b, hipStreamSynchronize(b->stream));
+  NB_BHIP(b, stage_counters(b->ctr, b->stream, &after));
+  b->ctr_last = after;
   auto t1 = std::chrono::steady_clock::now();
   const int64_t removed = (int64_t)(after.removed_total - before.removed_total);
   if (out) {
@@ -619,24 +662,29 @@ int nb_batch_store(nb_batch *b, double *x, double *y, double *z, double *vx, dou
   if (!b) return NB_E_INVALID;
   if (!b->items) return bfail(b, NB_E_STATE, "nb_batch_store: nothing loaded");
   NB_BHIP(b, hipSetDevice(b->device));
-  const int64_t n = b->n;
-  double *dst[6] = {x, y, z, vx, vy, vz};
+  const int64_t n = b->off[b->nsims];
+  if (n == 0) return NB_OK;
+  if (!b->unpad) NB_BHIP(b, hipMalloc((void **)&b->unpad, (size_t)n * (6 * sizeof(double) + 1)));
+  BatchUnpadArgs u;
   const double *src[6] = {b->x, b->y, b->z, b->vx, b->vy, b->vz};
-  std::vector<double> h((size_t)n);
-  for (int c = 0; c < 6; c++) {
-    if (!dst[c]) continue;
-    NB_BHIP(b, hipMemcpy(h.data(), src[c], (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
-    for (int k = 0; k < b->nsims; k++)
-      for (int64_t q = 0; q < b->off[k + 1] - b->off[k]; q++)
-        dst[c][b->off[k] + q] = h[(size_t)(b->poff[k] + q)];
-  }
-  if (flags) {
-    std::vector<uint8_t> hf((size_t)n);
-    NB_BHIP(b, hipMemcpy(hf.data(), b->flags, (size_t)n, hipMemcpyDeviceToHost));
-    for (int k = 0; k < b->nsims; k++)
-      for (int64_t q = 0; q < b->off[k + 1] - b->off[k]; q++)
-        flags[b->off[k] + q] = hf[(size_t)(b->poff[k] + q)];
-  }
+  for (int c = 0; c < 6; c++) u.src[c] = src[c];
+  u.flags = b->flags;
+  u.out = b->unpad;
+  u.out_flags = reinterpret_cast<uint8_t *>(b->unpad + 6 * n);
+  u.off = b->sim_off;
+  u.poff = b->sim_off + b->nsims + 1;
+  u.nsims = b->nsims;
+  u.n = n;
+  hipLaunchKernelGGL(k_batch_unpad, dim3((unsigned)((n + 255) / 256), 7), dim3(256), 0, b->stream,
+                     u);
+  NB_BHIP(b, hipGetLastError());
+  double *dst[6] = {x, y, z, vx, vy, vz};
+  Fetch seg[7];
+  int k = 0;
+  for (int c = 0; c < 6; c++)
+    if (dst[c]) seg[k++] = {dst[c], u.out + (int64_t)c * n, (size_t)n * sizeof(double)};
+  if (flags) seg[k++] = {flags, u.out_flags, (size_t)n};
+  NB_BHIP(b, stage_fetch(seg, k, b->stream));
   return NB_OK;
 }
 

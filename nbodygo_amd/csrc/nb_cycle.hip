@@ -1079,21 +1079,22 @@ hipError_t launch_diag(const double *x, const double *y, const double *z, const 
 }
 
 __global__ void k_render(const double *x, const double *y, const double *z, const uint8_t *flags,
-                         int n, float *xyz) {
+                         int n, float *xyz, uint8_t *exists) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const bool e = flags[i] & NB_F_EXISTS;
   // NewRenderable (renderable.go:22-40): float32 positions; zero for a non-existent body.
+  exists[i] = e ? 1 : 0;
   xyz[3 * (size_t)i] = e ? (float)x[i] : 0.f;
   xyz[3 * (size_t)i + 1] = e ? (float)y[i] : 0.f;
   xyz[3 * (size_t)i + 2] = e ? (float)z[i] : 0.f;
 }
 
 hipError_t launch_render(const double *x, const double *y, const double *z, const uint8_t *flags,
-                         int n, float *xyz, hipStream_t st) {
+                         int n, float *xyz, uint8_t *exists, hipStream_t st) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_render, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, y, z,
-                     flags, n, xyz);
+                     flags, n, xyz, exists);
   return hipGetLastError();
 }
 

@@ -129,6 +129,17 @@ struct ForceShape {
   int variant = 1;  // 1 = scalar-cache j stream, 2 = LDS-staged tiles, 3 = each pair once
 };
 
+// Device arrays into caller memory (nb_stage.hip), on the current device.  Both wait for the stream.
+constexpr int kFetchMax = 16;
+struct Fetch {
+  void *dst;
+  const void *src;
+  size_t bytes;
+};
+hipError_t stage_fetch(const Fetch *seg, int n, hipStream_t st);
+hipError_t stage_counters(const DevCounters *c, hipStream_t st, DevCounters *out);
+void stage_user(int add);  // +1 with a context or batch, -1 with its end
+
 struct Ctx {
   nb_params p{};
   int device = 0;
@@ -175,6 +186,9 @@ struct Ctx {
   int64_t pair_cap_pow2 = 0;
 
   DevCounters *ctr = nullptr;
+  // the counters as the last nb_step left them, while nothing else has counted since
+  DevCounters ctr_last{};
+  bool ctr_last_ok = false;
   // scratch of cap * 8 + 64 doubles: the diagnostics' reduction, and the staging area of
   // nb_compute_forces, nb_store_render and nb_accel_fp64 (each call completes before it returns)
   double *diag = nullptr;
@@ -421,7 +435,7 @@ hipError_t launch_diag(const double *x, const double *y, const double *z, const 
                        int n, double G, double eps, double *scratch, int64_t scratch_len,
                        hipStream_t st);
 hipError_t launch_render(const double *x, const double *y, const double *z, const uint8_t *flags,
-                         int n, float *xyz, hipStream_t st);
+                         int n, float *xyz, uint8_t *exists, hipStream_t st);
 
 // collection lifecycle
 struct CompactArgs {

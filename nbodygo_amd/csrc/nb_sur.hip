@@ -1812,6 +1812,7 @@ int nb_sur_error(nb_ctx *c, int32_t samples, int32_t use_mlp, double *err) {
   if (samples < 1 || samples > 65536) return fail_msg(c, NB_E_INVALID, "bad sample count");
   Sur *s = c->sur;
   NB_HIP(c, hipSetDevice(c->device));
+  c->ctr_last_ok = false;
   NB_HIP(c, launch_zero_counters(c->ctr, 0, c->stream));
   const bool mlp = use_mlp && s->trained;
   int rc = sur_pipeline(c, false, mlp, true, mlp);

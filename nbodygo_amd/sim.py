@@ -5,6 +5,7 @@ Exists/fragmenting/IsSun/Pinned, Body.r and FragFactor; cmd/body/body.go:34-52).
 one nb_ctx and exposes the entry points of include/nbody_gpu.h with numpy arrays.
 """
 import ctypes as C
+from concurrent.futures import ThreadPoolExecutor
 from dataclasses import dataclass, field
 
 import numpy as np
@@ -381,10 +382,23 @@ class NBodyBatch:
         return f.T.copy()
 
     def store(self):
-        b = self._all.copy()
-        self._check(lib.nb_batch_store(self._b, _dp(b.x), _dp(b.y), _dp(b.z), _dp(b.vx),
-                                       _dp(b.vy), _dp(b.vz), b.flags.ctypes.data_as(L._u8p)))
-        return b
+        a, n = self._all, self.n
+        f = [np.empty(n, np.float64) for _ in range(6)]
+        flags = np.empty(n, np.uint8)
+        kept = (a.m, a.r, a.beh, a.rest, a.frag, a.fstep)
+        # what the device does not change is copied beside the read-back once that takes longer
+        # than the threads' start (both leave the interpreter lock): 12.7 -> 5 ms for 2.2 million
+        # bodies
+        pool = ThreadPoolExecutor(4) if n > 200000 else None
+        if pool:
+            copies = [pool.submit(np.copy, v) for v in kept]
+        rc = lib.nb_batch_store(self._b, *(_dp(v) for v in f), flags.ctypes.data_as(L._u8p))
+        m, r, beh, rest, frag, fstep = ([c.result() for c in copies] if pool
+                                        else [v.copy() for v in kept])
+        if pool:
+            pool.shutdown()
+        self._check(rc)
+        return Bodies(*f, m, r, beh, flags, rest, frag, fstep)
 
     def shapes(self):
         s = (C.c_int32 * 3)()
