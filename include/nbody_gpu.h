@@ -340,6 +340,9 @@ int nb_batch_store(nb_batch *b, double *x, double *y, double *z, double *vx, dou
  * then times full launches of those per-bucket winners together and of every single (IPL,
  * tile) for all buckets, and keeps the fastest full launch; ipl3 (may be NULL) receives the
  * per-bucket IPL.
+ * Until a shape is set the launch takes each unordered pair once, whatever the shape words say
+ * (simulations of up to 32,768 bodies); nb_batch_set_shapes and nb_batch_set_tuning select the
+ * kernel above, and nb_batch_autotune whichever is faster.
  * Tuning words: cfg7 = {waves, ipl0, tile0, ipl1, tile1, ipl2, tile2}. */
 int nb_batch_get_shapes(nb_batch *b, int32_t *ipl3);
 int nb_batch_set_shapes(nb_batch *b, const int32_t *ipl3);

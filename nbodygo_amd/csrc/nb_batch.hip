@@ -17,6 +17,9 @@
 // nb_batch_autotune.  When every item has the same (IPL, tile) the launch uses the kernel
 // specialised to that shape, whose registers and LDS are sized for it alone.
 //
+// That is the kernel for a shape that the caller sets, and for simulations above 32,768 bodies;
+// otherwise the launch is nb_sym.hip's, which takes each unordered pair once.
+//
 // One nb_batch_step call runs nsteps cycles as one hipGraph launch: per cycle a fill kernel resets
 // the queue (no memset nodes), then the force kernel, then the update kernel.
 #include <algorithm>
@@ -38,6 +41,8 @@ constexpr int kSimPad = 64;
 constexpr int kBatchMaxTargets = 256; // 64 lanes * IPL (IPL <= 4)
 constexpr int kBuckets = 3;           // size buckets for shape selection
 constexpr int kBatchMaxTile = 256;    // sources per Kahan tile (64, 128 or 256)
+constexpr int kSymSlices = 8;         // ranges a block's tile list is cut into, at most
+constexpr int kSymTiles = 10;         // tiles per range aimed at
 
 struct BatchItem {
   int32_t t0;     // first target (global index)
@@ -297,6 +302,15 @@ struct nb_batch {
   BatchItem *items = nullptr;
   BatchQueue *queue = nullptr;
   int nitems = 0;
+  // each unordered pair once (nb_sym.hip): used until a shape is set, and if the tuner prefers it
+  bool once = true;
+  bool once_fits = false;  // the loaded simulations are within its sizes
+  BatchSymItem *sym_items = nullptr;
+  BatchSymSim *sym_sims = nullptr;
+  int32_t *tile_sim = nullptr;
+  double *sym_acc = nullptr;
+  float *sym_layer = nullptr;
+  int sym_nitems = 0;
   int bucket_ipl[kBuckets] = {2, 4, 4};
   int bucket_tile[kBuckets] = {64, 64, 64};
   int waves = 4;  // waves per work item (1, 2 or 4)
@@ -344,7 +358,8 @@ void free_batch(nb_batch *b) {
   drop_graph(b);
   void *ptrs[] = {b->x, b->y, b->z, b->vx, b->vy, b->vz, b->m, b->rest, b->acc,
                   b->flags, b->collided, b->js, b->ctr, b->items, b->queue,
-                  b->sim_off, b->unpad};
+                  b->sim_off, b->unpad, b->sym_items, b->sym_sims, b->tile_sim, b->sym_acc,
+                  b->sym_layer};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   b->x = b->y = b->z = b->vx = b->vy = b->vz = b->m = b->rest = b->acc = nullptr;
@@ -355,6 +370,13 @@ void free_batch(nb_batch *b) {
   b->queue = nullptr;
   b->sim_off = nullptr;
   b->unpad = nullptr;
+  b->sym_items = nullptr;
+  b->sym_sims = nullptr;
+  b->tile_sim = nullptr;
+  b->sym_acc = nullptr;
+  b->sym_layer = nullptr;
+  b->sym_nitems = 0;
+  b->once_fits = false;
 }
 
 // Build the item list (longest first) with the per-bucket IPL and tile.
@@ -399,6 +421,97 @@ int build_items(nb_batch *b, int only_bucket, int force_ipl, int force_tile = 0)
   return NB_OK;
 }
 
+// Items of the kernel that takes each pair once.  A block is 256 targets times the targets per
+// lane, and a block's tile list is cut into `slices` equal ranges.
+// Targets per lane: as many as the simulation's size earns (as in one context: 4 from 4,096 bodies,
+// 2 from 1,024), fewer for all when that leaves the chip short of work items.
+constexpr int kSymMaxBodies = 32768;  // above, a context of its own is the better place
+static int build_sym(nb_batch *b) {
+  b->once_fits = false;
+  int64_t most = 0, any = 0;
+  for (int k = 0; k < b->nsims; k++) {
+    const int64_t nk = b->off[k + 1] - b->off[k];
+    most = std::max(most, nk);
+    any += nk;
+  }
+  if (any == 0 || most > kSymMaxBodies) return NB_OK;
+  std::vector<BatchSymItem> items;
+  std::vector<BatchSymSim> sims;
+  std::vector<int32_t> tile_sim;
+  int slices = 1, layers = 1;
+  for (int top = 4; top >= 1; top >>= 1) {
+    items.clear();
+    sims.assign((size_t)b->nsims, BatchSymSim{});
+    tile_sim.assign((size_t)(b->n / 64), -1);
+    slices = layers = 1;
+    for (int k = 0; k < b->nsims; k++) {
+      const int64_t nk = b->off[k + 1] - b->off[k];
+      if (nk == 0) continue;
+      const int ntiles = (int)((nk + 63) / 64), p0 = (int)b->poff[k];
+      for (int t = 0; t < ntiles; t++) tile_sim[(size_t)(p0 / 64 + t)] = k;
+      const int ipl = std::min(top, nk >= 4096 ? 4 : nk >= 1024 ? 2 : 1), T = ipl * kBatchSymW;
+      const int nb = (ntiles + T - 1) / T, d = nb / 2;
+      const int longest = std::min(ntiles, (d + 1) * T);
+      const int S = std::max(1, std::min(kSymSlices, (longest + kSymTiles - 1) / kSymTiles));
+      slices = std::max(slices, S);
+      layers = std::max(layers, d);
+      BatchSymSim &m = sims[(size_t)k];
+      m.p0 = p0;
+      m.nb = nb;
+      m.ipl = (int16_t)ipl;
+      m.slices = (int16_t)S;
+      for (int row = 0; row < nb; row++) {
+        // blocks row .. row + dmax, possibly past the last one, which may be short
+        const int dmax = (nb - 1) / 2 + ((nb & 1) == 0 && row < nb / 2 ? 1 : 0);
+        auto upto = [&](int q) { return std::min(q * T, ntiles); };
+        const int end = row + dmax + 1;
+        const int len = (end > nb ? ntiles + upto(end - nb) : upto(end)) - upto(row);
+        for (int q = 0; q < S; q++) {
+          BatchSymItem it{};
+          it.p0 = p0;
+          it.ntiles = ntiles;
+          it.nb = nb;
+          it.row = row;
+          it.u0 = (int)((int64_t)len * q / S);
+          it.u1 = (int)((int64_t)len * (q + 1) / S);
+          it.ipl = (int16_t)ipl;
+          it.slice = (int16_t)q;
+          it.cost = ipl * (it.u1 - it.u0);
+          items.push_back(it);
+        }
+      }
+    }
+    if ((int64_t)items.size() >= (int64_t)b->cus * 16 / kBatchSymW) break;
+  }
+  std::stable_sort(items.begin(), items.end(), [](const BatchSymItem &x, const BatchSymItem &y) {
+    return x.cost > y.cost;
+  });
+  void *ptrs[] = {b->sym_items, b->sym_sims, b->tile_sim, b->sym_acc, b->sym_layer};
+  for (void *q : ptrs)
+    if (q) (void)hipFree(q);
+  b->sym_items = nullptr;
+  b->sym_sims = nullptr;
+  b->tile_sim = nullptr;
+  b->sym_acc = nullptr;
+  b->sym_layer = nullptr;
+  const size_t n3 = (size_t)3 * b->n;
+  NB_BHIP(b, hipMalloc((void **)&b->sym_items, items.size() * sizeof(BatchSymItem)));
+  NB_BHIP(b, hipMalloc((void **)&b->sym_sims, sims.size() * sizeof(BatchSymSim)));
+  NB_BHIP(b, hipMalloc((void **)&b->tile_sim, tile_sim.size() * sizeof(int32_t)));
+  NB_BHIP(b, hipMalloc((void **)&b->sym_acc, (size_t)slices * n3 * sizeof(double)));
+  NB_BHIP(b, hipMalloc((void **)&b->sym_layer, (size_t)layers * n3 * sizeof(float)));
+  NB_BHIP(b, hipMemcpyAsync(b->sym_items, items.data(), items.size() * sizeof(BatchSymItem),
+                            hipMemcpyHostToDevice, b->stream));
+  NB_BHIP(b, hipMemcpyAsync(b->sym_sims, sims.data(), sims.size() * sizeof(BatchSymSim),
+                            hipMemcpyHostToDevice, b->stream));
+  NB_BHIP(b, hipMemcpyAsync(b->tile_sim, tile_sim.data(), tile_sim.size() * sizeof(int32_t),
+                            hipMemcpyHostToDevice, b->stream));
+  NB_BHIP(b, hipStreamSynchronize(b->stream));
+  b->sym_nitems = (int)items.size();
+  b->once_fits = true;
+  return NB_OK;
+}
+
 template <int W>
 static const void *batch_kernel(int ipl, int tile) {
   switch (ipl * 1000 + tile) {
@@ -418,6 +531,20 @@ static const void *batch_kernel(int ipl, int tile) {
 hipError_t launch_batch_force(nb_batch *b) {
   hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, b->stream, b->queue);
   float eps2 = (float)(b->p.eps * b->p.eps);
+  if (b->once && b->once_fits) {
+    BatchSymArgs a;
+    a.items = b->sym_items;
+    a.sims = b->sym_sims;
+    a.tile_sim = b->tile_sim;
+    a.nitems = b->sym_nitems;
+    a.next = &b->queue->next;
+    a.js = b->js;
+    a.acc = b->sym_acc;
+    a.layer = b->sym_layer;
+    a.npad = (int)b->n;
+    a.eps2 = eps2;
+    return launch_batch_sym(a, b->acc, b->cus, b->stream);
+  }
   // items of one shape: the kernel specialised to it; otherwise the per-item dispatch
   const int ipl = b->items_ipl, tile = b->items_tile;
   // 32 waves per CU: 8 workgroups of 4 waves (W = 4, and W = 1 with independent waves), 16 of 2
@@ -571,6 +698,8 @@ int nb_batch_load(nb_batch *b, int32_t nsims, const int64_t *offsets, const doub
   b->ctr_last = DevCounters{};
   NB_BHIP(b, launch_write_stream(b->x, b->y, b->z, b->m, b->flags, b->js, (int)n, (int)n,
                                  b->stream));
+  const int rc = build_sym(b);
+  if (rc) return rc;
   return build_items(b, -1, 0);
 }
 
@@ -700,6 +829,8 @@ int nb_batch_set_shapes(nb_batch *b, const int32_t *ipl3) {
     if (ipl3[k] != 1 && ipl3[k] != 2 && ipl3[k] != 4)
       return bfail(b, NB_E_INVALID, "nb_batch_set_shapes: IPL must be 1, 2 or 4");
   for (int k = 0; k < kBuckets; k++) b->bucket_ipl[k] = ipl3[k];
+  b->once = false;
+  drop_graph(b);
   return b->items ? build_items(b, -1, 0) : NB_OK;
 }
 
@@ -723,6 +854,7 @@ int nb_batch_set_tuning(nb_batch *b, const int32_t *cfg7) {
       return bfail(b, NB_E_INVALID, "nb_batch_set_tuning: IPL in {1, 2, 4}, tile in {64, 128, 256}");
   }
   b->waves = cfg7[0];
+  b->once = false;
   for (int k = 0; k < kBuckets; k++) {
     b->bucket_ipl[k] = cfg7[1 + 2 * k];
     b->bucket_tile[k] = cfg7[2 + 2 * k];
@@ -754,6 +886,7 @@ int nb_batch_autotune(nb_batch *b, int32_t reps, int32_t *ipl3) {
     ms /= (float)reps;
     return NB_OK;
   };
+  b->once = false;  // the shapes first
   float best_total = 1e30f;
   int best_w = b->waves, best_ipl[kBuckets], best_tile[kBuckets];
   for (int k = 0; k < kBuckets; k++) best_ipl[k] = b->bucket_ipl[k], best_tile[k] = b->bucket_tile[k];
@@ -801,12 +934,18 @@ int nb_batch_autotune(nb_batch *b, int32_t reps, int32_t *ipl3) {
         }
       }
   }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
   b->waves = best_w;
   for (int k = 0; k < kBuckets; k++) b->bucket_ipl[k] = best_ipl[k], b->bucket_tile[k] = best_tile[k];
   int rc = build_items(b, -1, 0);
   if (rc) return rc;
+  if (b->once_fits) {  // each pair once, against the best shape
+    b->once = true;
+    float ms = 0;
+    if ((rc = time_launch(ms))) return rc;
+    b->once = ms < best_total;
+  }
+  (void)hipEventDestroy(e0);
+  (void)hipEventDestroy(e1);
   if (ipl3)
     for (int k = 0; k < kBuckets; k++) ipl3[k] = b->bucket_ipl[k];
   return NB_OK;

@@ -323,6 +323,33 @@ struct SymArgs {
 hipError_t launch_force_sym(const ForceShape &s, SymArgs a, double *out, int64_t layer_words,
                             bool detect, hipStream_t st);
 
+// The same for many sets of bodies at once (batched simulations).
+constexpr int kBatchSymW = 4;  // waves per workgroup
+struct BatchSymItem {
+  int32_t p0;             // first body of the simulation (a multiple of 64)
+  int32_t ntiles, nb;     // its tiles and blocks
+  int32_t row, u0, u1;    // block, and range of the block's tile list
+  int16_t ipl, slice;     // targets per lane; which of the block's ranges
+  int32_t cost;
+};
+struct BatchSymSim {
+  int32_t p0, nb;
+  int16_t ipl, slices;
+};
+struct BatchSymArgs {
+  const BatchSymItem *items;
+  const BatchSymSim *sims;
+  const int32_t *tile_sim;  // simulation of each 64-body tile (-1: padding)
+  int nitems;
+  uint32_t *next;           // queue head, zero at the launch
+  const float4 *js;
+  double *acc;              // [slices][3][npad]
+  float *layer;             // [distance][3][npad]
+  int npad;
+  float eps2;
+};
+hipError_t launch_batch_sym(const BatchSymArgs &b, double *out, int cus, hipStream_t st);
+
 struct FixupArgs {
   const double *x, *y, *z, *m, *r;
   const int32_t *beh;

@@ -34,6 +34,7 @@
 // Detection: as nb_force.hip's bound on the tile's smallest r^2, evaluated from the target's side
 // only (r^2 is symmetric); a flagged (target, tile) is re-tested at once in FP64 by the whole wave,
 // one source per lane, with the reference's test (body.go:196-202).
+#include <algorithm>
 #include <cfloat>
 #include <type_traits>
 
@@ -74,47 +75,45 @@ __device__ __forceinline__ void exact_tile(const SymArgs &a, Buf &found, int i, 
 #define NB_ROW __builtin_amdgcn_sched_barrier(0);
 
 template <int IPL, int W, bool DETECT>
-__global__ __launch_bounds__(64 * W)
-__attribute__((amdgpu_waves_per_eu(IPL == 1 ? 8 : IPL == 2 ? 6 : 4)))
-void k_force_sym(SymArgs a) {
+struct SymLds {
+  float4 sh[2][128];
+  float red[2][W][3][64];
+  double sums[W][IPL][3][64];  // the targets' sums over the tiles so far
+  PairBuf<DETECT ? 256 : 1> found;
+};
+
+// What one workgroup does: block `row` of a set of bodies against tiles u0 .. u1 - 1 of its list,
+// which starts at tile `first` and wraps at ntiles.
+struct SymWork {
+  const float4 *js;  // the set's bodies
+  int ntiles, nb, row, first, u0, u1;
+  int slot0;         // distance d's sums go to layer slot d - slot0
+  int limit;         // bodies a target's sums are written for
+  size_t stride;     // words between components in acc and layer
+  double *acc;
+  float *layer;
+};
+
+template <int IPL, int W, bool DETECT>
+__device__ __forceinline__ void sym_block(const SymWork &w, float eps2_s, const SymArgs &a,
+                                          SymLds<IPL, W, DETECT> &lds) {
   constexpr int T = IPL * W;  // tiles per block
-  __shared__ float4 sh[2][128];
-  __shared__ float red[2][W][3][64];
-  __shared__ double sums[W][IPL][3][64];  // the targets' sums over the tiles so far
-  __shared__ PairBuf<DETECT ? 256 : 1> found;
-  if (a.run_flag && *a.run_flag == 0u) return;  // conditional launch (surrogate fallback)
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int row = blockIdx.x, slice = blockIdx.y;
-  // the row's tiles: its own block's (first panel only), then those of blocks row + d0 .. row + d1
-  const int nb = a.nb, ntiles = a.ntiles;
-  const int dmax = (nb - 1) / 2 + ((nb & 1) == 0 && row < nb / 2 ? 1 : 0);
-  const int d1 = min(a.d1, dmax);
-  auto tiles_upto = [&](int b) { return min(b * T, ntiles); };  // b in [0, nb]
-  int len = 0;
-  if (d1 >= a.d0) {
-    const int b0 = row + a.d0, b1 = row + d1 + 1;  // blocks [b0, b1), possibly past nb
-    const int lo = b0 >= nb ? ntiles + tiles_upto(b0 - nb) : tiles_upto(b0);
-    const int hi = b1 > nb ? ntiles + tiles_upto(b1 - nb) : tiles_upto(b1);
-    len = hi - lo;
-  }
-  const int first = (row + a.d0) % nb * T;
-  const int u0 = (int)((int64_t)len * slice / a.slices);
-  const int u1 = (int)((int64_t)len * (slice + 1) / a.slices);
-
+  const int row = w.row, nb = w.nb, ntiles = w.ntiles, u0 = w.u0, u1 = w.u1;
   float xi[IPL], yi[IPL], zi[IPL], mi[IPL];
   float ri[IPL], amax[IPL];
   int live = 0;
 #pragma unroll
   for (int k = 0; k < IPL; k++) {
     const int i = (row * T + wave * IPL + k) * 64 + lane;
-    const float4 b = i < a.npad ? a.js[i] : make_float4(kSentinel, kSentinel, kSentinel, 0.f);
+    const float4 b = i < w.limit ? w.js[i] : make_float4(kSentinel, kSentinel, kSentinel, 0.f);
     xi[k] = b.x;
     yi[k] = b.y;
     zi[k] = b.z;
     mi[k] = b.w;
 #pragma unroll
-    for (int c = 0; c < 3; c++) sums[wave][k][c][lane] = 0.0;
+    for (int c = 0; c < 3; c++) lds.sums[wave][k][c][lane] = 0.0;
     if (DETECT) {
       const uint8_t f = i < a.n ? a.flags[i] : 0;
       if ((f & NB_F_EXISTS) && !(f & NB_F_FRAGMENTING)) live |= 1 << k;
@@ -122,7 +121,7 @@ void k_force_sym(SymArgs a) {
       amax[k] = fmaxf(fabsf(b.x), fmaxf(fabsf(b.y), fabsf(b.z)));
     }
   }
-  const float eps2 = to_vgpr(a.eps2);
+  const float eps2 = to_vgpr(eps2_s);
   // The cube of 1/r is formed once for both bodies where it cannot leave FP32's normal range:
   // eps^2 >= 1e-24 and coordinates within 2.8e11 (r^2 < 1e24).  Elsewhere the masses are multiplied
   // in before the cube, as nb_force.hip does (one multiplication more per pair).  Sentinels need
@@ -132,18 +131,18 @@ void k_force_sym(SymArgs a) {
     const bool sentinel = b.x == kSentinel && b.y == kSentinel && b.z == kSentinel && b.w == 0.f;
     return __ballot(!(m <= 2.8e11f) && !sentinel) == 0;
   };
-  bool near_range = a.eps2 >= 1e-24f;
+  bool near_range = eps2_s >= 1e-24f;
 #pragma unroll
   for (int k = 0; k < IPL; k++)
     near_range = near_range && tile_range(make_float4(xi[k], yi[k], zi[k], mi[k]));
 
-  int t = first + u0;
+  int t = w.first + u0;
   if (t >= ntiles) t -= ntiles;
-  if (DETECT && threadIdx.x == 0) found.clear();
+  if (DETECT && threadIdx.x == 0) lds.found.clear();
   if (u0 < u1 && wave == 0) {
-    const float4 b = a.js[(size_t)t * 64 + lane];
-    sh[0][lane] = b;
-    sh[0][64 + lane] = b;
+    const float4 b = w.js[(size_t)t * 64 + lane];
+    lds.sh[0][lane] = b;
+    lds.sh[0][64 + lane] = b;
   }
   __syncthreads();
   for (int u = u0; u < u1; u++) {
@@ -152,13 +151,13 @@ void k_force_sym(SymArgs a) {
     if (tn >= ntiles) tn -= ntiles;
     float4 next;
     const bool fetch = wave == 0 && u + 1 < u1;
-    if (fetch) next = a.js[(size_t)tn * 64 + lane];
+    if (fetch) next = w.js[(size_t)tn * 64 + lane];
     const int blk = t / T;
     const int d = blk >= row ? blk - row : blk - row + nb;
     float px[IPL], py[IPL], pz[IPL], rmin[IPL];
 #pragma unroll
     for (int k = 0; k < IPL; k++) px[k] = py[k] = pz[k] = 0.f, rmin[k] = FLT_MAX;
-    const float4 *tl = &sh[buf][lane];
+    const float4 *tl = &lds.sh[buf][lane];
     if (d != 0) {
       float qx = 0.f, qy = 0.f, qz = 0.f;
       // One step, written phase by phase over the targets with the order pinned: neighbouring
@@ -241,40 +240,70 @@ void k_force_sym(SymArgs a) {
         for (int s = 0; s < 64; s++) step(tl[s], std::true_type{});
       }
       // after step 63 lane l holds body (l + 63) mod 64: one more rotation brings it home
-      red[buf][wave][0][lane] = -from_next_lane(qx);
-      red[buf][wave][1][lane] = -from_next_lane(qy);
-      red[buf][wave][2][lane] = -from_next_lane(qz);
+      lds.red[buf][wave][0][lane] = -from_next_lane(qx);
+      lds.red[buf][wave][1][lane] = -from_next_lane(qy);
+      lds.red[buf][wave][2][lane] = -from_next_lane(qz);
     } else {
       // the block against itself, one-sided; a target's own entry is met at step 0 of its own tile
       // (it adds exactly zero, but must not count as a candidate)
+      float4 b = tl[0];
 #pragma unroll 2
       for (int s = 0; s < 64; s++) {
-        const float4 b = tl[s];
+        const float4 bn = tl[s + 1];
+        float dx[IPL], dy[IPL], dz[IPL], r2[IPL], gj[IPL];
+#pragma unroll
+        for (int k = 0; k < IPL; k++) dx[k] = b.x - xi[k];
+        NB_ROW
+#pragma unroll
+        for (int k = 0; k < IPL; k++) dy[k] = b.y - yi[k];
+        NB_ROW
+#pragma unroll
+        for (int k = 0; k < IPL; k++) r2[k] = __builtin_fmaf(dx[k], dx[k], eps2);
+        NB_ROW
+#pragma unroll
+        for (int k = 0; k < IPL; k++) dz[k] = b.z - zi[k];
+        NB_ROW
+#pragma unroll
+        for (int k = 0; k < IPL; k++) r2[k] = __builtin_fmaf(dy[k], dy[k], r2[k]);
+        NB_ROW
+#pragma unroll
+        for (int k = 0; k < IPL; k++) r2[k] = __builtin_fmaf(dz[k], dz[k], r2[k]);
+        NB_ROW
 #pragma unroll
         for (int k = 0; k < IPL; k++) {
-          const float dx = b.x - xi[k], dy = b.y - yi[k], dz = b.z - zi[k];
-          float r2 = __builtin_fmaf(dx, dx, eps2);
-          r2 = __builtin_fmaf(dy, dy, r2);
-          r2 = __builtin_fmaf(dz, dz, r2);
-          const float inv = __builtin_amdgcn_rsqf(r2);
-          const float gj = b.w * inv * (inv * inv);
-          px[k] = __builtin_fmaf(dx, gj, px[k]);
-          py[k] = __builtin_fmaf(dy, gj, py[k]);
-          pz[k] = __builtin_fmaf(dz, gj, pz[k]);
+          gj[k] = __builtin_amdgcn_rsqf(r2[k]);
           if (DETECT && !(s == 0 && t == row * T + wave * IPL + k))
-            rmin[k] = __builtin_fminf(rmin[k], r2);
+            rmin[k] = __builtin_fminf(rmin[k], r2[k]);
         }
+        NB_ROW
+#pragma unroll
+        for (int k = 0; k < IPL; k++) r2[k] = b.w * gj[k];
+        NB_ROW
+#pragma unroll
+        for (int k = 0; k < IPL; k++) gj[k] = gj[k] * gj[k];
+        NB_ROW
+#pragma unroll
+        for (int k = 0; k < IPL; k++) gj[k] = r2[k] * gj[k];
+#pragma unroll
+        for (int k = 0; k < IPL; k++) {
+          NB_ROW
+          px[k] = __builtin_fmaf(dx[k], gj[k], px[k]);
+          py[k] = __builtin_fmaf(dy[k], gj[k], py[k]);
+          pz[k] = __builtin_fmaf(dz[k], gj[k], pz[k]);
+        }
+        NB_ROW
+        b = bn;
       }
     }
     if (fetch) {
-      sh[buf ^ 1][lane] = next;
-      sh[buf ^ 1][64 + lane] = next;
+      lds.sh[buf ^ 1][lane] = next;
+      lds.sh[buf ^ 1][64 + lane] = next;
     }
 #pragma unroll
     for (int k = 0; k < IPL; k++) {
-      sums[wave][k][0][lane] += (double)px[k];
-      sums[wave][k][1][lane] += (double)py[k];
-      sums[wave][k][2][lane] += (double)pz[k];
+      lds.sums[wave][k][0][lane] += (double)px[k];
+      lds.sums[wave][k][1][lane] += (double)py[k];
+      lds.sums[wave][k][2][lane] += (double)pz[k];
     }
     if (DETECT) {
       const float rmax = a.rmax_tile[t];
@@ -283,51 +312,159 @@ void k_force_sym(SymArgs a) {
         // the bound of nb_force.hip's tile_end
         const float rs = ri[k] + rmax;
         const float e = 4.76837158e-7f * (amax[k] + rs);
-        const float w = rs + e;
-        const float thr = __builtin_fmaf(w, w, eps2) * 1.0000039f;
+        const float rse = rs + e;
+        const float thr = __builtin_fmaf(rse, rse, eps2) * 1.0000039f;
         uint64_t hit = __ballot(rmin[k] <= thr && (live >> k & 1));
         if (hit && lane == 0)
-          atomicAdd(&found.tiles, (uint32_t)__builtin_popcountll(hit));
+          atomicAdd(&lds.found.tiles, (uint32_t)__builtin_popcountll(hit));
         while (hit) {
           const int l = __builtin_ctzll(hit);
           hit &= hit - 1;
-          exact_tile(a, found, (row * T + wave * IPL + k) * 64 + l, t, d == 0);
+          exact_tile(a, lds.found, (row * T + wave * IPL + k) * 64 + l, t, d == 0);
         }
       }
     }
-    // one barrier per tile: the next tile is staged, every wave's sums are in red[buf] (which is
+    // one barrier per tile: the next tile is staged, every wave's sums are in lds.red[buf] (which is
     // written again two tiles on, after the next barrier)
     __syncthreads();
     if (d != 0) {
       for (int q = threadIdx.x; q < 192; q += 64 * W) {
         const int c = q >> 6, l = q & 63;
-        float s = red[buf][0][c][l];
+        float s = lds.red[buf][0][c][l];
 #pragma unroll
-        for (int w = 1; w < W; w++) s += red[buf][w][c][l];
-        a.layer[((size_t)(d - a.d0 + (a.d0 == 0 ? -1 : 0)) * 3 + c) * a.npad + t * 64 + l] = s;
+        for (int v = 1; v < W; v++) s += lds.red[buf][v][c][l];
+        w.layer[((size_t)(d - w.slot0) * 3 + c) * w.stride + t * 64 + l] = s;
       }
     }
     t = tn;
   }
-  double *o = a.acc + (size_t)slice * 3 * a.npad;
+  double *o = w.acc;
 #pragma unroll
   for (int k = 0; k < IPL; k++) {
     const int i = (row * T + wave * IPL + k) * 64 + lane;
-    if (i >= a.npad) continue;
-    o[i] = sums[wave][k][0][lane];
-    o[a.npad + i] = sums[wave][k][1][lane];
-    o[2 * (size_t)a.npad + i] = sums[wave][k][2][lane];
+    if (i >= w.limit) continue;
+    o[i] = lds.sums[wave][k][0][lane];
+    o[w.stride + i] = lds.sums[wave][k][1][lane];
+    o[2 * w.stride + i] = lds.sums[wave][k][2][lane];
   }
-  if (DETECT) found.flush(a.pairs, a.ctr, a.pair_cap);
+  if (DETECT) lds.found.flush(a.pairs, a.ctr, a.pair_cap);
+}
+
+template <int IPL, int W, bool DETECT>
+__global__ __launch_bounds__(64 * W)
+__attribute__((amdgpu_waves_per_eu(IPL == 1 ? 8 : IPL == 2 ? 6 : 4)))
+void k_force_sym(SymArgs a) {
+  constexpr int T = IPL * W;
+  __shared__ SymLds<IPL, W, DETECT> lds;
+  if (a.run_flag && *a.run_flag == 0u) return;  // conditional launch (surrogate fallback)
+  const int row = blockIdx.x, slice = blockIdx.y;
+  // the row's tiles: its own block's (first panel only), then those of blocks row + d0 .. row + d1
+  const int nb = a.nb, ntiles = a.ntiles;
+  const int dmax = (nb - 1) / 2 + ((nb & 1) == 0 && row < nb / 2 ? 1 : 0);
+  const int d1 = min(a.d1, dmax);
+  auto tiles_upto = [&](int b) { return min(b * T, ntiles); };  // b in [0, nb]
+  int len = 0;
+  if (d1 >= a.d0) {
+    const int b0 = row + a.d0, b1 = row + d1 + 1;  // blocks [b0, b1), possibly past nb
+    const int lo = b0 >= nb ? ntiles + tiles_upto(b0 - nb) : tiles_upto(b0);
+    const int hi = b1 > nb ? ntiles + tiles_upto(b1 - nb) : tiles_upto(b1);
+    len = hi - lo;
+  }
+  SymWork w;
+  w.js = a.js;
+  w.ntiles = ntiles;
+  w.nb = nb;
+  w.row = row;
+  w.first = (row + a.d0) % nb * T;
+  w.u0 = (int)((int64_t)len * slice / a.slices);
+  w.u1 = (int)((int64_t)len * (slice + 1) / a.slices);
+  w.slot0 = a.d0 == 0 ? 1 : a.d0;
+  w.limit = a.npad;
+  w.stride = (size_t)a.npad;
+  w.acc = a.acc + (size_t)slice * 3 * a.npad;
+  w.layer = a.layer;
+  sym_block<IPL, W, DETECT>(w, a.eps2, a, lds);
+}
+
+// Many sets of bodies (batched simulations) in one persistent launch: items are (simulation, block,
+// range of its tiles), longest first, taken from a device queue until it is exhausted.
+// 512 simulations of 256 to 8,192 bodies: 2.7 ms a step, 4,500 G interactions/s, FP32 VALU issue
+// (a simulation's blocks against themselves, a fifth of the tiles at 8,192 bodies, are one-sided);
+// the one-sided kernel of nb_batch.hip takes 4.3 ms in its default shape, 3.45 in its tuned one.
+// 8 simulations of 64 to 128 bodies: 0.041 -> 0.019 ms; 64 of 500 to 4,000: 0.29 -> 0.15 (tuned
+// 0.16).  Blocks of two waves or one: 2.73 and 2.70 ms for the first, 0.16 and 0.20 for the last.
+__global__ __launch_bounds__(64 * kBatchSymW) __attribute__((amdgpu_waves_per_eu(4)))
+void k_batch_sym(BatchSymArgs b) {
+  constexpr int W = kBatchSymW;
+  __shared__ __attribute__((aligned(16))) char raw[sizeof(SymLds<4, W, false>)];
+  __shared__ int cur;
+  SymArgs none{};
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) cur = (int)atomicAdd(b.next, 1u);
+    __syncthreads();
+    const int q = cur;
+    if (q >= b.nitems) break;
+    const BatchSymItem it = b.items[q];
+    SymWork w;
+    w.js = b.js + it.p0;
+    w.ntiles = it.ntiles;
+    w.nb = it.nb;
+    w.row = it.row;
+    w.first = it.row * it.ipl * W;
+    w.u0 = it.u0;
+    w.u1 = it.u1;
+    w.slot0 = 1;
+    w.limit = it.ntiles * 64;
+    w.stride = (size_t)b.npad;
+    w.acc = b.acc + (size_t)it.slice * 3 * b.npad + it.p0;
+    w.layer = b.layer + it.p0;
+    if (it.ipl == 4)
+      sym_block<4, W, false>(w, b.eps2, none, reinterpret_cast<SymLds<4, W, false> &>(raw));
+    else if (it.ipl == 2)
+      sym_block<2, W, false>(w, b.eps2, none, reinterpret_cast<SymLds<2, W, false> &>(raw));
+    else
+      sym_block<1, W, false>(w, b.eps2, none, reinterpret_cast<SymLds<1, W, false> &>(raw));
+  }
+}
+
+// The batch's k_sym_fold: a body's slices and distances follow from its simulation.
+__global__ __launch_bounds__(256) void k_batch_sym_fold(BatchSymArgs b, double *out) {
+  const int c = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;  // npad is a multiple of 256
+  const int64_t g = (int64_t)c * b.npad + i;
+  const int sim = b.tile_sim[i >> 6];
+  if (sim < 0) {
+    out[g] = 0.0;
+    return;
+  }
+  const BatchSymSim s = b.sims[sim];
+  const size_t st = (size_t)3 * b.npad;
+  double v = 0.0;
+  for (int q = 0; q < s.slices; q++) v += b.acc[q * st + g];
+  const int blk = (i - s.p0) / (s.ipl * 64 * kBatchSymW);
+  const int cnt = (s.nb - 1) / 2 + ((s.nb & 1) == 0 && blk >= s.nb / 2 ? 1 : 0);
+  const float *p = b.layer + (size_t)c * b.npad + i;
+  for (int q = 0; q < cnt; q++) v += p[(size_t)q * st];
+  out[g] = v;
+}
+
+hipError_t launch_batch_sym(const BatchSymArgs &b, double *out, int cus, hipStream_t st) {
+  // 16 waves per CU are resident at once
+  hipLaunchKernelGGL(k_batch_sym, dim3((unsigned)std::min(b.nitems, cus * 16 / kBatchSymW)),
+                     dim3(64 * kBatchSymW), 0, st, b);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_batch_sym_fold, dim3((unsigned)(b.npad / 256), 3), dim3(256), 0, st, b,
+                     out);
+  return hipGetLastError();
 }
 
 // out = (first panel: 0, later: out) + the target slices + the distances that reached the body's
 // block, in FP64 and in this order; one thread per word.
 __global__ __launch_bounds__(256) void k_sym_fold(SymArgs a, int T, double *out) {
   if (a.run_flag && *a.run_flag == 0u) return;
-  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (g >= (int64_t)3 * a.npad) return;
-  const int c = (int)(g / a.npad), i = (int)(g - (int64_t)c * a.npad);
+  const int c = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;  // npad is a multiple of 256
+  const int64_t g = (int64_t)c * a.npad + i;
   const size_t st = (size_t)3 * a.npad;
   double s = a.d0 == 0 ? 0.0 : out[g];
   for (int q = 0; q < a.slices; q++) s += a.acc[q * st + g];
@@ -384,7 +521,7 @@ hipError_t launch_force_sym(const ForceShape &s, SymArgs a, double *out, int64_t
       default: return hipErrorInvalidValue;
     }
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_sym_fold, dim3((unsigned)((per + 255) / 256)), dim3(256), 0, st, a, T,
+    hipLaunchKernelGGL(k_sym_fold, dim3((unsigned)(a.npad / 256), 3), dim3(256), 0, st, a, T,
                        out);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
