@@ -235,17 +235,25 @@ __global__ void k_mse(const float *Y, int ldy, const float *T, int rows, int dou
   lrow[r] = l;
 }
 
-__global__ void k_adam(float *w, const float *g, float *m1, float *m2, uint16_t *wb, int64_t n,
-                       float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float a = b1 * m1[i] + (1.f - b1) * gi;
-  const float b = b2 * m2[i] + (1.f - b2) * gi * gi;
+struct AdamArgs {
+  float lr, b1, b2, eps, c1, c2;
+};
+// One weight's Adam update; returns the new weight.
+__device__ __forceinline__ float adam_update(const AdamArgs &h, float gi, float *w, float *m1,
+                                             float *m2, int64_t i) {
+  const float a = h.b1 * m1[i] + (1.f - h.b1) * gi;
+  const float b = h.b2 * m2[i] + (1.f - h.b2) * gi * gi;
   m1[i] = a;
   m2[i] = b;
-  const float wi = w[i] - lr * (a / c1) / (sqrtf(b / c2) + eps);
+  const float wi = w[i] - h.lr * (a / h.c1) / (sqrtf(b / h.c2) + h.eps);
   w[i] = wi;
+  return wi;
+}
+__global__ void k_adam(float *w, const float *g, float *m1, float *m2, uint16_t *wb, int64_t n,
+                       AdamArgs h) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const float wi = adam_update(h, g[i], w, m1, m2, i);
   if (wb) wb[i] = f2bf(wi);
 }
 
@@ -450,6 +458,291 @@ __global__ __launch_bounds__(256) void k_mlp_infer_p(InferArgs a) {
   }
 }
 
+// ---- a training step in two launches ---------------------------------------------------------
+// For the shapes of the fused inference with up to three hidden layers.  A step layer by layer is
+// 45 small launches (GEMMs, split-K sums, column sums, GELU backward, Adam) that wait for each
+// other, 181 us for 512 rows; these two take 23 (8,192 rows: 725 and 69).  Every product, sum and
+// rounding is the layer-by-layer step's, in its order, so the weights are the same bit for bit.
+//
+// k_train_rows: one workgroup takes 16 rows through the forward pass, the loss and the backward
+// chain.  Pre-activations stay in registers, activations and gradients in LDS; what the weight
+// gradients need goes out transposed ([column][row]), four consecutive rows of a column being one
+// lane's MFMA results and, later, one lane's MFMA operand.
+// k_train_weights: one workgroup per 16 x 16 block of a layer's weights: the block's gradient over
+// the rows (the split-K ranges of the layer-by-layer GEMM dealt to the waves, summed in range
+// order), then Adam, the BF16 weights and their transpose; and one per 16 biases: the column sums
+// in k_colsum's order, then Adam.
+constexpr int kTrainRows = 16;
+struct TrainLayer {
+  float *w, *m1, *m2, *b, *bm1, *bm2;
+  uint16_t *wb, *wt;   // BF16 weights [in][out], [out][in]
+  int in, out;         // padded
+  int cols;            // columns with gradients: out, or 16 for the output layer
+  uint16_t *inT, *dT;  // layer input and gradient, [column][row]
+  float *d;            // FP32 gradient [row][cols]
+};
+struct TrainArgs {
+  const float *x, *t;
+  float *lrow;
+  int rows, din, dout;
+  TrainLayer l[4];
+  AdamArgs adam;
+  int layers;          // linear layers
+  int splits, kps;     // row ranges of the weight gradients
+};
+
+__device__ __forceinline__ void store4(uint16_t *p, const uint16_t (&v)[4]) {
+  *reinterpret_cast<uint2 *>(p) =
+      make_uint2((uint32_t)v[0] | (uint32_t)v[1] << 16, (uint32_t)v[2] | (uint32_t)v[3] << 16);
+}
+
+// A hidden layer's forward for the workgroup's 16 rows (infer_layer_w's products and epilogue),
+// keeping the pre-activations and writing the transposed activations.
+template <int K, int HID>
+__device__ __forceinline__ void train_forward(const uint16_t (*Hin)[kInferW + 8],
+                                              uint16_t (*Hout)[kInferW + 8],
+                                              const bf16x8 (&fb)[K / 32][HID / 64],
+                                              const float (&bc)[HID / 64], uint16_t *outT,
+                                              int rows, int r0, f32x4 (&z)[HID / 64], int w,
+                                              int lr, int lq) {
+  constexpr int NBW = HID / 64, KS = K / 32;
+#pragma unroll
+  for (int b = 0; b < NBW; b++) z[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) {
+    const bf16x8 fa = *(const bf16x8 *)&Hin[lr][ks * 32 + 2 * lq];
+#pragma unroll
+    for (int b = 0; b < NBW; b++)
+      z[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb[ks][b], z[b], 0, 0, 0);
+  }
+#pragma unroll
+  for (int b = 0; b < NBW; b++) {
+    const int col = w * (HID / 4) + b * 16 + lr;
+    uint16_t h[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      z[b][v] += bc[b];
+      h[v] = f2bf(gelu(z[b][v]));
+      Hout[lq + v][col] = h[v];
+    }
+    store4(outT + (size_t)col * rows + r0 + lq, h);
+  }
+}
+
+// The B fragments of G W^T (K columns of G) for the wave's columns: W's rows.
+template <int K, int HID>
+__device__ __forceinline__ void back_frags(bf16x4 (&fb)[K / 16][HID / 64], const TrainLayer &next,
+                                           int w, int lr, int lq) {
+#pragma unroll
+  for (int ks = 0; ks < K / 16; ks++)
+#pragma unroll
+    for (int b = 0; b < HID / 64; b++)
+      fb[ks][b] = *(const bf16x4 *)(next.wb + (size_t)(w * (HID / 4) + b * 16 + lr) * next.out +
+                                    ks * 16 + lq);
+}
+
+// A hidden layer's backward: the gradient of its output is G W^T (W the next layer's), times GELU'
+// of its pre-activations.
+template <int K, int HID>
+__device__ __forceinline__ void train_backward(const uint16_t (*G)[kInferW + 8],
+                                               uint16_t (*Gout)[kInferW + 8],
+                                               const bf16x4 (&fb)[K / 16][HID / 64],
+                                               const TrainLayer &l, int rows, int r0,
+                                               const f32x4 (&z)[HID / 64], int w, int lr,
+                                               int lq) {
+  constexpr int NBW = HID / 64, KS = K / 16;
+  f32x4 acc[NBW];
+#pragma unroll
+  for (int b = 0; b < NBW; b++) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) {
+    const bf16x4 fa = *(const bf16x4 *)&G[lr][ks * 16 + lq];
+#pragma unroll
+    for (int b = 0; b < NBW; b++)
+      acc[b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa, fb[ks][b], acc[b], 0, 0, 0);
+  }
+#pragma unroll
+  for (int b = 0; b < NBW; b++) {
+    const int col = w * (HID / 4) + b * 16 + lr;
+    uint16_t h[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const float g = acc[b][v] * gelu_grad(z[b][v]);
+      l.d[(size_t)(r0 + lq + v) * HID + col] = g;
+      h[v] = f2bf(g);
+      Gout[lq + v][col] = h[v];
+    }
+    store4(l.dT + (size_t)col * rows + r0 + lq, h);
+  }
+}
+
+// Every layer's weight fragments are requested at the start, so that their latency is paid once and
+// not once a layer: 14.5 us for 512 rows (64 rows a workgroup and each layer's fragments when it
+// comes: 23.3; whole steps 23 and 32 us, 69 and 70 with 8,192 rows).
+template <int DINP, int HID, int NH>
+__global__ __launch_bounds__(256) void k_train_rows(TrainArgs a) {
+  constexpr int KH = HID / 32;
+  __shared__ __attribute__((aligned(16))) uint16_t Hs[2][kTrainRows][kInferW + 8];
+  __shared__ float dsq[kTrainRows][17];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lq = 4 * (lane >> 4);
+  const int r0 = blockIdx.x * kTrainRows, R = a.rows;
+  bf16x8 f0[DINP / 32][HID / 64], fh[NH][KH][HID / 64], fo[KH];
+  bf16x4 g0[1][HID / 64], gh[NH][HID / 16][HID / 64];
+  float c0[HID / 64], ch[NH][HID / 64];
+  infer_frags<DINP, HID>(f0, c0, a.l[0].wt, a.l[0].b, w, lr, lq);
+#pragma unroll
+  for (int l = 1; l < NH; l++)
+    infer_frags<HID, HID>(fh[l - 1], ch[l - 1], a.l[l].wt, a.l[l].b, w, lr, lq);
+#pragma unroll
+  for (int ks = 0; ks < KH; ks++)
+    fo[ks] = *(const bf16x8 *)(a.l[NH].wt + (size_t)lr * HID + ks * 32 + 2 * lq);
+  back_frags<16, HID>(g0, a.l[NH], w, lr, lq);
+#pragma unroll
+  for (int l = NH - 2; l >= 0; l--) back_frags<HID, HID>(gh[l], a.l[l + 1], w, lr, lq);
+  for (int i = tid; i < DINP * kTrainRows / 4; i += 256) {  // four rows of one column
+    const int c = i % DINP, r = i / DINP * 4;
+    uint16_t h[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      h[v] = c < a.din ? f2bf(a.x[(size_t)(r0 + r + v) * a.din + c]) : 0;
+      Hs[0][r + v][c] = h[v];
+    }
+    store4(a.l[0].inT + (size_t)c * R + r0 + r, h);
+  }
+  __syncthreads();
+  f32x4 z[NH][HID / 64];
+  train_forward<DINP, HID>(Hs[0], Hs[1], f0, c0, a.l[1].inT, R, r0, z[0], w, lr, lq);
+  __syncthreads();
+  int cur = 1;
+#pragma unroll
+  for (int l = 1; l < NH; l++) {
+    train_forward<HID, HID>(Hs[cur], Hs[cur ^ 1], fh[l - 1], ch[l - 1], a.l[l + 1].inT, R, r0,
+                                z[l], w, lr, lq);
+    __syncthreads();
+    cur ^= 1;
+  }
+  // output layer, columns 0..15, and the loss (k_mse), by the first wave
+  if (w == 0) {
+    const TrainLayer &o = a.l[NH];
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KH; ks++) {
+      const bf16x8 fa = *(const bf16x8 *)&Hs[cur][lr][ks * 32 + 2 * lq];
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fo[ks], acc, 0, 0, 0);
+    }
+    const bool real = lr < a.dout;
+    const float bc = real ? o.b[lr] : 0.f;
+    const float sc = 2.f / ((float)R * (float)a.dout);
+    uint16_t h[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int row = lq + v;
+      float g = 0.f, d = 0.f;
+      if (real) {
+        d = (acc[v] + bc) - a.t[(size_t)(r0 + row) * a.dout + lr];
+        g = sc * d;
+      }
+      dsq[row][lr] = d * d;
+      o.d[(size_t)(r0 + row) * 16 + lr] = g;
+      h[v] = f2bf(g);
+      Hs[cur ^ 1][row][lr] = h[v];
+    }
+    store4(o.dT + (size_t)lr * R + r0 + lq, h);
+  }
+  __syncthreads();
+  if (tid < kTrainRows) {
+    float l = 0.f;
+    for (int c = 0; c < a.dout; c++) l += dsq[tid][c];
+    a.lrow[r0 + tid] = l;
+  }
+  // the output layer's padded columns carry zeros: its first 16 are all of its gradient
+  cur ^= 1;
+  train_backward<16, HID>(Hs[cur], Hs[cur ^ 1], g0, a.l[NH - 1], R, r0, z[NH - 1], w, lr, lq);
+  cur ^= 1;
+#pragma unroll
+  for (int l = NH - 2; l >= 0; l--) {
+    __syncthreads();
+    train_backward<HID, HID>(Hs[cur], Hs[cur ^ 1], gh[l], a.l[l], R, r0, z[l], w, lr, lq);
+    cur ^= 1;
+  }
+}
+
+constexpr int kTrainSplits = 64;
+__global__ __launch_bounds__(256) void k_train_weights(TrainArgs a) {
+  __shared__ float part[kTrainSplits][256];  // [range][4 x lane + v]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lq = 4 * (lane >> 4);
+  int b = blockIdx.x, l = 0;
+  for (; l < a.layers; l++) {
+    const int n = a.l[l].in / 16 * (a.l[l].cols / 16);
+    if (b < n) break;
+    b -= n;
+  }
+  if (l < a.layers) {
+    const TrainLayer &y = a.l[l];
+    const int nbc = y.cols / 16, mb = b / nbc * 16, nb = b % nbc * 16;
+    const uint16_t *pa = y.inT + (size_t)(mb + lr) * a.rows + lq;
+    const uint16_t *pb = y.dT + (size_t)(nb + lr) * a.rows + lq;
+    for (int s = w; s < a.splits; s += 4) {
+      const int k1 = min(a.rows, (s + 1) * a.kps);
+      f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int k = s * a.kps; k < k1; k += 128) {  // eight steps' operands in flight
+        bf16x4 fa[8], fb[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          const int at = min(k + 16 * u, k1 - 16);
+          fa[u] = *(const bf16x4 *)(pa + at);
+          fb[u] = *(const bf16x4 *)(pb + at);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+          if (k + 16 * u < k1)
+            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa[u], fb[u], acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; v++) part[s][lane * 4 + v] = acc[v];
+    }
+    __syncthreads();
+    // thread (i, j) of the block: accumulator register i % 4 of lane 16 (i / 4) + j
+    const int i = tid >> 4, j = tid & 15, src = ((i >> 2) * 16 + j) * 4 + (i & 3);
+    float g;
+    if (a.splits > 1) {  // k_splitk_sum
+      g = 0.f;
+      for (int s = 0; s < a.splits; s++) g += part[s][src];
+    } else {
+      g = part[0][src];
+    }
+    const int row = mb + i, col = nb + j;
+    const int64_t at = (int64_t)row * y.out + col;
+    const uint16_t wb = f2bf(adam_update(a.adam, g, y.w, y.m1, y.m2, at));
+    y.wb[at] = wb;
+    y.wt[(int64_t)col * y.in + row] = wb;
+    return;
+  }
+  // 16 biases: thread (g, c) sums rows g, g + 16, ... in order, then a tree over g (k_colsum)
+  for (l = 0; l < a.layers; l++) {
+    const int n = a.l[l].cols / 16;
+    if (b < n) break;
+    b -= n;
+  }
+  if (l >= a.layers) return;
+  const TrainLayer &y = a.l[l];
+  const int c = tid & 15, g = tid >> 4, col = b * 16 + c;
+  float s = 0.f;
+#pragma unroll 8
+  for (int r = g; r < a.rows; r += 16) s += y.d[(size_t)r * y.cols + col];
+  part[g][c] = s;
+  __syncthreads();
+  for (int q = 8; q > 0; q >>= 1) {
+    if (g < q) part[g][c] += part[g + q][c];
+    __syncthreads();
+  }
+  if (g == 0) (void)adam_update(a.adam, part[0][c], y.b, y.bm1, y.bm2, col);
+}
+
 }  // namespace nb
 
 // ---------------------------------------------------------------------------------------------
@@ -481,6 +774,11 @@ struct nb_mlp {
   // transposed BF16 weights for the fused inference kernel, rebuilt when wver moves
   std::vector<uint16_t *> WbT;
   int64_t wver = 0, wt_ver = -1;
+  // buffers of the two-launch training step: per linear layer the transposed input and gradient, and
+  // the FP32 gradient
+  std::vector<uint16_t *> inT, dT;
+  std::vector<float *> dF;
+  int64_t train_rows = 0;
   int infer_wgs = 0;  // resident workgroups of the persistent inference kernel (0: not yet known)
 };
 
@@ -644,20 +942,131 @@ int backward(nb_mlp *m, int64_t rows) {
   return NB_OK;
 }
 
-int adam_step(nb_mlp *m, float lr) {
+AdamArgs next_adam(nb_mlp *m, float lr) {
   m->adam_t++;
   m->wver++;
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.f - powf(b1, (float)m->adam_t), c2 = 1.f - powf(b2, (float)m->adam_t);
+  return AdamArgs{lr, b1, b2, 1e-8f, c1, c2};
+}
+
+int adam_step(nb_mlp *m, float lr) {
+  const AdamArgs h = next_adam(m, lr);
   for (int l = 0; l <= m->layers; l++) {
     const int64_t nw = (int64_t)m->in_dim[l] * m->out_dim[l];
     hipLaunchKernelGGL(k_adam, dim3(nblk(nw)), dim3(256), 0, m->stream, m->W[l], m->Wg[l],
-                       m->Wm1[l], m->Wm2[l], m->Wb[l], nw, lr, b1, b2, 1e-8f, c1, c2);
+                       m->Wm1[l], m->Wm2[l], m->Wb[l], nw, h);
     hipLaunchKernelGGL(k_adam, dim3(nblk(m->out_dim[l])), dim3(256), 0, m->stream, m->bvec[l],
                        m->bg[l], m->bm1[l], m->bm2[l], (uint16_t *)nullptr,
-                       (int64_t)m->out_dim[l], lr, b1, b2, 1e-8f, c1, c2);
+                       (int64_t)m->out_dim[l], h);
     NB_MHIP(m, hipGetLastError());
   }
+  return NB_OK;
+}
+
+// The shapes of the fused kernels.
+bool fused_shape(const nb_mlp *m) {
+  return m->dinp <= kInferW && m->hid <= kInferW && m->hid % 64 == 0 && m->dinp % 64 == 0 &&
+         m->dout <= 16 && m->layers <= kInferMaxLayers && m->layers >= 1;
+}
+
+// The transposed BF16 weights, made again if the weights have moved.
+int transposed_weights(nb_mlp *m, hipStream_t st) {
+  if (m->wt_ver == m->wver) return NB_OK;
+  if (m->WbT.empty())
+    for (int l = 0; l <= m->layers; l++) {
+      uint16_t *q = nullptr;
+      NB_MHIP(m, hipMalloc((void **)&q, (size_t)m->in_dim[l] * m->out_dim[l] * 2));
+      m->WbT.push_back(q);
+    }
+  for (int l = 0; l <= m->layers; l++) {
+    const int K = m->in_dim[l], N = m->out_dim[l];
+    hipLaunchKernelGGL(k_transpose_bf16, dim3(nblk((int64_t)K * N)), dim3(256), 0, st,
+                       m->Wb[l], K, N, m->WbT[l]);
+  }
+  NB_MHIP(m, hipGetLastError());
+  m->wt_ver = m->wver;
+  return NB_OK;
+}
+
+void free_train(nb_mlp *m) {
+  for (uint16_t *q : m->inT) (void)hipFree(q);
+  for (uint16_t *q : m->dT) (void)hipFree(q);
+  for (float *q : m->dF) (void)hipFree(q);
+  m->inT.clear();
+  m->dT.clear();
+  m->dF.clear();
+  m->train_rows = 0;
+}
+
+// A training step in two launches, on rows (a multiple of 64) of x and t on the device; per-row
+// losses to lrow.
+int train_step_fused(nb_mlp *m, const float *x, const float *t, int64_t rows, float lr,
+                     float *lrow, hipStream_t st) {
+  const int L = m->layers;
+  if (rows > m->train_rows) {
+    free_train(m);
+    for (int l = 0; l <= L; l++) {
+      uint16_t *a = nullptr, *d = nullptr;
+      float *f = nullptr;
+      const int cols = l == L ? 16 : m->hid;
+      NB_MHIP(m, hipMalloc((void **)&a, (size_t)rows * m->in_dim[l] * 2));
+      m->inT.push_back(a);
+      NB_MHIP(m, hipMalloc((void **)&d, (size_t)rows * cols * 2));
+      m->dT.push_back(d);
+      NB_MHIP(m, hipMalloc((void **)&f, (size_t)rows * cols * 4));
+      m->dF.push_back(f);
+    }
+    m->train_rows = rows;
+  }
+  int rc = transposed_weights(m, st);
+  if (rc) return rc;
+  TrainArgs a{};
+  a.x = x;
+  a.t = t;
+  a.lrow = lrow;
+  a.rows = (int)rows;
+  a.din = m->din;
+  a.dout = m->dout;
+  a.layers = L + 1;
+  unsigned blocks = 0;
+  for (int l = 0; l <= L; l++) {
+    TrainLayer &y = a.l[l];
+    y.w = m->W[l];
+    y.m1 = m->Wm1[l];
+    y.m2 = m->Wm2[l];
+    y.b = m->bvec[l];
+    y.bm1 = m->bm1[l];
+    y.bm2 = m->bm2[l];
+    y.wb = m->Wb[l];
+    y.wt = m->WbT[l];
+    y.in = m->in_dim[l];
+    y.out = m->out_dim[l];
+    y.cols = l == L ? 16 : m->hid;
+    y.inT = m->inT[l];
+    y.dT = m->dT[l];
+    y.d = m->dF[l];
+    blocks += (unsigned)(y.in / 16 * (y.cols / 16) + y.cols / 16);
+  }
+  // the row ranges of gemm()'s split-K
+  const int K = (int)rows, want = std::max(1, std::min(kTrainSplits, K / 256));
+  a.kps = ((K / 16 + want - 1) / want) * 16;
+  a.splits = (K + a.kps - 1) / a.kps;
+  a.adam = next_adam(m, lr);
+  const dim3 grid((unsigned)(rows / kTrainRows));
+#define NB_TRAIN(D, H)                                                                           \
+  if (L == 1) hipLaunchKernelGGL((k_train_rows<D, H, 1>), grid, dim3(256), 0, st, a);            \
+  else if (L == 2) hipLaunchKernelGGL((k_train_rows<D, H, 2>), grid, dim3(256), 0, st, a);       \
+  else hipLaunchKernelGGL((k_train_rows<D, H, 3>), grid, dim3(256), 0, st, a);
+  if (m->dinp == 64 && m->hid == 64) { NB_TRAIN(64, 64) }
+  else if (m->dinp == 128 && m->hid == 64) { NB_TRAIN(128, 64) }
+  else if (m->dinp == 64) { NB_TRAIN(64, 128) }
+  else { NB_TRAIN(128, 128) }
+#undef NB_TRAIN
+  NB_MHIP(m, hipGetLastError());
+  hipLaunchKernelGGL(k_train_weights, dim3(blocks), dim3(256), 0, st, a);
+  NB_MHIP(m, hipGetLastError());
+  m->wt_ver = m->wver;  // the transposed weights moved along
   return NB_OK;
 }
 
@@ -694,8 +1103,13 @@ int mlp_forward_device(nb_mlp *m, const float *x_dev, int64_t rows, const float 
 }
 
 // One Adam step on device-resident rows (features FP32 [rows x din], targets FP32 [rows x dout]).
+// lrow (may be null): per-row losses, in place of the object's own buffer.
 int mlp_train_step_device(nb_mlp *m, const float *x_dev, const float *t_dev, int64_t rows,
-                          float lr, hipStream_t st) {
+                          float lr, float *lrow, hipStream_t st) {
+  if (rows > 0 && rows % 64 == 0 && m->layers <= 3 && fused_shape(m)) {
+    int rc = ensure_rows(m, rows);  // (the per-row losses)
+    return rc ? rc : train_step_fused(m, x_dev, t_dev, rows, lr, lrow ? lrow : m->lrow, st);
+  }
   hipStream_t keep = m->stream;
   m->stream = st;
   int rc = ensure_rows(m, rows);
@@ -710,33 +1124,22 @@ int mlp_train_step_device(nb_mlp *m, const float *x_dev, const float *t_dev, int
   if (!rc) rc = forward(m, rows);
   if (!rc) rc = backward(m, rows);
   if (!rc) rc = adam_step(m, lr);
+  if (!rc && lrow &&
+      hipMemcpyAsync(lrow, m->lrow, (size_t)rows * 4, hipMemcpyDeviceToDevice, st) != hipSuccess)
+    rc = NB_E_HIP;
   m->stream = keep;
   return rc;
 }
 // Fused inference on device-resident FP32 rows [rows x din] into y [rows x dout].
 int mlp_infer_device(nb_mlp *m, const float *x_dev, int64_t rows, float *y_dev,
                      hipStream_t st) {
-  if (m->dinp > kInferW || m->hid > kInferW || m->hid % 64 || m->dinp % 64 || m->dout > 16 ||
-      m->layers > kInferMaxLayers || m->layers < 1) {
+  if (!fused_shape(m)) {
     m->err = "fused inference: shape beyond its limits";
     return NB_E_UNSUPPORTED;
   }
   if (rows <= 0) return NB_OK;
-  if (m->wt_ver != m->wver) {
-    if (m->WbT.empty())
-      for (int l = 0; l <= m->layers; l++) {
-        uint16_t *q = nullptr;
-        NB_MHIP(m, hipMalloc((void **)&q, (size_t)m->in_dim[l] * m->out_dim[l] * 2));
-        m->WbT.push_back(q);
-      }
-    for (int l = 0; l <= m->layers; l++) {
-      const int K = m->in_dim[l], N = m->out_dim[l];
-      hipLaunchKernelGGL(k_transpose_bf16, dim3(nblk((int64_t)K * N)), dim3(256), 0, st,
-                         m->Wb[l], K, N, m->WbT[l]);
-    }
-    NB_MHIP(m, hipGetLastError());
-    m->wt_ver = m->wver;
-  }
+  int rc = transposed_weights(m, st);
+  if (rc) return rc;
   InferArgs a;
   a.x = x_dev;
   a.rows = (int)rows;
@@ -901,6 +1304,7 @@ void nb_mlp_destroy(nb_mlp *m) {
   (void)hipSetDevice(m->device);
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   free_rows(m);
+  free_train(m);
   for (auto *v : {&m->W, &m->Wg, &m->Wm1, &m->Wm2, &m->bvec, &m->bg, &m->bm1, &m->bm2})
     for (float *q : *v) (void)hipFree(q);
   for (uint16_t *q : m->Wb) (void)hipFree(q);
@@ -971,8 +1375,8 @@ static int xfer_params(nb_mlp *m, float *host, int64_t count, bool to_dev, bool 
                          m->stream, W, m->Wb[l], (int64_t)full.size());
       NB_MHIP(m, hipStreamSynchronize(m->stream));
     } else {
-      NB_MHIP(m, hipMemcpy(full.data(), W, full.size() * 4, hipMemcpyDeviceToHost));
-      NB_MHIP(m, hipMemcpy(bf.data(), b, bf.size() * 4, hipMemcpyDeviceToHost));
+      const Fetch seg[2] = {{full.data(), W, full.size() * 4}, {bf.data(), b, bf.size() * 4}};
+      NB_MHIP(m, stage_fetch(seg, 2, m->stream));
       for (int i = 0; i < in; i++)
         for (int j = 0; j < o; j++) host[off + (int64_t)i * o + j] = full[(size_t)i * op + j];
       for (int j = 0; j < o; j++) host[off + (int64_t)in * o + j] = bf[j];
@@ -1056,29 +1460,45 @@ int nb_mlp_train(nb_mlp *m, const float *x, const float *t, int64_t rows, int32_
   if (hipMemcpy(dx, x, (size_t)rows * m->din * 4, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(dt, t, (size_t)rows * m->dout * 4, hipMemcpyHostToDevice) != hipSuccess)
     rc = NB_E_HIP;
+  // the losses of the last tenth of the steps, kept on the device and read in one copy at the end
+  // (whenever 64 MiB of them are there)
+  const int loss_steps = std::max(1, (16 << 20) / batch);
   double lsum = 0;
-  int lcount = 0;
+  int lcount = 0, held = 0;
   const int64_t nb = rows / batch;
-  std::vector<float> l((size_t)batch);
+  const int last = std::max(1, steps / 10);
+  float *dl = nullptr;
+  std::vector<float> l;
+  if (!rc && steps > 0 &&
+      hipMalloc((void **)&dl, (size_t)std::min(last, loss_steps) * batch * 4) != hipSuccess)
+    rc = NB_E_NOMEM;
   for (int s = 0; s < steps && !rc; s++) {
     const int64_t b0 = (s % nb) * batch;
-    rc = nb::mlp_train_step_device(m, dx + b0 * m->din, dt + b0 * m->dout, batch, lr, m->stream);
-    if (!rc && s >= steps - std::max(1, steps / 10)) {
-      if (hipMemcpyAsync(l.data(), m->lrow, l.size() * 4, hipMemcpyDeviceToHost, m->stream) !=
+    const bool count = s >= steps - last;
+    rc = nb::mlp_train_step_device(m, dx + b0 * m->din, dt + b0 * m->dout, batch, lr,
+                                   count ? dl + (size_t)held * batch : nullptr, m->stream);
+    if (rc || !count) continue;
+    if (++held == loss_steps || s + 1 == steps) {
+      l.resize((size_t)held * batch);
+      if (hipMemcpyAsync(l.data(), dl, l.size() * 4, hipMemcpyDeviceToHost, m->stream) !=
               hipSuccess ||
           hipStreamSynchronize(m->stream) != hipSuccess) {
         rc = NB_E_HIP;
         break;
       }
-      double q = 0;
-      for (float v : l) q += v;
-      lsum += q / ((double)batch * m->dout);
-      lcount++;
+      for (int k = 0; k < held; k++) {
+        double q = 0;
+        for (int r = 0; r < batch; r++) q += l[(size_t)k * batch + r];
+        lsum += q / ((double)batch * m->dout);
+        lcount++;
+      }
+      held = 0;
     }
   }
   (void)hipStreamSynchronize(m->stream);
   (void)hipFree(dx);
   (void)hipFree(dt);
+  if (dl) (void)hipFree(dl);
   if (loss_out) *loss_out = lcount ? (float)(lsum / lcount) : 0.f;
   return rc;
 }

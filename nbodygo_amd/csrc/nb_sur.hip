@@ -35,8 +35,6 @@ namespace nb {
 
 int mlp_infer_device(nb_mlp *m, const float *x_dev, int64_t rows, float *y_dev,
                      hipStream_t st);
-int mlp_train_step_device(nb_mlp *m, const float *x_dev, const float *t_dev, int64_t rows,
-                          float lr, hipStream_t st);
 
 constexpr int kCellRec = 16;  // COM(3), M, Qxx, Qyy, Qzz, Qxy, Qxz, Qyz, radius, ix, iy, iz, n, 0
 constexpr int kFarRec = 36;   // a(3), J(6: xx yy zz xy xz yz), H(10), T(15), 0, 0
