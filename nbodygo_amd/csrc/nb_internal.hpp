@@ -263,6 +263,9 @@ __device__ __forceinline__ float to_vgpr(float s) {
   return v;
 }
 
+// One row of independent instructions ends here: the scheduler keeps rows apart.
+#define NB_ROW __builtin_amdgcn_sched_barrier(0);
+
 // ---- kernels launched from nb_api.cpp (defined in the .hip files) ----------------------------
 struct ForceArgs {
   const float4 *js;

@@ -65,6 +65,7 @@ struct Sur {
   void *sort_tmp = nullptr;
   size_t sort_bytes = 0;
   int32_t *cstart = nullptr, *ccount = nullptr, *nelist = nullptr, *necount = nullptr;
+  float *srad = nullptr;                 // radii in sorted order, rounded up (collisions)
   float4 *sp = nullptr;
   float *crec = nullptr, *crec_ne = nullptr, *fexp = nullptr, *part = nullptr, *feat = nullptr;
   int2 *items = nullptr, *btot = nullptr;
@@ -297,12 +298,19 @@ __global__ __launch_bounds__(1024) void k_sur_scan(const int32_t *cstart, int nc
   for (int j = 0; j < b; j++) items[q + j] = make_int2(c, j);
 }
 
+__device__ __forceinline__ float round_up_f(double d) {  // smallest float >= d (d >= 0)
+  float f = (float)d;
+  if ((double)f < d) f = __uint_as_float(__float_as_uint(f) + 1u);
+  return f;
+}
+
 __global__ void k_sur_gather(const uint32_t *perm, const uint32_t *keys2, int n, int ncell,
                              const double *x, const double *y, const double *z, const double *m,
-                             const double *center, float4 *sp) {
+                             const double *center, float4 *sp, const double *r, float *srad) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n || (int)keys2[k] >= ncell) return;
   const uint32_t i = perm[k];
+  if (r) srad[k] = round_up_f(r[i]);
   sp[k] = make_float4((float)(x[i] - center[0]), (float)(y[i] - center[1]),
                       (float)(z[i] - center[2]), (float)m[i]);
 }
@@ -681,19 +689,58 @@ __device__ __forceinline__ void near_pair(float4 b, float4 me, float eps2, float
   near_pair(f4v{b.x, b.y, b.z, b.w}, me, eps2, px, py, pz);
 }
 
-// near_pair that also keeps the smallest r^2 = d^2 + eps^2 seen (collision candidates).
-__device__ __forceinline__ void near_pair_min(float4 b, float4 me, float eps2, float &px,
-                                              float &py, float &pz, float &r2min) {
-  const float dx = b.x - me.x, dy = b.y - me.y, dz = b.z - me.z;
-  float r2 = __builtin_fmaf(dx, dx, eps2);
-  r2 = __builtin_fmaf(dy, dy, r2);
-  r2 = __builtin_fmaf(dz, dz, r2);
-  r2min = fminf(r2min, r2);
-  const float inv = __builtin_amdgcn_rsqf(r2);
-  const float s = b.w * inv * inv * inv;
-  px = __builtin_fmaf(dx, s, px);
-  py = __builtin_fmaf(dy, s, py);
-  pz = __builtin_fmaf(dz, s, pz);
+// near_pair for four sources, row by row with the order pinned: neighbouring instructions are then
+// independent, which is what lets gfx950 issue two at a time.  The sums take the sources in order.
+// The next four (`tn`, LDS) are requested into b once it is used up.
+// MIN also keeps the smallest r^2 = d^2 + eps^2 seen (collision candidates), source `skip` left out.
+template <bool MIN>
+__device__ __forceinline__ void near_four(float4 (&b)[4], const float4 *tn, float4 me, float eps2,
+                                          float &px, float &py, float &pz, float &r2min,
+                                          int skip) {
+  float dx[4], dy[4], dz[4], r2[4], s[4], inv[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) dx[k] = b[k].x - me.x;
+  NB_ROW
+#pragma unroll
+  for (int k = 0; k < 4; k++) dy[k] = b[k].y - me.y;
+  NB_ROW
+#pragma unroll
+  for (int k = 0; k < 4; k++) r2[k] = __builtin_fmaf(dx[k], dx[k], eps2);
+  NB_ROW
+#pragma unroll
+  for (int k = 0; k < 4; k++) dz[k] = b[k].z - me.z;
+  NB_ROW
+#pragma unroll
+  for (int k = 0; k < 4; k++) r2[k] = __builtin_fmaf(dy[k], dy[k], r2[k]);
+  NB_ROW
+#pragma unroll
+  for (int k = 0; k < 4; k++) r2[k] = __builtin_fmaf(dz[k], dz[k], r2[k]);
+  NB_ROW
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    inv[k] = __builtin_amdgcn_rsqf(r2[k]);
+    if (MIN) r2min = fminf(r2min, k == skip ? FLT_MAX : r2[k]);
+  }
+  NB_ROW
+#pragma unroll
+  for (int k = 0; k < 4; k++) s[k] = b[k].w * inv[k];
+  NB_ROW
+#pragma unroll
+  for (int k = 0; k < 4; k++) b[k] = tn[k];
+  NB_ROW
+#pragma unroll
+  for (int k = 0; k < 4; k++) s[k] *= inv[k];
+  NB_ROW
+#pragma unroll
+  for (int k = 0; k < 4; k++) s[k] *= inv[k];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    NB_ROW
+    px = __builtin_fmaf(dx[k], s[k], px);
+    py = __builtin_fmaf(dy[k], s[k], py);
+    pz = __builtin_fmaf(dz[k], s[k], pz);
+  }
+  NB_ROW
 }
 
 struct NearArgs {
@@ -710,6 +757,7 @@ struct NearArgs {
   double *near_pairs;
   // collision detection (near field only; the grid keeps every overlapping pair adjacent)
   const uint32_t *perm;                // sorted position -> body index
+  const float *srad;                   // radii in sorted order, rounded up
   const double *x, *y, *z, *r;         // FP64 state
   const int32_t *beh;
   uint64_t *pairs;
@@ -717,12 +765,6 @@ struct NearArgs {
   int64_t pair_cap;
   int events;
 };
-
-__device__ __forceinline__ float round_up_f(double d) {  // smallest float >= d (d >= 0)
-  float f = (float)d;
-  if ((double)f < d) f = __uint_as_float(__float_as_uint(f) + 1u);
-  return f;
-}
 
 __device__ __forceinline__ float wave_maxf(float v) {
 #pragma unroll
@@ -767,8 +809,10 @@ __device__ void exact_chunk_pairs(const NearArgs &a, uint32_t i, int s0, int cnt
 // LDS: one 3 KB region per wave, used in turn for the wave's source tile (64 float4, 128 with
 // collisions), its staged shell records (64 x 3 float4) and, in waves 1-3, its partial sums for
 // wave 0 (3 x 64 doubles): 12 KB per workgroup.  Without collisions the kernel is held to 64
-// VGPRs, so 8 waves fit per SIMD; with collisions it is held to 80 VGPRs (6 waves per SIMD, no
-// spills; 94 VGPRs and 5 waves unconstrained).
+// VGPRs, so 8 waves fit per SIMD; with collisions to 96 (5 waves: 10.9 ms at 1,048,576 bodies in
+// two spheres, 64^3 cells; 6 waves spill, 11.2 ms).  Bound by FP32 issue: 14 instructions a pair
+// with collisions (the pair's own 13), 36e9 pairs, 3,300 G pairs/s at the 2.0 GHz that the card
+// holds here.  Sums before pinning the rows, and radii gathered through perm: 12.2 ms.
 template <bool COLL>
 __device__ __forceinline__ void near_item(const NearArgs &a, const int item,
                                           float4 (*wlds)[64 * 3]) {
@@ -800,7 +844,7 @@ __device__ __forceinline__ void near_item(const NearArgs &a, const int item,
   float ri = 0.f, me_inf = 0.f;
   if (COLL && tv) {
     i_body = a.perm[k];
-    ri = round_up_f(a.r[i_body]);
+    ri = a.srad[k];
     me_inf = fmaxf(fabsf(me.x), fmaxf(fabsf(me.y), fabsf(me.z)));
   }
   // The sources are the bodies of the 3 x 3 rows of three adjacent cells around the cell, each
@@ -863,7 +907,7 @@ __device__ __forceinline__ void near_item(const NearArgs &a, const int item,
           const float4 src = e < cnt ? a.sp[s0 + e] : make_float4(0.f, 0.f, 0.f, 0.f);
           tl[e] = src;
           if (COLL && e < cnt) {
-            rmax_c = fmaxf(rmax_c, round_up_f(a.r[a.perm[s0 + e]]));
+            rmax_c = fmaxf(rmax_c, a.srad[s0 + e]);
             xmax_c = fmaxf(xmax_c, fmaxf(fabsf(src.x), fmaxf(fabsf(src.y), fabsf(src.z))));
           }
         }
@@ -880,36 +924,25 @@ __device__ __forceinline__ void near_item(const NearArgs &a, const int item,
         const int cntp = (cnt + q4 - 1) / q4 * q4;
         const int len = cntp / copies;
         const float4 *tc = tl + cp * len;
+        // four sources a step, the next four on their way
+        auto walk = [&](auto min_k, auto own_k) {
+          constexpr bool MIN = decltype(min_k)::value, OWN = decltype(own_k)::value;
+          float4 b[4];
+#pragma unroll
+          for (int u = 0; u < 4; u++) b[u] = tc[u];
+          for (int j = 0; j < len; j += 4)
+            near_four<MIN>(b, tc + min(j + 4, len - 4), me, eps2, px, py, pz, r2min,
+                           OWN ? k - s0 - cp * len - j : -1);
+        };
         if (COLL) {
-          // the body's own entry (r^2 = eps^2) must not count as a candidate
-          if (s0 < t_end && s0 + cnt > t_begin) {
-            const int self = k - s0;
-            const int j1 = min(cp * len + len, cnt);
-            for (int j = cp * len; j < j1; j++) {
-              const float keep = r2min;
-              near_pair_min(tl[j], me, eps2, px, py, pz, r2min);
-              if (j == self) r2min = keep;
-            }
-          } else {
-            // zero-mass padding may only add candidates (an exact pass over the real sources)
-            for (int j = 0; j < len; j += 4) {
-              const float4 b0 = tc[j], b1 = tc[j + 1], b2 = tc[j + 2], b3 = tc[j + 3];
-              near_pair_min(b0, me, eps2, px, py, pz, r2min);
-              near_pair_min(b1, me, eps2, px, py, pz, r2min);
-              near_pair_min(b2, me, eps2, px, py, pz, r2min);
-              near_pair_min(b3, me, eps2, px, py, pz, r2min);
-            }
-          }
+          // the body's own entry (r^2 = eps^2) must not count as a candidate; zero-mass padding may
+          // only add candidates (an exact pass over the real sources)
+          if (s0 < t_end && s0 + cnt > t_begin) walk(std::true_type{}, std::true_type{});
+          else walk(std::true_type{}, std::false_type{});
           // the chunk's minimum over all copies, for the target's one decision below
           for (int o = cwid; o < 64; o <<= 1) r2min = fminf(r2min, __shfl_xor(r2min, o));
         } else {
-          for (int j = 0; j < len; j += 4) {
-            const float4 b0 = tc[j], b1 = tc[j + 1], b2 = tc[j + 2], b3 = tc[j + 3];
-            near_pair(b0, me, eps2, px, py, pz);
-            near_pair(b1, me, eps2, px, py, pz);
-            near_pair(b2, me, eps2, px, py, pz);
-            near_pair(b3, me, eps2, px, py, pz);
-          }
+          walk(std::false_type{}, std::false_type{});
         }
         wave_lds_sync();
         if (COLL && tv && cp == 0) {
@@ -1063,7 +1096,7 @@ __device__ __forceinline__ void near_item(const NearArgs &a, const int item,
 // further items; the barrier between two items keeps wave 0's reads of the partial sums ahead of
 // the other waves' next writes).
 template <bool COLL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(COLL ? 6 : 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(COLL ? 5 : 8)))
 void k_sur_near(NearArgs a) {
   __shared__ float4 wlds[4][64 * 3];
   const int nitems = *a.nitems;
@@ -1339,7 +1372,7 @@ void sur_free(Sur *s) {
   if (!s) return;
   if (s->nitems_host) (void)hipHostFree(s->nitems_host);
   void *ptrs[] = {s->keys, s->keys2, s->perm_in, s->perm, s->sort_tmp, s->cstart, s->ccount,
-                  s->nelist, s->necount, s->sp, s->crec, s->crec_ne, s->fexp, s->part,
+                  s->nelist, s->necount, s->sp, s->srad, s->crec, s->crec_ne, s->fexp, s->part,
                   s->items, s->nitems, s->btot, s->feat, s->base, s->center,
                   s->red, s->mu, s->sd, s->tx, s->ty, s->sidx, s->sexact, s->serr, s->flag,
                   s->sbody,
@@ -1365,6 +1398,7 @@ static int sur_ensure_bodies(Ctx *c) {
   NB_HIP(c, salloc(&s->perm_in, n));
   NB_HIP(c, salloc(&s->perm, n));
   NB_HIP(c, salloc(&s->sp, n));
+  NB_HIP(c, salloc(&s->srad, n));
   NB_HIP(c, salloc(&s->base, n));
   NB_HIP(c, salloc(&s->ymlp, n * 3));
   NB_HIP(c, salloc(&s->feat, n * kFeat));
@@ -1447,7 +1481,7 @@ static int sur_pipeline(Ctx *c, bool feat_raw, bool feat_norm, bool apply, bool 
                      s->cstart, ncell, s->btot, s->ccount, s->nelist, s->necount, s->items,
                      s->nitems, s->nitems_host_dev);
   hipLaunchKernelGGL(k_sur_gather, dim3(nb256(n)), dim3(256), 0, st, s->perm, s->keys2, n, ncell,
-                     c->x, c->y, c->z, c->m, s->center, s->sp);
+                     c->x, c->y, c->z, c->m, s->center, s->sp, detect ? c->r : nullptr, s->srad);
   hipLaunchKernelGGL(k_sur_moments, dim3((unsigned)ncell), dim3(64), 0, st, s->sp, s->cstart,
                      s->nelist, s->necount, G, s->crec, s->crec_ne);
   const float eps2 = (float)(c->p.eps * c->p.eps);
@@ -1476,6 +1510,7 @@ static int sur_pipeline(Ctx *c, bool feat_raw, bool feat_norm, bool apply, bool 
   na.r0 = (float)s->r0;
   na.near_pairs = s->near_pairs;
   na.perm = s->perm;
+  na.srad = s->srad;
   na.x = c->x;
   na.y = c->y;
   na.z = c->z;

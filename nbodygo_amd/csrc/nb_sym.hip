@@ -71,9 +71,6 @@ __device__ __forceinline__ void exact_tile(const SymArgs &a, Buf &found, int i, 
   found.add(a.pairs, a.ctr, a.pair_cap, min(i, j), max(i, j));
 }
 
-// One row of independent instructions ends here: the scheduler keeps rows apart.
-#define NB_ROW __builtin_amdgcn_sched_barrier(0);
-
 template <int IPL, int W, bool DETECT>
 struct SymLds {
   float4 sh[2][128];
