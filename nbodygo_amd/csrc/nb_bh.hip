@@ -686,27 +686,40 @@ __global__ __launch_bounds__(256) void k_bh_force(BhForceArgs a) {
 // 64 + 2 kBhGroupSpan bodies (or is one body, or one bucket).  Each group shares one traversal.
 // Without the cut, a run that straddles two large cells takes a box spanning both and opens
 // everything inside it to the leaves (on a Plummer sphere one such wave met 261,464 of the
-// 262,144 bodies and set the kernel's duration).  A node is accepted for the whole group when 2 half < theta * sqrt(d_box^2 + soft^2), d_box being
-// its centre of mass's distance to the group's bounding box: every body of the group is then at
-// least that far away, so each would accept it by the reference's own test (octree.go:299-309);
-// otherwise the node is opened.  The walk is breadth-parallel: each step pops up to 8 nodes from
-// a per-wave LDS stack and the 64 lanes examine their 64 child slots at once; accepted nodes and
-// leaves go to an LDS list of terms, opened nodes back to the stack.  Every 64 listed terms are
-// evaluated by all lanes against their own bodies like the direct FP32 kernel (sources broadcast
-// from LDS, coordinates relative to the group's centre, r^-3 from v_rsq_f32), the list's partial
-// sums are added into FP64 per lane, and the self term is skipped by body index.
+// 262,144 bodies and set the kernel's duration).  A node is accepted for the whole group when
+// 2 half < theta * sqrt(d_box^2 + soft^2), d_box being its centre of mass's distance to the
+// group's bounding box: every body of the group is then at least that far away, so each would
+// accept it by the reference's own test (octree.go:299-309); otherwise the node is opened.
+// A workgroup has the 64 bodies.  Its first wave walks: each step pops up to 8 nodes from an LDS
+// stack and the 64 lanes examine their 64 child slots at once; accepted nodes and leaves go to an
+// LDS list of terms, opened nodes back to the stack, and the next slots are requested before the
+// terms are listed.  The other three waves evaluate the list, 64 terms in a row each, a body per
+// lane, like the direct FP32 kernel (sources broadcast from LDS, coordinates relative to the
+// group's centre, r^-3 from v_rsq_f32), while the first fills another.  Each 64 terms' sums are
+// added into FP64 per lane; the self term is skipped by body index.  The walk is about a quarter of
+// the instructions and a chain of dependent loads; terms are 10,000 a body at theta 0.3 and want
+// all the issue slots.  One wave doing both, 64 bodies to each, left the longest of four waves a
+// SIMD 1.5 times over the mean: 2.35 ms for 262,144 bodies in a Plummer sphere (2.09 with the
+// terms' rows pinned and the slots requested ahead) against 1.65 now, and a step of 100,003 bodies
+// 1.99 ms against 1.17.  Two evaluating waves 2.55 ms a step of 262,144, three 2.36, four 2.42.
 constexpr int kBhGroupSpan = 512;   // see the group cut above
-// Per-wave stack entries.  The stack stays sorted by depth (each step pops the deepest entries
+// Stack entries.  The stack stays sorted by depth (each step pops the deepest entries
 // and pushes their children on top), so entries of depth d can only be pushed by a step that
 // popped every deeper-or-equal entry: at most 64 entries per depth, 21 depths below the root.
 constexpr int kBhFastStack = 64 * kBhLevels;
-constexpr int kBhFastList = 128;    // per-wave term list (< 64 kept + up to 64 added per step)
+constexpr int kBhFastEval = 3;      // waves of a workgroup that evaluate terms (one lists them)
+constexpr int kBhFastOut = 64 * kBhFastEval;        // terms handed over at a time
+constexpr int kBhFastList = kBhFastOut + 64;  // < 64 kept + up to 64 added per step
 
-struct BhFastLds {
-  int32_t stack[kBhFastStack];
+// A list of terms on its way from the listing wave to the others.
+struct BhFastSet {
   float4 term[kBhFastList];
   int32_t tidx[kBhFastList];  // body (sorted index) of a leaf term, -1 for a node
-  int32_t top, len;
+  int32_t len, ga, gb, last;  // terms, the group's lanes, whether this is the workgroup's last list
+};
+struct BhFastLds {
+  BhFastSet set[2];
+  int32_t stack[kBhFastStack];
 };
 
 __device__ __forceinline__ void fast_sync() {
@@ -715,82 +728,106 @@ __device__ __forceinline__ void fast_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// The first `cnt` listed terms against the lane's body; the rest of the list moves to the front.
-__device__ __forceinline__ void fast_flush(BhFastLds &L, int cnt, float tx, float ty, float tz,
-                                           float soft2, int s, bool act, double &ax, double &ay,
-                                           double &az, unsigned long long &nint) {
+// This lane's place among the lanes set in `bal`.
+__device__ __forceinline__ int lanes_below(unsigned long long bal) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0));
+}
+
+// Listed terms j .. j + T - 1 against the lane's body.  Four at a time they go row by row with the
+// order pinned (neighbouring instructions are then independent, which is what lets gfx950 issue two
+// at a time); the sums take them in order.  OWN: one of them may be the body itself.
+template <int T, bool OWN>
+__device__ __forceinline__ void fast_terms(const BhFastSet &L, int j, float tx, float ty, float tz,
+                                           float sf, int s, float &px, float &py, float &pz) {
+  float4 e[T];
+  float dx[T], dy[T], dz[T], r2[T], inv[T], w[T];
+#define NB_T _Pragma("unroll") for (int k = 0; k < T; k++)
+  NB_T e[k] = L.term[j + k];
+  NB_ROW
+  NB_T dx[k] = e[k].x - tx;
+  NB_ROW
+  NB_T dy[k] = e[k].y - ty;
+  NB_ROW
+  NB_T r2[k] = __builtin_fmaf(dx[k], dx[k], sf);
+  NB_ROW
+  NB_T dz[k] = e[k].z - tz;
+  NB_ROW
+  NB_T r2[k] = __builtin_fmaf(dy[k], dy[k], r2[k]);
+  NB_ROW
+  NB_T r2[k] = __builtin_fmaf(dz[k], dz[k], r2[k]);
+  NB_ROW
+  NB_T inv[k] = __builtin_amdgcn_rsqf(r2[k]);
+  NB_ROW
+  NB_T w[k] = e[k].w * inv[k];
+  NB_ROW
+  NB_T inv[k] *= inv[k];
+  NB_ROW
+  NB_T w[k] *= inv[k];
+  if (OWN) {
+    NB_T w[k] = L.tidx[j + k] == s ? 0.f : w[k];
+  }
+  NB_T {
+    NB_ROW
+    px = __builtin_fmaf(dx[k], w[k], px);
+    py = __builtin_fmaf(dy[k], w[k], py);
+    pz = __builtin_fmaf(dz[k], w[k], pz);
+  }
+  NB_ROW
+#undef NB_T
+}
+
+// Listed terms j0 .. j0 + cnt - 1 (64, fewer at a group's end) against the lane's body: one FP32
+// partial sum each.
+__device__ __forceinline__ void fast_chunk(const BhFastSet &L, int j0, int cnt, float tx, float ty,
+                                           float tz, float sf, int s, int g0, int g1, float &px,
+                                           float &py, float &pz) {
   const int lane = threadIdx.x & 63;
-  float px = 0.f, py = 0.f, pz = 0.f;
-  const float sf = to_vgpr(soft2);
-  for (int j = 0; j < cnt; j++) {
-    const float4 e = L.term[j];
-    const int id = L.tidx[j];
-    const float dx = e.x - tx, dy = e.y - ty, dz = e.z - tz;
-    float r2 = __builtin_fmaf(dx, dx, sf);
-    r2 = __builtin_fmaf(dy, dy, r2);
-    r2 = __builtin_fmaf(dz, dz, r2);
-    const float inv = __builtin_amdgcn_rsqf(r2);
-    float w = e.w * inv;
-    w = w * (inv * inv);
-    w = id == s ? 0.f : w;
-    px = __builtin_fmaf(dx, w, px);
-    py = __builtin_fmaf(dy, w, py);
-    pz = __builtin_fmaf(dz, w, pz);
+  const int id = lane < cnt ? L.tidx[j0 + lane] : -1;
+  const int c4 = j0 + (cnt & ~3), c1 = j0 + cnt;
+  if (__builtin_amdgcn_ballot_w64(id >= g0 && id < g1)) {  // the group's own bodies are rare
+    for (int j = j0; j < c4; j += 4) fast_terms<4, true>(L, j, tx, ty, tz, sf, s, px, py, pz);
+    for (int j = c4; j < c1; j++) fast_terms<1, true>(L, j, tx, ty, tz, sf, s, px, py, pz);
+  } else {
+    for (int j = j0; j < c4; j += 4) fast_terms<4, false>(L, j, tx, ty, tz, sf, s, px, py, pz);
+    for (int j = c4; j < c1; j++) fast_terms<1, false>(L, j, tx, ty, tz, sf, s, px, py, pz);
   }
-  if (act) {
-    ax += px;
-    ay += py;
-    az += pz;
-    nint += (unsigned long long)cnt;
-  }
-  fast_sync();
-  const int rest = L.len - cnt;
-  float4 mv = make_float4(0.f, 0.f, 0.f, 0.f);
-  int mi = -1;
-  if (lane < rest) {
-    mv = L.term[cnt + lane];
-    mi = L.tidx[cnt + lane];
-  }
-  fast_sync();
-  if (lane < rest) {
-    L.term[lane] = mv;
-    L.tidx[lane] = mi;
-  }
-  if (lane == 0) L.len = rest;
-  fast_sync();
 }
 
-// Appends one term per lane that has one (wave-wide, in lane order).
-__device__ __forceinline__ void fast_append(BhFastLds &L, bool has, float4 t, int id) {
-  const unsigned long long bal = __builtin_amdgcn_ballot_w64(has);
-  const int base = L.len;
-  if (has) {
-    const int pos = base + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
-                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0));
-    L.term[pos] = t;
-    L.tidx[pos] = id;
-  }
-  fast_sync();
-  if ((threadIdx.x & 63) == 0) L.len = base + __builtin_popcountll(bal);
-  fast_sync();
+// The box of the lanes of a group: centre and half extents (FP64), the same on every lane.
+struct BhBox {
+  double cx, cy, cz, hx, hy, hz;
+};
+__device__ __forceinline__ BhBox fast_box(bool mine, double px, double py, double pz) {
+  double glo[3] = {mine ? px : DBL_MAX, mine ? py : DBL_MAX, mine ? pz : DBL_MAX};
+  double ghi[3] = {mine ? px : -DBL_MAX, mine ? py : -DBL_MAX, mine ? pz : -DBL_MAX};
+  for (int o = 32; o > 0; o >>= 1)
+    for (int d = 0; d < 3; d++) {
+      glo[d] = fmin(glo[d], __shfl_xor(glo[d], o));
+      ghi[d] = fmax(ghi[d], __shfl_xor(ghi[d], o));
+    }
+  return BhBox{0.5 * (glo[0] + ghi[0]), 0.5 * (glo[1] + ghi[1]), 0.5 * (glo[2] + ghi[2]),
+               0.5 * (ghi[0] - glo[0]), 0.5 * (ghi[1] - glo[1]), 0.5 * (ghi[2] - glo[2])};
 }
 
-__global__ __launch_bounds__(256) void k_bh_force_fast(BhForceArgs a) {
-  __shared__ BhFastLds lds[4];
+__global__ __launch_bounds__(64 * (1 + kBhFastEval)) void k_bh_force_fast(BhForceArgs a) {
+  __shared__ BhFastLds L;
   __shared__ double h2s[kBhLevels + 1];
+  __shared__ double part[kBhFastEval][3][64];
+  __shared__ unsigned long long nints[kBhFastEval];
   const int M = a.cnt->M;
   if (M < 2) return;
   bh_half2_table(a.nbox, h2s);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  BhFastLds &L = lds[wv];
-  const int s = (blockIdx.x * 4 + wv) * 64 + lane;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int s = blockIdx.x * 64 + lane;
   bool act = s < M;
   int i = -1;
   if (act) {
     i = a.perm[s];
     act = !(a.flags[i] & NB_F_SUN);  // suns sum directly
   }
-  if (__builtin_amdgcn_ballot_w64(act) == 0) return;
+  if (__builtin_amdgcn_ballot_w64(act) == 0) return;  // the same in all four waves
   const double px = act ? a.sx[s] : 0, py = act ? a.sy[s] : 0, pz = act ? a.sz[s] : 0;
   // the group cut (wave-uniform): bit j of `starts` marks a group starting at lane j
   const int wbase = s - lane, nl = min(64, M - wbase);
@@ -822,68 +859,134 @@ __global__ __launch_bounds__(256) void k_bh_force_fast(BhForceArgs a) {
     }
     if (!cut) fin |= 1ull << ga;
   }
+  if (wv > 0) {  // evaluates the listed terms: 64 in a row to each of these waves in turn
+    double ax = 0, ay = 0, az = 0;
+    unsigned long long nint = 0;
+    float tx = 0.f, ty = 0.f, tz = 0.f;
+    bool mine = false;
+    const float sf = to_vgpr((float)a.soft2);
+    int ga = -1;
+    for (int set = 0;; set ^= 1) {
+      __syncthreads();
+      const BhFastSet &S = L.set[set];
+      const int len = S.len;
+      if (len > 0) {
+        const int gb = S.gb;
+        if (S.ga != ga) {  // another group: its bodies about its box's centre
+          ga = S.ga;
+          mine = act && lane >= ga && lane < gb;
+          const BhBox bx = fast_box(mine, px, py, pz);
+          tx = (float)(px - bx.cx);
+          ty = (float)(py - bx.cy);
+          tz = (float)(pz - bx.cz);
+        }
+        for (int j0 = (wv - 1) * 64; j0 < len; j0 += 64 * kBhFastEval) {
+          const int cnt = min(64, len - j0);
+          float qx = 0.f, qy = 0.f, qz = 0.f;
+          fast_chunk(S, j0, cnt, tx, ty, tz, sf, s, wbase + ga, wbase + gb, qx, qy, qz);
+          if (mine) {
+            ax += qx;
+            ay += qy;
+            az += qz;
+            nint += (unsigned long long)cnt;
+          }
+        }
+      }
+      if (S.last) break;
+    }
+    part[wv - 1][0][lane] = ax;
+    part[wv - 1][1][lane] = ay;
+    part[wv - 1][2][lane] = az;
+    for (int o = 32; o > 0; o >>= 1) nint += __shfl_xor(nint, o);
+    if (lane == 0) nints[wv - 1] = nint;
+    __syncthreads();
+    return;
+  }
+  // the first wave walks the tree and lists the terms; the others wait for it
   const double th2 = a.theta * a.theta, soft2 = a.soft2;
-  double ax = 0, ay = 0, az = 0;
-  unsigned long long nint = 0;
   bool overflow = false;
   const int node_lim = (int)min(a.node_cap, (int64_t)INT32_MAX / 8);
-  for (unsigned long long segs = starts; segs && !overflow;) {
-    const int ga = __builtin_ctzll(segs);
+  int set = 0, len = 0;  // the list being filled and its length
+  int ga = 0, gb = 0;
+  // The list goes to the evaluating waves, all of it at a group's end, else the whole rounds of 64;
+  // what is left starts the other list.
+  auto hand_over = [&](bool end, bool last) {
+    BhFastSet &S = L.set[set], &N = L.set[set ^ 1];
+    const int out = end ? len : kBhFastOut, rest = len - out;
+    float4 mv = make_float4(0.f, 0.f, 0.f, 0.f);
+    int mi = -1;
+    if (lane < rest) {
+      mv = S.term[out + lane];
+      mi = S.tidx[out + lane];
+    }
+    if (lane == 0) {
+      S.len = out;
+      S.ga = ga;
+      S.gb = gb;
+      S.last = last;
+    }
+    __syncthreads();  // the others are done with the other list and start on this one
+    if (lane < rest) {
+      N.term[lane] = mv;
+      N.tidx[lane] = mi;
+    }
+    set ^= 1;
+    len = rest;
+  };
+  // One term per lane that has one, in lane order.
+  auto append = [&](bool has, float4 t, int id) {
+    const unsigned long long bal = __builtin_amdgcn_ballot_w64(has);
+    if (has) {
+      const int pos = len + lanes_below(bal);
+      L.set[set].term[pos] = t;
+      L.set[set].tidx[pos] = id;
+    }
+    len += __builtin_popcountll(bal);
+    if (len >= kBhFastOut) hand_over(false, false);
+  };
+  for (unsigned long long segs = starts; segs;) {
+    ga = __builtin_ctzll(segs);
     segs &= segs - 1;
-    const int gb = segs ? __builtin_ctzll(segs) : nl;
+    gb = segs ? __builtin_ctzll(segs) : nl;
     const bool mine = act && lane >= ga && lane < gb;
     if (__builtin_amdgcn_ballot_w64(mine) == 0) continue;
-    // the group's box (FP64)
-    double glo[3] = {mine ? px : DBL_MAX, mine ? py : DBL_MAX, mine ? pz : DBL_MAX};
-    double ghi[3] = {mine ? px : -DBL_MAX, mine ? py : -DBL_MAX, mine ? pz : -DBL_MAX};
-    for (int o = 32; o > 0; o >>= 1)
-      for (int d = 0; d < 3; d++) {
-        glo[d] = fmin(glo[d], __shfl_xor(glo[d], o));
-        ghi[d] = fmax(ghi[d], __shfl_xor(ghi[d], o));
-      }
-    const double cx = 0.5 * (glo[0] + ghi[0]), cy = 0.5 * (glo[1] + ghi[1]),
-                 cz = 0.5 * (glo[2] + ghi[2]);
-    const double hx = 0.5 * (ghi[0] - glo[0]), hy = 0.5 * (ghi[1] - glo[1]),
-                 hz = 0.5 * (ghi[2] - glo[2]);
-    const float tx = (float)(px - cx), ty = (float)(py - cy), tz = (float)(pz - cz);
+    const BhBox bx = fast_box(mine, px, py, pz);
     // a node accepted for the group: (2 half)^2 < theta^2 (d_box^2 + soft^2)
     auto accept = [&](double x, double y, double z, double half) {
-      const double ex = fmax(fabs(x - cx) - hx, 0.0), ey = fmax(fabs(y - cy) - hy, 0.0),
-                   ez = fmax(fabs(z - cz) - hz, 0.0);
+      const double ex = fmax(fabs(x - bx.cx) - bx.hx, 0.0), ey = fmax(fabs(y - bx.cy) - bx.hy, 0.0),
+                   ez = fmax(fabs(z - bx.cz) - bx.hz, 0.0);
       return 4.0 * half * half < th2 * (ex * ex + ey * ey + ez * ez + soft2);
     };
-    if (lane == 0) {
-      L.top = 0;
-      L.len = 0;
-    }
-    fast_sync();
+    int top = 0;
     const double4 root = a.nmc[0];
     if (root.w != 0.0) {
       if (accept(root.x, root.y, root.z, a.nbox[0].w)) {
-        fast_append(L, lane == 0, make_float4((float)(root.x - cx), (float)(root.y - cy),
-                                              (float)(root.z - cz), (float)root.w), -1);
+        append(lane == 0, make_float4((float)(root.x - bx.cx), (float)(root.y - bx.cy),
+                                      (float)(root.z - bx.cz), (float)root.w), -1);
       } else {
-        if (lane == 0) {
-          L.stack[0] = 0;
-          L.top = 1;
-        }
-        fast_sync();
+        if (lane == 0) L.stack[0] = 0;
+        top = 1;
       }
     }
-    for (;;) {
-      const int top = L.top;
-      if (top == 0) break;
-      const int nn = min(8, top);
-      const int k = lane >> 3, c = lane & 7;
+    // Pops up to 8 nodes and requests their child slots, one per lane.
+    BhSlot sl;
+    bool have = false;
+    auto pop = [&]() {
+      fast_sync();
+      const int nn = min(8, top), k = lane >> 3;
       const int node = k < nn ? L.stack[top - nn + k] : -1;
+      have = node >= 0 && node < node_lim;
+      if (have) sl = a.slots[(size_t)node * 8 + (lane & 7)];
+      top -= nn;
       fast_sync();
-      if (lane == 0) L.top = top - nn;
-      fast_sync();
+    };
+    bool more = top > 0;
+    if (more) pop();
+    while (more) {
       bool term = false, open = false, bucket = false;
       float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
       int id = -1, code = -1;
-      if (node >= 0 && node < node_lim) {
-        const BhSlot sl = a.slots[(size_t)node * 8 + c];
+      if (have) {
         code = sl.code;
         if (code != -1 && sl.m > 0) {
           if (code <= -2) {  // a leaf: the body's own centre of mass (x*m)/m and mass 0 + m
@@ -897,26 +1000,22 @@ __global__ __launch_bounds__(256) void k_bh_force_fast(BhForceArgs a) {
             open = code < node_lim;
           }
           if (term)
-            t = make_float4((float)(sl.x - cx), (float)(sl.y - cy), (float)(sl.z - cz),
+            t = make_float4((float)(sl.x - bx.cx), (float)(sl.y - bx.cy), (float)(sl.z - bx.cz),
                             (float)sl.m);
         }
       }
-      fast_append(L, term, t, id);
-      if (L.len >= 64) fast_flush(L, 64, tx, ty, tz, (float)soft2, s, mine, ax, ay, az, nint);
-      // opened nodes onto the stack
+      // opened nodes onto the stack, and the next slots requested before the terms are listed
       const unsigned long long bo = __builtin_amdgcn_ballot_w64(open);
-      const int base = L.top, nopen = __builtin_popcountll(bo);
-      if (base + nopen > kBhFastStack) {
+      const int nopen = __builtin_popcountll(bo);
+      if (top + nopen > kBhFastStack) {
         overflow = true;
         break;
       }
-      if (open)
-        L.stack[base + (int)__builtin_amdgcn_mbcnt_hi(
-                           (uint32_t)(bo >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bo, 0))] =
-            code;
-      fast_sync();
-      if (lane == 0) L.top = base + nopen;
-      fast_sync();
+      if (open) L.stack[top + lanes_below(bo)] = code;
+      top += nopen;
+      more = top > 0;
+      if (more) pop();
+      append(term, t, id);
       // buckets (the depth limit): their bodies one by one, 64 at a time
       unsigned long long bb = __builtin_amdgcn_ballot_w64(bucket);
       while (bb) {
@@ -930,25 +1029,33 @@ __global__ __launch_bounds__(256) void k_bh_force_fast(BhForceArgs a) {
           const bool h = q0 + lane < bn;
           float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
           if (h)
-            e = make_float4((float)(a.sx[q] - cx), (float)(a.sy[q] - cy), (float)(a.sz[q] - cz),
-                            (float)a.sm[q]);
-          fast_append(L, h, e, q);
-          if (L.len >= 64)
-            fast_flush(L, 64, tx, ty, tz, (float)soft2, s, mine, ax, ay, az, nint);
+            e = make_float4((float)(a.sx[q] - bx.cx), (float)(a.sy[q] - bx.cy),
+                            (float)(a.sz[q] - bx.cz), (float)a.sm[q]);
+          append(h, e, q);
         }
       }
     }
-    if (L.len > 0) fast_flush(L, L.len, tx, ty, tz, (float)soft2, s, mine, ax, ay, az, nint);
+    hand_over(true, false);
   }
+  hand_over(true, true);  // (empty)
   if (overflow && lane == 0) atomicOr(&a.cnt_w->stack_overflow, 1u);
-  if (act) {
-    const double Gm = a.G * a.sm[s];
-    a.acc[i] = Gm * ax;
-    a.acc[a.npad + i] = Gm * ay;
-    a.acc[2 * a.npad + i] = Gm * az;
+  __syncthreads();
+  if (lane == 0) {
+    unsigned long long nint = 0;
+    for (int v = 0; v < kBhFastEval; v++) nint += nints[v];
+    atomicAdd(&a.cnt_w->interactions, nint);
   }
-  for (int o = 32; o > 0; o >>= 1) nint += __shfl_xor(nint, o);
-  if (lane == 0) atomicAdd(&a.cnt_w->interactions, nint);
+  if (act) {  // the evaluating waves' sums in wave order
+    double f[3];
+    for (int q = 0; q < 3; q++) {
+      f[q] = part[0][q][lane];
+      for (int v = 1; v < kBhFastEval; v++) f[q] += part[v][q][lane];
+    }
+    const double Gm = a.G * a.sm[s];
+    a.acc[i] = Gm * f[0];
+    a.acc[a.npad + i] = Gm * f[1];
+    a.acc[2 * a.npad + i] = Gm * f[2];
+  }
 }
 
 // Suns: directForce from every other existing, non-fragmenting body in array order.
@@ -1270,7 +1377,8 @@ int bh_force_phase(Ctx *c, bool timed, int ev_slot) {
   fa.soft2 = b->p.softening * b->p.softening;
   if (timed) NB_HIP(c, hipEventRecord(c->ev[2 * ev_slot], st));
   if (b->p.mode == 1)
-    hipLaunchKernelGGL(k_bh_force_fast, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, fa);
+    hipLaunchKernelGGL(k_bh_force_fast, dim3((unsigned)((n + 63) / 64)),
+                       dim3(64 * (1 + kBhFastEval)), 0, st, fa);
   else {
     // by default the shared-reciprocal term once the walk has four waves per SIMD (issue-bound)
     const int64_t waves = (n + fa.gsz - 1) / fa.gsz;
