@@ -49,8 +49,7 @@ constexpr int kSunChunk = 64;
 struct BhCounters {
   int32_t M;                         // bodies in the tree
   int32_t depth_max;                 // deepest leaf
-  int32_t level[kBhLevels + 2];      // first node of each level
-  int32_t lcount[kBhLevels + 2];     // nodes at each level
+  int32_t nodes;                     // nodes of two or more bodies
   uint32_t nsun;
   uint32_t buckets;
   uint32_t stack_overflow;
@@ -96,7 +95,11 @@ struct Bh {
   int32_t *nchild = nullptr;
   BhSlot *slots = nullptr;
   int32_t *pslot = nullptr;  // each node's slot in its parent
-  int2 *nrange = nullptr;
+  int2 *nrange = nullptr;    // each node's bodies
+  int2 *nstart = nullptr;    // each node's first body and depth
+  int32_t *first = nullptr;  // the first node that a body or a later one starts
+  int32_t *npart = nullptr, *cross = nullptr;
+  uint8_t *live = nullptr;
   double *bpart = nullptr;
   void *sort_tmp = nullptr;
   size_t sort_bytes = 0;
@@ -166,7 +169,7 @@ __global__ __launch_bounds__(256) void k_bh_box_part(const double *x, const doub
 // bookkeeping.  One block of 256: the partials are folded per thread, then in LDS (min, max and
 // sums of whole numbers are exact in any order).
 __global__ __launch_bounds__(256) void k_bh_root(const double *part, int nparts,
-                                                 BhCounters *cnt, double4 *nbox, int2 *nrange,
+                                                 BhCounters *cnt, double4 *nbox,
                                                  int32_t *nchild) {
   __shared__ double sh[7][256];
   double v[7] = {DBL_MAX, DBL_MAX, DBL_MAX, -DBL_MAX, -DBL_MAX, -DBL_MAX, 0.0};
@@ -198,12 +201,7 @@ __global__ __launch_bounds__(256) void k_bh_root(const double *part, int nparts,
   const int M = (int)v[6];
   cnt->M = M;
   cnt->depth_max = 0;
-  for (int d = 0; d < kBhLevels + 2; d++) {
-    cnt->level[d] = 0;
-    cnt->lcount[d] = 0;
-  }
-  cnt->level[1] = 1;
-  cnt->lcount[0] = M >= 2 ? 1 : 0;
+  cnt->nodes = 0;
   cnt->nsun = 0;
   cnt->buckets = 0;
   cnt->stack_overflow = 0;
@@ -214,7 +212,6 @@ __global__ __launch_bounds__(256) void k_bh_root(const double *part, int nparts,
   const double mx = ey > ez ? ey : ez;  // math.Max on finite values
   const double half = (ex > mx ? ex : mx) / 2 * 1.05;
   nbox[0] = make_double4((v[0] + v[3]) / 2, (v[1] + v[4]) / 2, (v[2] + v[5]) / 2, half);
-  nrange[0] = make_int2(0, M);
   for (int c = 0; c < 8; c++) nchild[c] = -1;
 }
 
@@ -255,11 +252,10 @@ __global__ __launch_bounds__(256) void k_bh_gather(const int32_t *perm, const do
                                                    const double *m, const BhCounters *cnt,
                                                    double *sx, double *sy, double *sz,
                                                    double *sm, double *lcx, double *lcy,
-                                                   double *lcz, int32_t *depth) {
+                                                   double *lcz) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= cnt->M) return;
   const int i = perm[s];
-  if (cnt->M == 1) depth[i] = 0;  // the root is the lone body's leaf
   const double px = x[i], py = y[i], pz = z[i], mm = m[i];
   const double zero = 0.0;
   const double tot = zero + mm;
@@ -272,217 +268,367 @@ __global__ __launch_bounds__(256) void k_bh_gather(const int32_t *perm, const do
   lcz[s] = (zero * zero + pz * mm) / tot;
 }
 
-// One level of the tree: each node of level d splits its run into octant runs.
-struct BhLevelArgs {
+// ---- nodes -------------------------------------------------------------------------------------
+// The tree follows from how many leading digits neighbours in key order share.  Let L(j) be that
+// number for bodies j - 1 and j (at most D; -1 before the first body and after the last).  A node of
+// depth d is a run of two or more bodies with d digits in common, so body j starts one for every d
+// with L(j) < d <= L(j + 1), and nodes numbered by their first body, then by depth, are in
+// depth-first order with the root first.  All of them can then be made at once (a launch per level,
+// 21 of them, was 380 us at 262,144 bodies, mostly launches and one counter of the next level's
+// nodes; these three take 30).
+__device__ __forceinline__ int bh_shared(const uint64_t *keys, int j, int M, int D) {
+  if (j <= 0 || j >= M) return -1;
+  const uint64_t x = keys[j - 1] ^ keys[j];
+  return x ? (__builtin_clzll(x) - 1) / 3 : D;  // keys use bits 0..62
+}
+
+constexpr int kBhRun = 1024;  // bodies per workgroup of the next two: four to a thread
+
+// Nodes started in each run of kBhRun bodies; every body's leaf depth.
+__global__ __launch_bounds__(256) void k_bh_count(const uint64_t *keys, const int32_t *perm, int D,
+                                                  BhCounters *cnt, int32_t *part,
+                                                  int32_t *depth) {
+  __shared__ int red[3][4];
+  const int M = cnt->M, j0 = blockIdx.x * kBhRun + threadIdx.x * 4;
+  int n = 0, buckets = 0, deep = 0;
+  int l = bh_shared(keys, j0, M, D);
+  for (int j = j0; j < min(j0 + 4, M); j++) {
+    const int l1 = bh_shared(keys, j + 1, M, D);
+    n += max(0, l1 - l);
+    buckets += l < D && l1 == D;
+    const int dep = min(max(l, l1) + 1, D);
+    depth[perm[j]] = dep;
+    deep = max(deep, dep);
+    l = l1;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    n += __shfl_xor(n, o);
+    buckets += __shfl_xor(buckets, o);
+    deep = max(deep, __shfl_xor(deep, o));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = n;
+    red[1][threadIdx.x >> 6] = buckets;
+    red[2][threadIdx.x >> 6] = deep;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  part[blockIdx.x] = red[0][0] + red[0][1] + red[0][2] + red[0][3];
+  buckets = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+  deep = max(max(red[2][0], red[2][1]), max(red[2][2], red[2][3]));
+  if (buckets) atomicAdd(&cnt->buckets, (uint32_t)buckets);
+  if (deep > 0) atomicMax(&cnt->depth_max, deep);
+}
+
+// first[j]: the first node that body j or a later one starts (first[M]: the number of nodes);
+// nstart[node] = (first body, depth).
+__global__ __launch_bounds__(256) void k_bh_starts(const uint64_t *keys, int D, BhCounters *cnt,
+                                                   const int32_t *part, int64_t node_cap,
+                                                   int32_t *first, int2 *nstart) {
+  __shared__ int wsum[4], base_s[4];
+  const int M = cnt->M, j0 = blockIdx.x * kBhRun + threadIdx.x * 4;
+  if ((int)(blockIdx.x * kBhRun) >= M) return;  // uniform
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int before = 0;
+  for (int b = threadIdx.x; b < (int)blockIdx.x; b += 256) before += part[b];
+  int l[5], n = 0;
+  for (int q = 0; q < 5; q++) l[q] = bh_shared(keys, j0 + q, M, D);
+  for (int q = 0; q < 4; q++) n += max(0, l[q + 1] - l[q]);
+  int scan = n;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(scan, o);
+    if (lane >= o) scan += v;
+  }
+  for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
+  if (lane == 63) {
+    wsum[w] = scan;
+    base_s[w] = before;
+  }
+  __syncthreads();
+  int id = base_s[0] + base_s[1] + base_s[2] + base_s[3] + scan - n;
+  for (int v = 0; v < w; v++) id += wsum[v];
+  for (int q = 0; q < 4 && j0 + q < M; q++) {
+    first[j0 + q] = id;
+    for (int d = l[q] + 1; d <= l[q + 1]; d++, id++)
+      if (id < node_cap) nstart[id] = make_int2(j0 + q, d);
+    if (j0 + q == M - 1) {
+      first[M] = id;
+      cnt->nodes = id;
+      if (id > node_cap) cnt->node_overflow = 1;
+    }
+  }
+}
+
+__device__ __forceinline__ int bh_nodes(const BhCounters *cnt, int64_t node_cap) {
+  return (int)min((int64_t)cnt->nodes, node_cap);
+}
+
+struct BhNodeArgs {
   const uint64_t *keys;
-  const int32_t *perm;
-  BhCounters *cnt;
+  const BhCounters *cnt;
+  const int32_t *first;
+  const int2 *nstart;
   double4 *nbox;
   int2 *nrange;
-  int32_t *nchild;
-  int32_t *depth;
+  int32_t *nchild, *pslot;
   int64_t node_cap;
-  int d, D;
+  int D;
 };
 
-// Eight lanes per node: lane c (1..7) finds by binary search the first body of the run whose
-// digit d is >= c, the group's boundaries go round by shuffles, and lane c makes child c.
-__global__ __launch_bounds__(256) void k_bh_level(BhLevelArgs a) {
-  BhCounters *cnt = a.cnt;
-  const int d = a.d;
-  const int begin = cnt->level[d], end = begin + cnt->lcount[d];
-  if (blockIdx.x == 0 && threadIdx.x == 0) cnt->level[d + 1] = end;
-  const int shift = 60 - 3 * d;
-  const int last = (int)min((int64_t)end, a.node_cap);  // nodes past the capacity were not made
-  const int c = threadIdx.x & 7;
+// Eight lanes per node.  The run's end by an eight-way search upwards from its start; then lane c
+// (1..7) finds by binary search the first body whose digit d is >= c, the boundaries go round by
+// shuffles, and lane c makes child c's code.  A child of two or more bodies is the node after this
+// one if it starts with it, else the first that its own first body starts.
+__global__ __launch_bounds__(256) void k_bh_nodes(BhNodeArgs a) {
+  const int nodes = bh_nodes(a.cnt, a.node_cap), M = a.cnt->M, D = a.D;
+  const int c = threadIdx.x & 7, gsh = threadIdx.x & 56;
   const int groups = gridDim.x * (blockDim.x >> 3);
-  // every lane runs the same number of iterations, so the shuffles see full groups
-  const int first = begin + (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 3);
-  for (int k0 = begin; k0 < last; k0 += groups) {
-    const int k = first + (k0 - begin);
-    const bool live = k < last;
-    int2 rg = make_int2(0, 0);
-    int lb = 0;
-    if (live) {
-      rg = a.nrange[k];
-      if (c == 0) {
-        lb = rg.x;
-      } else {  // first body whose digit is >= c
-        int lo = rg.x, hi = rg.y;
-        while (lo < hi) {
-          const int mid = (lo + hi) >> 1;
-          if ((int)((a.keys[mid] >> shift) & 7) < c)
-            lo = mid + 1;
-          else
-            hi = mid;
-        }
-        lb = lo;
+  const int mine = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 3);
+  // every lane runs the same number of iterations, so ballots and shuffles see full groups
+  for (int k0 = 0; k0 < nodes; k0 += groups) {
+    const int k = mine + k0;
+    const bool live = k < nodes;
+    const int2 st = live ? a.nstart[k] : make_int2(0, 0);
+    const int lo = st.x, d = st.y, sh = 63 - 3 * d;
+    const uint64_t pre = live ? a.keys[lo] >> sh : 0;
+    auto inside = [&](int t) { return live && t < M && (a.keys[t] >> sh) == pre; };
+    auto count = [&](bool in) {  // of the group's lanes; those inside come first
+      return __builtin_popcount((uint32_t)(__builtin_amdgcn_ballot_w64(in) >> gsh) & 255u);
+    };
+    // the bodies lo + 2, lo + 8, lo + 32, ...; then the range between the last inside (b0) and the
+    // first outside (b1) cut in nine, until they are neighbours
+    int n = count(inside(lo + (2 << (2 * c))));
+    int b0 = n ? lo + (2 << (2 * (n - 1))) : lo + 1;
+    int b1 = n < 8 ? min(M, lo + (2 << (2 * n))) : M;
+    if (!live) b1 = b0;
+    while (__builtin_amdgcn_ballot_w64(b1 - b0 > 1)) {
+      const int span = b1 - b0;
+      auto at = [&](int q) { return span <= 9 ? b0 + q + 1 : b0 + (int)((int64_t)span * (q + 1) / 9); };
+      const int t = at(c);
+      n = count(t < b1 && inside(t));
+      const int n0 = n ? at(n - 1) : b0, n1 = n < 8 ? min(b1, at(n)) : b1;
+      b0 = n0;
+      b1 = n1;
+    }
+    const int hi = b1;
+    const bool bucket = d == D;
+    int lb = lo;
+    if (live && !bucket && c > 0) {
+      const int dsh = 60 - 3 * d;
+      int p = lo, q = hi;
+      while (p < q) {
+        const int mid = (p + q) >> 1;
+        if ((int)((a.keys[mid] >> dsh) & 7) < c)
+          p = mid + 1;
+        else
+          q = mid;
       }
+      lb = p;
     }
     int ub = __shfl_down(lb, 1, 8);
-    if (c == 7) ub = rg.y;
+    if (c == 7) ub = hi;
     if (!live) continue;
-    const double4 bx = a.nbox[k];
-    const double q = bx.w / 2;
-    const int cn = ub - lb;
     int32_t code = -1;
-    if (cn == 1) {
+    if (bucket) {  // depth limit: a bucket of bodies in array order
+      code = c == 0 ? kBucket : c == 1 ? lo : c == 2 ? hi - lo : -1;
+    } else if (ub - lb == 1) {
       code = -2 - lb;
-      a.depth[a.perm[lb]] = d + 1;
-      atomicMax(&cnt->depth_max, d + 1);
-    } else if (cn >= 2) {
-      const int id = end + atomicAdd(&cnt->lcount[d + 1], 1);
-      if (id >= a.node_cap) {
-        atomicOr(&cnt->node_overflow, 1u);
-      } else {
-        a.nrange[id] = make_int2(lb, ub);
-        a.nbox[id] = make_double4((c & 1) ? bx.x + q : bx.x - q, (c & 2) ? bx.y + q : bx.y - q,
-                                  (c & 4) ? bx.z + q : bx.z - q, bx.w / 2);
-        int32_t *ch = a.nchild + (size_t)id * 8;
-        if (d + 1 == a.D) {  // depth limit: a bucket of bodies in array order
-          ch[0] = kBucket;
-          ch[1] = lb;
-          ch[2] = cn;
-          for (int q2 = 3; q2 < 8; q2++) ch[q2] = -1;
-          for (int s = lb; s < ub; s++) a.depth[a.perm[s]] = d + 1;
-          atomicAdd(&cnt->buckets, 1u);
-          atomicMax(&cnt->depth_max, d + 1);
-        } else {
-          for (int q2 = 0; q2 < 8; q2++) ch[q2] = -1;
-        }
+    } else if (ub - lb >= 2) {
+      const int id = lb == lo ? k + 1 : a.first[lb];
+      if (id < a.node_cap) {
         code = id;
+        a.pslot[id] = k * 8 + c;
       }
     }
     a.nchild[(size_t)k * 8 + c] = code;
+    if (c != 0) continue;
+    a.nrange[k] = make_int2(lo, hi);
+    if (k == 0) continue;  // the root's box is there
+    // centre and half from the root's, a digit at a time, as the keys were made
+    double4 bx = a.nbox[0];
+    const uint64_t key = a.keys[lo];
+    for (int e = 0; e < d; e++) {
+      const int o = (int)((key >> (60 - 3 * e)) & 7);
+      const double q = bx.w / 2;
+      bx.x = (o & 1) ? bx.x + q : bx.x - q;
+      bx.y = (o & 2) ? bx.y + q : bx.y - q;
+      bx.z = (o & 4) ? bx.z + q : bx.z - q;
+      bx.w = bx.w / 2;
+    }
+    a.nbox[k] = bx;
   }
 }
 
-// Mass and centre of mass of the nodes of level d, from their children (or, for a bucket, its
-// bodies folded in array order by updateMass).
+// ---- masses and links --------------------------------------------------------------------------
+// Bottom-up: mass and centre of mass of a node from its children (or, for a bucket, its bodies
+// folded in array order by updateMass), its children's slots, and which of them are live.
 struct BhMassArgs {
   const BhCounters *cnt;
-  const int32_t *nchild;
-  const int2 *nrange;
-  const double4 *nbox;
+  const int32_t *nchild, *first;
+  const int2 *nstart, *nrange;
   double4 *nmc;
   BhSlot *slots;
+  uint8_t *live;  // bit c: slot c of the node is live
+  int32_t *cross;
   const double *sx, *sy, *sz, *sm, *lcx, *lcy, *lcz;
   int64_t node_cap;
-  int d;
+  int D, blocks;
 };
 
-__global__ __launch_bounds__(256) void k_bh_mass(BhMassArgs a) {
-  const int begin = a.cnt->level[a.d];
-  const int end = (int)min((int64_t)begin + a.cnt->lcount[a.d], a.node_cap);
-  for (int k = begin + blockIdx.x * blockDim.x + threadIdx.x; k < end;
-       k += gridDim.x * blockDim.x) {
-    const int32_t *ch = a.nchild + (size_t)k * 8;
-    if (ch[0] == kBucket) {
-      double mt = 0, cx = 0, cy = 0, cz = 0;
-      for (int s = ch[1]; s < ch[1] + ch[2]; s++) {
-        const double mm = a.sm[s];
-        const double nt = mt + mm;
-        cx = (cx * mt + a.sx[s] * mm) / nt;
-        cy = (cy * mt + a.sy[s] * mm) / nt;
-        cz = (cz * mt + a.sz[s] * mm) / nt;
-        mt = nt;
-      }
-      a.nmc[k] = make_double4(cx, cy, cz, mt);
+__device__ __forceinline__ void bh_mass_node(const BhMassArgs &a, int k, int d) {
+  const int4 *cw = reinterpret_cast<const int4 *>(a.nchild + (size_t)k * 8);
+  const int4 c0 = cw[0], c1 = cw[1];
+  if (d == a.D) {
+    double mt = 0, cx = 0, cy = 0, cz = 0;
+    for (int s = c0.y; s < c0.y + c0.z; s++) {
+      const double mm = a.sm[s];
+      const double nt = mt + mm;
+      cx = (cx * mt + a.sx[s] * mm) / nt;
+      cy = (cy * mt + a.sy[s] * mm) / nt;
+      cz = (cz * mt + a.sz[s] * mm) / nt;
+      mt = nt;
+    }
+    a.nmc[k] = make_double4(cx, cy, cz, mt);
+    a.live[k] = 0;
+    return;
+  }
+  const int32_t code[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+  double x[8], y[8], z[8], m[8];
+  uint8_t cl[8];
+  // all of the children's loads at once (an empty slot reads its own node's words, unused)
+#pragma unroll
+  for (int c = 0; c < 8; c++) {
+    const bool leaf = code[c] <= -2;
+    const int s = leaf ? -2 - code[c] : 0, id = code[c] >= 0 ? code[c] : 0;
+    const double *v = reinterpret_cast<const double *>(a.nmc + id);
+    x[c] = *(leaf ? a.lcx + s : v);
+    y[c] = *(leaf ? a.lcy + s : v + 1);
+    z[c] = *(leaf ? a.lcz + s : v + 2);
+    m[c] = *(leaf ? a.sm + s : v + 3);
+    cl[c] = a.live[id];
+  }
+  double mt = 0, wx = 0, wy = 0, wz = 0;
+  uint32_t live = 0;
+#pragma unroll
+  for (int c = 0; c < 8; c++) {
+    if (code[c] == -1) {
+      x[c] = y[c] = z[c] = m[c] = 0.0;
       continue;
     }
-    double mt = 0, wx = 0, wy = 0, wz = 0;
-    BhSlot *sl = a.slots + (size_t)k * 8;
-    for (int c = 0; c < 8; c++) {
-      const int32_t code = ch[c];
-      BhSlot o;
-      o.code = code;
-      o.first = o.skip = -1;
-      o.dep = 0;
-      if (code == -1) {
-        o.x = o.y = o.z = o.m = 0.0;
-        sl[c] = o;
-        continue;
-      }
-      if (code <= -2) {
-        const int s = -2 - code;
-        o.m = 0.0 + a.sm[s];
-        o.x = a.lcx[s];
-        o.y = a.lcy[s];
-        o.z = a.lcz[s];
-      } else {
-        const double4 v = a.nmc[code];
-        o.m = v.w;
-        o.x = v.x;
-        o.y = v.y;
-        o.z = v.z;
-        o.dep = a.nchild[(size_t)code * 8] == kBucket ? -1 : a.d + 1;
-      }
-      sl[c] = o;
-      mt += o.m;
-      wx += o.x * o.m;
-      wy += o.y * o.m;
-      wz += o.z * o.m;
+    if (code[c] <= -2) m[c] = 0.0 + m[c];
+    mt += m[c];
+    wx += x[c] * m[c];
+    wy += y[c] * m[c];
+    wz += z[c] * m[c];
+    live |= (m[c] > 0 ? 1u : 0u) << c;
+  }
+  BhSlot *sl = a.slots + (size_t)k * 8;
+#pragma unroll
+  for (int c = 0; c < 8; c++) {
+    BhSlot o;
+    o.x = x[c];
+    o.y = y[c];
+    o.z = z[c];
+    o.m = m[c];
+    o.code = code[c];
+    o.dep = code[c] >= 0 ? (d + 1 == a.D ? -1 : d + 1) : 0;
+    const bool on = (live >> c) & 1;
+    o.first = on && o.code >= 0 && o.dep >= 0 && cl[c] ? o.code * 8 + __builtin_ctz(cl[c]) : -1;
+    // the next live sibling; the last one's comes from an ancestor, in k_bh_links
+    const uint32_t rest = live >> (c + 1);
+    o.skip = on && rest ? k * 8 + c + 1 + __builtin_ctz(rest) : -1;
+    sl[c] = o;
+  }
+  a.nmc[k] = make_double4(wx / mt, wy / mt, wz / mt, mt);
+  a.live[k] = (uint8_t)live;
+}
+
+// Nodes whose run lies within one block of kBhBlock bodies, a workgroup per block, deepest first;
+// their numbers are in one range and so is everything below them.  A node that crosses the block's
+// end is noted by depth (at most one each) for k_bh_mass_top.  (A launch per depth, 22 of them, was
+// 215 us at 262,144 bodies; the two take 60.)
+constexpr int kBhBlock = 512;
+constexpr int kBhBlockNodes = kBhBlock / 2 * (kBhLevels + 1) + kBhLevels + 1;
+__global__ __launch_bounds__(256) void k_bh_mass(BhMassArgs a) {
+  __shared__ int count[kBhLevels + 2], at[kBhLevels + 2];
+  __shared__ uint16_t order[kBhBlockNodes];
+  const int M = a.cnt->M, j0 = blockIdx.x * kBhBlock, tid = threadIdx.x;
+  if (j0 >= M) return;  // uniform
+  const int j1 = min(M, j0 + kBhBlock);
+  const int k0 = min(a.first[j0], bh_nodes(a.cnt, a.node_cap));
+  const int k1 = min(a.first[j1], bh_nodes(a.cnt, a.node_cap));
+  int32_t *cross = a.cross + (size_t)blockIdx.x * (kBhLevels + 1);
+  if (tid <= kBhLevels) {
+    count[tid] = 0;
+    cross[tid] = -1;
+  }
+  __syncthreads();
+  for (int k = k0 + tid; k < k1; k += 256) {
+    const int d = a.nstart[k].y;
+    if (a.nrange[k].y <= j1) atomicAdd(&count[d], 1);
+    else cross[d] = k;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int s = 0;
+    for (int d = 0; d <= kBhLevels; d++) {
+      at[d] = s;
+      s += count[d];
     }
-    a.nmc[k] = make_double4(wx / mt, wy / mt, wz / mt, mt);
+  }
+  __syncthreads();
+  for (int k = k0 + tid; k < k1; k += 256)
+    if (a.nrange[k].y <= j1) order[atomicAdd(&at[a.nstart[k].y], 1)] = (uint16_t)(k - k0);
+  __syncthreads();
+  for (int d = a.D; d >= 0; d--) {  // at[d] is now the end of depth d's part
+    const int n = count[d];
+    if (n == 0) continue;  // uniform
+    for (int i = tid; i < n; i += 256) bh_mass_node(a, k0 + order[at[d] - n + i], d);
+    __syncthreads();
   }
 }
 
-// ---- links -------------------------------------------------------------------------------------
-__device__ __forceinline__ int bh_nodes(const BhCounters *cnt, int D, int64_t node_cap) {
-  return (int)min((int64_t)cnt->level[D] + cnt->lcount[D], node_cap);
-}
-
-__device__ __forceinline__ bool bh_live(const BhSlot &sl) { return sl.code != -1 && sl.m > 0; }
-
-// Each node's slot in its parent (the root has none).
-__global__ __launch_bounds__(256) void k_bh_parent(const BhCounters *cnt, const int32_t *nchild,
-                                                   int D, int64_t node_cap, int32_t *pslot) {
-  const int nodes = bh_nodes(cnt, D, node_cap);
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nodes; k += gridDim.x * blockDim.x) {
-    const int32_t *ch = nchild + (size_t)k * 8;
-    if (ch[0] == kBucket) continue;
-    for (int c = 0; c < 8; c++)
-      if (ch[c] >= 0) pslot[ch[c]] = k * 8 + c;
+__global__ __launch_bounds__(1024) void k_bh_mass_top(BhMassArgs a) {
+  __shared__ uint32_t depths;
+  const int M = a.cnt->M, nb = min(a.blocks, (M + kBhBlock - 1) / kBhBlock), tid = threadIdx.x;
+  if (tid == 0) depths = 0;
+  __syncthreads();
+  uint32_t has = 0;
+  for (int i = tid; i < nb * (kBhLevels + 1); i += 1024)
+    if (a.cross[i] >= 0) has |= 1u << (i % (kBhLevels + 1));
+  if (has) atomicOr(&depths, has);
+  __syncthreads();
+  for (int d = a.D; d >= 0; d--) {
+    if (!((depths >> d) & 1)) continue;  // uniform
+    for (int b = tid; b < nb; b += 1024) {
+      const int k = a.cross[(size_t)b * (kBhLevels + 1) + d];
+      if (k >= 0) bh_mass_node(a, k, d);
+    }
+    __syncthreads();
   }
 }
 
-// first and skip of every live slot; the root's first live child goes to the counters.
-__global__ __launch_bounds__(256) void k_bh_links(BhCounters *cnt, const int32_t *nchild,
-                                                  const int32_t *pslot, int D, int64_t node_cap,
+// The slot after each node's last live child: the next live sibling of the nearest ancestor that
+// has one.  The root's first live child goes to the counters.
+__global__ __launch_bounds__(256) void k_bh_links(BhCounters *cnt, const int32_t *pslot,
+                                                  const uint8_t *live, int64_t node_cap,
                                                   BhSlot *slots) {
-  const int nodes = bh_nodes(cnt, D, node_cap);
+  const int nodes = bh_nodes(cnt, node_cap);
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nodes; k += gridDim.x * blockDim.x) {
-    if (nchild[(size_t)k * 8] == kBucket) continue;
-    BhSlot *sl = slots + (size_t)k * 8;
-    if (k == 0) {
-      int f = -1;
-      for (int c = 0; c < 8 && f < 0; c++)
-        if (bh_live(sl[c])) f = c;
-      cnt->root_first = f;
-    }
-    for (int c = 0; c < 8; c++) {
-      if (!bh_live(sl[c])) continue;
-      int first = -1;
-      const int32_t code = sl[c].code;
-      if (code >= 0 && sl[c].dep >= 0) {
-        const BhSlot *cs = slots + (size_t)code * 8;
-        for (int c2 = 0; c2 < 8 && first < 0; c2++)
-          if (bh_live(cs[c2])) first = code * 8 + c2;
+    const uint32_t on = live[k];
+    if (k == 0) cnt->root_first = on ? __builtin_ctz(on) : -1;
+    if (on == 0) continue;
+    int skip = -1;
+    for (int node = k; node != 0;) {
+      const int up = pslot[node];
+      node = up >> 3;
+      const uint32_t rest = (uint32_t)live[node] >> ((up & 7) + 1);
+      if (rest) {
+        skip = up + 1 + __builtin_ctz(rest);
+        break;
       }
-      // next live sibling of this slot, else of the nearest ancestor that has one
-      int skip = -1, node = k, cc = c;
-      for (;;) {
-        const BhSlot *ps = slots + (size_t)node * 8;
-        for (int c2 = cc + 1; c2 < 8 && skip < 0; c2++)
-          if (bh_live(ps[c2])) skip = node * 8 + c2;
-        if (skip >= 0 || node == 0) break;
-        const int up = pslot[node];
-        node = up >> 3;
-        cc = up & 7;
-      }
-      sl[c].first = first;
-      sl[c].skip = skip;
     }
+    slots[(size_t)k * 8 + (31 - __builtin_clz(on))].skip = skip;
   }
 }
 
@@ -1242,7 +1388,7 @@ void bh_free(Bh *b) {
   void *ps[] = {b->keys_in, b->keys, b->perm_in, b->perm, b->sx,     b->sy,     b->sz,
                 b->sm,      b->lcx,  b->lcy,     b->lcz,  b->depth,  b->suns,   b->nbox,
                 b->nmc,     b->nchild, b->nrange, b->bpart, b->sort_tmp, b->cnt, b->slots,
-                b->pslot};
+                b->pslot, b->nstart, b->first, b->npart, b->cross, b->live};
   for (void *p : ps)
     if (p) (void)hipFree(p);
   delete b;
@@ -1278,6 +1424,11 @@ static int bh_ensure(Ctx *c) {
   NB_HIP(c, balloc(&b->slots, (size_t)b->node_cap * 8));
   NB_HIP(c, balloc(&b->pslot, (size_t)b->node_cap));
   NB_HIP(c, balloc(&b->nrange, (size_t)b->node_cap));
+  NB_HIP(c, balloc(&b->nstart, (size_t)b->node_cap));
+  NB_HIP(c, balloc(&b->live, (size_t)b->node_cap));
+  NB_HIP(c, balloc(&b->first, n + 1));
+  NB_HIP(c, balloc(&b->npart, (n + kBhRun - 1) / kBhRun));
+  NB_HIP(c, balloc(&b->cross, (n + kBhBlock - 1) / kBhBlock * (kBhLevels + 1)));
   size_t bytes = 0;
   NB_HIP(c, rocprim::radix_sort_pairs(nullptr, bytes, b->keys_in, b->keys, b->perm_in, b->perm,
                                       n, 0, 64, c->stream));
@@ -1306,7 +1457,7 @@ int bh_force_phase(Ctx *c, bool timed, int ev_slot) {
   hipLaunchKernelGGL(k_bh_box_part, dim3(nparts), dim3(256), 0, st, c->x, c->y, c->z, c->flags,
                      n, b->bpart);
   hipLaunchKernelGGL(k_bh_root, dim3(1), dim3(256), 0, st, b->bpart, nparts, b->cnt, b->nbox,
-                     b->nrange, b->nchild);
+                     b->nchild);
   hipLaunchKernelGGL(k_bh_keys, dim3(nb256(n)), dim3(256), 0, st, c->x, c->y, c->z, c->flags, n,
                      b->nbox, D, b->keys_in, b->perm_in, b->depth);
   NB_HIP(c, hipGetLastError());
@@ -1314,42 +1465,45 @@ int bh_force_phase(Ctx *c, bool timed, int ev_slot) {
   NB_HIP(c, rocprim::radix_sort_pairs(b->sort_tmp, bytes, b->keys_in, b->keys, b->perm_in,
                                       b->perm, (size_t)n, 0, 64, st));
   hipLaunchKernelGGL(k_bh_gather, dim3(nb256(n)), dim3(256), 0, st, b->perm, c->x, c->y, c->z,
-                     c->m, b->cnt, b->sx, b->sy, b->sz, b->sm, b->lcx, b->lcy, b->lcz, b->depth);
-  const int gl = std::min(2048, nb256(std::max(1, n / 2)));          // one thread per node
-  const int gl8 = std::min(4096, nb256((int64_t)std::max(1, n / 2) * 8));  // eight per node
-  BhLevelArgs la;
-  la.keys = b->keys;
-  la.perm = b->perm;
-  la.cnt = b->cnt;
-  la.nbox = b->nbox;
-  la.nrange = b->nrange;
-  la.nchild = b->nchild;
-  la.depth = b->depth;
-  la.node_cap = b->node_cap;
-  la.D = D;
-  for (int d = 0; d < D; d++) {
-    la.d = d;
-    hipLaunchKernelGGL(k_bh_level, dim3(gl8), dim3(256), 0, st, la);
-  }
+                     c->m, b->cnt, b->sx, b->sy, b->sz, b->sm, b->lcx, b->lcy, b->lcz);
+  const unsigned runs = (unsigned)((n + kBhRun - 1) / kBhRun);
+  hipLaunchKernelGGL(k_bh_count, dim3(runs), dim3(256), 0, st, b->keys, b->perm, D, b->cnt,
+                     b->npart, b->depth);
+  hipLaunchKernelGGL(k_bh_starts, dim3(runs), dim3(256), 0, st, b->keys, D, b->cnt, b->npart,
+                     b->node_cap, b->first, b->nstart);
+  BhNodeArgs na;
+  na.keys = b->keys;
+  na.cnt = b->cnt;
+  na.first = b->first;
+  na.nstart = b->nstart;
+  na.nbox = b->nbox;
+  na.nrange = b->nrange;
+  na.nchild = b->nchild;
+  na.pslot = b->pslot;
+  na.node_cap = b->node_cap;
+  na.D = D;
+  // about half as many nodes as bodies: eight lanes for each
+  hipLaunchKernelGGL(k_bh_nodes, dim3(nb256((int64_t)std::max(1, n / 2) * 8)), dim3(256), 0, st,
+                     na);
   BhMassArgs ma;
   ma.cnt = b->cnt;
   ma.nchild = b->nchild;
+  ma.first = b->first;
+  ma.nstart = b->nstart;
   ma.nrange = b->nrange;
   ma.nmc = b->nmc;
-  ma.nbox = b->nbox;
   ma.slots = b->slots;
+  ma.live = b->live;
+  ma.cross = b->cross;
   ma.sx = b->sx; ma.sy = b->sy; ma.sz = b->sz; ma.sm = b->sm;
   ma.lcx = b->lcx; ma.lcy = b->lcy; ma.lcz = b->lcz;
   ma.node_cap = b->node_cap;
-  for (int d = D; d >= 0; d--) {
-    ma.d = d;
-    hipLaunchKernelGGL(k_bh_mass, dim3(gl), dim3(256), 0, st, ma);
-  }
-  const int gn = std::min(4096, nb256(std::max(1, n)));  // nodes < n
-  hipLaunchKernelGGL(k_bh_parent, dim3(gn), dim3(256), 0, st, b->cnt, b->nchild, D, b->node_cap,
-                     b->pslot);
-  hipLaunchKernelGGL(k_bh_links, dim3(gn), dim3(256), 0, st, b->cnt, b->nchild, b->pslot, D,
-                     b->node_cap, b->slots);
+  ma.D = D;
+  ma.blocks = (n + kBhBlock - 1) / kBhBlock;
+  hipLaunchKernelGGL(k_bh_mass, dim3((unsigned)ma.blocks), dim3(256), 0, st, ma);
+  hipLaunchKernelGGL(k_bh_mass_top, dim3(1), dim3(1024), 0, st, ma);
+  hipLaunchKernelGGL(k_bh_links, dim3(nb256(n)), dim3(256), 0, st, b->cnt, b->pslot,
+                     b->live, b->node_cap, b->slots);
   NB_HIP(c, hipGetLastError());
   BhForceArgs fa;
   fa.cnt = b->cnt;
@@ -1480,11 +1634,9 @@ int nb_bh_get_stats(nb_ctx *c, nb_bh_stats *out) {
   BhCounters h;
   NB_HIP(c, hipStreamSynchronize(c->stream));
   NB_HIP(c, hipMemcpy(&h, c->bh->cnt, sizeof h, hipMemcpyDeviceToHost));
-  int64_t nodes = 0;
-  for (int d = 0; d <= kBhLevels; d++) nodes += h.lcount[d];
   out->builds = c->bh->builds;
   out->bodies = h.M;
-  out->nodes = nodes;
+  out->nodes = h.nodes;
   out->buckets = h.buckets;
   out->interactions = (int64_t)h.interactions;
   out->depth_max = h.depth_max;
