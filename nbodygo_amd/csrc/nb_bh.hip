@@ -10,11 +10,12 @@
 //           childCenter: octree.go:55-88), one octal digit per level, max_depth levels
 //   sort    stable radix sort of the keys: every node's bodies are one contiguous run, and a
 //           bucket's bodies (the depth limit) stay in array order
-//   levels  one launch per level splits each node's run into its eight octant runs by binary
+//   nodes   from how many digits neighbours in key order share, every node's first body and depth;
+//           then each node splits its run into its eight octant runs by binary
 //           search on that level's digit.  Runs of two or more bodies become nodes, single
 //           bodies leaves -- the tree that leaf-capacity-1 insertion builds (insert, subdivide:
 //           octree.go:198-231): same topology, node centres, halves and leaf depths.
-//   mass    bottom-up per level.  A leaf's mass and centre of mass are updateMass's from zero,
+//   mass    bottom-up, deepest first.  A leaf's mass and centre of mass are updateMass's from zero,
 //           (0 + x*m) / (0 + m) (octree.go:91-97); a node sums its children in octant order.
 //           (The reference folds bodies into each node one at a time in array order, so a
 //           node's centre of mass can differ from it in the last bits; leaves are identical.)
@@ -275,7 +276,7 @@ __global__ __launch_bounds__(256) void k_bh_gather(const int32_t *perm, const do
 // with L(j) < d <= L(j + 1), and nodes numbered by their first body, then by depth, are in
 // depth-first order with the root first.  All of them can then be made at once (a launch per level,
 // 21 of them, was 380 us at 262,144 bodies, mostly launches and one counter of the next level's
-// nodes; these three take 30).
+// nodes; these three take 34).
 __device__ __forceinline__ int bh_shared(const uint64_t *keys, int j, int M, int D) {
   if (j <= 0 || j >= M) return -1;
   const uint64_t x = keys[j - 1] ^ keys[j];
@@ -546,8 +547,10 @@ __device__ __forceinline__ void bh_mass_node(const BhMassArgs &a, int k, int d) 
 // Nodes whose run lies within one block of kBhBlock bodies, a workgroup per block, deepest first;
 // their numbers are in one range and so is everything below them.  A node that crosses the block's
 // end is noted by depth (at most one each) for k_bh_mass_top.  (A launch per depth, 22 of them, was
-// 215 us at 262,144 bodies; the two take 60.)
-constexpr int kBhBlock = 512;
+// 215 us at 262,144 bodies; these two take 42 + 77, at 100,003 35 + 46.  Each is a chain of loads
+// and stores per depth: blocks of 512 38 + 115 and 32 + 61, of 2,048 52 + 55 and 50 + 38, but 20
+// more at 5,000.)
+constexpr int kBhBlock = 1024;
 constexpr int kBhBlockNodes = kBhBlock / 2 * (kBhLevels + 1) + kBhLevels + 1;
 __global__ __launch_bounds__(256) void k_bh_mass(BhMassArgs a) {
   __shared__ int count[kBhLevels + 2], at[kBhLevels + 2];

@@ -1,5 +1,5 @@
 """The octree's build where its parts meet: body counts at the edges of a thread's four bodies, of a
-block of 512 whose nodes one workgroup sums, and of a run of 1,024 that counts nodes; a tight clump
+block of 1,024 whose nodes one workgroup sums (and which counts nodes); a tight clump
 across a block's end, so that deep nodes cross it; depth limits that make buckets.  Against the
 host's insertion-built tree: leaf depths, node and bucket counts and, with theta = 0, the forces'
 bits; with theta = 0.3 the forces to 1e-11 (the bar of the larger scenes: centres of mass are summed
