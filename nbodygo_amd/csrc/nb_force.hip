@@ -308,35 +308,65 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 
 // Pairs and the tile count go through LDS: an atomic per record took most of the kernel's 0.88 ms
-// at n = 10,007 in the reference scene (55,000 records).  Without them, and with a source's words
-// requested together, 0.15 ms: 220 G pair tests/s, FP64 issue.
+// at n = 10,007 in the reference scene (55,000 records).  Without them 0.15 ms, two thirds of the
+// cycles taken by the sources' loads, 41 bytes a pair test.  Neighbouring records come from the
+// same wave of the force kernel and share most of their flagged tiles, so a wave takes kFixRecs of
+// them and loads a tile's sources once for those that have it flagged; and without softening one
+// square root serves the test and the force.  1 / 2 / 3 / 4 / 8 records 147 / 116 / 109 / 117 / 132
+// us: 300 G pair tests/s, two thirds of the FP64 issue.
+constexpr int kFixRecs = 3;
 __global__ __launch_bounds__(256) void k_fixup(FixupArgs a) {
   __shared__ PairBuf<512> found;
   if (threadIdx.x == 0) found.clear();
   __syncthreads();
   const int lane = threadIdx.x & 63;
-  const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int wave =
+      __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
   const int nwaves = (int)((gridDim.x * blockDim.x) >> 6);
   const int nrec = (int)min((int64_t)a.ctr->rec_count, a.rec_cap);
-  for (int rr = wave; rr < nrec; rr += nwaves) {
-    const int2 rec = a.recs[rr];
-    const int slice = rec.x, i = rec.y;
-    if (!active_body(a.flags[i])) continue;
-    const size_t q = (size_t)slice * a.npad + i;
-    const int cnt = a.fcnt[q];
-    const int4 lst = reinterpret_cast<const int4 *>(a.flist)[q];
-    const int t0 = slice * a.tiles_per_slice;
-    const int t1 = min(t0 + a.tiles_per_slice, a.tiles);
-    const bool all = cnt > kFlagSlots;
-    const int ntile = all ? (t1 - t0) : cnt;
-    const double xi = a.x[i], yi = a.y[i], zi = a.z[i], ri = a.r[i];
-    const int32_t bi = a.beh[i];
-    const bool ci = nb_may_pair(bi, a.events);
-    double ax = 0, ay = 0, az = 0;
-    for (int u = 0; u < ntile; u++) {
-      int t;
-      if (all) t = t0 + u;
-      else t = u == 0 ? lst.x : u == 1 ? lst.y : u == 2 ? lst.z : lst.w;
+  for (int r0 = wave * kFixRecs; r0 < nrec; r0 += nwaves * kFixRecs) {
+    constexpr int kNone = INT_MAX;
+    int slice[kFixRecs], ti[kFixRecs], cnt[kFixRecs], pos[kFixRecs], next[kFixRecs];
+    int4 lst[kFixRecs];
+    double xi[kFixRecs], yi[kFixRecs], zi[kFixRecs], ri[kFixRecs];
+    int32_t bi[kFixRecs];
+    double ax[kFixRecs], ay[kFixRecs], az[kFixRecs];
+    // a record's tiles in order: all of its slice's, or those on its list
+    auto tile_at = [&](int u, int p) {
+      if (cnt[u] > kFlagSlots) {
+        const int t = slice[u] * a.tiles_per_slice + p;
+        return p < a.tiles_per_slice && t < a.tiles ? t : kNone;
+      }
+      return p >= cnt[u] ? kNone : p == 0 ? lst[u].x : p == 1 ? lst[u].y : p == 2 ? lst[u].z : lst[u].w;
+    };
+#pragma unroll
+    for (int u = 0; u < kFixRecs; u++) {
+      const bool have = r0 + u < nrec;
+      const int2 rec = a.recs[have ? r0 + u : r0];
+      const int i = __builtin_amdgcn_readfirstlane(rec.y);
+      slice[u] = __builtin_amdgcn_readfirstlane(rec.x);
+      ti[u] = i;
+      pos[u] = 0;
+      const size_t q = (size_t)slice[u] * a.npad + i;
+      const int4 l = reinterpret_cast<const int4 *>(a.flist)[q];
+      lst[u] = make_int4(__builtin_amdgcn_readfirstlane(l.x), __builtin_amdgcn_readfirstlane(l.y),
+                         __builtin_amdgcn_readfirstlane(l.z), __builtin_amdgcn_readfirstlane(l.w));
+      const bool run = have && active_body(a.flags[i]);
+      cnt[u] = __builtin_amdgcn_readfirstlane(run ? (int)a.fcnt[q] : 0);
+      xi[u] = a.x[i];
+      yi[u] = a.y[i];
+      zi[u] = a.z[i];
+      ri[u] = a.r[i];
+      bi[u] = a.beh[i];
+      ax[u] = ay[u] = az[u] = 0;
+      if (!run) slice[u] = -1;
+      next[u] = run ? tile_at(u, 0) : kNone;
+    }
+    for (;;) {
+      int t = next[0];
+#pragma unroll
+      for (int u = 1; u < kFixRecs; u++) t = min(t, next[u]);
+      if (t == kNone) break;
       const int j0 = t * a.tile_j;
       const int j1 = min(j0 + a.tile_j, a.n);
       for (int jb = j0; jb < j1; jb += 64) {
@@ -344,43 +374,63 @@ __global__ __launch_bounds__(256) void k_fixup(FixupArgs a) {
         const int j = jb + lane, q = min(j, j1 - 1);
         const double xj = a.x[q], yj = a.y[q], zj = a.z[q], rj = a.r[q], mj = a.m[q];
         const uint8_t fj = a.flags[q];
-        const bool valid = j < j1 && j != i && active_body(fj);
-        const double dx = xj - xi;
-        const double dy = yj - yi;
-        const double dz = zj - zi;
-        const double d2 = dx * dx + dy * dy + dz * dz;
-        const double dist = __builtin_sqrt(d2);
-        const bool overlap = !(dist > ri + rj);
-        if (valid && overlap && a.collisions && i < j && ci &&
-            nb_pair_event(bi, a.beh[j], ri, rj, dist, a.events))
-          found.add(a.pairs, a.ctr, a.pair_cap, i, j);
-        if (a.recompute) {
-          const double ds = d2 + a.eps2;
-          const double w = mj / (ds * __builtin_sqrt(ds));
-          const bool add = valid && !(overlap && a.cutoff);
-          ax += add ? w * dx : 0.0;
-          ay += add ? w * dy : 0.0;
-          az += add ? w * dz : 0.0;
+        const bool there = j < j1 && active_body(fj);
+#pragma unroll
+        for (int u = 0; u < kFixRecs; u++) {
+          if (next[u] != t) continue;  // uniform
+          const int i = ti[u];
+          const bool valid = there && j != i;
+          const double dx = xj - xi[u];
+          const double dy = yj - yi[u];
+          const double dz = zj - zi[u];
+          const double d2 = dx * dx + dy * dy + dz * dz;
+          const double dist = __builtin_sqrt(d2);
+          const bool overlap = !(dist > ri[u] + rj);
+          if (valid && overlap && a.collisions && i < j && nb_may_pair(bi[u], a.events) &&
+              nb_pair_event(bi[u], a.beh[j], ri[u], rj, dist, a.events))
+            found.add(a.pairs, a.ctr, a.pair_cap, i, j);
+          if (a.recompute) {
+            const double ds = d2 + a.eps2;
+            // without softening ds is d2 (a sum with zero changes no bit of a square's)
+            double sd = dist;
+            if (a.eps2 != 0.0) {
+              __asm__ volatile("");  // a real branch
+              sd = __builtin_sqrt(ds);
+            }
+            const double w = mj / (ds * sd);
+            const bool add = valid && !(overlap && a.cutoff);
+            ax[u] += add ? w * dx : 0.0;
+            ay[u] += add ? w * dy : 0.0;
+            az[u] += add ? w * dz : 0.0;
+          }
         }
       }
+#pragma unroll
+      for (int u = 0; u < kFixRecs; u++)
+        if (next[u] == t) next[u] = tile_at(u, ++pos[u]);
     }
-    if (a.recompute) {
-      ax = wave_sum(ax);
-      ay = wave_sum(ay);
-      az = wave_sum(az);
-    }
-    if (lane == 0) {
-      atomicAdd(&found.tiles, (uint32_t)ntile);
+#pragma unroll
+    for (int u = 0; u < kFixRecs; u++) {
+      if (slice[u] < 0) continue;  // uniform
       if (a.recompute) {
-        double *o = a.acc + (size_t)slice * 3 * a.npad;
-        if (all) {
-          o[i] = ax;
-          o[a.npad + i] = ay;
-          o[2 * a.npad + i] = az;
-        } else {
-          o[i] += ax;
-          o[a.npad + i] += ay;
-          o[2 * a.npad + i] += az;
+        ax[u] = wave_sum(ax[u]);
+        ay[u] = wave_sum(ay[u]);
+        az[u] = wave_sum(az[u]);
+      }
+      if (lane == 0) {
+        atomicAdd(&found.tiles, (uint32_t)pos[u]);
+        if (a.recompute) {
+          double *o = a.acc + (size_t)slice[u] * 3 * a.npad;
+          const int i = ti[u];
+          if (cnt[u] > kFlagSlots) {
+            o[i] = ax[u];
+            o[a.npad + i] = ay[u];
+            o[2 * a.npad + i] = az[u];
+          } else {
+            o[i] += ax[u];
+            o[a.npad + i] += ay[u];
+            o[2 * a.npad + i] += az[u];
+          }
         }
       }
     }
