@@ -7,7 +7,6 @@
 #include <cstring>
 #include <new>
 
-#include <rocprim/rocprim.hpp>
 
 #include "nb_internal.hpp"
 
@@ -50,7 +49,7 @@ static void free_spare(Ctx *c) {
   auto &S = c->spare;
   for (auto *&q : S.a)
     if (q) (void)hipFree(q), q = nullptr;
-  void *ps[] = {S.beh, S.flags, S.collided, S.fstep, S.fst, c->cyc_keep, c->cyc_pos, c->cyc_tmp};
+  void *ps[] = {S.beh, S.flags, S.collided, S.fstep, S.fst, c->cyc_part};
   for (void *p : ps)
     if (p) (void)hipFree(p);
   S.beh = nullptr;
@@ -58,9 +57,7 @@ static void free_spare(Ctx *c) {
   S.fstep = nullptr;
   S.fst = nullptr;
   S.cap = 0;
-  c->cyc_keep = c->cyc_pos = nullptr;
-  c->cyc_tmp = nullptr;
-  c->cyc_tmp_bytes = 0;
+  c->cyc_part = nullptr;
   c->cyc_cap = 0;
 }
 
@@ -965,11 +962,9 @@ static int refresh_rmax(Ctx *c) {
   unsigned long long *d = c->small, h = 0;
   NB_HIP(c, hipMemsetAsync(d, 0, sizeof h, c->stream));
   NB_HIP(c, launch_rmax_active(c->r, c->flags, (int)c->n, d, c->stream));
-  NB_HIP(c, hipMemcpyAsync(&h, d, sizeof h, hipMemcpyDeviceToHost, c->stream));
-  NB_HIP(c, hipStreamSynchronize(c->stream));
-  double v;
-  memcpy(&v, &h, sizeof v);
-  c->rmax = v;
+  const Fetch f = {&h, d, sizeof h};
+  NB_HIP(c, stage_fetch(&f, 1, c->stream));
+  memcpy(&c->rmax, &h, sizeof c->rmax);
   return NB_OK;
 }
 
@@ -988,9 +983,12 @@ int nb_add_bodies(nb_ctx *c, int64_t k, const double *x, const double *y, const 
     return fail(c, NB_E_INVALID, "nb_add_bodies: NULL array");
   const double *src[10] = {x, y, z, vx, vy, vz, m, r, nullptr, frag};
   auto &A = c->adds;
-  for (int q = 0; q < 10; q++)
-    for (int64_t i = 0; i < k; i++) A.a[q].push_back(src[q] ? src[q][i] : (q == 8 ? 1.0 : 0.0));
-  for (int64_t i = 0; i < k; i++) A.fstep.push_back(frag_step ? frag_step[i] : 0.0);
+  auto queue = [k](std::vector<double> &v, const double *s, double otherwise) {
+    if (s) v.insert(v.end(), s, s + k);
+    else v.insert(v.end(), (size_t)k, otherwise);
+  };
+  for (int q = 0; q < 10; q++) queue(A.a[q], src[q], q == 8 ? 1.0 : 0.0);
+  queue(A.fstep, frag_step, 0.0);
   A.beh.insert(A.beh.end(), beh, beh + k);
   A.flags.insert(A.flags.end(), flags, flags + k);
   return NB_OK;
@@ -1007,28 +1005,15 @@ int nb_cycle(nb_ctx *c, double R, int64_t *n_out) {
   int64_t nk = 0;
   if (n > 0) {
     if (c->cyc_cap < n) {
-      NB_HIP(c, dalloc(&c->cyc_keep, (size_t)c->cap));
-      NB_HIP(c, dalloc(&c->cyc_pos, (size_t)c->cap));
+      NB_HIP(c, dalloc(&c->cyc_part, (size_t)(c->cap + 1023) / 1024));
       c->cyc_cap = c->cap;
     }
-    int32_t *keep = c->cyc_keep, *pos = c->cyc_pos;
-    NB_HIP(c, launch_keep_flags(c->flags, (int)n, keep, st));
-    size_t tb = 0;
-    NB_HIP(c, rocprim::exclusive_scan(nullptr, tb, keep, pos, 0, (size_t)n,
-                                      rocprim::plus<int32_t>(), st));
-    if (tb > c->cyc_tmp_bytes) {
-      if (c->cyc_tmp) (void)hipFree(c->cyc_tmp);
-      c->cyc_tmp = nullptr;
-      NB_HIP(c, hipMalloc(&c->cyc_tmp, tb));
-      c->cyc_tmp_bytes = tb;
-    }
-    NB_HIP(c, rocprim::exclusive_scan(c->cyc_tmp, tb, keep, pos, 0, (size_t)n,
-                                      rocprim::plus<int32_t>(), st));
-    int32_t lp = 0, lk = 0;
-    NB_HIP(c, hipMemcpyAsync(&lp, pos + n - 1, 4, hipMemcpyDeviceToHost, st));
-    NB_HIP(c, hipMemcpyAsync(&lk, keep + n - 1, 4, hipMemcpyDeviceToHost, st));
-    NB_HIP(c, hipStreamSynchronize(st));
-    nk = (int64_t)lp + lk;
+    const int run = cycle_run(n);
+    NB_HIP(c, launch_keep_count(c->flags, (int)n, run, c->cyc_part, st));
+    std::vector<int32_t> part((size_t)(n + run - 1) / run);
+    const Fetch f = {part.data(), c->cyc_part, part.size() * sizeof(int32_t)};
+    NB_HIP(c, stage_fetch(&f, 1, st));
+    for (int32_t p : part) nk += p;
   }
   int64_t nq = 0;  // fragments waiting in the device queue
   if (c->p.events) {
@@ -1079,13 +1064,6 @@ int nb_cycle(nb_ctx *c, double R, int64_t *n_out) {
   double *fs = c->p.events ? S.fstep : nullptr;
   FragState *fst = c->p.events ? S.fst : nullptr;
   hipError_t e = hipSuccess;
-  for (int q = 0; q < 10 && e == hipSuccess; q++)
-    e = hipMemsetAsync(d[q], 0, (size_t)cap_new * 8, st);
-  if (e == hipSuccess) e = hipMemsetAsync(beh, 0, (size_t)cap_new * 4, st);
-  if (e == hipSuccess) e = hipMemsetAsync(fl, 0, (size_t)cap_new, st);
-  if (e == hipSuccess) e = hipMemsetAsync(col, 0, (size_t)cap_new, st);
-  if (e == hipSuccess && fs) e = hipMemsetAsync(fs, 0, (size_t)cap_new * 8, st);
-  if (e == hipSuccess && fst) e = hipMemsetAsync(fst, 0, (size_t)cap_new * sizeof(FragState), st);
   CompactArgs ca;
   const double *olds[10] = {c->x, c->y, c->z, c->vx, c->vy, c->vz, c->m, c->r, c->rest, c->frag};
   for (int q = 0; q < 10; q++) {
@@ -1096,34 +1074,36 @@ int nb_cycle(nb_ctx *c, double R, int64_t *n_out) {
   ca.beh_dst = beh;
   ca.flags_src = c->flags;
   ca.flags_dst = fl;
-  ca.pos = c->cyc_pos;
+  ca.collided_dst = col;
+  ca.part = c->cyc_part;
   ca.fstep_src = c->fstep;
   ca.fstep_dst = fs;
   ca.fst_src = c->fst;
   ca.fst_dst = fst;
   ca.n = (int)n;
-  if (e == hipSuccess) e = launch_compact(ca, st);
+  ca.run = cycle_run(std::max<int64_t>(n, 1));
+  ca.kept = nk;
+  ca.cap = cap_new;
+  e = launch_compact(ca, st);
   // the device's fragments first (the newest events), then the host's queue
   if (e == hipSuccess && nq) e = launch_append_frags(c, nq, d, beh, fl, fs, fst, nk, R, st);
   // queued adds go after the survivors, newest first, each with restitution R: the reference
   // keeps its events with PushFront (body_collection.go:100) and Cycle walks them from the front
   // (body_collection.go:273-279, 286-290)
   auto &A = c->adds;
-  std::fill(A.a[8].begin(), A.a[8].end(), R);
-  for (int q = 0; q < 10; q++) std::reverse(A.a[q].begin(), A.a[q].end());
-  std::reverse(A.beh.begin(), A.beh.end());
-  std::reverse(A.flags.begin(), A.flags.end());
-  std::reverse(A.fstep.begin(), A.fstep.end());
-  const int64_t at = nk + nq;
-  for (int q = 0; q < 10 && e == hipSuccess && nadd; q++)
-    e = hipMemcpyAsync(d[q] + at, A.a[q].data(), (size_t)nadd * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess && nadd)
-    e = hipMemcpyAsync(beh + at, A.beh.data(), (size_t)nadd * 4, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess && nadd)
-    e = hipMemcpyAsync(fl + at, A.flags.data(), (size_t)nadd, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess && nadd && fs)
-    e = hipMemcpyAsync(fs + at, A.fstep.data(), (size_t)nadd * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  if (e == hipSuccess && nadd) {
+    std::fill(A.a[8].begin(), A.a[8].end(), R);
+    const int64_t at = nk + nq;
+    Send seg[13];
+    int ns = 0;
+    for (int q = 0; q < 10; q++) seg[ns++] = {d[q] + at, A.a[q].data(), 8};
+    seg[ns++] = {beh + at, A.beh.data(), 4};
+    seg[ns++] = {fl + at, A.flags.data(), 1};
+    if (fs) seg[ns++] = {fs + at, A.fstep.data(), 8};
+    e = stage_send_reversed(seg, ns, nadd, st);
+  } else if (e == hipSuccess) {
+    e = hipStreamSynchronize(st);
+  }
   NB_HIP(c, e);
   // swap the sets: the compacted arrays go live, the old ones become the second set
   const int64_t live_cap = S.cap;  // >= cap_new >= c->cap
@@ -1186,17 +1166,19 @@ int nb_remove_bodies(nb_ctx *c, int64_t count, int64_t *removed) {
   const bool all = count == -1;
   const int64_t step = all ? 1 : (count > n ? 1 : n / count);
   const int64_t npoints = all ? n : (n + step - 1) / step;
-  unsigned long long *cnt = c->small, h[2] = {0, 0};
+  unsigned long long *cnt = c->small, h[3] = {0, 0, 0};  // removed, of them active, rmax's bits
   NB_HIP(c, hipMemsetAsync(cnt, 0, sizeof h, c->stream));
   NB_HIP(c, launch_remove_walk(c->flags, c->m, (int)n, (int)step, (int)npoints, all ? 1 : 0, cnt,
                                c->stream));
-  NB_HIP(c, hipMemcpyAsync(h, cnt, sizeof h, hipMemcpyDeviceToHost, c->stream));
   NB_HIP(c, launch_write_stream(c->x, c->y, c->z, c->m, c->flags, c->js, (int)n, (int)c->npad,
                                 c->stream));
-  NB_HIP(c, hipStreamSynchronize(c->stream));
+  NB_HIP(c, launch_rmax_active(c->r, c->flags, (int)n, cnt + 2, c->stream));
+  const Fetch f = {h, cnt, sizeof h};
+  NB_HIP(c, stage_fetch(&f, 1, c->stream));
   c->n_active = std::max<int64_t>(0, c->n_active - (int64_t)h[1]);
+  memcpy(&c->rmax, &h[2], sizeof c->rmax);
   if (removed) *removed = (int64_t)h[0];
-  return refresh_rmax(c);
+  return NB_OK;
 }
 
 int nb_get_body(nb_ctx *c, int64_t index, nb_body *out) {

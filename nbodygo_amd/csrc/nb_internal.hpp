@@ -138,6 +138,13 @@ struct Fetch {
 };
 hipError_t stage_fetch(const Fetch *seg, int n, hipStream_t st);
 hipError_t stage_counters(const DevCounters *c, hipStream_t st, DevCounters *out);
+// The other way, last element first: dst[i] = src[count - 1 - i], elements of 8, 4 or 1 bytes.
+struct Send {
+  void *dst;
+  const void *src;
+  int width;
+};
+hipError_t stage_send_reversed(const Send *seg, int n, int64_t count, hipStream_t st);
 void stage_user(int add);  // +1 with a context or batch, -1 with its end
 
 struct Ctx {
@@ -225,9 +232,7 @@ struct Ctx {
     FragState *fst = nullptr;
     int64_t cap = 0;
   } spare;
-  int32_t *cyc_keep = nullptr, *cyc_pos = nullptr;  // keep flags and their prefix sum
-  void *cyc_tmp = nullptr;
-  size_t cyc_tmp_bytes = 0;
+  int32_t *cyc_part = nullptr;  // bodies kept in each run of a compaction
   int64_t cyc_cap = 0;
 
   // bodies queued by nb_add_bodies, appended by the next nb_cycle
@@ -475,14 +480,19 @@ struct CompactArgs {
   int32_t *beh_dst;
   const uint8_t *flags_src;
   uint8_t *flags_dst;
-  const int32_t *pos;  // exclusive prefix sum of the keep flags
+  uint8_t *collided_dst;
+  const int32_t *part;  // bodies kept in each run
   const double *fstep_src;  // events: FragStep and fragmentation state (may be null)
   double *fstep_dst;
   const FragState *fst_src;
   FragState *fst_dst;
-  int n;
+  int n, run;
+  int64_t kept, cap;  // survivors; capacity of the destination
 };
-hipError_t launch_keep_flags(const uint8_t *flags, int n, int32_t *keep, hipStream_t st);
+// Bodies per workgroup of a compaction: 1,024, more where there would be over 8,192 workgroups (each
+// adds up the counts of those before it).
+constexpr int cycle_run(int64_t n) { return 1024 * (int)(1 + (n - 1) / ((int64_t)8192 * 1024)); }
+hipError_t launch_keep_count(const uint8_t *flags, int n, int run, int32_t *part, hipStream_t st);
 hipError_t launch_compact(const CompactArgs &a, hipStream_t st);
 hipError_t launch_rmax_active(const double *r, const uint8_t *flags, int n,
                               unsigned long long *out, hipStream_t st);

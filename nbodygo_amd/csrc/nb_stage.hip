@@ -149,6 +149,66 @@ hipError_t stage_counters(const DevCounters *c, hipStream_t st, DevCounters *out
   return e;
 }
 
+// Slices of host arrays, read by the kernel over the bus.
+struct SendArgs {
+  void *dst[kFetchMax];
+  uint32_t at[kFetchMax];  // offset in src
+  int width[kFetchMax];
+  const char *src;
+  int count;
+};
+__global__ __launch_bounds__(256) void k_send_reversed(SendArgs a) {
+  const int c = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x, j = a.count - 1 - i;
+  if (j < 0) return;
+  const char *s = a.src + a.at[c];
+  if (a.width[c] == 8) static_cast<uint64_t *>(a.dst[c])[j] = ((const uint64_t *)s)[i];
+  else if (a.width[c] == 4) static_cast<uint32_t *>(a.dst[c])[j] = ((const uint32_t *)s)[i];
+  else static_cast<uint8_t *>(a.dst[c])[j] = ((const uint8_t *)s)[i];
+}
+
+hipError_t stage_send_reversed(const Send *seg, int n, int64_t count, hipStream_t st) {
+  size_t each = 0;  // bytes of one element of every array
+  for (int k = 0; k < n; k++) each += (size_t)seg[k].width;
+  const size_t pad = (size_t)16 * n;
+  Lease l((size_t)count * each + pad);
+  if (!l.b) {  // no pinned memory to be had: reversed copies, one array at a time
+    std::vector<char> rev;
+    for (int k = 0; k < n; k++) {
+      const size_t w = (size_t)seg[k].width;
+      rev.resize((size_t)count * w);
+      for (int64_t i = 0; i < count; i++)
+        memcpy(rev.data() + i * w, static_cast<const char *>(seg[k].src) + (count - 1 - i) * w, w);
+      const hipError_t e = hipMemcpyAsync(seg[k].dst, rev.data(), rev.size(),
+                                          hipMemcpyHostToDevice, st);
+      if (e != hipSuccess) return e;
+      const hipError_t e2 = hipStreamSynchronize(st);
+      if (e2 != hipSuccess) return e2;
+    }
+    return hipSuccess;
+  }
+  const int64_t most = (int64_t)((l.b->bytes - pad) / each);
+  for (int64_t i0 = 0; i0 < count; i0 += most) {
+    SendArgs a;
+    a.src = static_cast<const char *>(l.dev);
+    a.count = (int)std::min(most, count - i0);
+    size_t at = 0;
+    for (int k = 0; k < n; k++) {
+      const size_t w = (size_t)seg[k].width, bytes = (size_t)a.count * w;
+      memcpy(l.b->buf + at, static_cast<const char *>(seg[k].src) + (size_t)i0 * w, bytes);
+      a.dst[k] = static_cast<char *>(seg[k].dst) + (size_t)(count - i0 - a.count) * w;
+      a.at[k] = (uint32_t)at;
+      a.width[k] = seg[k].width;
+      at += (bytes + 15) / 16 * 16;
+    }
+    hipLaunchKernelGGL(k_send_reversed, dim3((unsigned)((a.count + 255) / 256), (unsigned)n),
+                       dim3(256), 0, st, a);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 static int copy_threads(size_t bytes) {
   cpu_set_t set;
   CPU_ZERO(&set);
