@@ -27,8 +27,6 @@
 #include <random>
 #include <vector>
 
-#include <rocprim/rocprim.hpp>
-
 #include "nb_internal.hpp"
 
 namespace nb {
@@ -41,12 +39,7 @@ constexpr int kFarRec = 36;   // a(3), J(6: xx yy zz xy xz yz), H(10), T(15), 0,
 constexpr int kFarUsed = 34;  // words of the record the far-field kernel writes
 constexpr int kFeat = 30;     // MLP input width
 constexpr int kMaxGrid = 64;  // cell keys 0..64^3 (the last for inactive bodies): 19 bits
-// Bits of the cell keys 0..ncell sorted by the radix sort (16 up to 40^3 cells).
-// Stable radix sort by onesweep passes at every size (rocPRIM's default sorts inputs below a
-// million items by block sort plus merge passes: 17 launches for 262,144 keys).
-using SortCfg = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
-                                           rocprim::default_config, 0>;
-
+// Bits of the cell keys 0..ncell (16 up to 40^3 cells).
 static unsigned key_bits(int ncell) { return 32u - (unsigned)__builtin_clz((unsigned)ncell); }
 
 typedef float f4v __attribute__((ext_vector_type(4)));
@@ -62,8 +55,8 @@ struct Sur {
   double r0 = 0;
   int64_t cap = 0;
   uint32_t *keys = nullptr, *keys2 = nullptr, *perm_in = nullptr, *perm = nullptr;
-  void *sort_tmp = nullptr;
-  size_t sort_bytes = 0;
+  uint32_t *keys1 = nullptr;               // between the sort's passes
+  int32_t *sort_cnt = nullptr, *sort_tot = nullptr;
   int32_t *cstart = nullptr, *ccount = nullptr, *nelist = nullptr, *necount = nullptr;
   float *srad = nullptr;                 // radii in sorted order, rounded up (collisions)
   float4 *sp = nullptr;
@@ -185,14 +178,156 @@ __device__ __forceinline__ int cell_of(double dx, double dy, double dz, double r
 
 __global__ void k_sur_keys(const double *x, const double *y, const double *z,
                            const uint8_t *flags, int n, const double *center, double r0, int G,
-                           uint32_t *keys, uint32_t *perm_in) {
+                           uint32_t *keys) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   uint32_t key = (uint32_t)(G * G * G);
   if (act(flags[i]))
     key = (uint32_t)cell_of(x[i] - center[0], y[i] - center[1], z[i] - center[2], r0, G);
   keys[i] = key;
-  perm_in[i] = (uint32_t)i;
+}
+
+// Orders this wave's writes of its private LDS tile before its later reads (and the reads before
+// the next overwrite); the waitcnt of a workgroup-scope fence covers the LDS queue.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// ---- bodies by cell ------------------------------------------------------------------------
+// A stable sort of the bodies' cell keys: one or two counting passes of up to 10 bits.  A workgroup
+// has 256 IT neighbouring bodies; it counts its digits, a wave per digit turns the counts into places
+// among the workgroups, and it puts its bodies there: a body's place within its wave is the count
+// of equal digits before it, by ballots.  Three short launches a pass, 34 us at 262,144 bodies and
+// 16 bits: the radix sort of rocPRIM took 61 us of kernels and, with its four clears, 117 in all.
+constexpr int kSortBins = 1024;
+struct SortArgs {
+  const uint32_t *key, *idx;  // idx null: the bodies in order
+  uint32_t *key_out, *idx_out;
+  int32_t *cnt, *tot;         // [digit][workgroup], [digit]
+  int n, nblk, shift, bits;
+};
+
+template <int IT>
+__global__ __launch_bounds__(256) void k_sort_count(SortArgs a) {
+  __shared__ int h[kSortBins];
+  const int bins = 1 << a.bits;
+  for (int b = threadIdx.x; b < bins; b += 256) h[b] = 0;
+  __syncthreads();
+  const int i0 = blockIdx.x * 256 * IT + threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < IT; q++)
+    if (i0 + q * 256 < a.n) atomicAdd(&h[(a.key[i0 + q * 256] >> a.shift) & (bins - 1)], 1);
+  __syncthreads();
+  for (int b = threadIdx.x; b < bins; b += 256) a.cnt[(size_t)b * a.nblk + blockIdx.x] = h[b];
+}
+
+// A wave per digit: its counts become exclusive sums over the workgroups, and their total.
+__global__ __launch_bounds__(256) void k_sort_places(SortArgs a) {
+  const int b = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (b >= 1 << a.bits) return;
+  int32_t *c = a.cnt + (size_t)b * a.nblk;
+  int run = 0;
+  for (int k0 = 0; k0 < a.nblk; k0 += 64) {
+    const int k = k0 + lane, v = k < a.nblk ? c[k] : 0;
+    int t = v;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(t, o);
+      if (lane >= o) t += u;
+    }
+    if (k < a.nblk) c[k] = run + t - v;
+    run += __shfl(t, 63);
+  }
+  if (lane == 0) a.tot[b] = run;
+}
+
+template <int IT>
+__global__ __launch_bounds__(256) void k_sort_scatter(SortArgs a) {
+  __shared__ int h[4][kSortBins];
+  __shared__ int wsum[4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int bins = 1 << a.bits;
+  for (int b = tid; b < 4 * kSortBins; b += 256) (&h[0][0])[b] = 0;
+  // thread t's four digits 4 t .. 4 t + 3: where each starts for this workgroup
+  int tot[4], start = 0;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    tot[e] = tid * 4 + e < bins ? a.tot[tid * 4 + e] : 0;
+    start += tot[e];
+  }
+  const int mine = start;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(start, o);
+    if (lane >= o) start += u;
+  }
+  if (lane == 63) wsum[w] = start;
+  __syncthreads();
+  start -= mine;
+  for (int v = 0; v < w; v++) start += wsum[v];
+  // each body's place among the wave's equal digits, in order
+  const int i0 = blockIdx.x * 256 * IT + w * 64 * IT + lane;
+  uint32_t key[IT];
+  int rank[IT];
+#pragma unroll
+  for (int q = 0; q < IT; q++) key[q] = i0 + q * 64 < a.n ? a.key[i0 + q * 64] : 0;
+#pragma unroll
+  for (int q = 0; q < IT; q++) {
+    const bool there = i0 + q * 64 < a.n;
+    const int d = (int)(key[q] >> a.shift) & (bins - 1);
+    uint64_t peers = __builtin_amdgcn_ballot_w64(there);
+    for (int e = 0; e < a.bits; e++) {
+      const bool on = (d >> e) & 1;
+      const uint64_t bal = __builtin_amdgcn_ballot_w64(on);
+      peers &= on ? bal : ~bal;
+    }
+    const int below = __builtin_popcountll(peers & ((1ull << lane) - 1));
+    const int before = h[w][d];
+    rank[q] = before + below;
+    wave_lds_sync();
+    if (there && below == 0) h[w][d] = before + __builtin_popcountll(peers);
+    wave_lds_sync();
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const int b = tid * 4 + e;
+    if (b < bins) {
+      int o = start + a.cnt[(size_t)b * a.nblk + blockIdx.x];
+      for (int v = 0; v < 4; v++) {
+        const int c = h[v][b];
+        h[v][b] = o;
+        o += c;
+      }
+    }
+    start += tot[e];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < IT; q++) {
+    const int i = i0 + q * 64;
+    if (i >= a.n) continue;
+    const int at = h[w][(key[q] >> a.shift) & (bins - 1)] + rank[q];
+    a.key_out[at] = key[q];
+    a.idx_out[at] = a.idx ? a.idx[i] : (uint32_t)i;
+  }
+}
+
+// Bodies per thread: 4 up to 524,288 bodies (enough workgroups), 16 above (fewer counts).
+static int sort_items(int64_t n) { return n <= 524288 ? 4 : 16; }
+static int sort_blocks(int64_t n) {
+  const int64_t per = 256 * (int64_t)sort_items(n);
+  return (int)((n + per - 1) / per);
+}
+static hipError_t sort_pass(const SortArgs &a, hipStream_t st) {
+  const dim3 grid((unsigned)a.nblk), block(256);
+  if (sort_items(a.n) == 4) hipLaunchKernelGGL(k_sort_count<4>, grid, block, 0, st, a);
+  else hipLaunchKernelGGL(k_sort_count<16>, grid, block, 0, st, a);
+  hipLaunchKernelGGL(k_sort_places, dim3((unsigned)(((1 << a.bits) + 3) / 4)), block, 0, st, a);
+  if (sort_items(a.n) == 4) hipLaunchKernelGGL(k_sort_scatter<4>, grid, block, 0, st, a);
+  else hipLaunchKernelGGL(k_sort_scatter<16>, grid, block, 0, st, a);
+  return hipGetLastError();
 }
 
 // cstart[c] = first sorted position whose key is >= c, for c = 0..ncell (inactive bodies carry
@@ -326,14 +461,6 @@ __device__ __forceinline__ double wmax(double v) {
 #pragma unroll
   for (int m = 32; m > 0; m >>= 1) v = fmax(v, __shfl_xor(v, m, 64));
   return v;
-}
-
-// Orders this wave's writes of its private LDS tile before its later reads (and the reads before
-// the next overwrite); the waitcnt of a workgroup-scope fence covers the LDS queue.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
 // Cell moments about the cell's centre of mass (FP64 accumulation), one wave per nonempty cell:
@@ -1371,7 +1498,7 @@ static hipError_t salloc(T **p, size_t count) {
 void sur_free(Sur *s) {
   if (!s) return;
   if (s->nitems_host) (void)hipHostFree(s->nitems_host);
-  void *ptrs[] = {s->keys, s->keys2, s->perm_in, s->perm, s->sort_tmp, s->cstart, s->ccount,
+  void *ptrs[] = {s->keys, s->keys2, s->perm_in, s->perm, s->keys1, s->sort_cnt, s->sort_tot, s->cstart, s->ccount,
                   s->nelist, s->necount, s->sp, s->srad, s->crec, s->crec_ne, s->fexp, s->part,
                   s->items, s->nitems, s->btot, s->feat, s->base, s->center,
                   s->red, s->mu, s->sd, s->tx, s->ty, s->sidx, s->sexact, s->serr, s->flag,
@@ -1402,15 +1529,11 @@ static int sur_ensure_bodies(Ctx *c) {
   NB_HIP(c, salloc(&s->base, n));
   NB_HIP(c, salloc(&s->ymlp, n * 3));
   NB_HIP(c, salloc(&s->feat, n * kFeat));
-  size_t bytes = 0;
-  NB_HIP(c, rocprim::radix_sort_pairs<SortCfg>(
-                nullptr, bytes, s->keys, s->keys2, s->perm_in, s->perm, (size_t)n, 0u,
-                key_bits(kMaxGrid * kMaxGrid * kMaxGrid), c->stream));
-  void *tmp = nullptr;
-  NB_HIP(c, hipMalloc(&tmp, bytes ? bytes : 1));
-  if (s->sort_tmp) (void)hipFree(s->sort_tmp);
-  s->sort_tmp = tmp;
-  s->sort_bytes = bytes;
+  NB_HIP(c, salloc(&s->keys1, n));
+  // (a smaller count can have more workgroups: four bodies a thread)
+  const int64_t blocks = std::max<int64_t>(sort_blocks(n), sort_blocks(std::min<size_t>(n, 524288)));
+  NB_HIP(c, salloc(&s->sort_cnt, (size_t)blocks * kSortBins));
+  NB_HIP(c, salloc(&s->sort_tot, kSortBins));
   s->cap = c->cap;
   return NB_OK;
 }
@@ -1470,11 +1593,21 @@ static int sur_pipeline(Ctx *c, bool feat_raw, bool feat_norm, bool apply, bool 
                      c->flags, n, s->red, zero_counters ? c->ctr : nullptr);
   hipLaunchKernelGGL(k_sur_com_final, dim3(1), dim3(256), 0, st, s->red, nbk, s->center);
   hipLaunchKernelGGL(k_sur_keys, dim3(nb256(n)), dim3(256), 0, st, c->x, c->y, c->z, c->flags,
-                     n, s->center, s->r0, G, s->keys, s->perm_in);
+                     n, s->center, s->r0, G, s->keys);
   NB_HIP(c, hipGetLastError());
-  size_t bytes = s->sort_bytes;
-  NB_HIP(c, rocprim::radix_sort_pairs<SortCfg>(s->sort_tmp, bytes, s->keys, s->keys2, s->perm_in,
-                                               s->perm, (size_t)n, 0u, key_bits(ncell), st));
+  {
+    const int bits = (int)key_bits(ncell), low = bits <= 10 ? bits : bits / 2;
+    SortArgs sa{s->keys, nullptr, s->keys2, s->perm, s->sort_cnt, s->sort_tot,
+                n,       sort_blocks(n), 0, low};
+    if (bits > low) {
+      sa.key_out = s->keys1;
+      sa.idx_out = s->perm_in;
+      NB_HIP(c, sort_pass(sa, st));
+      sa = SortArgs{s->keys1, s->perm_in, s->keys2, s->perm, s->sort_cnt, s->sort_tot,
+                    n,        sort_blocks(n), low, bits - low};
+    }
+    NB_HIP(c, sort_pass(sa, st));
+  }
   hipLaunchKernelGGL(k_sur_bounds, dim3((unsigned)(ncell / 1024 + 1)), dim3(1024), 0, st,
                      s->keys2, n, ncell, s->cstart, s->btot);
   hipLaunchKernelGGL(k_sur_scan, dim3((unsigned)((ncell + 1023) / 1024)), dim3(1024), 0, st,
