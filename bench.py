@@ -193,7 +193,8 @@ def plain_leg(n, steps, warmup, pinned, tune, seed=2024):
         "roofline": {"bound": "mfma", "bound_detail": BOUND_FP32, "achieved": achieved / 1e12,
                      "peak": PEAK_FP32 / 1e12, "unit": "TFLOP/s", "frac": achieved / PEAK_FP32,
                      "traffic": traffic, "traffic_source": tsrc,
-                     "kernel": "k_force_lds / k_force_scalar (FP32 pairwise force)",
+                     "kernel": ("k_force_sym" if shape.get("variant") == 3 else
+                                "k_force_lds / k_force_scalar") + " (FP32 pairwise force)",
                      "flops_per_interaction": FLOPS_PER_INTERACTION,
                      "interactions_per_launch": per_launch, "avg_launch_ms": launch_ms},
         "force_error": force_error(g, b),

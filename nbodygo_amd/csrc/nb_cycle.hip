@@ -70,7 +70,7 @@ __device__ __forceinline__ void three_quotients(const double n[3], double d, boo
 // one barrier per round.
 // One lane per target (sources staged in LDS) left most of the chip idle below 65,536 bodies, each
 // lane in a serial chain of square roots and divisions: 0.413 ms at n = 1,000, 6.69 at 16,384,
-// 26.6 at 65,536, 283 at 262,144.  This form, same bits: 0.018, 1.22, 16.7 and 256 ms.  What bounds
+// 26.6 at 65,536, 283 at 262,144.  This form, same bits: 0.018, 1.22, 17.1 and 263 ms.  What bounds
 // it now is FP64 issue (about 110 VALU instructions a pair), and for small n the serial additions.
 constexpr int kF64Term = 13, kF64Sum = 3;
 template <int TL, int UN>
