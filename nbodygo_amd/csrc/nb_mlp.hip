@@ -239,13 +239,20 @@ struct AdamArgs {
   float lr, b1, b2, eps, c1, c2;
 };
 // One weight's Adam update; returns the new weight.
-__device__ __forceinline__ float adam_update(const AdamArgs &h, float gi, float *w, float *m1,
-                                             float *m2, int64_t i) {
-  const float a = h.b1 * m1[i] + (1.f - h.b1) * gi;
-  const float b = h.b2 * m2[i] + (1.f - h.b2) * gi * gi;
+struct AdamState {
+  float w, m1, m2;
+};
+__device__ __forceinline__ AdamState adam_load(const float *w, const float *m1, const float *m2,
+                                               int64_t i) {
+  return AdamState{w[i], m1[i], m2[i]};
+}
+__device__ __forceinline__ float adam_update(const AdamArgs &h, float gi, const AdamState &v, float *w,
+                                             float *m1, float *m2, int64_t i) {
+  const float a = h.b1 * v.m1 + (1.f - h.b1) * gi;
+  const float b = h.b2 * v.m2 + (1.f - h.b2) * gi * gi;
   m1[i] = a;
   m2[i] = b;
-  const float wi = w[i] - h.lr * (a / h.c1) / (sqrtf(b / h.c2) + h.eps);
+  const float wi = v.w - h.lr * (a / h.c1) / (sqrtf(b / h.c2) + h.eps);
   w[i] = wi;
   return wi;
 }
@@ -253,7 +260,7 @@ __global__ void k_adam(float *w, const float *g, float *m1, float *m2, uint16_t 
                        AdamArgs h) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const float wi = adam_update(h, g[i], w, m1, m2, i);
+  const float wi = adam_update(h, g[i], adam_load(w, m1, m2, i), w, m1, m2, i);
   if (wb) wb[i] = f2bf(wi);
 }
 
@@ -461,7 +468,7 @@ __global__ __launch_bounds__(256) void k_mlp_infer_p(InferArgs a) {
 // ---- a training step in two launches ---------------------------------------------------------
 // For the shapes of the fused inference with up to three hidden layers.  A step layer by layer is
 // 45 small launches (GEMMs, split-K sums, column sums, GELU backward, Adam) that wait for each
-// other, 181 us for 512 rows; these two take 23 (8,192 rows: 725 and 69).  Every product, sum and
+// other, 181 us for 512 rows; these two take 21 (8,192 rows: 725 and 66).  Every product, sum and
 // rounding is the layer-by-layer step's, in its order, so the weights are the same bit for bit.
 //
 // k_train_rows: one workgroup takes 16 rows through the forward pass, the loss and the backward
@@ -501,44 +508,43 @@ __device__ __forceinline__ void store4(uint16_t *p, const uint16_t (&v)[4]) {
 template <int K, int HID>
 __device__ __forceinline__ void train_forward(const uint16_t (*Hin)[kInferW + 8],
                                               uint16_t (*Hout)[kInferW + 8],
-                                              const bf16x8 (&fb)[K / 32][HID / 64],
-                                              const float (&bc)[HID / 64], uint16_t *outT,
-                                              int rows, int r0, f32x4 (&z)[HID / 64], int w,
-                                              int lr, int lq) {
-  constexpr int NBW = HID / 64, KS = K / 32;
+                                              const bf16x8 (&fb)[K / 32], float bc, uint16_t *outT,
+                                              int rows, int r0, f32x4 &z, int w, int lr,
+                                              int lq) {
+  z = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int b = 0; b < NBW; b++) z[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ks = 0; ks < KS; ks++) {
+  for (int ks = 0; ks < K / 32; ks++) {
     const bf16x8 fa = *(const bf16x8 *)&Hin[lr][ks * 32 + 2 * lq];
-#pragma unroll
-    for (int b = 0; b < NBW; b++)
-      z[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb[ks][b], z[b], 0, 0, 0);
+    z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb[ks], z, 0, 0, 0);
   }
+  const int col = w * 16 + lr;
+  uint16_t h[4];
 #pragma unroll
-  for (int b = 0; b < NBW; b++) {
-    const int col = w * (HID / 4) + b * 16 + lr;
-    uint16_t h[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      z[b][v] += bc[b];
-      h[v] = f2bf(gelu(z[b][v]));
-      Hout[lq + v][col] = h[v];
-    }
-    store4(outT + (size_t)col * rows + r0 + lq, h);
+  for (int v = 0; v < 4; v++) {
+    z[v] += bc;
+    h[v] = f2bf(gelu(z[v]));
+    Hout[lq + v][col] = h[v];
   }
+  store4(outT + (size_t)col * rows + r0 + lq, h);
+}
+
+// The B fragments of a forward layer for the wave's 16 columns, and its bias.
+template <int K>
+__device__ __forceinline__ void train_frags(bf16x8 (&fb)[K / 32], float &bc, const TrainLayer &l,
+                                            int w, int lr, int lq) {
+#pragma unroll
+  for (int ks = 0; ks < K / 32; ks++)
+    fb[ks] = *(const bf16x8 *)(l.wt + (size_t)(w * 16 + lr) * K + ks * 32 + 2 * lq);
+  bc = l.b[w * 16 + lr];
 }
 
 // The B fragments of G W^T (K columns of G) for the wave's columns: W's rows.
-template <int K, int HID>
-__device__ __forceinline__ void back_frags(bf16x4 (&fb)[K / 16][HID / 64], const TrainLayer &next,
-                                           int w, int lr, int lq) {
+template <int K>
+__device__ __forceinline__ void back_frags(bf16x4 (&fb)[K / 16], const TrainLayer &next, int w,
+                                           int lr, int lq) {
 #pragma unroll
   for (int ks = 0; ks < K / 16; ks++)
-#pragma unroll
-    for (int b = 0; b < HID / 64; b++)
-      fb[ks][b] = *(const bf16x4 *)(next.wb + (size_t)(w * (HID / 4) + b * 16 + lr) * next.out +
-                                    ks * 16 + lq);
+    fb[ks] = *(const bf16x4 *)(next.wb + (size_t)(w * 16 + lr) * next.out + ks * 16 + lq);
 }
 
 // A hidden layer's backward: the gradient of its output is G W^T (W the next layer's), times GELU'
@@ -546,81 +552,98 @@ __device__ __forceinline__ void back_frags(bf16x4 (&fb)[K / 16][HID / 64], const
 template <int K, int HID>
 __device__ __forceinline__ void train_backward(const uint16_t (*G)[kInferW + 8],
                                                uint16_t (*Gout)[kInferW + 8],
-                                               const bf16x4 (&fb)[K / 16][HID / 64],
+                                               const bf16x4 (&fb)[K / 16],
                                                const TrainLayer &l, int rows, int r0,
-                                               const f32x4 (&z)[HID / 64], int w, int lr,
-                                               int lq) {
-  constexpr int NBW = HID / 64, KS = K / 16;
-  f32x4 acc[NBW];
+                                               const f32x4 &z, int w, int lr, int lq) {
+  float gg[4];  // (does not wait for the product)
 #pragma unroll
-  for (int b = 0; b < NBW; b++) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int v = 0; v < 4; v++) gg[v] = gelu_grad(z[v]);
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) {
+  for (int ks = 0; ks < K / 16; ks++) {
     const bf16x4 fa = *(const bf16x4 *)&G[lr][ks * 16 + lq];
-#pragma unroll
-    for (int b = 0; b < NBW; b++)
-      acc[b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa, fb[ks][b], acc[b], 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa, fb[ks], acc, 0, 0, 0);
   }
+  const int col = w * 16 + lr;
+  uint16_t h[4];
 #pragma unroll
-  for (int b = 0; b < NBW; b++) {
-    const int col = w * (HID / 4) + b * 16 + lr;
-    uint16_t h[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const float g = acc[b][v] * gelu_grad(z[b][v]);
-      l.d[(size_t)(r0 + lq + v) * HID + col] = g;
-      h[v] = f2bf(g);
-      Gout[lq + v][col] = h[v];
-    }
-    store4(l.dT + (size_t)col * rows + r0 + lq, h);
+  for (int v = 0; v < 4; v++) {
+    const float g = acc[v] * gg[v];
+    l.d[(size_t)(r0 + lq + v) * HID + col] = g;
+    h[v] = f2bf(g);
+    Gout[lq + v][col] = h[v];
   }
+  store4(l.dT + (size_t)col * rows + r0 + lq, h);
 }
 
-// Every layer's weight fragments are requested at the start, so that their latency is paid once and
-// not once a layer: 14.5 us for 512 rows (64 rows a workgroup and each layer's fragments when it
-// comes: 23.3; whole steps 23 and 32 us, 69 and 70 with 8,192 rows).
+// The workgroup's LDS is in order across it; global stores and loads stay in flight (__syncthreads
+// would wait for them).
+__device__ __forceinline__ void lds_barrier() {
+  __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  __asm__ volatile("" ::: "memory");
+}
+
+// A wave per 16 columns.  The rows, every layer's weight fragments and the targets are requested at
+// the start, so that their latency is paid once and not once a layer: 12.8 us for 512 rows (two
+// column blocks a wave 14.0; 64 rows a workgroup and each layer's fragments when it comes 23.3).
 template <int DINP, int HID, int NH>
-__global__ __launch_bounds__(256) void k_train_rows(TrainArgs a) {
-  constexpr int KH = HID / 32;
+__global__ __launch_bounds__(4 * HID) void k_train_rows(TrainArgs a) {
+  constexpr int KH = HID / 32, NT = 4 * HID, XE = (DINP * 4 + NT - 1) / NT;
   __shared__ __attribute__((aligned(16))) uint16_t Hs[2][kTrainRows][kInferW + 8];
   __shared__ float dsq[kTrainRows][17];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lq = 4 * (lane >> 4);
   const int r0 = blockIdx.x * kTrainRows, R = a.rows;
-  bf16x8 f0[DINP / 32][HID / 64], fh[NH][KH][HID / 64], fo[KH];
-  bf16x4 g0[1][HID / 64], gh[NH][HID / 16][HID / 64];
-  float c0[HID / 64], ch[NH][HID / 64];
-  infer_frags<DINP, HID>(f0, c0, a.l[0].wt, a.l[0].b, w, lr, lq);
+  bf16x8 f0[DINP / 32], fh[NH][KH], fo[KH];
+  bf16x4 g0[1], gh[NH][HID / 16];
+  float c0, ch[NH];
+  // the rows first: what is requested first arrives first
+  float xv[XE][4];
 #pragma unroll
-  for (int l = 1; l < NH; l++)
-    infer_frags<HID, HID>(fh[l - 1], ch[l - 1], a.l[l].wt, a.l[l].b, w, lr, lq);
+  for (int e = 0; e < XE; e++) {
+    const int i = tid + e * NT, c = i % DINP, r = i / DINP * 4;
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+      xv[e][v] = c < a.din && r < kTrainRows ? a.x[(size_t)(r0 + r + v) * a.din + c] : 0.f;
+  }
+  train_frags<DINP>(f0, c0, a.l[0], w, lr, lq);
+#pragma unroll
+  for (int l = 1; l < NH; l++) train_frags<HID>(fh[l - 1], ch[l - 1], a.l[l], w, lr, lq);
 #pragma unroll
   for (int ks = 0; ks < KH; ks++)
     fo[ks] = *(const bf16x8 *)(a.l[NH].wt + (size_t)lr * HID + ks * 32 + 2 * lq);
-  back_frags<16, HID>(g0, a.l[NH], w, lr, lq);
+  const bool real = lr < a.dout;
+  const float co = real ? a.l[NH].b[lr] : 0.f;
+  float tv[4];
 #pragma unroll
-  for (int l = NH - 2; l >= 0; l--) back_frags<HID, HID>(gh[l], a.l[l + 1], w, lr, lq);
-  for (int i = tid; i < DINP * kTrainRows / 4; i += 256) {  // four rows of one column
-    const int c = i % DINP, r = i / DINP * 4;
+  for (int v = 0; v < 4; v++) tv[v] = real ? a.t[(size_t)(r0 + lq + v) * a.dout + lr] : 0.f;
+  back_frags<16>(g0, a.l[NH], w, lr, lq);
+#pragma unroll
+  for (int l = NH - 2; l >= 0; l--) back_frags<HID>(gh[l], a.l[l + 1], w, lr, lq);
+#pragma unroll
+  for (int e = 0; e < XE; e++) {  // four rows of one column
+    const int i = tid + e * NT, c = i % DINP, r = i / DINP * 4;
+    if (r >= kTrainRows) break;
     uint16_t h[4];
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      h[v] = c < a.din ? f2bf(a.x[(size_t)(r0 + r + v) * a.din + c]) : 0;
+      h[v] = f2bf(xv[e][v]);
       Hs[0][r + v][c] = h[v];
     }
     store4(a.l[0].inT + (size_t)c * R + r0 + r, h);
   }
-  __syncthreads();
-  f32x4 z[NH][HID / 64];
+  lds_barrier();
+  f32x4 z[NH];
   train_forward<DINP, HID>(Hs[0], Hs[1], f0, c0, a.l[1].inT, R, r0, z[0], w, lr, lq);
-  __syncthreads();
+  lds_barrier();
   int cur = 1;
 #pragma unroll
   for (int l = 1; l < NH; l++) {
     train_forward<HID, HID>(Hs[cur], Hs[cur ^ 1], fh[l - 1], ch[l - 1], a.l[l + 1].inT, R, r0,
-                                z[l], w, lr, lq);
-    __syncthreads();
+                            z[l], w, lr, lq);
+    lds_barrier();
     cur ^= 1;
   }
   // output layer, columns 0..15, and the loss (k_mse), by the first wave
@@ -632,8 +655,6 @@ __global__ __launch_bounds__(256) void k_train_rows(TrainArgs a) {
       const bf16x8 fa = *(const bf16x8 *)&Hs[cur][lr][ks * 32 + 2 * lq];
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fo[ks], acc, 0, 0, 0);
     }
-    const bool real = lr < a.dout;
-    const float bc = real ? o.b[lr] : 0.f;
     const float sc = 2.f / ((float)R * (float)a.dout);
     uint16_t h[4];
 #pragma unroll
@@ -641,7 +662,7 @@ __global__ __launch_bounds__(256) void k_train_rows(TrainArgs a) {
       const int row = lq + v;
       float g = 0.f, d = 0.f;
       if (real) {
-        d = (acc[v] + bc) - a.t[(size_t)(r0 + row) * a.dout + lr];
+        d = (acc[v] + co) - tv[v];
         g = sc * d;
       }
       dsq[row][lr] = d * d;
@@ -651,7 +672,7 @@ __global__ __launch_bounds__(256) void k_train_rows(TrainArgs a) {
     }
     store4(o.dT + (size_t)lr * R + r0 + lq, h);
   }
-  __syncthreads();
+  lds_barrier();
   if (tid < kTrainRows) {
     float l = 0.f;
     for (int c = 0; c < a.dout; c++) l += dsq[tid][c];
@@ -663,13 +684,14 @@ __global__ __launch_bounds__(256) void k_train_rows(TrainArgs a) {
   cur ^= 1;
 #pragma unroll
   for (int l = NH - 2; l >= 0; l--) {
-    __syncthreads();
+    lds_barrier();
     train_backward<HID, HID>(Hs[cur], Hs[cur ^ 1], gh[l], a.l[l], R, r0, z[l], w, lr, lq);
     cur ^= 1;
   }
 }
 
 constexpr int kTrainSplits = 64;
+constexpr int kTrainAhead = 8;
 __global__ __launch_bounds__(256) void k_train_weights(TrainArgs a) {
   __shared__ float part[kTrainSplits][256];  // [range][4 x lane + v]
   const int tid = threadIdx.x, lane = tid & 63;
@@ -686,19 +708,25 @@ __global__ __launch_bounds__(256) void k_train_weights(TrainArgs a) {
     const int nbc = y.cols / 16, mb = b / nbc * 16, nb = b % nbc * 16;
     const uint16_t *pa = y.inT + (size_t)(mb + lr) * a.rows + lq;
     const uint16_t *pb = y.dT + (size_t)(nb + lr) * a.rows + lq;
+    // thread (i, j) of the block: accumulator register i % 4 of lane 16 (i / 4) + j; its weight's
+    // state is on its way while the gradient is made
+    const int i = tid >> 4, j = tid & 15, src = ((i >> 2) * 16 + j) * 4 + (i & 3);
+    const int row = mb + i, col = nb + j;
+    const int64_t at = (int64_t)row * y.out + col;
+    const AdamState v0 = adam_load(y.w, y.m1, y.m2, at);
     for (int s = w; s < a.splits; s += 4) {
       const int k1 = min(a.rows, (s + 1) * a.kps);
       f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int k = s * a.kps; k < k1; k += 128) {  // eight steps' operands in flight
-        bf16x4 fa[8], fb[8];
+      for (int k = s * a.kps; k < k1; k += 16 * kTrainAhead) {  // so many steps' operands in flight
+        bf16x4 fa[kTrainAhead], fb[kTrainAhead];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
+        for (int u = 0; u < kTrainAhead; u++) {
           const int at = min(k + 16 * u, k1 - 16);
           fa[u] = *(const bf16x4 *)(pa + at);
           fb[u] = *(const bf16x4 *)(pb + at);
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++)
+        for (int u = 0; u < kTrainAhead; u++)
           if (k + 16 * u < k1)
             acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa[u], fb[u], acc, 0, 0, 0);
       }
@@ -706,8 +734,6 @@ __global__ __launch_bounds__(256) void k_train_weights(TrainArgs a) {
       for (int v = 0; v < 4; v++) part[s][lane * 4 + v] = acc[v];
     }
     __syncthreads();
-    // thread (i, j) of the block: accumulator register i % 4 of lane 16 (i / 4) + j
-    const int i = tid >> 4, j = tid & 15, src = ((i >> 2) * 16 + j) * 4 + (i & 3);
     float g;
     if (a.splits > 1) {  // k_splitk_sum
       g = 0.f;
@@ -715,9 +741,7 @@ __global__ __launch_bounds__(256) void k_train_weights(TrainArgs a) {
     } else {
       g = part[0][src];
     }
-    const int row = mb + i, col = nb + j;
-    const int64_t at = (int64_t)row * y.out + col;
-    const uint16_t wb = f2bf(adam_update(a.adam, g, y.w, y.m1, y.m2, at));
+    const uint16_t wb = f2bf(adam_update(a.adam, g, v0, y.w, y.m1, y.m2, at));
     y.wb[at] = wb;
     y.wt[(int64_t)col * y.in + row] = wb;
     return;
@@ -740,7 +764,8 @@ __global__ __launch_bounds__(256) void k_train_weights(TrainArgs a) {
     if (g < q) part[g][c] += part[g + q][c];
     __syncthreads();
   }
-  if (g == 0) (void)adam_update(a.adam, part[0][c], y.b, y.bm1, y.bm2, col);
+  if (g == 0)
+    (void)adam_update(a.adam, part[0][c], adam_load(y.b, y.bm1, y.bm2, col), y.b, y.bm1, y.bm2, col);
 }
 
 }  // namespace nb
@@ -1055,9 +1080,9 @@ int train_step_fused(nb_mlp *m, const float *x, const float *t, int64_t rows, fl
   a.adam = next_adam(m, lr);
   const dim3 grid((unsigned)(rows / kTrainRows));
 #define NB_TRAIN(D, H)                                                                           \
-  if (L == 1) hipLaunchKernelGGL((k_train_rows<D, H, 1>), grid, dim3(256), 0, st, a);            \
-  else if (L == 2) hipLaunchKernelGGL((k_train_rows<D, H, 2>), grid, dim3(256), 0, st, a);       \
-  else hipLaunchKernelGGL((k_train_rows<D, H, 3>), grid, dim3(256), 0, st, a);
+  if (L == 1) hipLaunchKernelGGL((k_train_rows<D, H, 1>), grid, dim3(4 * H), 0, st, a);          \
+  else if (L == 2) hipLaunchKernelGGL((k_train_rows<D, H, 2>), grid, dim3(4 * H), 0, st, a);     \
+  else hipLaunchKernelGGL((k_train_rows<D, H, 3>), grid, dim3(4 * H), 0, st, a);
   if (m->dinp == 64 && m->hid == 64) { NB_TRAIN(64, 64) }
   else if (m->dinp == 128 && m->hid == 64) { NB_TRAIN(128, 64) }
   else if (m->dinp == 64) { NB_TRAIN(64, 128) }
