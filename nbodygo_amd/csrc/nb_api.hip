@@ -5,8 +5,8 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <new>
-
 
 #include "nb_internal.hpp"
 
@@ -1010,10 +1010,12 @@ int nb_cycle(nb_ctx *c, double R, int64_t *n_out) {
     }
     const int run = cycle_run(n);
     NB_HIP(c, launch_keep_count(c->flags, (int)n, run, c->cyc_part, st));
-    std::vector<int32_t> part((size_t)(n + run - 1) / run);
-    const Fetch f = {part.data(), c->cyc_part, part.size() * sizeof(int32_t)};
+    const size_t runs = (size_t)(n + run - 1) / run;
+    std::unique_ptr<int32_t[]> part(new (std::nothrow) int32_t[runs]);
+    if (!part) return fail(c, NB_E_NOMEM, "nb_cycle: host allocation failed");
+    const Fetch f = {part.get(), c->cyc_part, runs * sizeof(int32_t)};
     NB_HIP(c, stage_fetch(&f, 1, st));
-    for (int32_t p : part) nk += p;
+    for (size_t k = 0; k < runs; k++) nk += part[k];
   }
   int64_t nq = 0;  // fragments waiting in the device queue
   if (c->p.events) {

@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <system_error>
@@ -175,13 +176,13 @@ hipError_t stage_send_reversed(const Send *seg, int n, int64_t count, hipStream_
   const size_t pad = (size_t)16 * n;
   Lease l((size_t)count * each + pad);
   if (!l.b) {  // no pinned memory to be had: reversed copies, one array at a time
-    std::vector<char> rev;
+    std::unique_ptr<char[]> rev(new (std::nothrow) char[(size_t)count * 8]);
+    if (!rev) return hipErrorOutOfMemory;
     for (int k = 0; k < n; k++) {
       const size_t w = (size_t)seg[k].width;
-      rev.resize((size_t)count * w);
       for (int64_t i = 0; i < count; i++)
-        memcpy(rev.data() + i * w, static_cast<const char *>(seg[k].src) + (count - 1 - i) * w, w);
-      const hipError_t e = hipMemcpyAsync(seg[k].dst, rev.data(), rev.size(),
+        memcpy(rev.get() + i * w, static_cast<const char *>(seg[k].src) + (count - 1 - i) * w, w);
+      const hipError_t e = hipMemcpyAsync(seg[k].dst, rev.get(), (size_t)count * w,
                                           hipMemcpyHostToDevice, st);
       if (e != hipSuccess) return e;
       const hipError_t e2 = hipStreamSynchronize(st);
