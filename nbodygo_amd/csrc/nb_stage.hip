@@ -11,10 +11,10 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 
 #include "nb_internal.hpp"
@@ -25,6 +25,7 @@ constexpr size_t kStageMax = (size_t)32 << 20;    // bytes of a pinned buffer at
 constexpr size_t kStagePiece = (size_t)1 << 20;   // bytes a thread moves at a time
 constexpr size_t kStageSlice = (size_t)4 << 20;   // bytes per launch (and per event)
 constexpr size_t kStageSmall = (size_t)1 << 20;   // total up to which one launch and one thread do
+constexpr int kStageSlices = 64;                  // slices in flight at most (8 of full size fit)
 
 // Pieces of device arrays to pinned host memory: the kernel's stores go over the bus in whole lines,
 // as fast as the copy engine's (about 53 GB/s), and a launch takes up to 16 pieces where a copy call
@@ -65,31 +66,42 @@ __global__ void k_publish(const DevCounters *c, DevCounters *host) {
 // of a millisecond, so they outlive a context: idle ones wait here, at most kStageIdle of at most
 // kStageMax bytes each, and all are freed when the last context or batch of the process goes.  A
 // buffer belongs to one call at a time, so any number of threads and streams may fetch at once.
+// Its lists have fixed room: the calls are C entries, from which nothing may be thrown.
+struct Piece {
+  char *dst;
+  size_t at, bytes;
+  int slice;
+};
 struct StageBuf {
   int device = 0;
   char *buf = nullptr;
   size_t bytes = 0;
-  std::vector<hipEvent_t> ev;
+  int nev = 0;
+  hipEvent_t ev[kStageSlices];
+  Piece window[kStageSlices * kFetchMax];  // a call's pieces, as many as the staging holds
 };
-constexpr size_t kStageIdle = 4;
+constexpr int kStageIdle = 4;
 static std::mutex g_mutex;
-static std::vector<StageBuf *> g_idle;
+static StageBuf *g_idle[kStageIdle];
+static int g_nidle = 0;
 static int g_users = 0;
 
 static void destroy(StageBuf *b) {
-  for (hipEvent_t e : b->ev) (void)hipEventDestroy(e);
+  for (int k = 0; k < b->nev; k++) (void)hipEventDestroy(b->ev[k]);
   if (b->buf) (void)hipHostFree(b->buf);
   delete b;
 }
 
 void stage_user(int add) {
-  std::vector<StageBuf *> gone;
+  StageBuf *gone[kStageIdle];
+  int n = 0;
   {
     std::lock_guard<std::mutex> lock(g_mutex);
     g_users += add;
-    if (g_users == 0) gone.swap(g_idle);
+    if (g_users == 0)
+      while (g_nidle > 0) gone[n++] = g_idle[--g_nidle];
   }
-  for (StageBuf *b : gone) destroy(b);
+  for (int k = 0; k < n; k++) destroy(gone[k]);
 }
 
 namespace {
@@ -101,9 +113,13 @@ struct Lease {  // a buffer for one call
     if (hipGetDevice(&device) != hipSuccess) return;
     {
       std::lock_guard<std::mutex> lock(g_mutex);
-      for (size_t k = 0; k < g_idle.size(); k++)
-        if (g_idle[k]->device == device && (!b || g_idle[k]->bytes > b->bytes)) b = g_idle[k];
-      if (b) g_idle.erase(std::find(g_idle.begin(), g_idle.end(), b));
+      int at = -1;
+      for (int k = 0; k < g_nidle; k++)
+        if (g_idle[k]->device == device && (at < 0 || g_idle[k]->bytes > g_idle[at]->bytes)) at = k;
+      if (at >= 0) {
+        b = g_idle[at];
+        g_idle[at] = g_idle[--g_nidle];
+      }
     }
     if (!b && !(b = new (std::nothrow) StageBuf())) return;
     b->device = device;
@@ -129,8 +145,8 @@ struct Lease {  // a buffer for one call
     if (!b) return;
     {
       std::lock_guard<std::mutex> lock(g_mutex);
-      if (g_users > 0 && g_idle.size() < kStageIdle) {
-        g_idle.push_back(b);
+      if (g_users > 0 && g_nidle < kStageIdle) {
+        g_idle[g_nidle++] = b;
         b = nullptr;
       }
     }
@@ -235,21 +251,15 @@ hipError_t stage_fetch(const Fetch *seg, int n, hipStream_t st) {
   }
   char *const buf = l.b->buf;
   const size_t bytes = l.b->bytes;
-  std::vector<hipEvent_t> &ev = l.b->ev;
-  struct Piece {
-    char *dst;
-    size_t at, bytes;
-    int slice;
-  };
-  std::vector<Piece> window;  // as many pieces as the staging holds
+  hipEvent_t *const ev = l.b->ev;
+  Piece *const window = l.b->window;
   int k = 0;
   size_t off = 0;
   while (k < n) {
-    window.clear();
-    size_t at = 0;
+    size_t at = 0, pieces = 0;
     int slice = 0;
     hipError_t r = hipSuccess;
-    while (k < n && at < bytes && r == hipSuccess) {
+    while (k < n && at < bytes && slice < kStageSlices && r == hipSuccess) {
       PackArgs a;
       a.dst = static_cast<char *>(l.dev);
       int np = 0;
@@ -261,7 +271,7 @@ hipError_t stage_fetch(const Fetch *seg, int n, hipStream_t st) {
           a.bytes[np] = (uint32_t)take;
           a.at[np] = (uint32_t)at;
           np++;
-          window.push_back({static_cast<char *>(seg[k].dst) + off, at, take, slice});
+          window[pieces++] = {static_cast<char *>(seg[k].dst) + off, at, take, slice};
         }
         at += (take + 15) / 16 * 16;
         off += take;
@@ -277,10 +287,9 @@ hipError_t stage_fetch(const Fetch *seg, int n, hipStream_t st) {
       hipLaunchKernelGGL(k_pack, dim3(gx, (unsigned)np), dim3(256), 0, st, a);
       r = hipGetLastError();
       if (total > kStageSmall && r == hipSuccess) {
-        if ((int)ev.size() == slice) {
-          hipEvent_t e;
-          r = hipEventCreateWithFlags(&e, hipEventDisableTiming);
-          if (r == hipSuccess) ev.push_back(e);
+        if (l.b->nev == slice) {
+          r = hipEventCreateWithFlags(&ev[slice], hipEventDisableTiming);
+          if (r == hipSuccess) l.b->nev++;
         }
         if (r == hipSuccess) r = hipEventRecord(ev[slice], st);
       }
@@ -293,8 +302,8 @@ hipError_t stage_fetch(const Fetch *seg, int n, hipStream_t st) {
     if (total <= kStageSmall) {
       r = hipStreamSynchronize(st);
       if (r != hipSuccess) return r;
-      for (const Piece &p : window) memcpy(p.dst, buf + p.at, p.bytes);
-      return hipSuccess;
+      for (size_t q = 0; q < pieces; q++) memcpy(window[q].dst, buf + window[q].at, window[q].bytes);
+      continue;  // (a great many short arrays take further windows)
     }
     std::atomic<size_t> next{0};
     std::atomic<int> bad{(int)hipSuccess};
@@ -302,7 +311,7 @@ hipError_t stage_fetch(const Fetch *seg, int n, hipStream_t st) {
     (void)hipGetDevice(&device);
     auto work = [&]() {
       (void)hipSetDevice(device);
-      for (size_t q; (q = next.fetch_add(1)) < window.size();) {
+      for (size_t q; (q = next.fetch_add(1)) < pieces;) {
         const hipError_t w = hipEventSynchronize(ev[window[q].slice]);
         if (w != hipSuccess) {
           bad = (int)w;
@@ -316,8 +325,8 @@ hipError_t stage_fetch(const Fetch *seg, int n, hipStream_t st) {
     for (int t = 1; t < nt; t++) {
       try {
         pool[t] = std::thread(work);
-      } catch (const std::system_error &) {
-        break;  // no thread to be had: the others take its pieces
+      } catch (const std::exception &) {
+        break;  // no thread (or memory for one) to be had: the others take its pieces
       }
     }
     work();

@@ -1,0 +1,31 @@
+"""Host memory that runs out inside a call of the C interface: an error code or success, never an
+exception out of the call (which would end the process)."""
+import pytest
+
+import host_only
+
+STORE = """
+b = gen.plummer(%d, 1)
+g = NBodyGPU(G=1.0, eps=0.01, overlap_cutoff=False, collisions=False)
+g.load(b)
+for k in range(60):
+    fake.fake_fail_new(k)
+    try:
+        g.store()
+        g.render()
+    except L.NBodyError as e:
+        assert e.code in (L.NB_E_HIP, L.NB_E_NOMEM), e
+    if fake.fake_new_left() >= 0:
+        break                     # fewer than k allocations: all of them have failed once
+    fake.fake_fail_new(-1)
+    g.store()
+fake.fake_fail_new(-1)
+g.close()
+print("done", k)
+"""
+
+
+@pytest.mark.parametrize("n", [1000, 100000, 600000])  # one launch; threads; several windows
+def test_read_back_without_host_memory(n):
+    rc, out = host_only.run(STORE % n)
+    assert rc == 0 and "done" in out, (rc, out)
