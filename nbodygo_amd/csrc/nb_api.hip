@@ -983,14 +983,22 @@ int nb_add_bodies(nb_ctx *c, int64_t k, const double *x, const double *y, const 
     return fail(c, NB_E_INVALID, "nb_add_bodies: NULL array");
   const double *src[10] = {x, y, z, vx, vy, vz, m, r, nullptr, frag};
   auto &A = c->adds;
+  const size_t had = A.beh.size();
   auto queue = [k](std::vector<double> &v, const double *s, double otherwise) {
     if (s) v.insert(v.end(), s, s + k);
     else v.insert(v.end(), (size_t)k, otherwise);
   };
-  for (int q = 0; q < 10; q++) queue(A.a[q], src[q], q == 8 ? 1.0 : 0.0);
-  queue(A.fstep, frag_step, 0.0);
-  A.beh.insert(A.beh.end(), beh, beh + k);
-  A.flags.insert(A.flags.end(), flags, flags + k);
+  try {
+    for (int q = 0; q < 10; q++) queue(A.a[q], src[q], q == 8 ? 1.0 : 0.0);
+    queue(A.fstep, frag_step, 0.0);
+    A.flags.insert(A.flags.end(), flags, flags + k);
+    A.beh.insert(A.beh.end(), beh, beh + k);
+  } catch (const std::exception &) {  // the queue is as it was before the call
+    for (auto &v : A.a) v.resize(std::min(v.size(), had));
+    A.fstep.resize(std::min(A.fstep.size(), had));
+    A.flags.resize(std::min(A.flags.size(), had));
+    return fail(c, NB_E_NOMEM, "nb_add_bodies: host allocation failed");
+  }
   return NB_OK;
 }
 

@@ -29,3 +29,26 @@ print("done", k)
 def test_read_back_without_host_memory(n):
     rc, out = host_only.run(STORE % n)
     assert rc == 0 and "done" in out, (rc, out)
+
+
+def test_add_without_host_memory_leaves_the_queue_alone():
+    rc, out = host_only.run("""
+    g = NBodyGPU(G=1.0, eps=0.01, overlap_cutoff=False, collisions=False)
+    g.load(gen.plummer(100, 1))
+    a = gen.plummer(10, 2)
+    failed = 0
+    for k in range(40):
+        fake.fake_fail_new(k)
+        try:
+            g.add_bodies(a)
+        except L.NBodyError as e:
+            assert e.code == L.NB_E_NOMEM, e
+            failed += 1
+        if fake.fake_new_left() >= 0:
+            break
+    fake.fake_fail_new(-1)
+    n = g.cycle(1.0)              # (no kernel runs: nothing of the first 100 survives)
+    assert failed >= 3 and n == 10 * (k + 1 - failed), (failed, k, n)
+    print("done")
+    """)
+    assert rc == 0 and "done" in out, (rc, out)
