@@ -125,7 +125,9 @@ static int64_t sym_blocks(const ForceShape &s, int64_t n) {
 // 0.054 at n = 10,000, 0.084 / 0.083 / 0.082 at 16,384, 0.175 / 0.167 / 0.172 at 25,000,
 // 0.254 / 0.244 / 0.239 at 32,768, 0.934 / 0.863 / 0.826 at 65,536.
 // Slices: about 8,192 workgroups, at least 12 and at most 48 slices a row (small n: 16, where each
-// more costs a longer fold): with 12 / 24 / 48 slices at 262,144 12.6 / 12.25 / 12.2 ms.
+// more costs a longer fold): with 12 / 24 / 48 slices at 262,144 12.6 / 12.25 / 12.2 ms.  A slice
+// takes 24 bytes a body, so the 12 become fewer once the rows alone are 8,192 workgroups (8.4
+// million bodies): one slice from 100 million on, where twelve would take 31 GB.
 static ForceShape sym_shape(int64_t n) {
   ForceShape s;
   s.variant = 3;
@@ -133,8 +135,9 @@ static ForceShape sym_shape(int64_t n) {
   s.block = 256;
   s.ipl = n < 12288 ? 1 : n < 28672 ? 2 : 4;
   const int64_t nb = std::max<int64_t>(sym_blocks(s, n), 1);
+  const int64_t least = std::min<int64_t>(12, (12 * 8192 + nb - 1) / nb);
   s.jsplit = s.ipl == 1 ? 16 : s.ipl == 2 ? 24
-                             : (int)std::min<int64_t>(48, std::max<int64_t>(12, 8192 / nb));
+                             : (int)std::min<int64_t>(48, std::max<int64_t>(least, 8192 / nb));
   return s;
 }
 
@@ -159,7 +162,7 @@ int ensure_acc(Ctx *c, int split) {
 }
 
 // (Re)size the per-slice and per-tile buffers for the current shape.
-static int prepare_shape(Ctx *c) {
+static int size_shape(Ctx *c) {
   if (!shape_valid(c->shape, c->npad) || (c->shape.variant == 3 && !sym_possible(c)))
     return fail(c, NB_E_INVALID, "invalid FP32 force kernel shape for this body count");
   const int split = c->p.precision == NB_PREC_FP64 ? 1
@@ -190,6 +193,23 @@ static int prepare_shape(Ctx *c) {
   NB_HIP(c, launch_rmax_tile(c->r, c->flags, (int)c->n, c->shape.tile_j, tiles, c->rmax_tile,
                              c->stream));
   return NB_OK;
+}
+
+// The same; a shape that takes each pair once gives way to one that needs no workspace for it (and
+// a quarter of the slices) when the device has no room, unless the caller asked for that variant.
+static int prepare_shape(Ctx *c) {
+  int rc = size_shape(c);
+  if (rc != NB_E_HIP || c->shape.variant != 3 || c->p.variant == 3) return rc;
+  (void)hipGetLastError();  // or the next launch would report it
+  if (c->acc) (void)hipFree(c->acc);
+  if (c->layer) (void)hipFree(c->layer);
+  c->acc = nullptr;
+  c->layer = nullptr;
+  c->acc_split = 0;
+  c->layer_words = 0;
+  c->shape = default_shape(c->npad);
+  c->shape_tuned = false;
+  return size_shape(c);
 }
 
 // Keeps a tuned shape that still fits the padded count; else the default with the params'
@@ -928,7 +948,10 @@ int nb_autotune(nb_ctx *c, int32_t reps, int32_t *cfg) {
     }
     if (dup) continue;
     c->shape = s;
-    if (prepare_shape(c)) continue;
+    if (size_shape(c)) {  // (no room for this one)
+      (void)hipGetLastError();
+      continue;
+    }
     if (launch_plain(c, detect_needed(c), nullptr) != hipSuccess) continue;  // warm-up
     NB_HIP(c, hipEventRecord(e0, c->stream));
     for (int k = 0; k < reps; k++) (void)launch_plain(c, detect_needed(c), nullptr);

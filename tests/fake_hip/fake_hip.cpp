@@ -25,6 +25,8 @@ static long host_mallocs = 0, dev_mallocs = 0;
 static long publish_pairs = -1;
 static std::atomic<long> new_countdown{-1};
 
+static hipError_t last_error = hipSuccess;
+
 struct Head {
   size_t bytes, pad[31];
 };
@@ -74,9 +76,10 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
   launched += n + "\n";
   // the counters' copy to pinned memory: the first word is the pair count
   if (n.find("k_publish") != std::string::npos) {
-    char *dst = *static_cast<char **>(args[1]);
-    const uint32_t p = publish_pairs < 0 ? **static_cast<uint32_t **>(args[0]) : publish_pairs;
-    memcpy(dst, &p, sizeof p);
+    char *dst = *static_cast<char **>(args[1]), *src = *static_cast<char **>(args[0]);
+    memcpy(dst, src, (reinterpret_cast<Head *>(src) - 1)->bytes);
+    const uint32_t p = publish_pairs;
+    if (publish_pairs >= 0) memcpy(dst, &p, sizeof p);
   }
   return hipSuccess;
 }
@@ -86,7 +89,7 @@ hipError_t hipMalloc(void **p, size_t bytes) {
   std::lock_guard<std::mutex> l(mu);
   dev_mallocs++;
   *p = nullptr;
-  if (bytes > budget) return hipErrorOutOfMemory;
+  if (bytes > budget) return last_error = hipErrorOutOfMemory;
   Head *h = static_cast<Head *>(calloc(1, sizeof(Head) + bytes));
   if (!h) return hipErrorOutOfMemory;
   h->bytes = bytes;
@@ -153,7 +156,11 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, in
   return *n = 2, hipSuccess;
 }
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
-hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipGetLastError(void) {
+  const hipError_t e = last_error;
+  last_error = hipSuccess;
+  return e;
+}
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
   *s = reinterpret_cast<hipStream_t>(8);
   return hipSuccess;

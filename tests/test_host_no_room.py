@@ -1,0 +1,53 @@
+"""Device memory that runs out: workspaces of the kernels that take each pair once are given up for
+the kernels that need none, and the call succeeds as it did before there were such workspaces."""
+import host_only
+
+
+def test_a_context_without_room_for_the_workspace():
+    rc, out = host_only.run("""
+    n = 262144
+    b = gen.plummer(n, 1)
+    kw = dict(G=1.0, eps=0.01, overlap_cutoff=False, collisions=True)
+    g = NBodyGPU(variant=2, **kw)
+    g.load(b)
+    need = fake.fake_in_use()           # one evaluation per ordered pair
+    g.close()
+    for room in (1 << 20, 100 << 20, 300 << 20, 1 << 30):
+        fake.fake_budget(need + room)
+        g = NBodyGPU(**kw)
+        g.load(b)
+        v = g.config()["variant"]
+        assert v == (3 if room >= 1 << 30 else 2), (room, v)
+        g.step(1e-3, 1.0)               # (no error left over from the failed allocation)
+        fake.fake_budget(200 << 20)     # (cycle's second set)
+        g.add_bodies(gen.plummer(5, 2))
+        g.cycle(1.0)
+        g.autotune(1)
+        g.step(1e-3, 1.0)
+        g.close()
+        assert fake.fake_in_use() == 0
+    fake.fake_budget(need + (300 << 20))
+    g = NBodyGPU(variant=3, **kw)       # asked for: refused
+    try:
+        g.load(b)
+        raise SystemExit("accepted")
+    except L.NBodyError as e:
+        assert e.code == L.NB_E_HIP, e
+    print("done")
+    """)
+    assert rc == 0 and "done" in out, (rc, out)
+
+
+def test_slices_of_very_many_bodies():
+    """12,288 rows of 1,024 bodies: 8 slices of 24 bytes a body, not 12."""
+    rc, out = host_only.run("""
+    n = 12288 * 1024
+    z = np.zeros(n)
+    from nbodygo_amd import Bodies
+    g = NBodyGPU(G=1.0, eps=0.01, overlap_cutoff=False, collisions=False)
+    g.load(Bodies(z, z, z, z, z, z, z, z))
+    c = g.config()
+    assert c["variant"] == 3 and c["jsplit"] == 8, c
+    print("done")
+    """)
+    assert rc == 0 and "done" in out, (rc, out)
