@@ -28,6 +28,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <new>
 #include <string>
@@ -304,7 +305,8 @@ struct nb_batch {
   int nitems = 0;
   // each unordered pair once (nb_sym.hip): used until a shape is set, and if the tuner prefers it
   bool once = true;
-  bool once_fits = false;  // the loaded simulations are within its sizes
+  bool once_fits = false;  // the loaded simulations are within its sizes, and its workspace is there
+  char *sym_mem = nullptr; // what the next five point into
   BatchSymItem *sym_items = nullptr;
   BatchSymSim *sym_sims = nullptr;
   int32_t *tile_sim = nullptr;
@@ -358,8 +360,7 @@ void free_batch(nb_batch *b) {
   drop_graph(b);
   void *ptrs[] = {b->x, b->y, b->z, b->vx, b->vy, b->vz, b->m, b->rest, b->acc,
                   b->flags, b->collided, b->js, b->ctr, b->items, b->queue,
-                  b->sim_off, b->unpad, b->sym_items, b->sym_sims, b->tile_sim, b->sym_acc,
-                  b->sym_layer};
+                  b->sim_off, b->unpad, b->sym_mem};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   b->x = b->y = b->z = b->vx = b->vy = b->vz = b->m = b->rest = b->acc = nullptr;
@@ -370,11 +371,7 @@ void free_batch(nb_batch *b) {
   b->queue = nullptr;
   b->sim_off = nullptr;
   b->unpad = nullptr;
-  b->sym_items = nullptr;
-  b->sym_sims = nullptr;
-  b->tile_sim = nullptr;
-  b->sym_acc = nullptr;
-  b->sym_layer = nullptr;
+  b->sym_mem = nullptr;
   b->sym_nitems = 0;
   b->once_fits = false;
 }
@@ -425,8 +422,10 @@ int build_items(nb_batch *b, int only_bucket, int force_ipl, int force_tile = 0)
 // lane, and a block's tile list is cut into `slices` equal ranges.
 // Targets per lane: as many as the simulation's size earns (as in one context: 4 from 4,096 bodies,
 // 2 from 1,024), fewer for all when that leaves the chip short of work items.
+// tables: the host's copy of the items and the two tables, which the caller keeps until the stream has
+// been waited for.  Without room for the workspace (or these) the other kernel does the work.
 constexpr int kSymMaxBodies = 32768;  // above, a context of its own is the better place
-static int build_sym(nb_batch *b) {
+static int build_sym(nb_batch *b, std::vector<char> &tables) {
   b->once_fits = false;
   int64_t most = 0, any = 0;
   for (int k = 0; k < b->nsims; k++) {
@@ -486,27 +485,29 @@ static int build_sym(nb_batch *b) {
   std::stable_sort(items.begin(), items.end(), [](const BatchSymItem &x, const BatchSymItem &y) {
     return x.cost > y.cost;
   });
-  void *ptrs[] = {b->sym_items, b->sym_sims, b->tile_sim, b->sym_acc, b->sym_layer};
-  for (void *q : ptrs)
-    if (q) (void)hipFree(q);
-  b->sym_items = nullptr;
-  b->sym_sims = nullptr;
-  b->tile_sim = nullptr;
-  b->sym_acc = nullptr;
-  b->sym_layer = nullptr;
+  // one allocation: the tables, then the workspace
+  auto up = [](size_t v) { return (v + 255) / 256 * 256; };
   const size_t n3 = (size_t)3 * b->n;
-  NB_BHIP(b, hipMalloc((void **)&b->sym_items, items.size() * sizeof(BatchSymItem)));
-  NB_BHIP(b, hipMalloc((void **)&b->sym_sims, sims.size() * sizeof(BatchSymSim)));
-  NB_BHIP(b, hipMalloc((void **)&b->tile_sim, tile_sim.size() * sizeof(int32_t)));
-  NB_BHIP(b, hipMalloc((void **)&b->sym_acc, (size_t)slices * n3 * sizeof(double)));
-  NB_BHIP(b, hipMalloc((void **)&b->sym_layer, (size_t)layers * n3 * sizeof(float)));
-  NB_BHIP(b, hipMemcpyAsync(b->sym_items, items.data(), items.size() * sizeof(BatchSymItem),
-                            hipMemcpyHostToDevice, b->stream));
-  NB_BHIP(b, hipMemcpyAsync(b->sym_sims, sims.data(), sims.size() * sizeof(BatchSymSim),
-                            hipMemcpyHostToDevice, b->stream));
-  NB_BHIP(b, hipMemcpyAsync(b->tile_sim, tile_sim.data(), tile_sim.size() * sizeof(int32_t),
-                            hipMemcpyHostToDevice, b->stream));
-  NB_BHIP(b, hipStreamSynchronize(b->stream));
+  const size_t at_sims = up(items.size() * sizeof(BatchSymItem));
+  const size_t at_tiles = at_sims + up(sims.size() * sizeof(BatchSymSim));
+  const size_t end = at_tiles + up(tile_sim.size() * sizeof(int32_t));
+  const size_t acc_bytes = up((size_t)slices * n3 * sizeof(double));
+  if (hipMalloc((void **)&b->sym_mem, end + acc_bytes + (size_t)layers * n3 * sizeof(float)) !=
+      hipSuccess) {
+    (void)hipGetLastError();  // or the next launch would report it
+    b->sym_mem = nullptr;
+    return NB_OK;
+  }
+  tables.resize(end);
+  memcpy(tables.data(), items.data(), items.size() * sizeof(BatchSymItem));
+  memcpy(tables.data() + at_sims, sims.data(), sims.size() * sizeof(BatchSymSim));
+  memcpy(tables.data() + at_tiles, tile_sim.data(), tile_sim.size() * sizeof(int32_t));
+  NB_BHIP(b, hipMemcpyAsync(b->sym_mem, tables.data(), end, hipMemcpyHostToDevice, b->stream));
+  b->sym_items = reinterpret_cast<BatchSymItem *>(b->sym_mem);
+  b->sym_sims = reinterpret_cast<BatchSymSim *>(b->sym_mem + at_sims);
+  b->tile_sim = reinterpret_cast<int32_t *>(b->sym_mem + at_tiles);
+  b->sym_acc = reinterpret_cast<double *>(b->sym_mem + end);
+  b->sym_layer = reinterpret_cast<float *>(b->sym_mem + end + acc_bytes);
   b->sym_nitems = (int)items.size();
   b->once_fits = true;
   return NB_OK;
@@ -631,10 +632,9 @@ void nb_batch_destroy(nb_batch *b) {
 
 const char *nb_batch_last_error(const nb_batch *b) { return b ? b->err.c_str() : "NULL batch"; }
 
-int nb_batch_load(nb_batch *b, int32_t nsims, const int64_t *offsets, const double *x,
-                  const double *y, const double *z, const double *vx, const double *vy,
-                  const double *vz, const double *m, const uint8_t *flags) {
-  if (!b) return NB_E_INVALID;
+static int batch_load(nb_batch *b, int32_t nsims, const int64_t *offsets, const double *x,
+                      const double *y, const double *z, const double *vx, const double *vy,
+                      const double *vz, const double *m, const uint8_t *flags) {
   if (nsims < 1 || !offsets) return bfail(b, NB_E_INVALID, "nb_batch_load: need nsims >= 1");
   if (offsets[0] != 0) return bfail(b, NB_E_INVALID, "nb_batch_load: offsets[0] must be 0");
   for (int k = 0; k < nsims; k++)
@@ -698,9 +698,27 @@ int nb_batch_load(nb_batch *b, int32_t nsims, const int64_t *offsets, const doub
   b->ctr_last = DevCounters{};
   NB_BHIP(b, launch_write_stream(b->x, b->y, b->z, b->m, b->flags, b->js, (int)n, (int)n,
                                  b->stream));
-  const int rc = build_sym(b);
+  std::vector<char> tables;
+  int rc = NB_OK;
+  try {
+    rc = build_sym(b, tables);
+  } catch (const std::exception &) {  // no host memory for the lists: the other kernel's are shorter
+  }
   if (rc) return rc;
-  return build_items(b, -1, 0);
+  return build_items(b, -1, 0);  // (waits for the copies)
+}
+
+int nb_batch_load(nb_batch *b, int32_t nsims, const int64_t *offsets, const double *x,
+                  const double *y, const double *z, const double *vx, const double *vy,
+                  const double *vz, const double *m, const uint8_t *flags) {
+  if (!b) return NB_E_INVALID;
+  try {
+    return batch_load(b, nsims, offsets, x, y, z, vx, vy, vz, m, flags);
+  } catch (const std::exception &) {
+    (void)hipStreamSynchronize(b->stream);
+    free_batch(b);
+    return bfail(b, NB_E_NOMEM, "nb_batch_load: host allocation failed");
+  }
 }
 
 int nb_batch_set_graph(nb_batch *b, int32_t enable) {

@@ -51,3 +51,33 @@ def test_slices_of_very_many_bodies():
     print("done")
     """)
     assert rc == 0 and "done" in out, (rc, out)
+
+
+BATCH = """
+sims = [gen.plummer(4000 + k, k) for k in range(16)]
+g = NBodyBatch(G=1.0, eps=0.01)
+g.load(sims)
+full = fake.fake_in_use()
+g.step(1e-3, 1.0)
+assert any("k_batch_sym" in k for k in launched())
+g.close()
+assert fake.fake_in_use() == 0
+"""
+
+
+def test_a_batch_without_room_for_the_workspace():
+    rc, out = host_only.run(BATCH + """
+fake.fake_clear()
+fake.fake_budget(full - (1 << 20))
+g = NBodyBatch(G=1.0, eps=0.01)
+g.load(sims)
+g.step(1e-3, 1.0)
+assert any("k_batch_force" in k for k in launched())
+assert not any("k_batch_sym" in k for k in launched())
+g.load(sims[:4])                        # fewer: there is room again
+g.step(1e-3, 1.0)
+assert any("k_batch_sym" in k for k in launched())
+g.close()
+print("done")
+""")
+    assert rc == 0 and "done" in out, (rc, out)

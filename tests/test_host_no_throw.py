@@ -52,3 +52,27 @@ def test_add_without_host_memory_leaves_the_queue_alone():
     print("done")
     """)
     assert rc == 0 and "done" in out, (rc, out)
+
+
+def test_batch_load_without_host_memory():
+    rc, out = host_only.run("""
+    sims = [gen.plummer(300 + k, k) for k in range(8)]
+    g = NBodyBatch(G=1.0, eps=0.01)
+    loaded = failed = 0
+    for k in range(200):
+        fake.fake_fail_new(k)
+        try:
+            g.load(sims)
+            loaded += 1
+        except L.NBodyError as e:
+            assert e.code == L.NB_E_NOMEM, e
+            failed += 1
+        if fake.fake_new_left() >= 0:
+            break
+    fake.fake_fail_new(-1)
+    assert failed and loaded > 1, (failed, loaded)   # (without the pairs-once lists it still loads)
+    g.load(sims)
+    g.step(1e-3, 1.0)
+    print("done")
+    """)
+    assert rc == 0 and "done" in out, (rc, out)
