@@ -811,9 +811,30 @@ int nb_batch_store(nb_batch *b, double *x, double *y, double *z, double *vx, dou
   NB_BHIP(b, hipSetDevice(b->device));
   const int64_t n = b->off[b->nsims];
   if (n == 0) return NB_OK;
-  if (!b->unpad) NB_BHIP(b, hipMalloc((void **)&b->unpad, (size_t)n * (6 * sizeof(double) + 1)));
-  BatchUnpadArgs u;
   const double *src[6] = {b->x, b->y, b->z, b->vx, b->vy, b->vz};
+  double *dst[6] = {x, y, z, vx, vy, vz};
+  if (!b->unpad &&
+      hipMalloc((void **)&b->unpad, (size_t)n * (6 * sizeof(double) + 1)) != hipSuccess) {
+    // no room for the arrays in the caller's order: simulation by simulation from the padded ones
+    (void)hipGetLastError();
+    b->unpad = nullptr;
+    for (int c = 0; c < 7; c++) {
+      char *to = reinterpret_cast<char *>(c < 6 ? (void *)dst[c] : (void *)flags);
+      const char *from = reinterpret_cast<const char *>(c < 6 ? (const void *)src[c] : b->flags);
+      const size_t w = c < 6 ? sizeof(double) : 1;
+      Fetch seg[64];
+      int q = 0;
+      for (int k = 0; to && k < b->nsims; k++) {
+        seg[q++] = {to + b->off[k] * w, from + b->poff[k] * w, (size_t)(b->off[k + 1] - b->off[k]) * w};
+        if (q == 64 || k + 1 == b->nsims) {
+          NB_BHIP(b, stage_fetch(seg, q, b->stream));
+          q = 0;
+        }
+      }
+    }
+    return NB_OK;
+  }
+  BatchUnpadArgs u;
   for (int c = 0; c < 6; c++) u.src[c] = src[c];
   u.flags = b->flags;
   u.out = b->unpad;
@@ -825,7 +846,6 @@ int nb_batch_store(nb_batch *b, double *x, double *y, double *z, double *vx, dou
   hipLaunchKernelGGL(k_batch_unpad, dim3((unsigned)((n + 255) / 256), 7), dim3(256), 0, b->stream,
                      u);
   NB_BHIP(b, hipGetLastError());
-  double *dst[6] = {x, y, z, vx, vy, vz};
   Fetch seg[7];
   int k = 0;
   for (int c = 0; c < 6; c++)

@@ -1,5 +1,5 @@
 // A stand-in for the HIP runtime, for tests of the library's host code without a GPU.  Device and
-// pinned memory are host memory, kernels do nothing, and the test sets what fails and reads what was
+// pinned memory are host memory, kernels do nothing but the read-back's two, and the test sets what fails and reads what was
 // called.  Loaded with RTLD_GLOBAL before libnbgpu.so, its definitions are the ones that the library
 // binds to (operator new among them).
 #include <dlfcn.h>
@@ -70,7 +70,12 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t 
   *g = cfg_grid, *b = cfg_block, *lds = cfg_lds, *st = cfg_stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t) {
+struct PackArgs {  // nb_stage.hip's
+  const void *src[16];
+  uint32_t bytes[16], at[16];
+  char *dst;
+};
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, hipStream_t) {
   std::lock_guard<std::mutex> l(mu);
   const std::string &n = names()[f];
   launched += n + "\n";
@@ -80,6 +85,10 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
     memcpy(dst, src, (reinterpret_cast<Head *>(src) - 1)->bytes);
     const uint32_t p = publish_pairs;
     if (publish_pairs >= 0) memcpy(dst, &p, sizeof p);
+  }
+  if (n.find("k_pack") != std::string::npos) {
+    const PackArgs &a = *static_cast<PackArgs *>(args[0]);
+    for (unsigned c = 0; c < grid.y; c++) memcpy(a.dst + a.at[c], a.src[c], a.bytes[c]);
   }
   return hipSuccess;
 }

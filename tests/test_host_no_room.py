@@ -81,3 +81,20 @@ g.close()
 print("done")
 """)
     assert rc == 0 and "done" in out, (rc, out)
+
+
+def test_a_batch_read_back_without_room_to_reorder():
+    rc, out = host_only.run(BATCH + """
+sims = [gen.plummer(1 + 37 * (k % 9), k) for k in range(150)]
+g = NBodyBatch(G=1.0, eps=0.01)
+g.load(sims)
+fake.fake_budget(1000)
+got = g.store()
+exp = gen.concat(*sims)
+for k in ("x", "y", "z", "vx", "vy", "vz", "flags"):
+    np.testing.assert_array_equal(getattr(got, k), getattr(exp, k))
+g.step(1e-3, 1.0)
+g.close()
+print("done")
+""")
+    assert rc == 0 and "done" in out, (rc, out)
