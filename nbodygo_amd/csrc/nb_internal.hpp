@@ -145,7 +145,7 @@ struct Send {
   int width;
 };
 hipError_t stage_send_reversed(const Send *seg, int n, int64_t count, hipStream_t st);
-void stage_user(int add);  // +1 with a context or batch, -1 with its end
+void stage_user(int add);  // +1 with a context, batch or network, -1 with its end
 
 struct Ctx {
   nb_params p{};

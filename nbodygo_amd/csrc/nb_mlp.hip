@@ -1262,6 +1262,7 @@ int nb_mlp_create(int32_t device, int32_t din, int32_t hidden, int32_t layers, i
       return hip_fail("stream", e);
     }
   }
+  stage_user(1);  // (nb_mlp_destroy, from here on)
   std::mt19937_64 rng(seed);
   for (int l = 0; l <= layers; l++) {
     const int in = l == 0 ? m->dinp : hidden;
@@ -1337,6 +1338,7 @@ void nb_mlp_destroy(nb_mlp *m) {
   if (m->splitbuf) (void)hipFree(m->splitbuf);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
+  stage_user(-1);
 }
 
 const char *nb_mlp_last_error(const nb_mlp *m) { return m ? m->err.c_str() : "NULL mlp"; }
@@ -1383,14 +1385,33 @@ static int xfer_params(nb_mlp *m, float *host, int64_t count, bool to_dev, bool 
   }
   NB_MHIP(m, hipSetDevice(m->device));
   NB_MHIP(m, hipStreamSynchronize(m->stream));
+  // reading: every layer's padded arrays in one call (0.30 ms for three hidden layers of 128 when each
+  // layer had a call and pinned memory of its own, 0.20 by plain copies)
+  std::vector<float> padded;
+  if (!to_dev) {
+    size_t words = 0;
+    for (int l = 0; l <= m->layers; l++) words += (size_t)(m->in_dim[l] + 1) * m->out_dim[l];
+    padded.resize(words);
+    Fetch seg[2 * 9];  // at most 8 hidden layers
+    int k = 0;
+    float *to = padded.data();
+    for (int l = 0; l <= m->layers; l++) {
+      const size_t nw = (size_t)m->in_dim[l] * m->out_dim[l], nb = (size_t)m->out_dim[l];
+      seg[k++] = {to, grads ? m->Wg[l] : m->W[l], nw * 4};
+      seg[k++] = {to + nw, grads ? m->bg[l] : m->bvec[l], nb * 4};
+      to += nw + nb;
+    }
+    NB_MHIP(m, stage_fetch(seg, k, m->stream));
+  }
+  size_t at = 0;
   int64_t off = 0;
   for (int l = 0; l <= m->layers; l++) {
     const int in = l == 0 ? m->din : m->hid, o = l == m->layers ? m->dout : m->hid;
     const int op = m->out_dim[l];
     float *W = grads ? m->Wg[l] : m->W[l];
     float *b = grads ? m->bg[l] : m->bvec[l];
-    std::vector<float> full((size_t)m->in_dim[l] * op, 0.f), bf((size_t)op, 0.f);
     if (to_dev) {
+      std::vector<float> full((size_t)m->in_dim[l] * op, 0.f), bf((size_t)op, 0.f);
       for (int i = 0; i < in; i++)
         for (int j = 0; j < o; j++) full[(size_t)i * op + j] = host[off + (int64_t)i * o + j];
       for (int j = 0; j < o; j++) bf[j] = host[off + (int64_t)in * o + j];
@@ -1399,12 +1420,12 @@ static int xfer_params(nb_mlp *m, float *host, int64_t count, bool to_dev, bool 
       hipLaunchKernelGGL(k_f32_to_bf16, dim3(nblk((int64_t)full.size())), dim3(256), 0,
                          m->stream, W, m->Wb[l], (int64_t)full.size());
       NB_MHIP(m, hipStreamSynchronize(m->stream));
-    } else {
-      const Fetch seg[2] = {{full.data(), W, full.size() * 4}, {bf.data(), b, bf.size() * 4}};
-      NB_MHIP(m, stage_fetch(seg, 2, m->stream));
+    } else {  // from the padded copy
+      const float *full = padded.data() + at, *bf = full + (size_t)m->in_dim[l] * op;
       for (int i = 0; i < in; i++)
         for (int j = 0; j < o; j++) host[off + (int64_t)i * o + j] = full[(size_t)i * op + j];
       for (int j = 0; j < o; j++) host[off + (int64_t)in * o + j] = bf[j];
+      at += (size_t)(m->in_dim[l] + 1) * op;
     }
     off += (int64_t)in * o + o;
   }

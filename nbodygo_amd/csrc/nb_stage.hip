@@ -64,9 +64,9 @@ __global__ void k_publish(const DevCounters *c, DevCounters *host) {
 
 // The pinned buffers, with the events recorded beside them.  Allocating one takes the better part
 // of a millisecond, so they outlive a context: idle ones wait here, at most kStageIdle of at most
-// kStageMax bytes each, and all are freed when the last context or batch of the process goes.  A
-// buffer belongs to one call at a time, so any number of threads and streams may fetch at once.
-// Its lists have fixed room: the calls are C entries, from which nothing may be thrown.
+// kStageMax bytes each, and all are freed when the last context, batch or network of the process
+// goes.  A buffer belongs to one call at a time, so any number of threads and streams may fetch at
+// once.  Its lists have fixed room: the calls are C entries, from which nothing may be thrown.
 struct Piece {
   char *dst;
   size_t at, bytes;
