@@ -16,6 +16,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <new>
 #include <random>
 #include <string>
@@ -797,12 +798,13 @@ struct nb_mlp {
   int64_t adam_t = 0;
   int64_t splitbuf_len = 0;
   // transposed BF16 weights for the fused inference kernel, rebuilt when wver moves
-  std::vector<uint16_t *> WbT;
+  uint16_t *WbT[9] = {};
   int64_t wver = 0, wt_ver = -1;
-  // buffers of the two-launch training step: per linear layer the transposed input and gradient, and
-  // the FP32 gradient
-  std::vector<uint16_t *> inT, dT;
-  std::vector<float *> dF;
+  // buffers of the two-launch training step, in one allocation: per linear layer the transposed
+  // input and gradient, and the FP32 gradient
+  char *train_mem = nullptr;
+  uint16_t *inT[4] = {}, *dT[4] = {};
+  float *dF[4] = {};
   int64_t train_rows = 0;
   int infer_wgs = 0;  // resident workgroups of the persistent inference kernel (0: not yet known)
 };
@@ -998,12 +1000,9 @@ bool fused_shape(const nb_mlp *m) {
 // The transposed BF16 weights, made again if the weights have moved.
 int transposed_weights(nb_mlp *m, hipStream_t st) {
   if (m->wt_ver == m->wver) return NB_OK;
-  if (m->WbT.empty())
-    for (int l = 0; l <= m->layers; l++) {
-      uint16_t *q = nullptr;
-      NB_MHIP(m, hipMalloc((void **)&q, (size_t)m->in_dim[l] * m->out_dim[l] * 2));
-      m->WbT.push_back(q);
-    }
+  for (int l = 0; l <= m->layers; l++)
+    if (!m->WbT[l])
+      NB_MHIP(m, hipMalloc((void **)&m->WbT[l], (size_t)m->in_dim[l] * m->out_dim[l] * 2));
   for (int l = 0; l <= m->layers; l++) {
     const int K = m->in_dim[l], N = m->out_dim[l];
     hipLaunchKernelGGL(k_transpose_bf16, dim3(nblk((int64_t)K * N)), dim3(256), 0, st,
@@ -1015,35 +1014,43 @@ int transposed_weights(nb_mlp *m, hipStream_t st) {
 }
 
 void free_train(nb_mlp *m) {
-  for (uint16_t *q : m->inT) (void)hipFree(q);
-  for (uint16_t *q : m->dT) (void)hipFree(q);
-  for (float *q : m->dF) (void)hipFree(q);
-  m->inT.clear();
-  m->dT.clear();
-  m->dF.clear();
+  if (m->train_mem) (void)hipFree(m->train_mem);
+  m->train_mem = nullptr;
   m->train_rows = 0;
 }
 
+// The buffers for so many rows; false if the device has no room for them.
+bool ensure_train(nb_mlp *m, int64_t rows) {
+  if (rows <= m->train_rows) return true;
+  free_train(m);
+  size_t at[3][4], end = 0;
+  for (int l = 0; l <= m->layers; l++) {
+    const size_t cols = l == m->layers ? 16 : (size_t)m->hid;
+    const size_t bytes[3] = {(size_t)rows * m->in_dim[l] * 2, rows * cols * 2, rows * cols * 4};
+    for (int q = 0; q < 3; q++) {
+      at[q][l] = end;
+      end += (bytes[q] + 255) / 256 * 256;
+    }
+  }
+  if (hipMalloc((void **)&m->train_mem, end) != hipSuccess) {
+    (void)hipGetLastError();  // or the next launch would report it
+    m->train_mem = nullptr;
+    return false;
+  }
+  for (int l = 0; l <= m->layers; l++) {
+    m->inT[l] = reinterpret_cast<uint16_t *>(m->train_mem + at[0][l]);
+    m->dT[l] = reinterpret_cast<uint16_t *>(m->train_mem + at[1][l]);
+    m->dF[l] = reinterpret_cast<float *>(m->train_mem + at[2][l]);
+  }
+  m->train_rows = rows;
+  return true;
+}
+
 // A training step in two launches, on rows (a multiple of 64) of x and t on the device; per-row
-// losses to lrow.
+// losses to lrow.  The buffers are there.
 int train_step_fused(nb_mlp *m, const float *x, const float *t, int64_t rows, float lr,
                      float *lrow, hipStream_t st) {
   const int L = m->layers;
-  if (rows > m->train_rows) {
-    free_train(m);
-    for (int l = 0; l <= L; l++) {
-      uint16_t *a = nullptr, *d = nullptr;
-      float *f = nullptr;
-      const int cols = l == L ? 16 : m->hid;
-      NB_MHIP(m, hipMalloc((void **)&a, (size_t)rows * m->in_dim[l] * 2));
-      m->inT.push_back(a);
-      NB_MHIP(m, hipMalloc((void **)&d, (size_t)rows * cols * 2));
-      m->dT.push_back(d);
-      NB_MHIP(m, hipMalloc((void **)&f, (size_t)rows * cols * 4));
-      m->dF.push_back(f);
-    }
-    m->train_rows = rows;
-  }
   int rc = transposed_weights(m, st);
   if (rc) return rc;
   TrainArgs a{};
@@ -1133,7 +1140,9 @@ int mlp_train_step_device(nb_mlp *m, const float *x_dev, const float *t_dev, int
                           float lr, float *lrow, hipStream_t st) {
   if (rows > 0 && rows % 64 == 0 && m->layers <= 3 && fused_shape(m)) {
     int rc = ensure_rows(m, rows);  // (the per-row losses)
-    return rc ? rc : train_step_fused(m, x_dev, t_dev, rows, lr, lrow ? lrow : m->lrow, st);
+    if (rc) return rc;
+    if (ensure_train(m, rows))
+      return train_step_fused(m, x_dev, t_dev, rows, lr, lrow ? lrow : m->lrow, st);
   }
   hipStream_t keep = m->stream;
   m->stream = st;
@@ -1254,6 +1263,8 @@ int nb_mlp_create(int32_t device, int32_t din, int32_t hidden, int32_t layers, i
   m->layers = layers;
   m->dout = dout;
   m->doutp = 64;
+  m->Z.reserve((size_t)layers);  // (so that later calls allocate nothing of their own)
+  m->Hb.reserve((size_t)layers);
   {
     hipError_t e = hipSetDevice(device);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking);
@@ -1334,7 +1345,8 @@ void nb_mlp_destroy(nb_mlp *m) {
   for (auto *v : {&m->W, &m->Wg, &m->Wm1, &m->Wm2, &m->bvec, &m->bg, &m->bm1, &m->bm2})
     for (float *q : *v) (void)hipFree(q);
   for (uint16_t *q : m->Wb) (void)hipFree(q);
-  for (uint16_t *q : m->WbT) (void)hipFree(q);
+  for (uint16_t *q : m->WbT)
+    if (q) (void)hipFree(q);
   if (m->splitbuf) (void)hipFree(m->splitbuf);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
@@ -1496,28 +1508,36 @@ int nb_mlp_train(nb_mlp *m, const float *x, const float *t, int64_t rows, int32_
   if (!m || !x || !t || rows < batch || batch <= 0 || batch % 64 || steps < 0)
     return NB_E_INVALID;
   NB_MHIP(m, hipSetDevice(m->device));
-  float *dx = nullptr, *dt = nullptr;
-  NB_MHIP(m, hipMalloc((void **)&dx, (size_t)rows * m->din * 4));
-  if (hipMalloc((void **)&dt, (size_t)rows * m->dout * 4) != hipSuccess) {
-    (void)hipFree(dx);
+  // the losses of the last tenth of the steps are kept on the device and read in one copy at the end
+  // (whenever 64 MiB of them are there; step by step if there is no room for more)
+  const int last = std::max(1, steps / 10);
+  int loss_steps = std::min(last, std::max(1, (16 << 20) / batch));
+  const size_t nx = (size_t)rows * m->din, nt = (size_t)rows * m->dout;
+  std::unique_ptr<float[]> l(new (std::nothrow) float[(size_t)loss_steps * batch]);
+  if (!l && loss_steps > 1) l.reset(new (std::nothrow) float[batch]), loss_steps = 1;
+  if (!l) {
+    m->err = "nb_mlp_train: host allocation failed";
     return NB_E_NOMEM;
   }
+  float *dx = nullptr;
+  auto alloc = [&]() {
+    return hipMalloc((void **)&dx, (nx + nt + (size_t)loss_steps * batch) * 4);
+  };
+  hipError_t e = alloc();
+  if (e != hipSuccess && loss_steps > 1) {
+    (void)hipGetLastError();  // or the next launch would report it
+    loss_steps = 1;
+    e = alloc();
+  }
+  NB_MHIP(m, e);
+  float *dt = dx + nx, *dl = dt + nt;
   int rc = NB_OK;
-  if (hipMemcpy(dx, x, (size_t)rows * m->din * 4, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(dt, t, (size_t)rows * m->dout * 4, hipMemcpyHostToDevice) != hipSuccess)
+  if (hipMemcpy(dx, x, nx * 4, hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(dt, t, nt * 4, hipMemcpyHostToDevice) != hipSuccess)
     rc = NB_E_HIP;
-  // the losses of the last tenth of the steps, kept on the device and read in one copy at the end
-  // (whenever 64 MiB of them are there)
-  const int loss_steps = std::max(1, (16 << 20) / batch);
   double lsum = 0;
   int lcount = 0, held = 0;
   const int64_t nb = rows / batch;
-  const int last = std::max(1, steps / 10);
-  float *dl = nullptr;
-  std::vector<float> l;
-  if (!rc && steps > 0 &&
-      hipMalloc((void **)&dl, (size_t)std::min(last, loss_steps) * batch * 4) != hipSuccess)
-    rc = NB_E_NOMEM;
   for (int s = 0; s < steps && !rc; s++) {
     const int64_t b0 = (s % nb) * batch;
     const bool count = s >= steps - last;
@@ -1525,9 +1545,8 @@ int nb_mlp_train(nb_mlp *m, const float *x, const float *t, int64_t rows, int32_
                                    count ? dl + (size_t)held * batch : nullptr, m->stream);
     if (rc || !count) continue;
     if (++held == loss_steps || s + 1 == steps) {
-      l.resize((size_t)held * batch);
-      if (hipMemcpyAsync(l.data(), dl, l.size() * 4, hipMemcpyDeviceToHost, m->stream) !=
-              hipSuccess ||
+      if (hipMemcpyAsync(l.get(), dl, (size_t)held * batch * 4, hipMemcpyDeviceToHost,
+                         m->stream) != hipSuccess ||
           hipStreamSynchronize(m->stream) != hipSuccess) {
         rc = NB_E_HIP;
         break;
@@ -1543,8 +1562,6 @@ int nb_mlp_train(nb_mlp *m, const float *x, const float *t, int64_t rows, int32_
   }
   (void)hipStreamSynchronize(m->stream);
   (void)hipFree(dx);
-  (void)hipFree(dt);
-  if (dl) (void)hipFree(dl);
   if (loss_out) *loss_out = lcount ? (float)(lsum / lcount) : 0.f;
   return rc;
 }

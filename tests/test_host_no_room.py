@@ -98,3 +98,33 @@ g.close()
 print("done")
 """)
     assert rc == 0 and "done" in out, (rc, out)
+
+
+def test_training_without_room_for_the_two_launch_step():
+    """Layer by layer, the losses read step by step: as much memory as before there were its buffers."""
+    rc, out = host_only.run("""
+    from nbodygo_amd.mlp import MLP
+    B, steps = 1 << 20, 40
+    x, t = np.zeros((B, 30), np.float32), np.zeros((B, 3), np.float32)
+    m = MLP(30, hidden=128, layers=3, d_out=3, seed=1)
+    m.grad(x, t)                                  # (the layer-by-layer buffers)
+    m.train(x, t, steps, batch=B)
+    assert sum("k_train_rows" in k for k in launched()) == steps
+    m.close()
+    for room in (0, 4 << 20):
+        m = MLP(30, hidden=128, layers=3, d_out=3, seed=1)
+        m.grad(x, t)
+        fake.fake_clear()
+        fake.fake_budget(B * 34 * 4 + room)       # rows, targets and one step's losses
+        m.train(x, t, steps, batch=B)
+        assert not any("k_train_rows" in k for k in launched())
+        assert sum("k_adam" in k for k in launched()) == 8 * steps
+        fake.fake_budget((1 << 64) - 1)
+        fake.fake_clear()
+        m.train(x, t, 3, batch=B)
+        assert sum("k_train_rows" in k for k in launched()) == 3
+        m.close()
+    assert fake.fake_in_use() == 0
+    print("done")
+    """)
+    assert rc == 0 and "done" in out, (rc, out)

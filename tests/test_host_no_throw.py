@@ -76,3 +76,24 @@ def test_batch_load_without_host_memory():
     print("done")
     """)
     assert rc == 0 and "done" in out, (rc, out)
+
+
+def test_training_without_host_memory():
+    rc, out = host_only.run("""
+    from nbodygo_amd.mlp import MLP
+    x, t = np.zeros((256, 30), np.float32), np.zeros((256, 3), np.float32)
+    m = MLP(30, hidden=64, layers=2, d_out=3, seed=1)
+    for k in range(20):
+        fake.fake_fail_new(k)
+        try:
+            m.train(x, t, 50, batch=64)
+        except L.NBodyError as e:
+            assert e.code == L.NB_E_NOMEM, e
+        if fake.fake_new_left() >= 0:
+            break
+        if k == 0:
+            m.close()
+            m = MLP(30, hidden=64, layers=2, d_out=3, seed=1)
+    print("done", k)
+    """)
+    assert rc == 0 and "done" in out, (rc, out)
