@@ -515,6 +515,7 @@ int nb_load(nb_ctx *c, int64_t n, const double *x, const double *y, const double
     return fail(c, NB_E_INVALID, "nb_load: NULL array");
   NB_HIP(c, hipSetDevice(c->device));
   c->ctr_last_ok = false;
+  c->pairs_seen = kPairsUnknown;
   const int64_t npad = std::max<int64_t>(round_up(n, kPad), kPad);
   if (npad > c->cap) {
     free_all(c);
@@ -619,7 +620,15 @@ int nb_step(nb_ctx *c, double dt, double R, int32_t nsteps, nb_stats *out) {
     int rc = events_ensure_queue(c);
     if (rc) return rc;
   }
+  int look = c->pairs_seen == kPairsUnknown ? 1 : kPairLook;
   for (int s = 0; s < nsteps && c->n > 0; s++) {
+    // the pair list's launches follow the pairs there are, also within a call of many cycles
+    if (s == look && c->p.collisions && c->n <= kPairSmallN) {
+      DevCounters h;
+      NB_HIP(c, stage_counters(c->ctr, c->stream, &h));
+      c->pairs_seen = h.pair_count;
+      look = s + kPairLook;
+    }
     if (c->p.events) {  // fragment() of the fragmenting bodies, in Compute (body.go:152-154)
       int rc = events_emit(c);
       if (rc) return rc;

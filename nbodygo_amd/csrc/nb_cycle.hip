@@ -497,8 +497,8 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
 // successors.  One workgroup resolves the ready pairs round by round.
 //
 // Up to kPairSmallN bodies one workgroup does all of it in one launch, the counts in LDS; above, or
-// when the last cycle had more than kPairSmallPairs pairs, the list takes five launches, the chains
-// and the rounds one each (one workgroup / seven launches, reference scene: 0.020 / 0.033 ms with 63
+// when the last count read is more than kPairSmallPairs (or a scene's first is still to come), the
+// list takes five launches, the chains and the rounds one each (one workgroup / seven launches, reference scene: 0.020 / 0.033 ms with 63
 // pairs, 0.045 / 0.057 with 1,074, 0.072 / 0.074 with 2,439, 0.184 / 0.114 with 6,998).
 // A sort of the keys, one of the swapped keys and binary searches took 11 to 23 launches.
 //
@@ -508,7 +508,6 @@ __global__ __launch_bounds__(64) void k_resolve(ResolveArgs a) {
 // rounds), 0.63 -> 0.11 at 10,007 (6,998 pairs, 16 rounds), 1.30 -> 0.24 at 16,384 (18,696 pairs,
 // 40 rounds).
 // ---------------------------------------------------------------------------------------------
-constexpr int kPairSmallN = 16384;        // bodies whose two count arrays fit one workgroup's LDS
 constexpr int kPairThreads = 512;         // coll3d keeps its 140 VGPRs (1,024 threads would spill)
 constexpr int kPairLdsPend = 128 * 1024;  // pairs whose predecessor counts fit in LDS, one byte each
 

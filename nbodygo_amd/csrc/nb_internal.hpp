@@ -16,6 +16,7 @@ constexpr int kPad = 1024;           // body arrays are padded to a multiple of 
 constexpr int kFlagSlots = 4;        // flagged tiles remembered per (slice, target)
 constexpr int kMaxSplit = 64;        // max source-range slices
 constexpr int64_t kLayerWords = (int64_t)1 << 28;  // floats of variant 3's workspace (1 GiB)
+constexpr int64_t kPairsUnknown = INT64_MAX;  // no pair count read of a scene just loaded: many
 constexpr float kSentinel = 1.0e18f; // position of padding / inactive sources in the FP32 stream
 
 // Device counters, one struct per context (zeroed by a fill kernel, never by hipMemset, so the
@@ -188,7 +189,7 @@ struct Ctx {
   int32_t *pair_words = nullptr, *pair_body = nullptr;
   double *pair_geom = nullptr;
   int64_t pair_body_cap = 0;
-  int64_t pairs_seen = 0;  // pairs of the last cycle read back (chooses the list's launches)
+  int64_t pairs_seen = kPairsUnknown;  // pairs of the last cycle read back (chooses the list's launches)
   int64_t pair_cap = 0;
   int64_t pair_cap_pow2 = 0;
 
@@ -437,7 +438,12 @@ struct PairArgs {
   double *geom;  // 6 words for the first geom_cap pairs
   int64_t geom_cap;
 };
+constexpr int kPairSmallN = 16384;         // bodies whose two count arrays fit one workgroup's LDS
 constexpr int64_t kPairSmallPairs = 2500;  // pairs up to which one workgroup does the whole pass
+// Cycles of one call after which the host waits for the pair count (10 us) and chooses again: one
+// workgroup takes any number of pairs, but many times as long as the whole chip (a list costs the
+// square of its length).
+constexpr int kPairLook = 32;
 constexpr int64_t kPairGeom = 1 << 18;     // pairs whose positions' half of coll3d is kept
 // r: resolve too.  expect: about how many pairs there are (chooses the launches, not the result).
 hipError_t launch_pairs(const PairArgs &a, const ResolveArgs *r, int64_t expect, hipStream_t st);
