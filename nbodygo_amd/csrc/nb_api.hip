@@ -230,6 +230,7 @@ static void choose_shape(Ctx *c) {
 
 // Pair buffers for n bodies (collisions on), grown in powers of two.
 constexpr int kPairWords = 11;  // int32 words per pair of PairArgs' per-pair arrays
+static int64_t pair_longs(int64_t pairs) { return 2 * (pairs / kPairLong); }  // own and reach lists
 static int size_pairs(Ctx *c, int64_t n) {
   const int64_t pcap =
       c->p.pair_capacity > 0 ? c->p.pair_capacity : std::max<int64_t>(4 * n, 65536);
@@ -241,7 +242,7 @@ static int size_pairs(Ctx *c, int64_t n) {
     c->pair_cap_pow2 = 0;
     NB_HIP(c, dalloc(&c->pairs, (size_t)pow2));
     NB_HIP(c, dalloc(&c->pairs_sorted, (size_t)pow2));
-    NB_HIP(c, dalloc(&c->pair_words, (size_t)pow2 * kPairWords));
+    NB_HIP(c, dalloc(&c->pair_words, (size_t)pow2 * kPairWords + pair_longs(pow2) + 2));
     NB_HIP(c, dalloc(&c->pair_geom, (size_t)std::min(pow2, kPairGeom) * 6));
     c->pair_cap_pow2 = pow2;
   }
@@ -279,6 +280,8 @@ static PairArgs make_pair_args(Ctx *c) {
   a.by_hi = w + 4 * pair;
   a.place = w + 5 * pair;
   a.pend = w + 6 * pair;
+  a.nlong = reinterpret_cast<uint32_t *>(w + 7 * pair);
+  a.longs = a.nlong + 2;
   a.geom = c->pair_geom;
   a.geom_cap = std::min(pair, kPairGeom);
   return a;

@@ -437,9 +437,12 @@ struct PairArgs {
   int2 *succ, *role;
   double *geom;  // 6 words for the first geom_cap pairs
   int64_t geom_cap;
+  // lists of more than kPairLong pairs: their number (one word), and body * 2 + (0 own, 1 reach)
+  uint32_t *nlong, *longs;
 };
 constexpr int kPairSmallN = 16384;         // bodies whose two count arrays fit one workgroup's LDS
 constexpr int64_t kPairSmallPairs = 2500;  // pairs up to which one workgroup does the whole pass
+constexpr int kPairLong = 512;             // pairs above which a list is put in order beforehand
 // Cycles of one call after which the host waits for the pair count (10 us) and chooses again: one
 // workgroup takes any number of pairs, but many times as long as the whole chip (a list costs the
 // square of its length).
