@@ -1155,12 +1155,12 @@ int mlp_train_step_device(nb_mlp *m, const float *x_dev, const float *t_dev, int
         hipSuccess)
       rc = NB_E_HIP;
   }
+  float *keep_lrow = m->lrow;
+  if (!rc && lrow) m->lrow = lrow;
   if (!rc) rc = forward(m, rows);
   if (!rc) rc = backward(m, rows);
   if (!rc) rc = adam_step(m, lr);
-  if (!rc && lrow &&
-      hipMemcpyAsync(lrow, m->lrow, (size_t)rows * 4, hipMemcpyDeviceToDevice, st) != hipSuccess)
-    rc = NB_E_HIP;
+  m->lrow = keep_lrow;
   m->stream = keep;
   return rc;
 }

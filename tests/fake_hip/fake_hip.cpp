@@ -21,7 +21,7 @@ static std::map<const void *, std::string> &names() {
 }
 static std::string launched;  // names of the kernels launched, one a line
 static size_t budget = SIZE_MAX, in_use = 0;
-static long host_mallocs = 0, dev_mallocs = 0;
+static long host_mallocs = 0, dev_mallocs = 0, dev_copies = 0;
 static long publish_pairs = -1;
 static std::atomic<long> new_countdown{-1};
 
@@ -36,6 +36,7 @@ void fake_budget(size_t bytes) { budget = bytes; }       // device memory left t
 size_t fake_in_use() { return in_use; }
 long fake_host_mallocs() { return host_mallocs; }
 long fake_dev_mallocs() { return dev_mallocs; }
+long fake_dev_copies() { return dev_copies; }  // copies from device to device asked of the runtime
 // the library's n-th operator new from now (0: the next one) fails, once; -1: none
 void fake_fail_new(long n) { new_countdown = n; }
 long fake_new_left() { return new_countdown; }
@@ -134,7 +135,8 @@ hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
   memcpy(d, s, n);
   return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) {
+  if (k == hipMemcpyDeviceToDevice) dev_copies++;
   memcpy(d, s, n);
   return hipSuccess;
 }

@@ -16,7 +16,7 @@ import ctypes as C, sys
 fake = C.CDLL({fake!r}, C.RTLD_GLOBAL)
 fake.fake_budget.argtypes = [C.c_size_t]
 fake.fake_in_use.restype = C.c_size_t
-for f in ("fake_host_mallocs", "fake_dev_mallocs", "fake_new_left"):
+for f in ("fake_host_mallocs", "fake_dev_mallocs", "fake_dev_copies", "fake_new_left"):
     getattr(fake, f).restype = C.c_long
 fake.fake_fail_new.argtypes = fake.fake_pairs.argtypes = [C.c_long]
 fake.fake_launched.restype = C.c_char_p

@@ -1,4 +1,4 @@
-"""Pinned memory of the read-backs: allocated once while anything of the library is alive."""
+"""Copies and pinned memory of the read-backs: what a call asks of the runtime."""
 import host_only
 
 
@@ -15,6 +15,20 @@ def test_a_network_alone_keeps_its_staging():
     assert fake.fake_host_mallocs() - before <= 1, fake.fake_host_mallocs()
     m.close()
     assert fake.fake_in_use() == 0
+    print("done")
+    """)
+    assert rc == 0 and "done" in out, (rc, out)
+
+
+def test_losses_of_a_layer_by_layer_step_are_written_where_they_are_kept():
+    rc, out = host_only.run("""
+    from nbodygo_amd.mlp import MLP
+    x, t = np.zeros((256, 30), np.float32), np.zeros((256, 3), np.float32)
+    m = MLP(30, hidden=128, layers=5, d_out=3, seed=1)
+    for steps in (1, 10, 40):
+        before = fake.fake_dev_copies()
+        m.train(x, t, steps, batch=64)
+        assert fake.fake_dev_copies() - before == steps   # the targets', once a step
     print("done")
     """)
     assert rc == 0 and "done" in out, (rc, out)
