@@ -5,7 +5,7 @@ Exists/fragmenting/IsSun/Pinned, Body.r and FragFactor; cmd/body/body.go:34-52).
 one nb_ctx and exposes the entry points of include/nbody_gpu.h with numpy arrays.
 """
 import ctypes as C
-from concurrent.futures import ThreadPoolExecutor
+import threading
 from dataclasses import dataclass, field
 
 import numpy as np
@@ -388,15 +388,24 @@ class NBodyBatch:
         kept = (a.m, a.r, a.beh, a.rest, a.frag, a.fstep)
         # what the device does not change is copied beside the read-back once that takes longer
         # than the threads' start (both leave the interpreter lock): 12.7 -> 5 ms for 2.2 million
-        # bodies
-        pool = ThreadPoolExecutor(4) if n > 200000 else None
-        if pool:
-            copies = [pool.submit(np.copy, v) for v in kept]
+        # bodies.  What no thread could be had for (the interpreter is ending) is copied here.
+        copies, threads = [None] * len(kept), []
+
+        def copy(k):
+            copies[k] = kept[k].copy()
+
+        try:
+            for k in range(len(kept) if n > 200000 else 0):
+                t = threading.Thread(target=copy, args=(k,))
+                t.start()
+                threads.append(t)
+        except RuntimeError:
+            pass
         rc = lib.nb_batch_store(self._b, *(_dp(v) for v in f), flags.ctypes.data_as(L._u8p))
-        m, r, beh, rest, frag, fstep = ([c.result() for c in copies] if pool
-                                        else [v.copy() for v in kept])
-        if pool:
-            pool.shutdown()
+        for t in threads:
+            t.join()
+        m, r, beh, rest, frag, fstep = (c if c is not None else v.copy()
+                                        for c, v in zip(copies, kept))
         self._check(rc)
         return Bodies(*f, m, r, beh, flags, rest, frag, fstep)
 
