@@ -624,6 +624,10 @@ int nb_step(nb_ctx *c, double dt, double R, int32_t nsteps, nb_stats *out) {
     if (rc) return rc;
   }
   int look = c->pairs_seen == kPairsUnknown ? 1 : kPairLook;
+  // a small scene's first cycle is taken for one of few pairs: the launches for many cost it 13 us,
+  // and its lists are short enough for one workgroup whatever they hold
+  if (c->pairs_seen == kPairsUnknown && c->n <= kPairFreshN && c->pair_cap <= kPairFreshCap)
+    c->pairs_seen = 0;
   for (int s = 0; s < nsteps && c->n > 0; s++) {
     // the pair list's launches follow the pairs there are, also within a call of many cycles
     if (s == look && c->p.collisions && c->n <= kPairSmallN) {

@@ -443,6 +443,10 @@ struct PairArgs {
 constexpr int kPairSmallN = 16384;         // bodies whose two count arrays fit one workgroup's LDS
 constexpr int64_t kPairSmallPairs = 2500;  // pairs up to which one workgroup does the whole pass
 constexpr int kPairLong = 512;             // pairs above which a list is put in order beforehand
+// Bodies and room for pairs up to which one workgroup takes the first cycle of a scene, whose count is
+// still to come: the launches for many would cost every small scene 13 us, and here one cycle 12 ms
+// more at worst (15 bodies that overlap all of 4,096: 33 ms for 21, once).
+constexpr int64_t kPairFreshN = 4096, kPairFreshCap = 65536;
 // Cycles of one call after which the host waits for the pair count (10 us) and chooses again: one
 // workgroup takes any number of pairs, but many times as long as the whole chip (a list costs the
 // square of its length).

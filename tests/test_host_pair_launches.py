@@ -21,18 +21,19 @@ g.load(b)
 """
 
 
-@pytest.mark.parametrize("n", [300, 16384])
-def test_many_cycles_after_a_load(n):
-    rc, out = host_only.run(SETUP % n + """
+@pytest.mark.parametrize("n,first", [(300, "small"), (4096, "small"), (4097, "wide"),
+                                     (16384, "wide")])
+def test_many_cycles_after_a_load(n, first):
+    rc, out = host_only.run(SETUP % n + "first = %r" % first + """
 fake.fake_pairs(60000)
 fake.fake_clear()
 g.step(1e-3, 1.0, nsteps=40)
-assert per_cycle() == ["wide"] * 40, per_cycle()
+assert per_cycle() == [first] + ["wide"] * 39, per_cycle()
 fake.fake_pairs(100)                    # few: from the second cycle of the load's first call on
 g.load(b)
 fake.fake_clear()
 g.step(1e-3, 1.0, nsteps=5)
-assert per_cycle() == ["wide"] + ["small"] * 4, per_cycle()
+assert per_cycle() == [first] + ["small"] * 4, per_cycle()
 fake.fake_clear()
 g.step(1e-3, 1.0, nsteps=3)
 assert per_cycle() == ["small"] * 3, per_cycle()
@@ -40,6 +41,18 @@ fake.fake_pairs(5000)                   # the scene contracts during a call
 fake.fake_clear()
 g.step(1e-3, 1.0, nsteps=70)
 assert per_cycle() == ["small"] * 32 + ["wide"] * 38, per_cycle()
+print("done")
+""")
+    assert rc == 0 and "done" in out, (rc, out)
+
+
+def test_room_for_many_pairs_in_a_small_scene():
+    rc, out = host_only.run(SETUP % 1000 + """
+g = NBodyGPU(collisions=True, pair_capacity=500000)
+g.load(b)
+fake.fake_clear()
+g.step(1e-3, 1.0)
+assert per_cycle() == ["wide"], per_cycle()
 print("done")
 """)
     assert rc == 0 and "done" in out, (rc, out)
