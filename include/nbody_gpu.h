@@ -52,8 +52,9 @@ extern "C" {
 #define NB_CB_FRAGMENT 3
 
 /* ---- precision modes ---------------------------------------------------------------------- */
-#define NB_PREC_FP32 0 /* FP32 pairwise force with per-tile Kahan summation, FP64 exact
-                          overlap/collision tests, FP64 integration (production path) */
+#define NB_PREC_FP32 0 /* FP32 pairwise force, FP64 exact overlap/collision tests, FP64 integration
+                          (production path).  Each pair once (variant 3): FP32 sums over up to 1,024
+                          bodies at a time, added in FP64; one-sided: Kahan sums over tiles */
 #define NB_PREC_FP64 1 /* FP64 force in the reference's operation order (bit-identical to the
                           reference's arithmetic for the force and update) */
 
@@ -68,8 +69,8 @@ typedef struct nb_params {
   int32_t device;         /* HIP device ordinal */
   int64_t pair_capacity;  /* max collision pairs per step; 0 = default (max(4N, 65536)) */
   int32_t ipl;            /* FP32 force kernel: target bodies per lane (1,2,4); 0 = tuned */
-  int32_t tile_j;         /* FP32 force kernel: j bodies per Kahan tile (multiple of 64);
-                             0 = tuned */
+  int32_t tile_j;         /* FP32 force kernel: j bodies per tile (multiple of 64; variants 1 and 2
+                             add tiles by Kahan's method); 0 = tuned */
   int32_t jsplit;         /* FP32 force kernel: source-range slices; 0 = tuned */
   int32_t block;          /* FP32 force kernel: threads per workgroup (64..256); 0 = tuned */
   int32_t variant;        /* FP32 force kernel: 0 = tuned, 1 = scalar-cache j stream,
@@ -329,7 +330,7 @@ int nb_batch_forces(nb_batch *b, double *fx, double *fy, double *fz);
 int nb_batch_store(nb_batch *b, double *x, double *y, double *z, double *vx, double *vy,
                    double *vz, uint8_t *flags);
 
-/* Kernel shape of the batched force.  Work items are blocks of 64 x IPL targets of one
+/* Kernel shape of the batched one-sided force.  Work items are blocks of 64 x IPL targets of one
  * simulation; `waves` (1, 2 or 4) wavefronts share an item, splitting its sources; each wave
  * consumes its sources in Kahan tiles of `tile` (64, 128 or 256) sources.  IPL and tile are chosen
  * per size bucket (N < 1024, < 4096, >= 4096), waves for the whole launch.  When every bucket

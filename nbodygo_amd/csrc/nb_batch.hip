@@ -1,9 +1,9 @@
 // nb_batch.hip -- many independent simulations of uneven size in one persistent launch.
 //
 // No counterpart in the reference (it runs one BodyCollection per process); each simulation
-// follows the same per-cycle semantics as the single-context path: FP32 pairwise force with Kahan
-// tile sums (Body.Compute's force loop, body.go:156-170, :214-225, softened per octree.go:314-325)
-// and the FP64 Body.Update (body.go:114-139).  Collisions are not part of this path.
+// follows the same per-cycle semantics as the single-context path: FP32 pairwise force
+// (Body.Compute's force loop, body.go:156-170, :214-225, softened per octree.go:314-325) and the
+// FP64 Body.Update (body.go:114-139).  Collisions are not part of this path.
 //
 // Layout: the simulations' bodies are concatenated; each simulation is padded to a multiple of 64
 // with far-away massless sentinels (flags = 0), so no 64-source tile straddles two simulations.
@@ -17,8 +17,9 @@
 // nb_batch_autotune.  When every item has the same (IPL, tile) the launch uses the kernel
 // specialised to that shape, whose registers and LDS are sized for it alone.
 //
-// That is the kernel for a shape that the caller sets, and for simulations above 32,768 bodies;
-// otherwise the launch is nb_sym.hip's, which takes each unordered pair once.
+// That is the kernel for a shape that the caller sets, for simulations above 32,768 bodies, and where
+// the device has no room for the other's workspace; otherwise the launch is nb_sym.hip's, which takes
+// each unordered pair once.
 //
 // One nb_batch_step call runs nsteps cycles as one hipGraph launch: per cycle a fill kernel resets
 // the queue (no memset nodes), then the force kernel, then the update kernel.

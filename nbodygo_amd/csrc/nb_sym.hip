@@ -20,16 +20,24 @@
 // LDS; a tile body keeps plain FP32 sums over its 64 IPL partners per wave, the W waves are added
 // in wave order, and the block's contribution is one FP32 triple per (block distance, body).
 // k_sym_fold adds the target slices and the distances in FP64, in fixed order, so results do not
-// depend on scheduling.  Against FP64 the error is the one-sided kernel's or less: 6.6e-8 (was
-// 6.9e-8) global at N = 262,144, 1.26e-7 (was 1.33e-7) at 65,536, 3.8e-7 (was 4.4e-7) at 4,096.
+// depend on scheduling.  The tile bodies' sums are the ones in fewest bits: FP32 without compensation
+// over up to 1,024 partners (64 steps of 4 in a chain, then 4 waves), as the one-sided kernel's are
+// over the 512 of its tile.  Against FP64 the error is the one-sided kernel's or less, global / 99 of
+// 100 bodies: 6.7e-8 / 2.1e-7 (one-sided 7.0e-8 / 2.2e-7) for a Plummer sphere of 262,144, 1.5e-7 /
+// 4.7e-7 (1.5e-7 / 4.7e-7) of 65,536, 3.3e-7 / 9.6e-7 (3.6e-7 / 9.9e-7) of 4,096; and with masses far
+// apart, where those sums matter most, at 65,536: lognormal with sigma 3 6.1e-7 / 8.4e-7 (7.4e-7 /
+// 1.4e-6), one body with all of the mass 1.9e-7 / 3.1e-7 (the same), every seventh 64 bodies 1e5 times
+// the others 3.8e-7 / 9.4e-7 (4.9e-7 / 1.9e-6).
 //
 // What bounds it: FP32 VALU issue.  gfx950 issues two independent FP32 instructions at a time, and
 // the compiler's own order of a step (chains one target after another) leaves every second slot
 // empty: 4,700 G interactions/s at N = 262,144.  With the step written as rows of independent
-// instructions and the rows kept apart by scheduling barriers it is 5,600, against a ceiling of
-// 5,680 from the measured issue rates of the instructions alone.  The one-sided kernel does 3,660
-// there.  Per force phase: 18.6 -> 12.3 ms at N = 262,144, 1.17 -> 0.83 at 65,536, 0.297 -> 0.240
-// at 32,768; with detection 1.26 -> 0.87 at 65,536 and 0.084 -> 0.050 at 10,000.
+// instructions and the rows kept apart by scheduling barriers it is 5,560 to 5,650, against a ceiling
+// of 5,790 from the measured issue rates of the instructions alone (at 2.4 GHz; the card holds 2.34).
+// The one-sided kernel does 3,600 to 3,660 there.  Per force phase in a long run: 19.1 -> 12.2 to 12.4
+// ms at N = 262,144, 1.18 -> 0.83 at 65,536, 0.30 -> 0.25 at 32,768; with detection 20.2 -> 12.8, 1.29
+// -> 0.86 and 0.37 -> 0.26, 0.084 -> 0.050 at 10,000.  The first launches after an idle card are
+// slower: 14.5, 12.8, 12.25 ms at 262,144, 0.95 to 1.0 for some thirty at 65,536.
 //
 // Detection: as nb_force.hip's bound on the tile's smallest r^2, evaluated from the target's side
 // only (r^2 is symmetric); a flagged (target, tile) is re-tested at once in FP64 by the whole wave,
