@@ -517,10 +517,12 @@ __device__ __forceinline__ int64_t pair_total(const PairArgs &a) {
   return min((int64_t)a.ctr->pair_count, a.cap);
 }
 
-// The next place in body i's list.  The lanes that share the first one's body take theirs with one
-// atomic (2 million pairs among 2,000 bodies: 0.63 ms with one each).
-template <class P>
+// The next place in body i's list.  In memory, the lanes that share the first one's body take theirs
+// with one atomic (2 million pairs among 2,000 bodies: 0.63 ms with one each, 0.32 so); in LDS, where
+// the pairs are few, that costs more than it saves.
+template <bool LDS, class P>
 __device__ __forceinline__ int next_place(P counts, int i) {
+  if (LDS) return atomicAdd(&counts[i], 1);
   const bool same = i == __builtin_amdgcn_readfirstlane(i);
   const uint64_t peers = __builtin_amdgcn_ballot_w64(same);
   const int rank = (int)__builtin_amdgcn_mbcnt_hi(
@@ -532,13 +534,13 @@ __device__ __forceinline__ int next_place(P counts, int i) {
 }
 
 // A pair's place in its two bodies' lists, in arrival order.
-template <class P>
+template <bool LDS, class P>
 __device__ __forceinline__ void pair_count(const PairArgs &a, int64_t cnt, P own, P reach,
                                            int64_t k0, int64_t step) {
   for (int64_t k = k0; k < cnt; k += step) {
     const uint64_t key = a.raw[k];
-    a.slot_own[k] = next_place(own, (int)(key >> 32));
-    a.slot_reach[k] = next_place(reach, (int)(key & 0xffffffffu));
+    a.slot_own[k] = next_place<LDS>(own, (int)(key >> 32));
+    a.slot_reach[k] = next_place<LDS>(reach, (int)(key & 0xffffffffu));
   }
 }
 
@@ -740,7 +742,7 @@ __global__ __launch_bounds__(kPairThreads) void k_pairs_small(PairArgs a, Resolv
   }
   for (int i = tid; i <= a.n; i += nt) own[i] = reach[i] = 0;
   __syncthreads();
-  pair_count(a, cnt, own, reach, tid, nt);
+  pair_count<true>(a, cnt, own, reach, tid, nt);
   __syncthreads();
   const int per = (a.n + nt - 1) / nt, i0 = min(tid * per, a.n), i1 = min(i0 + per, a.n);
   int2 v = make_int2(0, 0), total;
@@ -768,7 +770,7 @@ __global__ __launch_bounds__(kPairThreads) void k_pairs_small(PairArgs a, Resolv
 // The same over the whole chip.  The counts are zero between uses.
 __global__ __launch_bounds__(256) void k_pair_count(PairArgs a) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *a.nlong = 0;
-  pair_count(a, pair_total(a), a.own, a.reach, (int64_t)blockIdx.x * 256 + threadIdx.x,
+  pair_count<false>(a, pair_total(a), a.own, a.reach, (int64_t)blockIdx.x * 256 + threadIdx.x,
              (int64_t)gridDim.x * 256);
 }
 
